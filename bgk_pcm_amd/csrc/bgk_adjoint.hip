@@ -839,7 +839,7 @@ bool reverse_steps(int a, int b, int sa, std::vector<int>& freev, Advance& advan
     for (int k = b; k > a; --k) {
       int st = sa;
       if (k - 1 > a) {
-        st = -1 - ((k - 1 - a - 1) & 1);  // the work slot the last step lands in
+        st = -1 - ((k - 1 - a - 1) & 1);  // a work state
         if (!advance(sa, a, k - 1, st)) return false;
       }
       if (!adjoint(k, st)) return false;
@@ -1034,9 +1034,10 @@ hipError_t launch_adjoint(bgk_handle* h, AdjCtx* x, const StatePtrs& sprev, int 
   return hipGetLastError();
 }
 
-// one forward step from state `in` to state `out` (explicit buffers)
-hipError_t fwd_step(bgk_handle* h, const StatePtrs& in, const StatePtrs& out, double* probe_out,
-                    const int* probe_idx, bool write_all, double* const* macro) {
+// T forward steps from state `in` to state `out` (explicit buffers) in one launch
+hipError_t fwd_steps(bgk_handle* h, int T, const StatePtrs& in, const StatePtrs& out,
+                     double* probe_out, const int* probe_idx, int np, bool write_all,
+                     double* const* macro) {
   mom::MomStep st;
   st.in = mom::MomIn{in.a, in.b, in.c};
   st.out = mom::MomOut{out.a, out.b, out.c};
@@ -1047,8 +1048,9 @@ hipError_t fwd_step(bgk_handle* h, const StatePtrs& in, const StatePtrs& out, do
   st.write_all = write_all;
   st.probe_idx = probe_idx;
   st.probe_out = probe_out;
+  st.probe_np = np;
   for (int m = 0; m < 4; ++m) st.macro[m] = macro ? macro[m] : nullptr;
-  return launch_mom_step(h, st);
+  return launch_mom_steps(h, st, T);
 }
 
 }  // namespace
@@ -1145,12 +1147,12 @@ hipError_t adj_forward(bgk_handle* h, double* probe_T_host) {
   // east column of the initial state (T(Nx, :) as the first BC_g reads it)
   if (e == hipSuccess) e = launch_teast_prologue(h);
   if (e != hipSuccess) return e;
-  int te = 0;  // teast[te] holds the current column
   size_t next_chain = 0;
-  for (int n = 0; n < x->nsteps; ++n) {
+  const int lvl1 = x->seg1 > 0 ? x->seg1 : x->seg;
+  for (int n = 0; n < x->nsteps;) {
     const int a = h->cur, b = 1 - h->cur;
-    StatePtrs in{h->ma[a], h->mb[a], h->mc[a], h->phi[h->pc], h->teast[te]};
-    StatePtrs out{h->ma[b], h->mb[b], h->mc[b], h->phi[1 - h->pc], h->teast[1 - te]};
+    StatePtrs in{h->ma[a], h->mb[a], h->mc[a], h->phi[h->pc], h->teast[h->te_cur]};
+    StatePtrs out{h->ma[b], h->mb[b], h->mc[b], h->phi[1 - h->pc], h->teast[1 - h->te_cur]};
     const StatePtrs* keep = nullptr;
     if (x->nsnap > 0) {
       if (n == 0) {
@@ -1159,22 +1161,29 @@ hipError_t adj_forward(bgk_handle* h, double* probe_T_host) {
         keep = &x->snap[next_chain + 1];
         ++next_chain;
       }
-    } else {
-      const int lvl1 = x->seg1 > 0 ? x->seg1 : x->seg;
-      if (n % lvl1 == 0) keep = &x->ckpt[(size_t)(n / lvl1)];
+    } else if (n % lvl1 == 0) {
+      keep = &x->ckpt[(size_t)(n / lvl1)];
     }
     if (keep) {
       e = copy_state(h, *keep, in.a, in.b, in.c, in.phi, in.te);
       if (e != hipSuccess) return e;
     }
-    e = fwd_step(h, in, out, x->probe_T + (size_t)n * x->np, x->probe_idx, n == x->nsteps - 1,
-                 nullptr);
+    // steps to the next state to keep
+    int stop = x->nsteps;
+    if (x->nsnap > 0) {
+      if (next_chain < x->chain.size()) stop = std::min(stop, x->chain[next_chain]);
+    } else {
+      stop = std::min(stop, (n / lvl1 + 1) * lvl1);
+    }
+    const int T = mom_next_steps(h, stop - n);
+    e = fwd_steps(h, T, in, out, x->np > 0 ? x->probe_T + (size_t)n * x->np : nullptr,
+                  x->probe_idx, x->np, mom_write_all(h, T, x->nsteps - n - T), nullptr);
     if (e != hipSuccess) return e;
     h->cur = b;
     h->pc = 1 - h->pc;
-    te = 1 - te;
+    h->te_cur = 1 - h->te_cur;
+    n += T;
   }
-  // the handle's teast convention: bgk_step recomputes it from T at entry
   if (x->np > 0)
     e = hipMemcpyAsync(probe_T_host, x->probe_T, (size_t)x->nsteps * x->np * sizeof(double),
                        hipMemcpyDeviceToHost, h->stream);
@@ -1211,21 +1220,34 @@ hipError_t adj_backward(bgk_handle* h, const double* seeds_host, double grad[3])
     has_next = true;
     return e == hipSuccess;
   };
-  auto step = [&](const StatePtrs& in, const StatePtrs& out) {
-    ++x->recomputed;
-    e = fwd_step(h, in, out, nullptr, nullptr, false, x->macro);
+  auto steps = [&](int T, const StatePtrs& in, const StatePtrs& out) {
+    x->recomputed += T;
+    e = fwd_steps(h, T, in, out, nullptr, nullptr, 0, false, x->macro);
     return e == hipSuccess;
+  };
+  auto step = [&](const StatePtrs& in, const StatePtrs& out) { return steps(1, in, out); };
+  // from state `src` on by n steps to state `dst`, through two scratch states,
+  // of which `dst` may be one
+  auto run = [&](const StatePtrs& src, int n, const StatePtrs& dst, const StatePtrs* scratch) {
+    int launches = 0;
+    for (int left = n; left > 0; ++launches) left -= mom_next_steps(h, left);
+    // launch m writes scratch (k + m) & 1: the one before last not `dst`
+    int k = (&dst == &scratch[0] ? 1 : 0) ^ (launches & 1);
+    const StatePtrs* in = &src;
+    for (int left = n; left > 0; k ^= 1) {
+      const int T = mom_next_steps(h, left);
+      left -= T;
+      const StatePtrs* out = left == 0 ? &dst : &scratch[k];
+      if (!steps(T, *in, *out)) return false;
+      in = out;
+    }
+    return true;
   };
   if (x->nsnap > 0) {
     // binomial schedule: slots >= 0 are snapshots, -1 and -2 the work states
     auto at = [&](int sl) -> const StatePtrs& { return sl >= 0 ? x->snap[(size_t)sl] : x->work[-1 - sl]; };
     auto advance = [&](int src, int from, int to, int dst) {
-      for (int t = from; t < to; ++t) {
-        const StatePtrs& in = t == from ? at(src) : x->work[(t - from - 1) & 1];
-        const StatePtrs& out = t == to - 1 ? at(dst) : x->work[(t - from) & 1];
-        if (!step(in, out)) return false;
-      }
-      return true;
+      return run(at(src), to - from, at(dst), x->work);
     };
     auto adjoint = [&](int n, int sl) { return adjoint_step(n, at(sl)); };
     int right = x->nsteps;
@@ -1256,12 +1278,7 @@ hipError_t adj_backward(bgk_handle* h, const double* seeds_host, double grad[3])
         // slot[0] and slot[1]
         auto c2 = [&](int k) -> const StatePtrs& { return k == 0 ? x->ckpt[s1] : x->ckpt2[k - 1]; };
         for (int k = 1; k < ns2 && e == hipSuccess; ++k) {
-          const StatePtrs* src = &c2(k - 1);
-          for (int i = 0; i < x->seg && e == hipSuccess; ++i) {
-            const StatePtrs* dst = (i == x->seg - 1) ? &x->ckpt2[k - 1] : &x->slot[i & 1];
-            step(*src, *dst);
-            src = dst;
-          }
+          run(c2(k - 1), x->seg, x->ckpt2[k - 1], x->slot.data());
         }
         for (int s2 = ns2 - 1; s2 >= 0 && e == hipSuccess; --s2)
           inner(c2(s2), m0 + s2 * x->seg, std::min(m0 + (s2 + 1) * x->seg, m1));

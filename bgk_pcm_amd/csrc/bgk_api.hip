@@ -274,6 +274,7 @@ int run_stage(bgk_handle* h, hipError_t (*fn)(bgk_handle*), const char* name) {
   int rc = check_handle(h);
   if (rc) return rc;
   if ((rc = need_fp64(h, name))) return rc;
+  h->te_ok = false;
   return launched(fn(h), name);
 }
 
@@ -369,6 +370,8 @@ int bgk_create(const bgk_params* p, bgk_handle** out) {
   h->cur = 0;
   h->pc = 0;
   h->rc = 0;
+  h->te_cur = 0;
+  h->te_ok = false;
   h->since_rebase = 0;
   // steps between re-basings of the FP32 populations' row densities
   // (BGK_REBASE_EVERY, 0: never); a tuning knob, every value is correct
@@ -377,10 +380,10 @@ int bgk_create(const bgk_params* p, bgk_handle** out) {
     h->rebase_every = std::max(0, std::atoi(env));
   std::memset(&h->ext, 0, sizeof h->ext);
   h->ext.k_ratio = 1.0;
-  // tiling of the moment kernel: BGK_MOM_ROWS (rows per strip; default
-  // about 64, or 32 for tau_f != 1, fitted to the device) and
-  // BGK_MOM_VARIANT (1..8: workgroup width 64/128/256/512 with a 4- or
-  // 3-row ring; 0: chosen from Nx) override the defaults; tuning knobs,
+  // BGK_MOM_ROWS (rows per strip of the moment kernels; default: fitted to
+  // the lattice and the device) and BGK_MOM_VARIANT (1..3: at most that many
+  // steps per launch of the streaming kernel; 4 and up: one step per launch
+  // of the ring kernel where it exists) override the defaults; tuning knobs,
   // every value is correct
   h->strip_rows = 0;
   h->mom_variant = 0;
@@ -452,6 +455,7 @@ int bgk_initialization(bgk_handle* h) {
   int rc = check_handle(h);
   if (rc) return rc;
   bgk::adj_invalidate(h);
+  h->te_ok = false;
   if (h->prm.precision == BGK_FP32_DEV) return launched(bgk::launch_initialization32(h), "initialization");
   if (h->prm.precision == BGK_FP32_MOM || h->prm.precision == BGK_FP64_MOM)
     return launched(bgk::launch_initialization_mom(h), "initialization");
@@ -486,6 +490,7 @@ int bgk_upload(bgk_handle* h, int32_t field, const double* src, int64_t ld) {
   FieldRef r;
   if ((rc = resolve(h, field, &r))) return rc;
   bgk::adj_invalidate(h);
+  h->te_ok = false;
   // the stored f of an FP32 handle depend on phi through their reference
   // density: a new phi is staged and the f re-expressed before it lands
   const bool phi_via_tmp = h->prm.precision == BGK_FP32_DEV && field == BGK_PHI;
@@ -545,16 +550,18 @@ int bgk_step(bgk_handle* h, int32_t nsteps) {
   if (h->fused_ok) {
     if ((rc = launched(bgk::launch_teast_prologue(h), "teast prologue"))) return rc;
     const int prec = h->prm.precision;
+    if (prec >= BGK_FP32_MOM)
+      return launched(bgk::launch_fused_steps_mom(h, nsteps), "fused steps");
     for (int s = 0; s < nsteps; ++s) {
       const bool last = (s == nsteps - 1);
-      hipError_t e = prec == BGK_FP32_DEV   ? bgk::launch_fused_step32(h, s, last)
-                     : prec >= BGK_FP32_MOM ? bgk::launch_fused_step_mom(h, s, last)
-                                            : bgk::launch_fused_step64(h, s, last);
+      hipError_t e = prec == BGK_FP32_DEV ? bgk::launch_fused_step32(h, last)
+                                          : bgk::launch_fused_step64(h, last);
       if (e != hipSuccess) return hip_fail(e, "fused step");
     }
     return BGK_OK;
   }
   if ((rc = need_fp64(h, "bgk_step with these boundary types"))) return rc;
+  h->te_ok = false;
   for (int s = 0; s < nsteps; ++s) {
     hipError_t e;
     if ((e = bgk::launch_bc_f(h)) != hipSuccess) return hip_fail(e, "BC_f");

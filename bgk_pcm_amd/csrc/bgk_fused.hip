@@ -203,20 +203,23 @@ __global__ __launch_bounds__(TILE_W) void k_fused64(Pairs64 A, Pairs64 B,
 }  // namespace
 
 hipError_t launch_teast_prologue(bgk_handle* h) {
+  if (h->te_ok) return hipSuccess;
   const Geom& g = h->geom;
   hipLaunchKernelGGL(k_teast_prologue, dim3((unsigned)((g.ny + 2 + 255) / 256)), dim3(256), 0,
-                     h->stream, h->T, h->teast[0], g);
-  return hipGetLastError();
+                     h->stream, h->T, h->teast[h->te_cur], g);
+  const hipError_t e = hipGetLastError();
+  h->te_ok = e == hipSuccess;
+  return e;
 }
 
-hipError_t launch_fused_step64(bgk_handle* h, int step_parity, bool write_all) {
+hipError_t launch_fused_step64(bgk_handle* h, bool write_all) {
   const Geom& g = h->geom;
   const TileGrid tg = make_tile_grid(g);
   dim3 blk(TILE_W);
   dim3 grd((unsigned)(tg.per * NXCD));
   Macro m{h->rho, h->u, h->v, h->T};
-  const double* te_in = h->teast[step_parity & 1];
-  double* te_out = h->teast[(step_parity + 1) & 1];
+  const double* te_in = h->teast[h->te_cur];
+  double* te_out = h->teast[1 - h->te_cur];
   const int a = h->cur, b = 1 - h->cur;
   if (h->prm.rounding == BGK_ROUND_STEP7)
     hipLaunchKernelGGL(k_fused64<true>, grd, blk, 0, h->stream, pairs(h->f[a]), pairs(h->f[b]), h->phi[h->pc], h->phi[1 - h->pc], te_in,
@@ -228,6 +231,7 @@ hipError_t launch_fused_step64(bgk_handle* h, int step_parity, bool write_all) {
   if (e == hipSuccess) {
     h->cur = b;
     h->pc = 1 - h->pc;
+    h->te_cur = 1 - h->te_cur;
   }
   return e;
 }

@@ -526,7 +526,7 @@ hipError_t launch_rephase32(bgk_handle* h, const double* phi_new) {
   return hipGetLastError();
 }
 
-hipError_t launch_fused_step32(bgk_handle* h, int step_parity, bool write_all) {
+hipError_t launch_fused_step32(bgk_handle* h, bool write_all) {
   if (h->rebase_every > 0 && h->since_rebase >= h->rebase_every) {
     hipError_t e = launch_rebase32(h);
     if (e != hipSuccess) return e;
@@ -536,8 +536,8 @@ hipError_t launch_fused_step32(bgk_handle* h, int step_parity, bool write_all) {
   dim3 blk(TILE_W);
   dim3 grd((unsigned)(tg.per * NXCD));
   Macro m{h->rho, h->u, h->v, h->T};
-  const double* te_in = h->teast[step_parity & 1];
-  double* te_out = h->teast[(step_parity + 1) & 1];
+  const double* te_in = h->teast[h->te_cur];
+  double* te_out = h->teast[1 - h->te_cur];
   const int a = h->cur, b = 1 - h->cur;
   const double* tab = h->rref[h->rc];
   if (h->prm.fp32_collision)
@@ -552,6 +552,7 @@ hipError_t launch_fused_step32(bgk_handle* h, int step_parity, bool write_all) {
   if (e == hipSuccess) {
     h->cur = b;
     h->pc = 1 - h->pc;
+    h->te_cur = 1 - h->te_cur;
     ++h->since_rebase;
   }
   return e;

@@ -1,4 +1,7 @@
-// bgk_fused_mom.hip -- the fused time step with moment storage.
+// bgk_fused_mom.hip -- moment storage: the choice of kernel and of the steps
+// per launch, the initialization, and the ring kernel, one step per launch
+// through LDS, which large FP32-moment lattices take for a step alone (see
+// ring_step; every other launch is bgk_stream_mom.hip's).
 //
 // The node state is the ten moments of bgk_mom.h (rho, T - T_crit in FP64;
 // u, v and the scaled non-equilibrium second moments in R = float or
@@ -342,12 +345,12 @@ __global__ void k_initialization_mom(MomOut st, Macro m, double* phi, double* ph
   phip[q] = s0.phi;
 }
 
-template <int W, int NS, typename R, bool EQF>
-hipError_t launch_mom_t(bgk_handle* h, const MomStep& st) {
+template <int W, int NS, bool EQF>
+hipError_t launch_ring(bgk_handle* h, const MomStep& st) {
   // resident workgroups per CU of this instantiation (LDS and registers)
   static const int per_cu = [] {
     int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_fused_mom<W, NS, R, EQF>, W, 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_fused_mom<W, NS, float, EQF>, W, 0) !=
         hipSuccess)
       n = 0;
     return n;
@@ -358,23 +361,21 @@ hipError_t launch_mom_t(bgk_handle* h, const MomStep& st) {
   const int64_t nwg = (int64_t)sg.nmain + (nedge + W - 1) / W;
   Macro m{h->rho, h->u, h->v, h->T};
   if (st.macro[0]) m = Macro{st.macro[0], st.macro[1], st.macro[2], st.macro[3]};
-  hipLaunchKernelGGL((k_fused_mom<W, NS, R, EQF>), dim3((unsigned)nwg), dim3(W), 0, h->stream,
+  hipLaunchKernelGGL((k_fused_mom<W, NS, float, EQF>), dim3((unsigned)nwg), dim3(W), 0, h->stream,
                      st.in, st.out, st.pa, st.pb, st.te_in, st.te_out, m, h->c, h->geom, sg,
                      st.write_all ? 1 : 0, st.probe_idx, st.probe_out);
   return hipGetLastError();
 }
 
-// FP64 moments take at most 256 columns per workgroup (the 512-wide ring
-// of 88-byte nodes exceeds the 160 KiB of LDS).
-template <int W, int NS>
-hipError_t launch_mom(bgk_handle* h, const MomStep& st) {
-  constexpr int W64 = W > 256 ? 256 : W;
-  const bool f64 = h->prm.precision == BGK_FP64_MOM;
-  if (h->mom_eqf)
-    return f64 ? launch_mom_t<W64, NS, double, true>(h, st)
-               : launch_mom_t<W, NS, float, true>(h, st);
-  return f64 ? launch_mom_t<W64, NS, double, false>(h, st)
-             : launch_mom_t<W, NS, float, false>(h, st);
+// Whether one step alone goes through the ring kernel.  Measured per step on
+// MI355X, ring against the streaming kernel with T = 1, FP32 moments: 4096^2
+// 362 / 394 us (omega_f = 1: 290 / 329), 2048^2 107 / 104 (89 / 84), 512^2
+// 20.2 / 11.8 (17.6 / 10.4); FP64 moments are faster or within 4% with the
+// streaming kernel at every size.
+bool ring_step(const bgk_handle* h) {
+  if (h->prm.precision != BGK_FP32_MOM) return false;
+  if (h->mom_variant != 0) return h->mom_variant >= 4;
+  return (int64_t)h->nx * h->ny >= (int64_t)1 << 23;
 }
 
 template <typename R, bool EQF>
@@ -387,47 +388,70 @@ void launch_init(bgk_handle* h, const MomOut& st, dim3 grd) {
 
 }  // namespace
 
-hipError_t launch_mom_step(bgk_handle* h, const MomStep& st) {
-  // Tiling (workgroup width W, ring rows NS).  Measured at 4096^2 on MI355X
-  // with FP32 moments: omega_f = 1 (36-byte nodes, 64-row strips) W = 512 /
-  // NS = 4 57.2 GLUPS, 512/3 53.1, 256/4 53.9 (32-row strips), 128/4 45.1,
-  // 64/4 45.8; general layout (48 bytes, 32-row strips) 512/3 45.9, 512/4
-  // 45.6, 256/3 42.0.  Wider segments stream longer contiguous runs of each
-  // row.  FP64 moments take the same tiling with half the workgroups per CU.
-  int v = h->mom_variant;
-  if (v == 0)
-    v = h->nx >= 2048 ? (h->mom_eqf ? 7 : 8) : h->nx >= 512 ? 5 : h->nx >= 128 ? 3 : 1;
-  switch (v) {
-    case 1: return launch_mom<64, 4>(h, st);
-    case 2: return launch_mom<64, 3>(h, st);
-    case 3: return launch_mom<128, 4>(h, st);
-    case 4: return launch_mom<128, 3>(h, st);
-    case 5: return launch_mom<256, 4>(h, st);
-    case 6: return launch_mom<256, 3>(h, st);
-    case 7: return launch_mom<512, 4>(h, st);
-    default: return launch_mom<512, 3>(h, st);
-  }
+// Most steps per launch.  Two halve the HBM bytes of a step; three pay only
+// where a node is large and its update small (FP64 moments with omega_f = 1:
+// 4096^2 188 against 239 us per step, 2048^2 62 against 64, smaller lattices
+// lose).  FP32 moments with omega_f = 1 take one step per launch beyond 2^25
+// nodes: there the cost of the adjoint is held to three plain forward steps,
+// and its own kernel, at 50% of the memory rate, cannot follow a forward step
+// of half the time.
+int mom_most_steps(const bgk_handle* h) {
+  const bool f64 = h->prm.precision == BGK_FP64_MOM;
+  const int64_t nodes = (int64_t)h->nx * h->ny;
+  if (h->mom_variant >= 4) return 1;
+  if (h->mom_variant > 0) return h->mom_variant == 3 && !(f64 && h->mom_eqf) ? 2 : h->mom_variant;
+  if (!f64 && h->mom_eqf && nodes > (int64_t)1 << 25) return 1;
+  return f64 && h->mom_eqf && nodes >= (int64_t)1 << 21 ? 3 : 2;
 }
 
-hipError_t launch_fused_step_mom(bgk_handle* h, int step_parity, bool write_all) {
-  const int a = h->cur, b = 1 - h->cur;
-  MomStep st;
-  st.in = MomIn{h->ma[a], h->mb[a], h->mc[a]};
-  st.out = MomOut{h->ma[b], h->mb[b], h->mc[b]};
-  st.pa = h->phi[h->pc];
-  st.pb = h->phi[1 - h->pc];
-  st.te_in = h->teast[step_parity & 1];
-  st.te_out = h->teast[(step_parity + 1) & 1];
-  st.write_all = write_all;
-  st.probe_idx = nullptr;
-  st.probe_out = nullptr;
-  for (int k = 0; k < 4; ++k) st.macro[k] = nullptr;
-  hipError_t e = launch_mom_step(h, st);
-  if (e == hipSuccess) {
+// Of `left` steps, how many the next launch takes: an odd rest first, so that
+// a call ends with a launch of several steps (which knows the state before
+// the last one, for the halo).
+int mom_next_steps(const bgk_handle* h, int left) {
+  const int most = mom_most_steps(h);
+  return left % most ? left % most : most;
+}
+
+// Whether a launch of T steps has to write the macroscopic fields: the last of
+// a call; and the one before a last launch of one step, which takes the halo
+// from them, unless it is a ring launch (these keep the boundary nodes
+// current).
+bool mom_write_all(const bgk_handle* h, int T, int left) {
+  return left == 0 || (left == 1 && !(T == 1 && ring_step(h)));
+}
+
+hipError_t launch_mom_steps(bgk_handle* h, const MomStep& st, int T) {
+  if (T > 1 || !ring_step(h)) return launch_mom_stream(h, st, T);
+  // Ring tiling (workgroup width / ring rows), measured at 4096^2: omega_f = 1
+  // (36-byte nodes, 64-row strips) 512/4 57.2 GLUPS, 512/3 53.1, 256/4 53.9;
+  // general layout (48 bytes, 32-row strips) 512/3 45.9, 512/4 45.6
+  return h->mom_eqf ? launch_ring<512, 4, true>(h, st) : launch_ring<512, 3, false>(h, st);
+}
+
+hipError_t launch_fused_steps_mom(bgk_handle* h, int nsteps) {
+  for (int left = nsteps; left > 0;) {
+    const int T = mom_next_steps(h, left);
+    left -= T;
+    const int a = h->cur, b = 1 - h->cur;
+    MomStep st;
+    st.in = MomIn{h->ma[a], h->mb[a], h->mc[a]};
+    st.out = MomOut{h->ma[b], h->mb[b], h->mc[b]};
+    st.pa = h->phi[h->pc];
+    st.pb = h->phi[1 - h->pc];
+    st.te_in = h->teast[h->te_cur];
+    st.te_out = h->teast[1 - h->te_cur];
+    st.write_all = mom_write_all(h, T, left);
+    st.probe_idx = nullptr;
+    st.probe_out = nullptr;
+    st.probe_np = 0;
+    for (int k = 0; k < 4; ++k) st.macro[k] = nullptr;
+    const hipError_t e = launch_mom_steps(h, st, T);
+    if (e != hipSuccess) return e;
     h->cur = b;
     h->pc = 1 - h->pc;
+    h->te_cur = 1 - h->te_cur;
   }
-  return e;
+  return hipSuccess;
 }
 
 hipError_t launch_initialization_mom(bgk_handle* h) {

@@ -57,14 +57,18 @@ struct bgk_handle {
   void* mb[2];    // float4 (FP32 moments) or double4 (FP64 moments) planes
   void* mc[2];    // the same, or float / double planes when mom_eqf
   bool mom_eqf;   // omega_f == 1: Pf vanishes, mb = (u, v, Pg_xx, Pg_yy), mc = Pg_xy
-  int strip_rows;   // rows per workgroup strip of the moment kernel (0: default)
-  int mom_variant;  // tiling variant of the moment kernel (0: default)
+  int strip_rows;   // rows per strip of the moment kernels (0: default)
+  int mom_variant;  // steps per launch of the moment step (0: by rule, see mom_most_steps)
   int cur;
 
   double* phi[2];
   int pc;
   double *rho, *u, *v, *T, *rho2, *u2, *v2, *T2;
-  double* teast[2];  // averaged T(Nx, 0..Ny+1) of the previous step, ping-pong
+  // averaged T(Nx, 0..Ny+1) of the previous step, ping-pong; teast[te_cur] is
+  // current when te_ok (else the next step copies the column from T)
+  double* teast[2];
+  int te_cur;
+  bool te_ok;
   // FP32 population handles: solid and liquid reference densities of rows
   // 0..Ny+1 ([0, Ny+2) and [Ny+2, 2(Ny+2)) of rref[rc]; the other is the
   // next table) the f members are stored against, and the re-basing cadence
@@ -97,13 +101,15 @@ hipError_t launch_collision(bgk_handle* h);
 hipError_t launch_moments(bgk_handle* h);
 
 // ---- fused step (bgk_fused.hip / bgk_fused32.hip)
-// Copy averaged T(Nx, :) into teast[cur] before the first fused step of a call.
+// Make teast[te_cur] hold the averaged T(Nx, :) before the first fused step of
+// a call: a launch only where something but the fused step wrote T since.
 hipError_t launch_teast_prologue(bgk_handle* h);
 // One fused FP64 step from buffer cur to 1-cur; write_all: write the
 // moments of every node (else only the boundary-adjacent ones).
-hipError_t launch_fused_step64(bgk_handle* h, int step_parity, bool write_all);
-hipError_t launch_fused_step32(bgk_handle* h, int step_parity, bool write_all);
-hipError_t launch_fused_step_mom(bgk_handle* h, int step_parity, bool write_all);
+hipError_t launch_fused_step64(bgk_handle* h, bool write_all);
+hipError_t launch_fused_step32(bgk_handle* h, bool write_all);
+// nsteps moment steps
+hipError_t launch_fused_steps_mom(bgk_handle* h, int nsteps);
 hipError_t launch_initialization_mom(bgk_handle* h);
 
 // ---- plane conversions (bgk_fused32.hip); strides in elements.  The base

@@ -360,13 +360,14 @@ struct NodeOut {
   double rho, Tav, uav, vav;
 };
 
-// One launch of the moment-storage step: state and phi in and out, the
-// east-wall temperature column of the previous and of this step, an
-// optional probe record (T averaged as moments.f90 at the nodes whose
-// probe_idx is >= 0, written to probe_out[probe_idx]; probe_idx in column 0
-// of a row is >= 0 when the row holds a probe) and optional
-// macroscopic planes rho, u, v, T to write instead of the handle's (their
-// halo columns of u, v must hold the ghost velocities).
+// One launch of T moment-storage steps: state and phi in and out, the
+// east-wall temperature column before and after, an optional probe record (T
+// averaged as moments.f90 at the nodes whose probe_idx is >= 0, after step t
+// of the launch to probe_out[t*probe_np + probe_idx]; probe_idx in column 0 of
+// a row is >= 0 when the row holds a probe).  write_all: the macroscopic
+// fields of every node and the halo.  One-step launches of the ring kernel
+// write those of the boundary nodes in any case, to the handle's planes or to
+// `macro` (whose halo columns of u, v must hold the ghost velocities).
 struct MomStep {
   double* macro[4];
   MomIn in;
@@ -378,11 +379,17 @@ struct MomStep {
   bool write_all;
   const int* probe_idx;
   double* probe_out;
+  int probe_np;
 };
 
 }  // namespace mom
 
-hipError_t launch_mom_step(bgk_handle* h, const mom::MomStep& st);
+// T steps in one launch (bgk_fused_mom.hip; T at most mom_next_steps), and the
+// streaming kernel's share of them (bgk_stream_mom.hip)
+hipError_t launch_mom_steps(bgk_handle* h, const mom::MomStep& st, int T);
+hipError_t launch_mom_stream(bgk_handle* h, const mom::MomStep& st, int T);
+int mom_next_steps(const bgk_handle* h, int left);
+bool mom_write_all(const bgk_handle* h, int T, int left);
 }  // namespace bgk
 
 #endif  // BGK_MOM_H

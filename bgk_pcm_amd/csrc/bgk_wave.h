@@ -1,0 +1,163 @@
+// bgk_wave.h -- building blocks of the wave-streaming kernels that advance
+// several time steps per launch (bgk_stream_mom.hip).
+//
+// One wavefront owns 64 neighbouring columns and walks up a strip of rows.
+// Lane L holds column i0 - T + L of the row being processed, so a pull from
+// the column to the west or east is a shift by one lane (v_mov_b32 with the
+// DPP control wave_shr:1 / wave_shl:1, full rate, no LDS and no barrier), and
+// a pull from the row below or above is a value kept in registers while the
+// walk goes on.  A launch of T steps feeds each row through T levels: level t
+// completes row r - t - 1 when row r arrives, and hands it to level t + 1 in
+// the same iteration.  T lanes at each end of the wave and T rows at each end
+// of a strip are recomputed by the neighbour, so HBM sees the state once in
+// and once out per T steps.
+#ifndef BGK_WAVE_H
+#define BGK_WAVE_H
+
+#include <algorithm>
+
+#include "bgk_internal.h"
+
+namespace bgk {
+namespace wave {
+
+constexpr int kLanes = 64;
+constexpr int kDppShr1 = 0x138;  // lane L reads lane L - 1
+constexpr int kDppShl1 = 0x130;  // lane L reads lane L + 1
+
+// The value of the lane to the west (column i - 1); 0 in lane 0.
+__device__ __forceinline__ double from_west(double x) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, kDppShr1, 0xf,
+                                                            0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), kDppShr1,
+                                                            0xf, 0xf, true);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+// The value of the lane to the east (column i + 1); 0 in lane 63.
+__device__ __forceinline__ double from_east(double x) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, kDppShl1, 0xf,
+                                                            0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), kDppShl1,
+                                                            0xf, 0xf, true);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// Buffer descriptor of n elements at p (wave-uniform), and a store of one
+// element at offset q that the hardware drops where q >= n.  kPastStrip times
+// an element's size (4 to 32 bytes) stays within 32 bits and past any strip
+// (kMaxStrip elements, see make_wave_grid).
+constexpr int kPastStrip = 0x07ffffff;
+constexpr int kMaxStrip = 0x03ffffff;
+template <typename E>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t strip_buffer(E* p, int n) {
+  return __builtin_amdgcn_make_buffer_rsrc(p, 0, n * (int)sizeof(E), 0x00020000);
+}
+constexpr int kNonTemporal = 2;
+template <typename E>
+__device__ __forceinline__ void buffer_put(__amdgpu_buffer_rsrc_t r, int q, const E& x) {
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  const int off = (int)((unsigned)q * (unsigned)sizeof(E));
+  if constexpr (sizeof(E) == 4) {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x), r, off, 0, kNonTemporal);
+  } else if constexpr (sizeof(E) == 8) {
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), r, off, 0, kNonTemporal);
+  } else if constexpr (sizeof(E) == 16) {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, off, 0, kNonTemporal);
+  } else {
+    static_assert(sizeof(E) == 32, "element size");
+    struct Two {
+      u32x4 lo, hi;
+    };
+    const Two t = __builtin_bit_cast(Two, x);
+    __builtin_amdgcn_raw_buffer_store_b128(t.lo, r, off, 0, kNonTemporal);
+    __builtin_amdgcn_raw_buffer_store_b128(t.hi, r, off + 16, 0, kNonTemporal);
+  }
+}
+
+// A copy of x in registers of its own, so that a load issued next can reuse
+// x's (otherwise the compiler loads into others and moves them, with a wait,
+// at the end of the loop).
+__device__ __forceinline__ double taken(double x) {
+  double y;
+  asm("v_mov_b64 %0, %1" : "=v"(y) : "v"(x));
+  return y;
+}
+
+// s_waitcnt operand: all loads and stores done (vmcnt 0; the others free).  Set
+// before a loop whose loads stay in flight across its back edge, so that the
+// waits inside need not cover the loop's entry.
+constexpr int kWaitLoads = 0x0f70;
+
+// A read-only array through the scalar cache (uniform index).
+typedef const __attribute__((address_space(4))) double* scalar_ptr;
+__device__ __forceinline__ scalar_ptr as_scalar(const double* p) {
+  return (scalar_ptr)(uintptr_t)p;
+}
+
+// Work split of a launch: column segments of `cols` output columns, strips of
+// `rows` rows, one wave (and workgroup) for each pair.
+constexpr int kMaxRows = 64;
+struct WaveGrid {
+  int nseg;    // column segments
+  int rows;    // rows per strip
+  int nstrip;  // strips
+  int nwg;     // workgroups, padded to a multiple of 8 (the XCDs)
+};
+
+// Segment and strip of this workgroup; false for the padding.  Workgroup b
+// runs on XCD b % 8: each XCD takes a contiguous run of (strip, segment)
+// pairs, so the columns and rows that neighbours share are hits in its L2.
+__device__ __forceinline__ bool wave_tile(const WaveGrid& g, int* seg, int* strip) {
+  const int b = (int)blockIdx.x;
+  const int k = (b % NXCD) * (g.nwg / NXCD) + b / NXCD;
+  *strip = k / g.nseg;
+  *seg = k % g.nseg;
+  return *strip < g.nstrip;
+}
+
+// The strip height, 1..most.  A strip of h rows costs its wave h + 2T row
+// iterations.  Up to one wave per SIMD (4 n_cu) they all run at once at full
+// speed; two waves on a SIMD slow each other by 1.2 to 1.6 (measured, large to
+// small lattices); beyond 8 n_cu waves the launch takes that many rounds, the
+// last one half empty on average.  Taller strips repeat fewer rows but are capped at `most`:
+// the more rows lie between the strips walked at once, the slower memory
+// serves them (figures at the callers).
+inline int strip_rows(int nseg, int ny, int T, int most, int n_cu) {
+  int best = 1;
+  double cost = -1.0;
+  for (int h = 1; h <= most && h <= ny; ++h) {
+    const double waves = (double)nseg * ((ny + h - 1) / h), slots = 8.0 * n_cu;
+    const double iters = h + 2 * T;
+    const double c = waves <= 0.5 * slots ? iters
+                     : waves <= slots     ? 1.35 * iters
+                                          : 1.35 * (waves / slots + 0.5) * iters;
+    if (cost < 0.0 || c < cost) {
+      cost = c;
+      best = h;
+    }
+  }
+  return best;
+}
+
+// rows_override > 0 fixes the strip height.
+inline WaveGrid make_wave_grid(int nx, int ny, int cols, int T, int most, int n_cu,
+                               int rows_override) {
+  WaveGrid g;
+  g.nseg = (nx + cols - 1) / cols;
+  g.rows = rows_override > 0 ? std::min(rows_override, std::min(ny, kMaxRows))
+                             : strip_rows(g.nseg, ny, T, most, n_cu);
+  // (offsets within a strip stay below kMaxStrip elements)
+  g.rows = std::max(1, std::min(g.rows, (int)(kMaxStrip / (int64_t)(nx + 256))));
+  g.nstrip = (ny + g.rows - 1) / g.rows;
+  const int64_t n = (int64_t)g.nseg * g.nstrip;
+  g.nwg = (int)((n + NXCD - 1) / NXCD * NXCD);
+  return g;
+}
+
+}  // namespace wave
+}  // namespace bgk
+
+#endif  // BGK_WAVE_H
