@@ -13,8 +13,8 @@
 // FP32 moments); two steps per launch halve the bytes and leave it bound by
 // VALU issue at two waves per SIMD (FP32 moments: 212 VGPRs).  Measured at
 // 4096^2, us per step, against one step per launch of the ring kernel:
-// FP32 moments 209 (362), with omega_f = 1 174 (290), FP64 moments 320 (648),
-// with omega_f = 1 188 (462, three steps per launch).  FP32 moments with three
+// FP32 moments 203 (362), with omega_f = 1 168 (290), FP64 moments 323 (648),
+// with omega_f = 1 180 (462, three steps per launch).  FP32 moments with three
 // steps per launch: 230 (spills), with omega_f = 1 172.
 #include <algorithm>
 
@@ -537,17 +537,13 @@ __device__ __forceinline__ void stream_strip(const StreamArgs& A, int i0, int j0
 
 template <int T, typename R, bool EQF, int MODE>
 __global__ __launch_bounds__(kLanes, 2) void k_stream_mom(StreamArgs A) {
-  int seg, strip;
-  if (!wave_tile(A.g, &seg, &strip)) return;
-  const int nx = A.nx, ny = A.ny;
+  int seg, j0, j1;
+  bool edge;
+  if (!wave_tile(A.g, A.ny, &seg, &j0, &j1, &edge)) return;
   const int i0 = seg * (kLanes - 2 * T) + 1;
-  const int j0 = strip * A.g.rows + 1;
-  const int j1 = min(j0 + A.g.rows - 1, ny);
   const int i = i0 - T + (int)threadIdx.x;
-  const bool has_w = i0 - T <= 1;
-  const bool has_e = i0 - T + kLanes - 1 >= nx;
-  if (has_w || has_e || j0 - T <= 1 || j1 + T >= ny)
-    stream_strip<T, R, EQF, true, MODE>(A, i0, j0, j1, i, has_w, has_e);
+  if (edge)
+    stream_strip<T, R, EQF, true, MODE>(A, i0, j0, j1, i, i0 - T <= 1, i0 - T + kLanes - 1 >= A.nx);
   else
     stream_strip<T, R, EQF, false, MODE>(A, i0, j0, j1, i, false, false);
 }
@@ -591,12 +587,13 @@ hipError_t launch_t(bgk_handle* h, const MomStep& st) {
   a.probe_idx = st.probe_idx;
   a.probe_out = st.probe_out;
   a.probe_np = st.probe_np;
-  // strips of at most 32 rows with FP32 moments, 16 with FP64 (24 with three
-  // steps per launch); measured at 4096^2, T = 2, us per step at 8 / 16 / 32 /
-  // 64 / 138 rows: FP32 234 / 213 / 209 / 243 / 314, FP64 321 / 320 / 333 /
-  // 359 / 420
-  constexpr int most = sizeof(R) == sizeof(float) ? 32 : T == 3 ? 24 : 16;
-  a.g = make_wave_grid(h->nx, h->ny, kLanes - 2 * T, T, most, h->n_cu, h->strip_rows);
+  // Strips of at most 64 rows with FP32 moments, 16 with FP64; a row beside a
+  // wall counts 1.4 (measured at 1.2 / 1.6 / 2.2, us per step: 512^2 8.9 / 9.5
+  // / 10.9, 1003 x 777 15.2 / 15.3 / 17.4, 4096^2 210 / 202 / 209; all strips
+  // alike, walls in turn: 11.0, 18.5, 210).  FP64 moments at 4096^2 with at most
+  // 16 / 32 rows: 323 / 334.
+  constexpr int most = sizeof(R) == sizeof(float) ? 64 : 16;
+  a.g = make_wave_grid(h->nx, h->ny, kLanes - 2 * T, T, 2 * T, 1.4, most, h->n_cu, h->strip_rows);
   const dim3 grd((unsigned)a.g.nwg);
   if (st.write_all)
     hipLaunchKernelGGL((k_stream_mom<T, R, EQF, kFinal>), grd, dim3(kLanes), 0, h->stream, a);

@@ -97,64 +97,103 @@ __device__ __forceinline__ scalar_ptr as_scalar(const double* p) {
   return (scalar_ptr)(uintptr_t)p;
 }
 
-// Work split of a launch: column segments of `cols` output columns, strips of
-// `rows` rows, one wave (and workgroup) for each pair.
+// Work split of a launch: column segments of `cols` output columns, and for
+// each segment strips of rows, one wave (and workgroup) per strip.  Waves that
+// meet a wall (the first segment, the last one or two, and the lowest and
+// highest strip of the others) run the walls' code and take longer per row:
+// their strips are shorter, and they are dispatched first, so that none of
+// them is left when the others are done.
 constexpr int kMaxRows = 64;
 struct WaveGrid {
-  int nseg;    // column segments
-  int rows;    // rows per strip
-  int nstrip;  // strips
-  int nwg;     // workgroups, padded to a multiple of 8 (the XCDs)
+  int nseg, nright;  // segments; those that meet the east wall
+  int ne;            // segments whose every strip meets a wall: 1 + nright, or all
+  int re, nse;       // rows per strip of those, strips
+  int ra;            // rows of the lowest and highest strip of the others
+  int rows, nmid;    // rows per strip between them, strips
+  int nedge;         // workgroups of the walls
+  int nwg;           // all, the others padded to a multiple of 8 (the XCDs)
 };
 
-// Segment and strip of this workgroup; false for the padding.  Workgroup b
-// runs on XCD b % 8: each XCD takes a contiguous run of (strip, segment)
-// pairs, so the columns and rows that neighbours share are hits in its L2.
-__device__ __forceinline__ bool wave_tile(const WaveGrid& g, int* seg, int* strip) {
-  const int b = (int)blockIdx.x;
-  const int k = (b % NXCD) * (g.nwg / NXCD) + b / NXCD;
-  *strip = k / g.nseg;
-  *seg = k % g.nseg;
-  return *strip < g.nstrip;
+// Segment and rows j0..j1 of this workgroup; false for the padding.  Workgroup
+// b runs on XCD b % 8: of the strips away from the walls each XCD takes a
+// contiguous run of (strip, segment) pairs, so the columns and rows that
+// neighbours share are hits in its L2.
+__device__ __forceinline__ bool wave_tile(const WaveGrid& g, int ny, int* seg, int* j0, int* j1,
+                                          bool* edge) {
+  int b = (int)blockIdx.x;
+  *edge = b < g.nedge;
+  if (*edge) {
+    if (b < g.ne * g.nse) {
+      const int e = b % g.ne;
+      *seg = e == 0 ? 0 : g.nseg - g.ne + e;
+      *j0 = b / g.ne * g.re + 1;
+      *j1 = min(*j0 + g.re - 1, ny);
+    } else {
+      b -= g.ne * g.nse;
+      *seg = 1 + b / 2;
+      *j0 = b % 2 == 0 ? 1 : ny - g.ra + 1;
+      *j1 = *j0 + g.ra - 1;
+    }
+    return true;
+  }
+  b -= g.nedge;
+  const int inner = g.nseg - g.ne, per = (g.nwg - g.nedge) / NXCD;
+  const int k = b % NXCD * per + b / NXCD;
+  *seg = 1 + k % inner;
+  *j0 = g.ra + 1 + k / inner * g.rows;
+  *j1 = min(*j0 + g.rows - 1, ny - g.ra);
+  return k / inner < g.nmid;
 }
 
-// The strip height, 1..most.  A strip of h rows costs its wave h + 2T row
-// iterations.  Up to one wave per SIMD (4 n_cu) they all run at once at full
-// speed; two waves on a SIMD slow each other by 1.2 to 1.6 (measured, large to
-// small lattices); beyond 8 n_cu waves the launch takes that many rounds, the
-// last one half empty on average.  Taller strips repeat fewer rows but are capped at `most`:
-// the more rows lie between the strips walked at once, the slower memory
-// serves them (figures at the callers).
-inline int strip_rows(int nseg, int ny, int T, int most, int n_cu) {
-  int best = 1;
+// The split with strips of h rows (walls: of equal duration, at `slow` times
+// the cost per row iteration).  A strip of h rows takes h + extra iterations.
+inline WaveGrid split_waves(int nx, int ny, int cols, int T, int extra, double slow, int h) {
+  WaveGrid g{};
+  g.nseg = (nx + cols - 1) / cols;
+  const int last = nx - (g.nseg - 1) * cols;  // columns of the last segment
+  g.nright = last <= T ? 2 : 1;
+  g.re = std::max(1, std::min({ny, h, (int)((h + extra) / slow) - extra}));
+  g.ra = std::max(g.re, T + 1);
+  g.ne = g.nseg <= 1 + g.nright || ny <= 2 * g.ra ? g.nseg : 1 + g.nright;
+  g.nse = (ny + g.re - 1) / g.re;
+  g.rows = h;
+  const int64_t inner = g.nseg - g.ne;
+  g.nmid = inner > 0 ? (ny - 2 * g.ra + h - 1) / h : 0;
+  g.nedge = (int)((int64_t)g.ne * g.nse + 2 * inner);
+  g.nwg = g.nedge + (int)((inner * g.nmid + NXCD - 1) / NXCD * NXCD);
+  return g;
+}
+
+// The strip height, 1..most, by a model of the launch.  Up to one wave per SIMD
+// (4 n_cu) all run at once at full speed; two waves on a SIMD slow each other
+// by 1.2 to 1.6 (measured, large to small lattices); beyond 8 n_cu waves the
+// launch takes its work at that rate, plus half a strip for the last waves.
+// Taller strips repeat fewer rows.  rows_override > 0 fixes the height.
+inline WaveGrid make_wave_grid(int nx, int ny, int cols, int T, int extra, double slow, int most,
+                               int n_cu, int rows_override) {
+  // (offsets within a strip stay below kMaxStrip elements)
+  most = std::max(1, std::min({most, ny, kMaxRows, (int)(kMaxStrip / (int64_t)(nx + 256))}));
+  if (rows_override > 0)
+    return split_waves(nx, ny, cols, T, extra, slow, std::min(rows_override, most));
+  WaveGrid best{};
   double cost = -1.0;
-  for (int h = 1; h <= most && h <= ny; ++h) {
-    const double waves = (double)nseg * ((ny + h - 1) / h), slots = 8.0 * n_cu;
-    const double iters = h + 2 * T;
-    const double c = waves <= 0.5 * slots ? iters
-                     : waves <= slots     ? 1.35 * iters
-                                          : 1.35 * (waves / slots + 0.5) * iters;
+  for (int h = 1; h <= most; ++h) {
+    const WaveGrid g = split_waves(nx, ny, cols, T, extra, slow, h);
+    const double inner = g.nseg - g.ne, slots = 8.0 * n_cu;
+    const double waves = g.nedge + inner * g.nmid;
+    const double te = slow * (std::max(g.re, inner > 0 ? g.ra : 0) + extra);
+    const double longest = std::max(te, g.nmid > 0 ? (double)(h + extra) : 0.0);
+    const double work = slow * ((double)g.ne * g.nse * (g.re + extra) + 2 * inner * (g.ra + extra)) +
+                        inner * g.nmid * (h + extra);
+    const double c = waves <= 0.5 * slots ? longest
+                     : waves <= slots     ? 1.35 * longest
+                                          : 1.35 * (work / slots + 0.5 * longest);
     if (cost < 0.0 || c < cost) {
       cost = c;
-      best = h;
+      best = g;
     }
   }
   return best;
-}
-
-// rows_override > 0 fixes the strip height.
-inline WaveGrid make_wave_grid(int nx, int ny, int cols, int T, int most, int n_cu,
-                               int rows_override) {
-  WaveGrid g;
-  g.nseg = (nx + cols - 1) / cols;
-  g.rows = rows_override > 0 ? std::min(rows_override, std::min(ny, kMaxRows))
-                             : strip_rows(g.nseg, ny, T, most, n_cu);
-  // (offsets within a strip stay below kMaxStrip elements)
-  g.rows = std::max(1, std::min(g.rows, (int)(kMaxStrip / (int64_t)(nx + 256))));
-  g.nstrip = (ny + g.rows - 1) / g.rows;
-  const int64_t n = (int64_t)g.nseg * g.nstrip;
-  g.nwg = (int)((n + NXCD - 1) / NXCD * NXCD);
-  return g;
 }
 
 }  // namespace wave
