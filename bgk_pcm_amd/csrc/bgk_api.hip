@@ -372,6 +372,7 @@ int bgk_create(const bgk_params* p, bgk_handle** out) {
   h->rc = 0;
   h->te_cur = 0;
   h->te_ok = false;
+  h->ghost_uv = false;
   h->since_rebase = 0;
   // steps between re-basings of the FP32 populations' row densities
   // (BGK_REBASE_EVERY, 0: never); a tuning knob, every value is correct
@@ -380,15 +381,18 @@ int bgk_create(const bgk_params* p, bgk_handle** out) {
     h->rebase_every = std::max(0, std::atoi(env));
   std::memset(&h->ext, 0, sizeof h->ext);
   h->ext.k_ratio = 1.0;
-  // BGK_MOM_ROWS (rows per strip of the moment kernels; default: fitted to
+  // BGK_MOM_ROWS (rows per strip of the streaming kernels; default: fitted to
   // the lattice and the device) and BGK_MOM_VARIANT (1..3: at most that many
   // steps per launch of the streaming kernel; 4 and up: one step per launch
   // of the ring kernel where it exists) override the defaults; tuning knobs,
   // every value is correct
   h->strip_rows = 0;
   h->mom_variant = 0;
+  h->pop_variant = 0;
   h->mom_eqf = (1.0 / p->tau_f) == 1.0;
   if (const char* env = std::getenv("BGK_MOM_ROWS")) h->strip_rows = std::max(0, std::atoi(env));
+  // the same for the population kernels: BGK_POP_VARIANT 1 or 2 steps per launch
+  if (const char* env = std::getenv("BGK_POP_VARIANT")) h->pop_variant = std::max(0, std::atoi(env));
   if (const char* env = std::getenv("BGK_MOM_VARIANT")) h->mom_variant = std::max(0, std::atoi(env));
   set_constants(h);
 
@@ -456,6 +460,7 @@ int bgk_initialization(bgk_handle* h) {
   if (rc) return rc;
   bgk::adj_invalidate(h);
   h->te_ok = false;
+  h->ghost_uv = true;
   if (h->prm.precision == BGK_FP32_DEV) return launched(bgk::launch_initialization32(h), "initialization");
   if (h->prm.precision == BGK_FP32_MOM || h->prm.precision == BGK_FP64_MOM)
     return launched(bgk::launch_initialization_mom(h), "initialization");
@@ -491,6 +496,7 @@ int bgk_upload(bgk_handle* h, int32_t field, const double* src, int64_t ld) {
   if ((rc = resolve(h, field, &r))) return rc;
   bgk::adj_invalidate(h);
   h->te_ok = false;
+  if (field == BGK_U || field == BGK_V) h->ghost_uv = false;
   // the stored f of an FP32 handle depend on phi through their reference
   // density: a new phi is staged and the f re-expressed before it lands
   const bool phi_via_tmp = h->prm.precision == BGK_FP32_DEV && field == BGK_PHI;
@@ -552,10 +558,15 @@ int bgk_step(bgk_handle* h, int32_t nsteps) {
     const int prec = h->prm.precision;
     if (prec >= BGK_FP32_MOM)
       return launched(bgk::launch_fused_steps_mom(h, nsteps), "fused steps");
-    for (int s = 0; s < nsteps; ++s) {
-      const bool last = (s == nsteps - 1);
-      hipError_t e = prec == BGK_FP32_DEV ? bgk::launch_fused_step32(h, last)
-                                          : bgk::launch_fused_step64(h, last);
+    for (int left = nsteps; left > 0;) {
+      // an odd step first: the last launch of a call knows the state before
+      // its last step, for the halo
+      const bool many =
+          prec == BGK_FP64 && left % bgk::kSteps64 == 0 && bgk::stream64(h);
+      left -= many ? bgk::kSteps64 : 1;
+      hipError_t e = prec == BGK_FP32_DEV ? bgk::launch_fused_step32(h, left == 0)
+                     : many               ? bgk::launch_stream64(h, left == 0)
+                                          : bgk::launch_fused_step64(h, left == 0);
       if (e != hipSuccess) return hip_fail(e, "fused step");
     }
     return BGK_OK;

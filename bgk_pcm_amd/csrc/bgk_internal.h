@@ -57,7 +57,8 @@ struct bgk_handle {
   void* mb[2];    // float4 (FP32 moments) or double4 (FP64 moments) planes
   void* mc[2];    // the same, or float / double planes when mom_eqf
   bool mom_eqf;   // omega_f == 1: Pf vanishes, mb = (u, v, Pg_xx, Pg_yy), mc = Pg_xy
-  int strip_rows;   // rows per strip of the moment kernels (0: default)
+  int strip_rows;   // rows per strip of the streaming and ring kernels (0: default)
+  int pop_variant;  // steps per launch of the population kernels (0: by rule)
   int mom_variant;  // steps per launch of the moment step (0: by rule, see mom_most_steps)
   int cur;
 
@@ -69,6 +70,8 @@ struct bgk_handle {
   double* teast[2];
   int te_cur;
   bool te_ok;
+  // the ghost columns of u and v hold the initial velocities (no upload since)
+  bool ghost_uv;
   // FP32 population handles: solid and liquid reference densities of rows
   // 0..Ny+1 ([0, Ny+2) and [Ny+2, 2(Ny+2)) of rref[rc]; the other is the
   // next table) the f members are stored against, and the re-basing cadence
@@ -107,6 +110,10 @@ hipError_t launch_teast_prologue(bgk_handle* h);
 // One fused FP64 step from buffer cur to 1-cur; write_all: write the
 // moments of every node (else only the boundary-adjacent ones).
 hipError_t launch_fused_step64(bgk_handle* h, bool write_all);
+// kSteps64 FP64 steps in one launch (bgk_stream64.hip), where stream64(h)
+constexpr int kSteps64 = 2;
+bool stream64(const bgk_handle* h);
+hipError_t launch_stream64(bgk_handle* h, bool write_all);
 hipError_t launch_fused_step32(bgk_handle* h, bool write_all);
 // nsteps moment steps
 hipError_t launch_fused_steps_mom(bgk_handle* h, int nsteps);
