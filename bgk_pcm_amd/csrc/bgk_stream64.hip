@@ -20,8 +20,8 @@
 // What bounds it: HBM (152 B per node and step, 304 with one step per launch);
 // a row costs its wave 1330 VALU instructions at two waves per SIMD, 75% of
 // its time at the memory rate.  Measured, us per step, against bgk_fused.hip:
-// 4096^2 571 (893), 2048^2 155 (228), 1003 x 777 36 (49), 512^2 21.5 (20.6),
-// 256^2 15.6 (9.4): below 2^19 nodes one step per launch stays (stream64).
+// 4096^2 552 (893), 2048^2 152 (228), 1003 x 777 34.9 (49), 512^2 18.1 (20.6),
+// 256^2 12.6 (9.4): below 2^17 nodes one step per launch stays (stream64).
 #include <algorithm>
 
 #include "bgk_wave.h"
@@ -36,7 +36,7 @@ struct Macro {
 };
 
 struct Args64 {
-  Pairs64 A, B;
+  Planes<double2> A, B;
   const double* pa;
   double* pb;
   const double* te_in;
@@ -119,18 +119,12 @@ __device__ __forceinline__ Avg averaged(const Done& o) {
   return a;
 }
 
-// An element at a lane's 32-bit byte offset from a uniform address.
-template <typename E>
-__device__ __forceinline__ E at(const E* base, unsigned off) {
-  return *reinterpret_cast<const E*>(reinterpret_cast<const char*>(base) + off);
-}
-
 // Populations of row j already pulled: population k of node (i - cx_k, j -
 // cy_k).  off: byte offset of column i in a row of pairs.
 __device__ __forceinline__ void load_pulled(const Args64& A, unsigned off, int j, Row& r) {
 #pragma unroll
   for (int k = 0; k < 9; ++k) {
-    const double2 v = at(A.A.p[k] + ((int64_t)(j - CY[k]) * A.pitch - CX[k]), off);
+    const double2 v = at(A.A.row(k, (int64_t)(j - CY[k]) * A.pitch - CX[k]), off);
     r.f[k] = v.x;
     r.g[k] = v.y;
   }
@@ -149,10 +143,10 @@ __device__ __forceinline__ void load_pulled_edge(const Args64& A, const unsigned
 #pragma unroll
   for (int k = 0; k < 9; ++k) {
     const int sj = min(max(j - CY[k], 1), A.ny);
-    const double2 v = at(A.A.p[k] + (int64_t)sj * A.pitch, offs[1 - CX[k]]);
+    const double2 v = at(A.A.row(k, (int64_t)sj * A.pitch), offs[1 - CX[k]]);
     e.r.f[k] = v.x;
     e.r.g[k] = v.y;
-    if (k > 0) e.own[k] = at(&A.A.p[k][(int64_t)j * A.pitch].x, offs[1]);
+    if (k > 0) e.own[k] = at(&A.A.row(k, (int64_t)j * A.pitch)->x, offs[1]);
   }
 }
 
@@ -338,29 +332,22 @@ __device__ __forceinline__ void halo(const Args64& A, int jc, int i, const Avg& 
   }
 }
 
-// The stores of a strip: nine pair planes, phi, and the macroscopic fields
-// after a call's last step.
+// The stores of a row: nine pair planes, phi, and the macroscopic fields after
+// a call's last step.
 template <bool FINAL>
 struct Store64 {
-  __amdgpu_buffer_rsrc_t out[9], phi;
-  __device__ __forceinline__ Store64(const Args64& A, int j0, int j1) {
-    const int64_t qs = (int64_t)j0 * A.pitch;
-    const int n = (j1 - j0 + 1) * (int)A.pitch;
+  __device__ __forceinline__ static void put(const Args64& A, int jc, int j0, int j1, int i,
+                                             bool own, bool own_phi, const Done& o) {
+    const bool on = jc >= j0 && jc <= j1;
+    const int64_t qr = (int64_t)jc * A.pitch;
+    const int qa = on && own ? i : kPastStrip;
 #pragma unroll
-    for (int k = 0; k < 9; ++k) out[k] = strip_buffer(A.B.p[k] + qs, n);
-    phi = strip_buffer(A.pb + qs, n);
-  }
-  __device__ __forceinline__ void put(const Args64& A, int jc, int j0, int j1, int i, bool own,
-                                      bool own_phi, const Done& o) const {
-    const bool on = jc >= j0;
-    const int q = (jc - j0) * (int)A.pitch + i;
-    const int qa = on && own ? q : kPastStrip;
-#pragma unroll
-    for (int k = 0; k < 9; ++k) buffer_put(out[k], qa, make_double2(o.f[k], o.g[k]));
-    buffer_put(phi, on && own_phi ? q : kPastStrip, o.phi);
-    if (FINAL && on && jc <= j1 && own) {
+    for (int k = 0; k < 9; ++k)
+      buffer_put(strip_buffer(A.B.row(k, qr), (int)A.pitch), qa, make_double2(o.f[k], o.g[k]));
+    buffer_put(strip_buffer(A.pb + qr, (int)A.pitch), on && own_phi ? i : kPastStrip, o.phi);
+    if (FINAL && on && own) {
       const Avg a = averaged(o);
-      const int64_t qg = (int64_t)jc * A.pitch + i;
+      const int64_t qg = qr + i;
       A.m.rho[qg] = a.rho;
       A.m.T[qg] = a.T;
       A.m.u[qg] = a.u;
@@ -374,7 +361,6 @@ template <int T, bool STEP7, bool FINAL>
 __device__ __forceinline__ void strip_mid(const Args64& A, int j0, int j1, int i) {
   const int lane = (int)threadIdx.x;
   const bool own = lane >= T && lane < kLanes - T;
-  const Store64<FINAL> out(A, j0, j1);
   Pend L[T - 1];
 #pragma unroll
   for (int t = 0; t < T - 1; ++t) L[t] = Pend{};
@@ -410,7 +396,7 @@ __device__ __forceinline__ void strip_mid(const Args64& A, int j0, int j1, int i
       feed<false>(A, L[t - 1], o, 0.0, j, i, false, false, 0.0, 0.0, fp, gp, tap);
       o = node_step<STEP7>(A.c, fp, gp, tap);
     }
-    out.put(A, r - (T - 1), j0, j1, i, own, own, o);
+    Store64<FINAL>::put(A, r - (T - 1), j0, j1, i, own, own, o);
   }
 }
 
@@ -429,11 +415,10 @@ __device__ __forceinline__ void strip_edge(const Args64& A, int j0, int j1, int 
   for (int d = 0; d < 3; ++d)
     offs[d] = (unsigned)min(max(i + d - 1, 1), nx) * (unsigned)sizeof(double2);
   const unsigned offp = (unsigned)min(max(i, 0), nx + 1) * (unsigned)sizeof(double);
-  const Store64<FINAL> out(A, j0, j1);
   const __amdgpu_buffer_rsrc_t te_out = strip_buffer(A.te_out, ny + 2);
   const scalar_ptr te_in = as_scalar(A.te_in);
-  const double frozen6 = A.A.p[6][nx + 1].x;
-  const double frozen7 = A.A.p[7][(int64_t)(ny + 1) * P + nx + 1].x;
+  const double frozen6 = A.A.row(6, nx + 1)->x;
+  const double frozen7 = A.A.row(7, (int64_t)(ny + 1) * P + nx + 1)->x;
   Pend L[T - 1];
 #pragma unroll
   for (int t = 0; t < T - 1; ++t) L[t] = Pend{};
@@ -484,12 +469,12 @@ __device__ __forceinline__ void strip_edge(const Args64& A, int j0, int j1, int 
         halo(A, j - 1, i, averaged(o), o.phi);
     }
     const int jc = r - (T - 1);  // row completed by the last level
-    out.put(A, jc, j0, j1, i, own, own_phi, o);
+    Store64<FINAL>::put(A, jc, j0, j1, i, own, own_phi, o);
     buffer_put(te_out, jc >= j0 && jc <= j1 && own && i == nx ? jc : kPastStrip, tav);
   }
   if (own && i == nx) {
-    if (j0 == 1) A.B.p[6][nx + 1].x = frozen6;
-    if (j1 == ny) A.B.p[7][(int64_t)(ny + 1) * P + nx + 1].x = frozen7;
+    if (j0 == 1) A.B.row(6, nx + 1)->x = frozen6;
+    if (j1 == ny) A.B.row(7, (int64_t)(ny + 1) * P + nx + 1)->x = frozen7;
   }
 }
 
@@ -508,22 +493,20 @@ __global__ __launch_bounds__(kLanes, 2) void k_stream64(Args64 A) {
 
 }  // namespace
 
-// Lattices below 2^19 nodes stay in the caches, and the few waves they give
+// Lattices below 2^17 nodes stay in the caches, and the few waves they give
 // are bound by the latency of their rows; a handle whose ghost velocities were
 // uploaded takes the general kernel.
 bool stream64(const bgk_handle* h) {
   if (!h->ghost_uv || h->pop_variant == 1) return false;
-  return h->pop_variant > 1 || (int64_t)h->nx * h->ny >= (int64_t)1 << 19;
+  return h->pop_variant > 1 || (int64_t)h->nx * h->ny >= (int64_t)1 << 17;
 }
 
 hipError_t launch_stream64(bgk_handle* h, bool write_all) {
   constexpr int T = kSteps64;
   Args64 a;
   const int ca = h->cur, cb = 1 - h->cur;
-  for (int k = 0; k < 9; ++k) {
-    a.A.p[k] = reinterpret_cast<double2*>(h->f[ca][k]);
-    a.B.p[k] = reinterpret_cast<double2*>(h->f[cb][k]);
-  }
+  a.A = planes_of<double2>(h->f[ca]);
+  a.B = planes_of<double2>(h->f[cb]);
   a.pa = h->phi[h->pc];
   a.pb = h->phi[1 - h->pc];
   a.te_in = h->teast[h->te_cur];

@@ -77,6 +77,12 @@ __device__ __forceinline__ void buffer_put(__amdgpu_buffer_rsrc_t r, int q, cons
   }
 }
 
+// An element at a lane's 32-bit byte offset from a uniform address.
+template <typename E>
+__device__ __forceinline__ E at(const E* base, unsigned off) {
+  return *reinterpret_cast<const E*>(reinterpret_cast<const char*>(base) + off);
+}
+
 // A copy of x in registers of its own, so that a load issued next can reuse
 // x's (otherwise the compiler loads into others and moves them, with a wait,
 // at the end of the loop).
@@ -84,6 +90,22 @@ __device__ __forceinline__ double taken(double x) {
   double y;
   asm("v_mov_b64 %0, %1" : "=v"(y) : "v"(x));
   return y;
+}
+
+// Nine pair planes at one spacing (a handle's planes of one buffer are carved
+// alike).  A kernel forms a plane's row address where it uses it, from the
+// row's: nine pointers or buffer descriptors held across the row loop spill
+// scalar registers (100 of 720 instructions per row of the FP32 kernel).
+template <typename P2>
+struct Planes {
+  P2* base;
+  int64_t stride;  // pairs
+  __device__ __forceinline__ P2* row(int k, int64_t q) const { return base + (q + k * stride); }
+};
+template <typename P2, typename E>
+inline Planes<P2> planes_of(E* const* p) {
+  P2* const b = reinterpret_cast<P2*>(p[0]);
+  return Planes<P2>{b, reinterpret_cast<P2*>(p[1]) - b};
 }
 
 // s_waitcnt operand: all loads and stores done (vmcnt 0; the others free).  Set
