@@ -558,15 +558,15 @@ int bgk_step(bgk_handle* h, int32_t nsteps) {
     const int prec = h->prm.precision;
     if (prec >= BGK_FP32_MOM)
       return launched(bgk::launch_fused_steps_mom(h, nsteps), "fused steps");
+    if (prec == BGK_FP32_DEV)
+      return launched(bgk::launch_fused_steps32(h, nsteps), "fused steps");
     for (int left = nsteps; left > 0;) {
       // an odd step first: the last launch of a call knows the state before
       // its last step, for the halo
-      const bool many =
-          prec == BGK_FP64 && left % bgk::kSteps64 == 0 && bgk::stream64(h);
+      const bool many = left % bgk::kSteps64 == 0 && bgk::stream64(h);
       left -= many ? bgk::kSteps64 : 1;
-      hipError_t e = prec == BGK_FP32_DEV ? bgk::launch_fused_step32(h, left == 0)
-                     : many               ? bgk::launch_stream64(h, left == 0)
-                                          : bgk::launch_fused_step64(h, left == 0);
+      hipError_t e =
+          many ? bgk::launch_stream64(h, left == 0) : bgk::launch_fused_step64(h, left == 0);
       if (e != hipSuccess) return hip_fail(e, "fused step");
     }
     return BGK_OK;

@@ -115,6 +115,12 @@ constexpr int kSteps64 = 2;
 bool stream64(const bgk_handle* h);
 hipError_t launch_stream64(bgk_handle* h, bool write_all);
 hipError_t launch_fused_step32(bgk_handle* h, bool write_all);
+// nsteps steps of an FP32 population handle; kSteps32 of them in one launch
+// (bgk_stream32.hip), where stream32(h)
+hipError_t launch_fused_steps32(bgk_handle* h, int nsteps);
+constexpr int kSteps32 = 2;
+bool stream32(const bgk_handle* h);
+hipError_t launch_stream32(bgk_handle* h, bool write_all);
 // nsteps moment steps
 hipError_t launch_fused_steps_mom(bgk_handle* h, int nsteps);
 hipError_t launch_initialization_mom(bgk_handle* h);

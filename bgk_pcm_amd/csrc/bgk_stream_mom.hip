@@ -18,8 +18,7 @@
 // steps per launch: 230 (spills), with omega_f = 1 172.
 #include <algorithm>
 
-#include "bgk_mom.h"
-#include "bgk_wave.h"
+#include "bgk_level.h"
 
 // Every multiply-add below is written out: contraction chosen by the compiler
 // could differ between instantiations, and a step has to give the same bits
@@ -29,8 +28,7 @@
 namespace bgk {
 namespace {
 
-using namespace mom;
-using namespace wave;
+using namespace level;
 
 struct Macro {
   double *rho, *u, *v, *T;
@@ -85,126 +83,6 @@ __device__ __forceinline__ NodeD widen(const Raw<R, EQF>& r) {
   return n;
 }
 
-// The nine populations of a node from (m0, m, j = m (u, v) and P): m0 = m =
-// rho for f; m0 = T - T_crit, m = T for g, whose populations are the
-// deviations g_k - w_k T_crit.  With Q = 9/2 (m u u + P), E = m0 - tr Q / 3:
-// p_k = w_k (E + c c : Q + 3 c . j).
-template <bool HAVE_P>
-__device__ __forceinline__ void populations(double m0, double m, double u, double v, double pxx,
-                                            double pyy, double pxy, double p[9]) {
-  const double jx = m * u, jy = m * v;
-  double qxx, qyy, qxy;
-  if constexpr (HAVE_P) {
-    qxx = 4.5 * fma(jx, u, pxx);
-    qyy = 4.5 * fma(jy, v, pyy);
-    qxy = 9.0 * fma(jx, v, pxy);
-  } else {
-    qxx = 4.5 * (jx * u);
-    qyy = 4.5 * (jy * v);
-    qxy = 9.0 * (jx * v);
-  }
-  const double s = qxx + qyy;
-  const double e = fma(s, -1.0 / 3.0, m0);
-  const double ax = (e + qxx) * (1.0 / 9.0), ay = (e + qyy) * (1.0 / 9.0), d = e + s;
-  const double dp = (d + qxy) * (1.0 / 36.0), dm = (d - qxy) * (1.0 / 36.0);
-  const double jp = jx + jy, jm = jx - jy;
-  p[0] = e * (4.0 / 9.0);
-  p[1] = fma(jx, 1.0 / 3.0, ax);
-  p[3] = fma(jx, -1.0 / 3.0, ax);
-  p[2] = fma(jy, 1.0 / 3.0, ay);
-  p[4] = fma(jy, -1.0 / 3.0, ay);
-  p[5] = fma(jp, 1.0 / 12.0, dp);
-  p[7] = fma(jp, -1.0 / 12.0, dp);
-  p[8] = fma(jm, 1.0 / 12.0, dm);
-  p[6] = fma(jm, -1.0 / 12.0, dm);
-}
-
-// What three neighbouring source nodes of one row give to a node's pulled
-// sums: their total, the total of the two diagonals, and the difference
-// (eastward - westward) of the diagonals.
-struct Triple {
-  double n, p, d;
-};
-__device__ __forceinline__ Triple triple(double c, double w, double e) {
-  const double p = w + e;
-  return Triple{c + p, p, w - e};
-}
-
-// Registers of one level between two rows.
-struct Level {
-  // row awaiting its northern neighbours: pulled sums so far, phi sums of
-  // its own and the southern row, its centre tap
-  PullSums s;
-  double t1, t2, pc;
-  // the southern share of the row after it
-  Triple sf, sg;
-  double n1, n2;
-};
-
-struct Updated {
-  double rho, dT, u, v, pfxx, pfyy, pfxy, pgxx, pgyy, pgxy, phi;  // stored
-  double dT2, u2, v2;                                              // before the forces
-};
-
-// momentsPre .. collision of one node (see core_forward_t in bgk_mom.h for
-// the citations), on explicit fused multiply-adds; st, st2: sums of the nine
-// phi_prec taps and of their squares, pc the centre tap.
-struct StepC {
-  double crit_shift, two_over_tw, half_dt_st, gb, t_ref, inv_omega_f, omf1, omega_g, alpha3,
-      k_ratio;
-};
-
-template <typename R, bool EQF>
-__device__ __forceinline__ Updated update(const StepC& c, const PullSums& S, double st, double st2,
-                                          double pc) {
-  Updated o;
-  o.rho = S.rho;
-  o.dT2 = S.dT;
-  const double irho = rcp_nr(S.rho);
-  o.u2 = S.jx * irho;
-  o.v2 = S.jy * irho;
-  // sum_m ((1 +/- t_m)/2)^2 = (9 +/- 2 sum t + sum t^2) / 4
-  const double h = 9.0 + st2;
-  const double kp = 0.25 * fma(2.0, st, h), km = 0.25 * fma(-2.0, st, h);
-  const bool react = !((kp == 0.0 || pc == 1.0) && (km == 0.0 || pc == -1.0));
-  double rm = 0.5;
-  if (react) rm = 1.0 / (1.0 + exp((o.dT2 + c.crit_shift) * c.two_over_tw));
-  const double rp = 1.0 - rm;
-  const double kpr = kp * 0.0625 * rp, kmr = km * 0.0625 * rm;
-  o.phi = pc + fma(kpr, 1.0 - pc, -(kmr * (1.0 + pc)));
-  o.dT = fma(-c.half_dt_st, o.phi - pc, o.dT2);
-  const double T = kTcrit + o.dT;
-  const double a = 0.5 - 0.5 * o.phi;
-  const double fy = fma(S.rho * c.gb, (T - c.t_ref) * fma(0.5, o.phi, 1.0), -(o.v2 * a));
-  const double sc = irho * c.inv_omega_f;
-  o.u = fma(-(o.u2 * a), sc, o.u2);
-  o.v = fma(fy, sc, o.v2);
-  double omg1;
-  if (c.k_ratio == 1.0) {
-    omg1 = 1.0 - c.omega_g;
-  } else {
-    const double fl = fma(0.5, o.phi, 0.5);
-    omg1 = 1.0 - rcp_nr(fma(c.alpha3, fma(c.k_ratio, 1.0 - fl, fl), 0.5));
-  }
-  const double Tu = T * o.u, Tv = T * o.v;
-  const double g0 = fma(o.dT2, -kCs2, S.gxx), g1 = fma(o.dT2, -kCs2, S.gyy);
-  o.pgxx = (double)(R)(omg1 * fma(-Tu, o.u, g0));
-  o.pgyy = (double)(R)(omg1 * fma(-Tv, o.v, g1));
-  o.pgxy = (double)(R)(omg1 * fma(-Tu, o.v, S.gxy));
-  if constexpr (EQF) {
-    o.pfxx = o.pfyy = o.pfxy = 0.0;
-  } else {
-    const double ru = S.rho * o.u, rv = S.rho * o.v;
-    const double f0 = fma(S.rho, -kCs2, S.fxx), f1 = fma(S.rho, -kCs2, S.fyy);
-    o.pfxx = (double)(R)(c.omf1 * fma(-ru, o.u, f0));
-    o.pfyy = (double)(R)(c.omf1 * fma(-rv, o.v, f1));
-    o.pfxy = (double)(R)(c.omf1 * fma(-ru, o.v, S.fxy));
-  }
-  o.u = (double)(R)o.u;
-  o.v = (double)(R)o.v;
-  return o;
-}
-
 // The initial phi of the ghost columns 0 and Nx+1, which no step changes
 // (STEP_7/initialization.f90:15-26: liquid for i <= Nx/40).
 constexpr double kPhiWest = 1.0, kPhiEast = -1.0;
@@ -254,122 +132,6 @@ struct StreamArgs {
   double* probe_out;
   int probe_np;
 };
-
-// Feed row j (1..Ny, or Ny+1: nothing more comes) of one level: nd holds the
-// row's nodes, one per lane.  Gives the completed pulled sums and tap sums of
-// row j - 1.  i: this lane's column; has_w / has_e: the wave holds column 1
-// / Nx (uniform).
-//
-// BC_f type 4 and BC_g (STEP_7/BC_f.f90:62-68,101-107,125-136,181-192;
-// BC_g.f90:9-64): the lanes of the ghost columns 0 and Nx+1 carry rho = 0
-// (their f vanish) and the wall's temperature and velocity (their g are the
-// thermal ghosts); bounce-back adds a node's own opposite populations; rows 0
-// and Ny+1 of g and phi are rows 1 and Ny.
-template <bool EQF, bool EDGE>
-__device__ __forceinline__ void feed(Level& L, const NodeD& nd, int j, int ny, int i, int nx,
-                                     bool has_w, bool has_e, double frozen6, double frozen7,
-                                     PullSums* S, double* st, double* st2, double* pc) {
-  *S = L.s;
-  *st = L.t1;
-  *st2 = L.t2;
-  *pc = L.pc;
-  if (EDGE && j > ny) return;
-  double f[9], g[9];
-  populations<!EQF>(nd.rho, nd.rho, nd.u, nd.v, nd.pfxx, nd.pfyy, nd.pfxy, f);
-  populations<true>(nd.th, kTcrit + nd.th, nd.u, nd.v, nd.pgxx, nd.pgyy, nd.pgxy, g);
-  // row sums of the phi taps
-  const double pw = from_west(nd.phi), pe = from_east(nd.phi);
-  const double r1 = (pw + pe) + nd.phi;
-  const double r2 = fma(nd.phi, nd.phi, fma(pw, pw, pe * pe));
-  // northern sources of row j - 1
-  const Triple nf = triple(f[4], from_west(f[8]), from_east(f[7]));
-  const Triple ng = triple(g[4], from_west(g[8]), from_east(g[7]));
-  S->rho += nf.n;
-  S->jx += nf.d;
-  S->jy -= nf.n;
-  S->fxx += nf.p;
-  S->fyy += nf.n;
-  S->fxy -= nf.d;
-  S->dT += ng.n;
-  S->gxx += ng.p;
-  S->gyy += ng.n;
-  S->gxy -= ng.d;
-  *st += r1;
-  *st2 += r2;
-  // southern sources of row j + 1
-  const Triple sf = triple(f[2], from_west(f[5]), from_east(f[6]));
-  const Triple sg = triple(g[2], from_west(g[5]), from_east(g[6]));
-  if (EDGE && j == 1) {  // row 0: bounce-back, copied g and phi
-    const double f6 = i == nx ? frozen6 : f[8];
-    L.sf = triple(f[4], f[7], f6);
-    L.sg = sg;
-    L.n1 = r1;
-    L.n2 = r2;
-  }
-  // row j: southern share, then its own row's sources
-  {
-    const Triple cf = triple(f[0], from_west(f[1]), from_east(f[3]));
-    const Triple cg = triple(g[0], from_west(g[1]), from_east(g[3]));
-    L.s.rho = L.sf.n + cf.n;
-    L.s.jx = L.sf.d + cf.d;
-    L.s.jy = L.sf.n;
-    L.s.fxx = L.sf.p + cf.p;
-    L.s.fyy = L.sf.n;
-    L.s.fxy = L.sf.d;
-    L.s.dT = L.sg.n + cg.n;
-    L.s.gxx = L.sg.p + cg.p;
-    L.s.gyy = L.sg.n;
-    L.s.gxy = L.sg.d;
-    L.t1 = L.n1 + r1;
-    L.t2 = L.n2 + r2;
-    L.pc = nd.phi;
-  }
-  if (EDGE) {
-    if (j == ny) {  // row Ny+1: bounce-back, copied g and phi
-      const Triple v = triple(f[2], f[6], i == nx ? frozen7 : f[5]);
-      L.s.rho += v.n;
-      L.s.jx += v.d;
-      L.s.jy -= v.n;
-      L.s.fxx += v.p;
-      L.s.fyy += v.n;
-      L.s.fxy -= v.d;
-      L.s.dT += ng.n;
-      L.s.gxx += ng.p;
-      L.s.gyy += ng.n;
-      L.s.gxy -= ng.d;
-      L.t1 += r1;
-      L.t2 += r2;
-    }
-    if (has_w) {  // column 1: directions 1, 5, 8 bounce back
-      const bool on = i == 1;
-      const double a = on ? f[3] : 0.0;
-      const double b = on && j != 1 ? f[7] : 0.0;
-      const double d = on && j != ny ? f[6] : 0.0;
-      L.s.rho += a + b + d;
-      L.s.jx += a + b + d;
-      L.s.jy += b - d;
-      L.s.fxx += a + b + d;
-      L.s.fyy += b + d;
-      L.s.fxy += b - d;
-    }
-    if (has_e) {  // column Nx: directions 3, 6, 7 bounce back
-      const bool on = i == nx;
-      const double a = on ? f[1] : 0.0;
-      const double b = on && j != 1 ? f[8] : 0.0;
-      const double d = on && j != ny ? f[5] : 0.0;
-      L.s.rho += a + b + d;
-      L.s.jx -= a + b + d;
-      L.s.jy += b - d;
-      L.s.fxx += a + b + d;
-      L.s.fyy += b + d;
-      L.s.fxy += d - b;
-    }
-  }
-  L.sf = sf;
-  L.sg = sg;
-  L.n1 = r1;
-  L.n2 = r2;
-}
 
 // What the last launch of a call adds for row jc (1..Ny) completed by level t
 // of T: the halo as BC_f / BC_g leave it at the start of the last step, and
@@ -500,8 +262,11 @@ __device__ __forceinline__ void stream_strip(const StreamArgs& A, int i0, int j0
       }
       PullSums S;
       double st, st2, pc;
-      feed<EQF, EDGE>(L[t], nd, j, ny, i, nx, has_w, has_e, A.frozen6, A.frozen7, &S, &st, &st2,
-                      &pc);
+      double f[9], g[9];
+      populations<!EQF>(nd.rho, nd.rho, nd.u, nd.v, nd.pfxx, nd.pfyy, nd.pfxy, f);
+      populations<true>(nd.th, kTcrit + nd.th, nd.u, nd.v, nd.pgxx, nd.pgyy, nd.pgxy, g);
+      feed<EDGE>(L[t], f, g, nd.phi, j, ny, i, nx, has_w, has_e, A.frozen6, A.frozen7, &S, &st,
+                 &st2, &pc);
       o = update<R, EQF>(A.c, S, st, st2, pc);
       tav = kTcrit + (o.dT + o.dT2) * 0.5;
       const int jd = j - 1 - j0;  // (rows outside the strip are its neighbours')
@@ -546,21 +311,6 @@ __global__ __launch_bounds__(kLanes, 2) void k_stream_mom(StreamArgs A) {
     stream_strip<T, R, EQF, true, MODE>(A, i0, j0, j1, i, i0 - T <= 1, i0 - T + kLanes - 1 >= A.nx);
   else
     stream_strip<T, R, EQF, false, MODE>(A, i0, j0, j1, i, false, false);
-}
-
-StepC step_constants(const Consts& c) {
-  StepC s;
-  s.crit_shift = c.crit_shift;
-  s.two_over_tw = c.two_over_tw;
-  s.half_dt_st = 0.5 * c.dt_st;
-  s.gb = c.grav * c.beta;
-  s.t_ref = c.t_ref;
-  s.inv_omega_f = c.inv_omega_f;
-  s.omf1 = 1.0 - c.omega_f;
-  s.omega_g = c.omega_g;
-  s.alpha3 = 3.0 * c.alpha_l;
-  s.k_ratio = c.k_ratio;
-  return s;
 }
 
 template <int T, typename R, bool EQF>
