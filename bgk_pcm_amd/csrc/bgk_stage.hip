@@ -6,6 +6,8 @@
 // serves every boundary type of the reference and is the path bgk_step takes
 // when the walls are not all no-slip.  Compiled with -ffp-contract=off: the
 // FP64 results equal the reference's bit for bit.
+#include <algorithm>
+
 #include "bgk_internal.h"
 
 namespace bgk {
@@ -23,6 +25,26 @@ inline Pops64 pops(double* const* p) {
   Pops64 r;
   for (int k = 0; k < 9; ++k) r.p[k].base = p[k];
   return r;
+}
+
+// pair view: plane k holds (f_k, g_k) per node.  One 16-byte access serves both
+// members; as two stride-2 accesses each cache line was requested twice.  A step
+// by subroutines, us, before and after pairs, merged boundary launches and no
+// copy of phi: 64^2 40 / 32, 512^2 90 / 79, 1024 x 512 151 / 130, 2048 x 1024
+// 610 / 530.
+inline Pairs64 pairs(double* const* fplanes) {
+  Pairs64 r;
+  for (int k = 0; k < 9; ++k) r.p[k] = reinterpret_cast<double2*>(fplanes[k]);
+  return r;
+}
+__device__ __forceinline__ void load_pairs(const Pairs64& p, int64_t q, double a[9],
+                                           double b[9]) {
+#pragma unroll
+  for (int k = 0; k < 9; ++k) {
+    const double2 v = p.p[k][q];
+    a[k] = v.x;
+    b[k] = v.y;
+  }
 }
 
 constexpr int TX = 64, TY = 4;
@@ -60,12 +82,16 @@ __global__ void k_initialization(Pops64 f, Pops64 g, Macro m, double* phi, doubl
   phip[q] = s0.phi;
 }
 
+// Boundary types of the four sides (input.dat).
+struct Walls {
+  int west, east, north, south;
+};
+
 // ----------------------------------------------------------------------- BC_f
-// West and east sides, one thread per row j = 0..Ny+1 (STEP_7/BC_f.f90:9-104).
-__global__ void k_bc_f_we(Pops64 F, Macro m, Consts c, Geom gm, int wbc, int ebc) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  const int nx = gm.nx, ny = gm.ny;
-  if (j > ny + 1) return;
+// West and east sides, row j = 0..Ny+1 (STEP_7/BC_f.f90:9-104).
+__device__ __forceinline__ void bc_f_we(const Pops64& F, const Macro& m, const Consts& c,
+                                        const Geom& gm, const Walls& w, int j) {
+  const int nx = gm.nx, ny = gm.ny, wbc = w.west, ebc = w.east;
   const int64_t P = gm.pitch;
   auto at = [&](int i, int jj) { return (int64_t)jj * P + i; };
   const Strided2<double>* f = F.p;
@@ -134,12 +160,11 @@ __global__ void k_bc_f_we(Pops64 F, Macro m, Consts c, Geom gm, int wbc, int ebc
   }
 }
 
-// North and south sides, one thread per column i = 0..Nx+1
-// (STEP_7/BC_f.f90:108-196); runs after k_bc_f_we.
-__global__ void k_bc_f_ns(Pops64 F, Macro m, Consts c, Geom gm, int nbc, int sbc) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int nx = gm.nx, ny = gm.ny;
-  if (i > nx + 1) return;
+// North and south sides, column i = 0..Nx+1 (STEP_7/BC_f.f90:108-196), after
+// bc_f_we.
+__device__ __forceinline__ void bc_f_ns(const Pops64& F, const Macro& m, const Consts& c,
+                                        const Geom& gm, const Walls& w, int i) {
+  const int nx = gm.nx, ny = gm.ny, nbc = w.north, sbc = w.south;
   const int64_t P = gm.pitch;
   auto at = [&](int ii, int jj) { return (int64_t)jj * P + ii; };
   const Strided2<double>* f = F.p;
@@ -196,11 +221,10 @@ __global__ void k_bc_f_ns(Pops64 F, Macro m, Consts c, Geom gm, int nbc, int sbc
 }
 
 // ----------------------------------------------------------------------- BC_g
-// West and east, rows j = 1..Ny (STEP_7/BC_g.f90:9-31).
-__global__ void k_bc_g_we(Pops64 G, Macro m, Consts c, Geom gm) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  const int nx = gm.nx, ny = gm.ny;
-  if (j > ny) return;
+// West and east, row j = 1..Ny (STEP_7/BC_g.f90:9-31).
+__device__ __forceinline__ void bc_g_we(const Pops64& G, const Macro& m, const Consts& c,
+                                        const Geom& gm, int j) {
+  const int nx = gm.nx;
   const int64_t P = gm.pitch;
   auto at = [&](int ii, int jj) { return (int64_t)jj * P + ii; };
   const Strided2<double>* g = G.p;
@@ -224,11 +248,11 @@ __global__ void k_bc_g_we(Pops64 G, Macro m, Consts c, Geom gm) {
   }
 }
 
-// North and south zero-gradient copies, i = 0..Nx+1 (STEP_7/BC_g.f90:36-64).
-__global__ void k_bc_g_ns(Pops64 G, Macro m, double* phi, Geom gm) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// North and south zero-gradient copies, column i = 0..Nx+1
+// (STEP_7/BC_g.f90:36-64), after bc_g_we.
+__device__ __forceinline__ void bc_g_ns(const Pops64& G, const Macro& m, double* phi,
+                                        const Geom& gm, int i) {
   const int ny = gm.ny;
-  if (i > gm.nx + 1) return;
   const int64_t P = gm.pitch;
   const int64_t qn = (int64_t)ny * P + i, qn1 = (int64_t)(ny + 1) * P + i;
   const int64_t q1 = P + i, q0 = i;
@@ -242,35 +266,61 @@ __global__ void k_bc_g_ns(Pops64 G, Macro m, double* phi, Geom gm) {
   phi[q0] = phi[q1];
 }
 
+// BC_f and/or BC_g.  The sides depend on each other in the reference's order
+// (west and east, then north and south; f before g).  PHASE 0: all of it by one
+// workgroup, which waits between the four parts; 1..4: one part, one thread per
+// node, for lattices whose sides one workgroup would walk too slowly.  What
+// bounds a part is the latency of a launch or of a few dependent accesses, so
+// one launch of one workgroup beats four.
+constexpr int kBcThreads = 1024;
+struct BcArgs {
+  Pops64 F, G;
+  Macro m;
+  double* phi;
+  Consts c;
+  Geom gm;
+  Walls w;
+  int do_f, do_g;
+};
+template <int PHASE>
+__global__ __launch_bounds__(kBcThreads) void k_bc(BcArgs a) {
+  const int nx = a.gm.nx, ny = a.gm.ny;
+  const int t0 = blockIdx.x * blockDim.x + threadIdx.x;
+  const int step = PHASE == 0 ? kBcThreads : nx + ny + 4;  // (1..4: one node each)
+  if ((PHASE == 0 && a.do_f) || PHASE == 1)
+    for (int j = t0; j <= ny + 1; j += step) bc_f_we(a.F, a.m, a.c, a.gm, a.w, j);
+  if (PHASE == 0 && a.do_f) __syncthreads();
+  if ((PHASE == 0 && a.do_f) || PHASE == 2)
+    for (int i = t0; i <= nx + 1; i += step) bc_f_ns(a.F, a.m, a.c, a.gm, a.w, i);
+  if (PHASE == 0 && a.do_f && a.do_g) __syncthreads();
+  if ((PHASE == 0 && a.do_g) || PHASE == 3)
+    for (int j = t0 + 1; j <= ny; j += step) bc_g_we(a.G, a.m, a.c, a.gm, j);
+  if (PHASE == 0 && a.do_g) __syncthreads();
+  if ((PHASE == 0 && a.do_g) || PHASE == 4)
+    for (int i = t0; i <= nx + 1; i += step) bc_g_ns(a.G, a.m, a.phi, a.gm, i);
+}
+
 // ------------------------------------------------------------------ streaming
 // Pull of f and g into fp and gp, STEP_7/streaming.f90:5-27.
-__global__ void k_streaming(Pops64 f, Pops64 fp, Pops64 g, Pops64 gp, Geom gm) {
+__global__ void k_streaming(Pairs64 f, Pairs64 fp, Geom gm) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
   const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
   if (i > gm.nx || j > gm.ny) return;
   const int64_t P = gm.pitch;
   const int64_t q = (int64_t)j * P + i;
 #pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    const int64_t s = q - CX[k] - (int64_t)CY[k] * P;
-    fp.p[k][q] = f.p[k][s];
-    gp.p[k][q] = g.p[k][s];
-  }
+  for (int k = 0; k < 9; ++k) fp.p[k][q] = f.p[k][q - CX[k] - (int64_t)CY[k] * P];
 }
 
 // ----------------------------------------------------------------- momentsPre
 // STEP_7/momentsPre.f90:8-21.
-__global__ void k_moments_pre(Pops64 fp, Pops64 gp, Macro m, Geom gm) {
+__global__ void k_moments_pre(Pairs64 fp, Macro m, Geom gm) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
   const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
   if (i > gm.nx || j > gm.ny) return;
   const int64_t q = (int64_t)j * gm.pitch + i;
   double a[9], b[9];
-#pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    a[k] = fp.p[k][q];
-    b[k] = gp.p[k][q];
-  }
+  load_pairs(fp, q, a, b);
   const double r = a[0] + a[1] + a[2] + a[3] + a[4] + a[5] + a[6] + a[7] + a[8];
   const double t = b[0] + b[1] + b[2] + b[3] + b[4] + b[5] + b[6] + b[7] + b[8];
   const double irho = 1.0 / r;
@@ -287,15 +337,20 @@ __global__ void k_moments_pre(Pops64 fp, Pops64 gp, Macro m, Geom gm) {
 }
 
 // ---------------------------------------------------------------- phase_field
-// Interior update from phi_prec (STEP_7/phase_field.f90:21-55); the copy
-// phi_prec(:,:) = phi(:,:) of :19 is a device copy before the launch.
+// STEP_7/phase_field.f90:19-55.  The copy phi_prec(:,:) = phi(:,:) of :19 is the
+// exchange of the two planes: pp holds the old phi, and the new one goes to the
+// other plane, with the halo nodes (which the update leaves) copied along.
 __global__ void k_phase_field(double* phi, const double* pp, const double* T, Consts c,
                               Geom gm) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
-  if (i > gm.nx || j > gm.ny) return;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int j = blockIdx.y * blockDim.y + threadIdx.y;
+  if (i > gm.nx + 1 || j > gm.ny + 1) return;
   const int64_t P = gm.pitch;
   const int64_t q = (int64_t)j * P + i;
+  if (i < 1 || i > gm.nx || j < 1 || j > gm.ny) {
+    phi[q] = pp[q];
+    return;
+  }
   const double tap[9] = {pp[q],         pp[q + 1],     pp[q + P],     pp[q - 1], pp[q - P],
                          pp[q + 1 + P], pp[q - 1 + P], pp[q - 1 - P], pp[q + 1 - P]};
   phi[q] = phase_update(c, T[q], tap);
@@ -323,39 +378,30 @@ __global__ void k_forces(Macro m, const double* phi, const double* pp, Consts c,
 // ------------------------------------------------------------------ collision
 // STEP_7/collision.f90:14-152.
 template <bool STEP7>
-__global__ void k_collision(Pops64 fp, Pops64 gp, Pops64 f, Pops64 g, Macro m,
-                            const double* __restrict__ phi, Consts c, Geom gm) {
+__global__ void k_collision(Pairs64 fp, Pairs64 f, Macro m, const double* __restrict__ phi,
+                            Consts c, Geom gm) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
   const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
   if (i > gm.nx || j > gm.ny) return;
   const int64_t q = (int64_t)j * gm.pitch + i;
   const double u = m.u[q], v = m.v[q];
-  double pop[9], out[9];
+  double a[9], b[9], fo[9], go[9];
+  load_pairs(fp, q, a, b);
+  regularised_bgk<STEP7>(c, c.omega_f, m.rho[q], u, v, a, fo);
+  regularised_bgk<STEP7>(c, omega_g_at(c, phi[q]), m.T[q], u, v, b, go);
 #pragma unroll
-  for (int k = 0; k < 9; ++k) pop[k] = fp.p[k][q];
-  regularised_bgk<STEP7>(c, c.omega_f, m.rho[q], u, v, pop, out);
-#pragma unroll
-  for (int k = 0; k < 9; ++k) f.p[k][q] = out[k];
-#pragma unroll
-  for (int k = 0; k < 9; ++k) pop[k] = gp.p[k][q];
-  regularised_bgk<STEP7>(c, omega_g_at(c, phi[q]), m.T[q], u, v, pop, out);
-#pragma unroll
-  for (int k = 0; k < 9; ++k) g.p[k][q] = out[k];
+  for (int k = 0; k < 9; ++k) f.p[k][q] = make_double2(fo[k], go[k]);
 }
 
 // -------------------------------------------------------------------- moments
 // STEP_7/moments.f90:11-25.
-__global__ void k_moments(Pops64 f, Pops64 g, Macro m, Geom gm) {
+__global__ void k_moments(Pairs64 f, Macro m, Geom gm) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
   const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
   if (i > gm.nx || j > gm.ny) return;
   const int64_t q = (int64_t)j * gm.pitch + i;
   double a[9], b[9];
-#pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    a[k] = f.p[k][q];
-    b[k] = g.p[k][q];
-  }
+  load_pairs(f, q, a, b);
   const double r = a[0] + a[1] + a[2] + a[3] + a[4] + a[5] + a[6] + a[7] + a[8];
   const double irho = 1.0 / r;
   const double tt = b[0] + b[1] + b[2] + b[3] + b[4] + b[5] + b[6] + b[7] + b[8];
@@ -383,46 +429,51 @@ hipError_t launch_initialization(bgk_handle* h) {
   return hipGetLastError();
 }
 
-hipError_t launch_bc_f(bgk_handle* h) {
+hipError_t launch_bc(bgk_handle* h, bool do_f, bool do_g) {
   const Geom& g = h->geom;
-  hipLaunchKernelGGL(k_bc_f_we, dim3(blocks1d(g.ny + 2, 256)), dim3(256), 0, h->stream,
-                     pops(h->f[h->cur]), macro_of(h), h->c, g, h->prm.west_bc, h->prm.east_bc);
-  hipLaunchKernelGGL(k_bc_f_ns, dim3(blocks1d(g.nx + 2, 256)), dim3(256), 0, h->stream,
-                     pops(h->f[h->cur]), macro_of(h), h->c, g, h->prm.north_bc,
-                     h->prm.south_bc);
+  BcArgs a{pops(h->f[h->cur]), pops(h->g[h->cur]), macro_of(h), h->phi[h->pc], h->c, g,
+           Walls{h->prm.west_bc, h->prm.east_bc, h->prm.north_bc, h->prm.south_bc},
+           do_f ? 1 : 0, do_g ? 1 : 0};
+  // one workgroup up to four rounds of its threads on a side
+  if (std::max(g.nx, g.ny) + 2 <= 4 * kBcThreads) {
+    hipLaunchKernelGGL(k_bc<0>, dim3(1), dim3(kBcThreads), 0, h->stream, a);
+    return hipGetLastError();
+  }
+  const dim3 we(blocks1d(g.ny + 2, 256)), ns(blocks1d(g.nx + 2, 256));
+  if (do_f) {
+    hipLaunchKernelGGL(k_bc<1>, we, dim3(256), 0, h->stream, a);
+    hipLaunchKernelGGL(k_bc<2>, ns, dim3(256), 0, h->stream, a);
+  }
+  if (do_g) {
+    hipLaunchKernelGGL(k_bc<3>, we, dim3(256), 0, h->stream, a);
+    hipLaunchKernelGGL(k_bc<4>, ns, dim3(256), 0, h->stream, a);
+  }
   return hipGetLastError();
 }
 
-hipError_t launch_bc_g(bgk_handle* h) {
-  const Geom& g = h->geom;
-  hipLaunchKernelGGL(k_bc_g_we, dim3(blocks1d(g.ny, 256)), dim3(256), 0, h->stream,
-                     pops(h->g[h->cur]), macro_of(h), h->c, g);
-  hipLaunchKernelGGL(k_bc_g_ns, dim3(blocks1d(g.nx + 2, 256)), dim3(256), 0, h->stream,
-                     pops(h->g[h->cur]), macro_of(h), h->phi[h->pc], g);
-  return hipGetLastError();
-}
+hipError_t launch_bc_f(bgk_handle* h) { return launch_bc(h, true, false); }
+hipError_t launch_bc_g(bgk_handle* h) { return launch_bc(h, false, true); }
 
 hipError_t launch_streaming(bgk_handle* h) {
   hipLaunchKernelGGL(k_streaming, interior_grid(h->geom), dim3(TX, TY), 0, h->stream,
-                     pops(h->f[h->cur]), pops(h->f[1 - h->cur]), pops(h->g[h->cur]),
-                     pops(h->g[1 - h->cur]), h->geom);
+                     pairs(h->f[h->cur]), pairs(h->f[1 - h->cur]), h->geom);
   return hipGetLastError();
 }
 
 hipError_t launch_moments_pre(bgk_handle* h) {
   hipLaunchKernelGGL(k_moments_pre, interior_grid(h->geom), dim3(TX, TY), 0, h->stream,
-                     pops(h->f[1 - h->cur]), pops(h->g[1 - h->cur]), macro_of(h), h->geom);
+                     pairs(h->f[1 - h->cur]), macro_of(h), h->geom);
   return hipGetLastError();
 }
 
 hipError_t launch_phase_field(bgk_handle* h) {
-  const size_t bytes = (size_t)h->plane_elems * sizeof(double);
-  hipError_t e = hipMemcpyAsync(h->phi[1 - h->pc], h->phi[h->pc], bytes,
-                                hipMemcpyDeviceToDevice, h->stream);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_phase_field, interior_grid(h->geom), dim3(TX, TY), 0, h->stream,
-                     h->phi[h->pc], h->phi[1 - h->pc], h->T, h->c, h->geom);
-  return hipGetLastError();
+  const Geom& g = h->geom;
+  const dim3 grd((unsigned)((g.nx + 2 + TX - 1) / TX), (unsigned)((g.ny + 2 + TY - 1) / TY));
+  hipLaunchKernelGGL(k_phase_field, grd, dim3(TX, TY), 0, h->stream, h->phi[1 - h->pc],
+                     h->phi[h->pc], h->T, h->c, g);
+  const hipError_t e = hipGetLastError();
+  if (e == hipSuccess) h->pc = 1 - h->pc;
+  return e;
 }
 
 hipError_t launch_forces(bgk_handle* h) {
@@ -434,18 +485,18 @@ hipError_t launch_forces(bgk_handle* h) {
 hipError_t launch_collision(bgk_handle* h) {
   if (h->prm.rounding == BGK_ROUND_STEP7)
     hipLaunchKernelGGL(k_collision<true>, interior_grid(h->geom), dim3(TX, TY), 0, h->stream,
-                       pops(h->f[1 - h->cur]), pops(h->g[1 - h->cur]), pops(h->f[h->cur]),
-                       pops(h->g[h->cur]), macro_of(h), h->phi[h->pc], h->c, h->geom);
+                       pairs(h->f[1 - h->cur]), pairs(h->f[h->cur]), macro_of(h), h->phi[h->pc],
+                       h->c, h->geom);
   else
     hipLaunchKernelGGL(k_collision<false>, interior_grid(h->geom), dim3(TX, TY), 0, h->stream,
-                       pops(h->f[1 - h->cur]), pops(h->g[1 - h->cur]), pops(h->f[h->cur]),
-                       pops(h->g[h->cur]), macro_of(h), h->phi[h->pc], h->c, h->geom);
+                       pairs(h->f[1 - h->cur]), pairs(h->f[h->cur]), macro_of(h), h->phi[h->pc],
+                       h->c, h->geom);
   return hipGetLastError();
 }
 
 hipError_t launch_moments(bgk_handle* h) {
   hipLaunchKernelGGL(k_moments, interior_grid(h->geom), dim3(TX, TY), 0, h->stream,
-                     pops(h->f[h->cur]), pops(h->g[h->cur]), macro_of(h), h->geom);
+                     pairs(h->f[h->cur]), macro_of(h), h->geom);
   return hipGetLastError();
 }
 
