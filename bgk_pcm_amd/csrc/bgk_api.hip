@@ -278,11 +278,20 @@ int run_stage(bgk_handle* h, hipError_t (*fn)(bgk_handle*), const char* name) {
   return launched(fn(h), name);
 }
 
-int copy_small_back(bgk_handle* h, double* out, int n) {
-  HIP_TRY(hipMemcpyAsync(out, h->small, (size_t)n * sizeof(double), hipMemcpyDeviceToHost,
-                         h->stream),
-          "hipMemcpyAsync(D2H)");
+// The n results of a reduction launched by `fn`, which its last kernel writes
+// where it is told: into pinned memory, or (none to be had) through a copy.
+int reduce_to_host(bgk_handle* h, hipError_t (*fn)(bgk_handle*, double*), const char* name,
+                   double* out, int n) {
+  bgk::Staging s;
+  double* const pinned = static_cast<double*>(s.ptr());
+  int rc = launched(fn(h, pinned ? pinned : h->small), name);
+  if (rc) return rc;
+  if (!pinned)
+    HIP_TRY(hipMemcpyAsync(out, h->small, (size_t)n * sizeof(double), hipMemcpyDeviceToHost,
+                           h->stream),
+            "hipMemcpyAsync(D2H)");
   HIP_TRY(hipStreamSynchronize(h->stream), "hipStreamSynchronize");
+  if (pinned) std::memcpy(out, pinned, (size_t)n * sizeof(double));
   return BGK_OK;
 }
 
@@ -429,6 +438,7 @@ int bgk_create(const bgk_params* p, bgk_handle** out) {
     delete h;
     return hip_fail(e, "hipMemset");
   }
+  bgk::staging_open();
   *out = h;
   return BGK_OK;
 }
@@ -438,6 +448,7 @@ int bgk_destroy(bgk_handle* h) {
   (void)hipSetDevice(h->device);
   hipError_t e1 = hipStreamSynchronize(h->stream);
   bgk::adj_free(h);
+  bgk::staging_close();
   hipError_t e2 = hipStreamDestroy(h->own_stream);
   hipError_t e3 = hipFree(h->pool);
   delete h;
@@ -523,11 +534,19 @@ int bgk_download(bgk_handle* h, int32_t field, double* dst, int64_t ld) {
   FieldRef r;
   if ((rc = resolve(h, field, &r))) return rc;
   const double* src = r.d64;
+  int stride = r.stride;
   if (r.d32) {
     HIP_TRY(bgk::launch_dev_to_f64(h, r.d32, 2, h->tmp, r.base, r.rho_table), "dev_to_f64");
     src = h->tmp;
-  } else if (r.stride != 1) {
-    HIP_TRY(bgk::launch_copy64(h, r.d64, r.stride, h->tmp, 1), "copy64");
+    stride = 1;
+  }
+  hipError_t e = hipSuccess;
+  if (bgk::download_staged(h, src, stride, dst, ld, &e)) {
+    if (e != hipSuccess) return hip_fail(e, "download");
+    return BGK_OK;
+  }
+  if (stride != 1) {
+    HIP_TRY(bgk::launch_copy64(h, src, stride, h->tmp, 1), "copy64");
     src = h->tmp;
   }
   HIP_TRY(hipMemcpy2DAsync(dst, (size_t)ld * sizeof(double), src, (size_t)h->pitch * sizeof(double),
@@ -596,9 +615,8 @@ int bgk_field_check(bgk_handle* h, double out[3]) {
   int rc = check_handle(h);
   if (rc) return rc;
   if (!out) return fail(BGK_E_INVALID, "null output");
-  if ((rc = launched(bgk::launch_field_sums(h, h->small), "field sums"))) return rc;
   double s[3];
-  if ((rc = copy_small_back(h, s, 3))) return rc;
+  if ((rc = reduce_to_host(h, bgk::launch_field_sums, "field sums", s, 3))) return rc;
   const double nn = nxny_as_reference(h);
   out[0] = s[0] / nn;
   out[1] = s[1] / nn;
@@ -633,9 +651,8 @@ int bgk_mass_check(bgk_handle* h, double out[3]) {
   int rc = check_handle(h);
   if (rc) return rc;
   if (!out) return fail(BGK_E_INVALID, "null output");
-  if ((rc = launched(bgk::launch_field_sums(h, h->small), "field sums"))) return rc;
   double s[3];
-  if ((rc = copy_small_back(h, s, 3))) return rc;
+  if ((rc = reduce_to_host(h, bgk::launch_field_sums, "field sums", s, 3))) return rc;
   const double nn = nxny_as_reference(h);
   out[0] = (nn * h->prm.rho0 - s[0]) * 100.0 / (nn * h->prm.rho0);
   out[1] = s[0] / nn;
@@ -649,8 +666,7 @@ int bgk_diag_sums(bgk_handle* h, double out[4]) {
   if (!out) return fail(BGK_E_INVALID, "null output");
   if (h->nx < 2)
     return fail(BGK_E_UNSUPPORTED, "diag reads T(1..3,j): needs Nx >= 2 (Nx=%d)", h->nx);
-  if ((rc = launched(bgk::launch_diag_sums(h, h->small), "diag sums"))) return rc;
-  if ((rc = copy_small_back(h, out, 4))) return rc;
+  if ((rc = reduce_to_host(h, bgk::launch_diag_sums, "diag sums", out, 4))) return rc;
   return nonfinite_check(out, 2, "diag sums");
 }
 
@@ -666,12 +682,32 @@ int bgk_gather(bgk_handle* h, int32_t field, int32_t n, const int32_t* i, const 
       return fail(BGK_E_INVALID, "node (%d,%d) outside 0..%d x 0..%d", i[k], j[k], h->nx + 1,
                   h->ny + 1);
   const double* plane = r.d64;
+  int stride = r.stride;
   if (r.d32) {
     HIP_TRY(bgk::launch_dev_to_f64(h, r.d32, 2, h->tmp, r.base, r.rho_table), "dev_to_f64");
     plane = h->tmp;
-  } else if (r.stride != 1) {
-    HIP_TRY(bgk::launch_copy64(h, r.d64, r.stride, h->tmp, 1), "copy64");
-    plane = h->tmp;
+    stride = 1;
+  }
+  {
+    // through pinned memory, which the kernel reads and writes: the pairs
+    // behind the results
+    bgk::Staging s;
+    if (s.ptr()) {
+      const int64_t chunk = (int64_t)(bgk::Staging::bytes() / (2 * sizeof(double)));
+      double* const res = static_cast<double*>(s.ptr());
+      int32_t* const ij = reinterpret_cast<int32_t*>(res + chunk);
+      for (int64_t base = 0; base < n; base += chunk) {
+        const int m = (int)std::min<int64_t>(chunk, n - base);
+        for (int k = 0; k < m; ++k) {
+          ij[2 * k] = i[base + k];
+          ij[2 * k + 1] = j[base + k];
+        }
+        HIP_TRY(bgk::launch_gather(h, plane, stride, m, ij, res), "gather");
+        HIP_TRY(hipStreamSynchronize(h->stream), "hipStreamSynchronize");
+        std::memcpy(out + base, res, (size_t)m * sizeof(double));
+      }
+      return BGK_OK;
+    }
   }
   // small buffer: first half outputs, second half (i,j) pairs
   const int64_t chunk = h->small_elems / 2;
@@ -686,7 +722,7 @@ int bgk_gather(bgk_handle* h, int32_t field, int32_t n, const int32_t* i, const 
     }
     hipError_t e = hipMemcpyAsync(ij_dev, pairs, (size_t)m * 2 * sizeof(int32_t),
                                   hipMemcpyHostToDevice, h->stream);
-    if (e == hipSuccess) e = bgk::launch_gather(h, plane, m, ij_dev, h->small);
+    if (e == hipSuccess) e = bgk::launch_gather(h, plane, stride, m, ij_dev, h->small);
     if (e == hipSuccess)
       e = hipMemcpyAsync(out + base, h->small, (size_t)m * sizeof(double), hipMemcpyDeviceToHost,
                          h->stream);

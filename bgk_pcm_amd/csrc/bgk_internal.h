@@ -146,8 +146,8 @@ hipError_t launch_initialization32(bgk_handle* h);
 hipError_t launch_field_sums(bgk_handle* h, double* out_dev);
 // diag sums (bgk_diag_sums layout)
 hipError_t launch_diag_sums(bgk_handle* h, double* out_dev);
-hipError_t launch_gather(bgk_handle* h, const double* plane, int n, const int32_t* ij_dev,
-                         double* out_dev);
+hipError_t launch_gather(bgk_handle* h, const double* plane, int stride, int n,
+                         const int32_t* ij_dev, double* out_dev);
 
 int reduce_partial_count(const bgk_handle* h);
 // field_check's sums over the interior of three caller-owned planes, with the
@@ -156,6 +156,28 @@ int reduce_partial_count(const bgk_handle* h);
 hipError_t field_sums_planes(const double* a, const double* b, const double* c3, const Geom& g,
                              hipStream_t stream, double out_host[3]);
 int max_scratch_devices();
+
+// ---- results to the host (bgk_transfer.hip)
+// every handle opens the staging at its creation and closes it at its end
+void staging_open();
+void staging_close();
+// a pinned, mapped buffer of bytes() bytes for one call; ptr() null: none to be had
+class Staging {
+ public:
+  Staging();
+  ~Staging();
+  Staging(const Staging&) = delete;
+  Staging& operator=(const Staging&) = delete;
+  void* ptr() const { return p_; }
+  static size_t bytes();
+
+ private:
+  void* p_;
+};
+// copies an FP64 plane (element stride `stride`) to the host array and waits;
+// false: no staging memory, nothing done
+bool download_staged(bgk_handle* h, const double* src, int stride, double* dst, int64_t ld,
+                     hipError_t* err);
 
 // ---- adjoint (bgk_adjoint.hip), FP64 moment handles
 // nsnap > 0: binomial checkpointing with nsnap snapshot slots; else the

@@ -134,11 +134,11 @@ __global__ __launch_bounds__(RB) void k_final(const CSum* __restrict__ part, int
     for (int k = 0; k < nk; ++k) out[k] = acc[k].s + acc[k].c;
 }
 
-__global__ void k_gather(const double* __restrict__ plane, int64_t pitch, int n,
+__global__ void k_gather(const double* __restrict__ plane, int stride, int64_t pitch, int n,
                          const int32_t* __restrict__ ij, double* __restrict__ out) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
-  out[t] = plane[(int64_t)ij[2 * t + 1] * pitch + ij[2 * t]];
+  out[t] = plane[((int64_t)ij[2 * t + 1] * pitch + ij[2 * t]) * stride];
 }
 
 inline int nparts(const Geom& g) { return g.ny < MAX_PARTS ? g.ny : MAX_PARTS; }
@@ -213,10 +213,10 @@ hipError_t launch_diag_sums(bgk_handle* h, double* out_dev) {
   return hipGetLastError();
 }
 
-hipError_t launch_gather(bgk_handle* h, const double* plane, int n, const int32_t* ij_dev,
-                         double* out_dev) {
+hipError_t launch_gather(bgk_handle* h, const double* plane, int stride, int n,
+                         const int32_t* ij_dev, double* out_dev) {
   hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream,
-                     plane, h->geom.pitch, n, ij_dev, out_dev);
+                     plane, stride, h->geom.pitch, n, ij_dev, out_dev);
   return hipGetLastError();
 }
 
