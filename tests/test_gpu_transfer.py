@@ -48,7 +48,8 @@ def test_two_threads_with_a_handle_each():
     def work(seed):
         p = Params(nx=900, ny=800)
         ext = dict(EXT, noise_seed=seed)
-        want = Oracle(p, **ext).field("T").copy()
+        o = Oracle(p, **ext)  # (owns the memory its fields are views of)
+        want = o.field("T").copy()
         with Lattice(p, **ext) as lat:
             for _ in range(5):
                 if not np.array_equal(lat.download("T"), want) or \
