@@ -593,15 +593,8 @@ int bgk_step(bgk_handle* h, int32_t nsteps) {
   if ((rc = need_fp64(h, "bgk_step with these boundary types"))) return rc;
   h->te_ok = false;
   for (int s = 0; s < nsteps; ++s) {
-    hipError_t e;
-    if ((e = bgk::launch_bc_f(h)) != hipSuccess) return hip_fail(e, "BC_f");
-    if ((e = bgk::launch_bc_g(h)) != hipSuccess) return hip_fail(e, "BC_g");
-    if ((e = bgk::launch_streaming(h)) != hipSuccess) return hip_fail(e, "streaming");
-    if ((e = bgk::launch_moments_pre(h)) != hipSuccess) return hip_fail(e, "momentsPre");
-    if ((e = bgk::launch_phase_field(h)) != hipSuccess) return hip_fail(e, "phase_field");
-    if ((e = bgk::launch_forces(h)) != hipSuccess) return hip_fail(e, "forces");
-    if ((e = bgk::launch_collision(h)) != hipSuccess) return hip_fail(e, "collision");
-    if ((e = bgk::launch_moments(h)) != hipSuccess) return hip_fail(e, "moments");
+    const hipError_t e = bgk::launch_general_step64(h, s == nsteps - 1);
+    if (e != hipSuccess) return hip_fail(e, "step");
   }
   return BGK_OK;
 }

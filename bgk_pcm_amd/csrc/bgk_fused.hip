@@ -25,7 +25,7 @@
 //  * the halo of rho, T, u, v and phi after a step holds what BC_f/BC_g
 //    wrote at the start of that step, i.e. previous-step values; the edge
 //    nodes write them so a download sees the reference's full arrays.
-#include "bgk_internal.h"
+#include "bgk_pop64.h"
 
 namespace bgk {
 namespace {
@@ -97,54 +97,20 @@ __global__ __launch_bounds__(TILE_W) void k_fused64(Pairs64 A, Pairs64 B,
     }
   }
 
-  // ---- momentsPre (STEP_7/momentsPre.f90:8-21)
-  const double rho = fp[0] + fp[1] + fp[2] + fp[3] + fp[4] + fp[5] + fp[6] + fp[7] + fp[8];
-  double T = gp[0] + gp[1] + gp[2] + gp[3] + gp[4] + gp[5] + gp[6] + gp[7] + gp[8];
-  double u, v;
-  {
-    const double irho = 1.0 / rho;
-    u = irho * (fp[1] - fp[3] + fp[5] - fp[6] - fp[7] + fp[8]);
-    v = irho * (fp[2] - fp[4] + fp[5] + fp[6] - fp[7] - fp[8]);
-  }
-  const double T2 = T, u2 = u, v2 = v;
-
-  // ---- phase_field (STEP_7/phase_field.f90:19-52), rows clamped per BC_g
+  // ---- momentsPre .. collision; phi_prec rows clamped per BC_g
   const int64_t rn = (int64_t)(j < ny ? j + 1 : ny) * P;
   const int64_t rs = (int64_t)(j > 1 ? j - 1 : 1) * P;
   const int64_t r0 = (int64_t)j * P;
   const double tap[9] = {pa[q],          pa[r0 + i + 1], pa[rn + i],     pa[r0 + i - 1], pa[rs + i],
                          pa[rn + i + 1], pa[rn + i - 1], pa[rs + i - 1], pa[rs + i + 1]};
-  const double phi = phase_update(c, T, tap);
-  const double pc = tap[0];
-
-  // ---- forces (STEP_7/forces.f90:18-26)
-  T = T - (c.dt_st * (phi - pc) / 2.0);
-  {
-    double fy = buoyancy(c, rho, T, phi);
-    const double fx = -(u * (1.0 - phi) * 0.5);
-    fy = fy - v * (1.0 - phi) * 0.5;
-    u = u + fx / (c.omega_f * rho);
-    v = v + fy / (c.omega_f * rho);
-  }
-
-  // ---- collision (STEP_7/collision.f90:14-150)
-  double fo[9], go[9];
-  regularised_bgk<STEP7>(c, c.omega_f, rho, u, v, fp, fo);
-  regularised_bgk<STEP7>(c, omega_g_at(c, phi), T, u, v, gp, go);
+  const Done o = node_step<STEP7>(c, fp, gp, tap);
 #pragma unroll
-  for (int k = 0; k < 9; ++k) stream_store(&B.p[k][q], fo[k], go[k]);
-  stream_store(&pb[q], phi);
+  for (int k = 0; k < 9; ++k) stream_store(&B.p[k][q], o.f[k], o.g[k]);
+  stream_store(&pb[q], o.phi);
 
   // ---- moments (STEP_7/moments.f90:11-25), where somebody reads them
   if (edge || write_all) {
-    const double r = fo[0] + fo[1] + fo[2] + fo[3] + fo[4] + fo[5] + fo[6] + fo[7] + fo[8];
-    const double irho = 1.0 / r;
-    const double tt = go[0] + go[1] + go[2] + go[3] + go[4] + go[5] + go[6] + go[7] + go[8];
-    const double tu = irho * (fo[1] - fo[3] + fo[5] - fo[6] - fo[7] + fo[8]);
-    const double tv = irho * (fo[2] - fo[4] + fo[5] + fo[6] - fo[7] - fo[8]);
-    const double Tav = (tt + T2) * 0.5;
-    const double uav = (tu + u2) * 0.5;
-    const double vav = (tv + v2) * 0.5;
+    const Avg a = averaged(o);
     if (edge) {
       // halo as BC_f / BC_g left it at the start of this step
       if (s_edge) {
@@ -179,7 +145,7 @@ __global__ __launch_bounds__(TILE_W) void k_fused64(Pairs64 A, Pairs64 B,
         const int64_t h = r0 + nx + 1;
         m.T[h] = east_T(c, te_in, j);
         pb[h] = pa[h];
-        te_out[j] = Tav;
+        te_out[j] = a.T;
         if (s_edge) {
           m.T[nx + 1] = east_T(c, te_in, 1);
           pb[nx + 1] = pa[P + nx + 1];
@@ -193,10 +159,62 @@ __global__ __launch_bounds__(TILE_W) void k_fused64(Pairs64 A, Pairs64 B,
         }
       }
     }
-    m.rho[q] = r;
-    m.T[q] = Tav;
-    m.u[q] = uav;
-    m.v[q] = vav;
+    m.rho[q] = a.rho;
+    m.T[q] = a.T;
+    m.u[q] = a.u;
+    m.v[q] = a.v;
+  }
+}
+
+// One step for any walls, after BC_f and BC_g (bgk_stage.hip) have written the
+// ghosts of A and pa: every pull and tap is a load.  The workgroups past the
+// tiles copy the ghosts, of which a boundary type may leave some unwritten, to
+// the next step's planes.  304 B per node as k_fused64, where the eight
+// subroutines move about 1.1 KB in ten launches (1024 x 512 channel, us per
+// step: 149 by subroutines, 48 in two launches).
+template <bool STEP7>
+__global__ __launch_bounds__(TILE_W) void k_general64(Pairs64 A, Pairs64 B,
+                                                      const double* __restrict__ pa,
+                                                      double* __restrict__ pb, Macro m, Consts c,
+                                                      Geom gm, TileGrid tg, int write_all) {
+  const int nx = gm.nx, ny = gm.ny;
+  const int64_t P = gm.pitch;
+  const int64_t past = (int64_t)blockIdx.x - tg.per * NXCD;
+  if (past >= 0) {
+    // ghost node e: rows 0 and Ny+1, then columns 0 and Nx+1 of rows 1..Ny
+    const int64_t e = past * TILE_W + threadIdx.x, row = nx + 2;
+    if (e >= 2 * row + 2 * (int64_t)ny) return;
+    const int64_t q = e < row       ? e
+                      : e < 2 * row ? (int64_t)(ny + 1) * P + (e - row)
+                                    : ((e - 2 * row) / 2 + 1) * P + ((e & 1) ? nx + 1 : 0);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) B.p[k][q] = A.p[k][q];
+    pb[q] = pa[q];
+    return;
+  }
+  int i, j;
+  if (!tile_node(tg, gm, &i, &j)) return;
+  const int64_t q = (int64_t)j * P + i;
+  double fp[9], gp[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) {
+    const double2 fg = stream_load(&A.p[k][q - CX[k] - (int64_t)CY[k] * P]);
+    fp[k] = fg.x;
+    gp[k] = fg.y;
+  }
+  const double tap[9] = {pa[q],         pa[q + 1],     pa[q + P],     pa[q - 1], pa[q - P],
+                         pa[q + 1 + P], pa[q - 1 + P], pa[q - 1 - P], pa[q + 1 - P]};
+  const Done o = node_step<STEP7>(c, fp, gp, tap);
+#pragma unroll
+  for (int k = 0; k < 9; ++k) stream_store(&B.p[k][q], o.f[k], o.g[k]);
+  stream_store(&pb[q], o.phi);
+  // BC_f and BC_g read the moments of the boundary-adjacent nodes
+  if (write_all || i == 1 || i == nx || j == 1 || j == ny) {
+    const Avg a = averaged(o);
+    m.rho[q] = a.rho;
+    m.T[q] = a.T;
+    m.u[q] = a.u;
+    m.v[q] = a.v;
   }
 }
 
@@ -232,6 +250,31 @@ hipError_t launch_fused_step64(bgk_handle* h, bool write_all) {
     h->cur = b;
     h->pc = 1 - h->pc;
     h->te_cur = 1 - h->te_cur;
+  }
+  return e;
+}
+
+hipError_t launch_general_step64(bgk_handle* h, bool write_all) {
+  hipError_t e = launch_bc(h, true, true);
+  if (e != hipSuccess) return e;
+  const Geom& g = h->geom;
+  const TileGrid tg = make_tile_grid(g);
+  const int64_t ghosts = 2 * ((int64_t)g.nx + 2) + 2 * (int64_t)g.ny;
+  const dim3 grd((unsigned)(tg.per * NXCD + (ghosts + TILE_W - 1) / TILE_W));
+  Macro m{h->rho, h->u, h->v, h->T};
+  const int a = h->cur, b = 1 - h->cur;
+  if (h->prm.rounding == BGK_ROUND_STEP7)
+    hipLaunchKernelGGL(k_general64<true>, grd, dim3(TILE_W), 0, h->stream, pairs(h->f[a]),
+                       pairs(h->f[b]), h->phi[h->pc], h->phi[1 - h->pc], m, h->c, g, tg,
+                       write_all ? 1 : 0);
+  else
+    hipLaunchKernelGGL(k_general64<false>, grd, dim3(TILE_W), 0, h->stream, pairs(h->f[a]),
+                       pairs(h->f[b]), h->phi[h->pc], h->phi[1 - h->pc], m, h->c, g, tg,
+                       write_all ? 1 : 0);
+  e = hipGetLastError();
+  if (e == hipSuccess) {
+    h->cur = b;
+    h->pc = 1 - h->pc;
   }
   return e;
 }

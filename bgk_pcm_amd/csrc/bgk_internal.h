@@ -94,6 +94,8 @@ namespace bgk {
 
 // ---- per-subroutine kernels (bgk_stage.hip), FP64 handles
 hipError_t launch_initialization(bgk_handle* h);
+// BC_f and / or BC_g; the entry points of one each
+hipError_t launch_bc(bgk_handle* h, bool do_f, bool do_g);
 hipError_t launch_bc_f(bgk_handle* h);
 hipError_t launch_bc_g(bgk_handle* h);
 hipError_t launch_streaming(bgk_handle* h);
@@ -110,6 +112,8 @@ hipError_t launch_teast_prologue(bgk_handle* h);
 // One fused FP64 step from buffer cur to 1-cur; write_all: write the
 // moments of every node (else only the boundary-adjacent ones).
 hipError_t launch_fused_step64(bgk_handle* h, bool write_all);
+// One FP64 step for any walls: BC_f and BC_g, then the rest fused.
+hipError_t launch_general_step64(bgk_handle* h, bool write_all);
 // kSteps64 FP64 steps in one launch (bgk_stream64.hip), where stream64(h)
 constexpr int kSteps64 = 2;
 bool stream64(const bgk_handle* h);

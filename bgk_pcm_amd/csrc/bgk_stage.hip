@@ -3,8 +3,8 @@
 // This is the per-subroutine path of the drop-in boundary: bgk_bc_f,
 // bgk_bc_g, bgk_streaming, ... each launch the kernels below on the handle's
 // stream, on the same fields the reference's `module shared` holds.  It
-// serves every boundary type of the reference and is the path bgk_step takes
-// when the walls are not all no-slip.  Compiled with -ffp-contract=off: the
+// serves every boundary type of the reference; bgk_step takes its boundary
+// launch when the walls are not all no-slip.  Compiled with -ffp-contract=off: the
 // FP64 results equal the reference's bit for bit.
 #include <algorithm>
 
@@ -29,9 +29,9 @@ inline Pops64 pops(double* const* p) {
 
 // pair view: plane k holds (f_k, g_k) per node.  One 16-byte access serves both
 // members; as two stride-2 accesses each cache line was requested twice.  A step
-// by subroutines, us, before and after pairs, merged boundary launches and no
-// copy of phi: 64^2 40 / 32, 512^2 90 / 79, 1024 x 512 151 / 130, 2048 x 1024
-// 610 / 530.
+// by subroutines, us, before and after pairs, one boundary launch each and no
+// copy of phi: 64^2 40 / 31, 512^2 90 / 65, 1024 x 512 151 / 106, 2048 x 1024
+// 610 / 462.
 inline Pairs64 pairs(double* const* fplanes) {
   Pairs64 r;
   for (int k = 0; k < 9; ++k) r.p[k] = reinterpret_cast<double2*>(fplanes[k]);
@@ -88,6 +88,34 @@ struct Walls {
 };
 
 // ----------------------------------------------------------------------- BC_f
+// Each routine below reads everything first and writes after: the planes may
+// alias for all the compiler knows, and a load behind a store waits for both
+// (channel 1024 x 512, us per step: 75 interleaved, 71 so).
+
+// The equilibria of directions a, b, d (one side's) for density r and velocity
+// (u, v), in the operand order of BC_f.f90.
+struct Three {
+  double a, b, d;
+};
+__device__ __forceinline__ Three west_eq(const Consts& c, double r, double u, double v) {
+  const double uu = u * u, vv = v * v, uv = 1.5 * (uu + vv), upv = u + v, umv = u - v;
+  return Three{c.w[1] * r * (1.0 + 3.0 * u + 4.5 * uu - uv),
+               c.w[5] * r * (1.0 + 3.0 * upv + 4.5 * upv * upv - uv),
+               c.w[8] * r * (1.0 + 3.0 * umv + 4.5 * umv * umv - uv)};
+}
+__device__ __forceinline__ Three east_eq(const Consts& c, double r, double u, double v) {
+  const double uu = u * u, vv = v * v, uv = 1.5 * (uu + vv), upv = u + v, umv = u - v;
+  return Three{c.w[3] * r * (1.0 - 3.0 * u + 4.5 * uu - uv),
+               c.w[6] * r * (1.0 - 3.0 * umv + 4.5 * umv * umv - uv),
+               c.w[7] * r * (1.0 - 3.0 * upv + 4.5 * upv * upv - uv)};
+}
+__device__ __forceinline__ Three north_eq(const Consts& c, double r, double u, double v) {
+  const double uu = u * u, vv = v * v, uv = 1.5 * (uu + vv), upv = u + v, umv = u - v;
+  return Three{c.w[4] * r * (1.0 - 3.0 * v + 4.5 * vv - uv),
+               c.w[7] * r * (1.0 - 3.0 * upv + 4.5 * upv * upv - uv),
+               c.w[8] * r * (1.0 + 3.0 * umv + 4.5 * umv * umv - uv)};
+}
+
 // West and east sides, row j = 0..Ny+1 (STEP_7/BC_f.f90:9-104).
 __device__ __forceinline__ void bc_f_we(const Pops64& F, const Macro& m, const Consts& c,
                                         const Geom& gm, const Walls& w, int j) {
@@ -96,66 +124,67 @@ __device__ __forceinline__ void bc_f_we(const Pops64& F, const Macro& m, const C
   auto at = [&](int i, int jj) { return (int64_t)jj * P + i; };
   const Strided2<double>* f = F.p;
   const bool inner = (j >= 1 && j <= ny);
-  double uu, vv, uv, upv, umv;
-  // WEST
+  // ---- read
+  double fw[9], fe[9];  // periodic
+  Three w3{}, e3{};     // directions 1, 5, 8 of the west, 3, 6, 7 of the east
+  double ru = 0.0, rv = 0.0, rr = 0.0, eu = 0.0, ev = 0.0;
   if (wbc == 0) {
 #pragma unroll
-    for (int k = 0; k < 9; ++k) f[k][at(0, j)] = f[k][at(nx, j)];
+    for (int k = 0; k < 9; ++k) fw[k] = f[k][at(nx, j)];
   } else if (wbc == 1) {
     if (inner) {
-      const double u0 = c.u0, v0 = c.v0;
-      uu = u0 * u0; vv = v0 * v0; uv = 1.5 * (uu + vv); upv = u0 + v0; umv = u0 - v0;
-      const double r1 = m.rho[at(1, j)];
-      f[1][at(0, j)] = c.w[1] * r1 * (1.0 + 3.0 * u0 + 4.5 * uu - uv);
-      f[5][at(0, j)] = c.w[5] * r1 * (1.0 + 3.0 * upv + 4.5 * upv * upv - uv);
-      f[8][at(0, j)] = c.w[8] * r1 * (1.0 + 3.0 * umv + 4.5 * umv * umv - uv);
-      m.u[at(0, j)] = u0;
-      m.v[at(0, j)] = v0;
-      m.rho[at(0, j)] = r1;
+      rr = m.rho[at(1, j)];
+      ru = c.u0;
+      rv = c.v0;
+      w3 = west_eq(c, rr, ru, rv);
     }
   } else if (wbc == 2) {
-    const double uw = m.u[at(0, j)], v0 = c.v0;
-    uu = uw * uw; vv = v0 * v0; uv = 1.5 * (uu + vv); upv = uw + v0; umv = uw - v0;
-    const double r1 = m.rho[at(1, j)];
-    f[1][at(0, j)] = c.w[1] * r1 * (1.0 + 3.0 * uw + 4.5 * uu - uv);
-    f[5][at(0, j)] = c.w[5] * r1 * (1.0 + 3.0 * upv + 4.5 * upv * upv - uv);
-    f[8][at(0, j)] = c.w[8] * r1 * (1.0 + 3.0 * umv + 4.5 * umv * umv - uv);
+    w3 = west_eq(c, m.rho[at(1, j)], m.u[at(0, j)], c.v0);
   } else if (wbc == 3) {
-    const double u1 = m.u[at(1, j)], v1 = m.v[at(1, j)];
-    uu = u1 * u1; vv = v1 * v1; uv = 1.5 * (uu + vv); upv = u1 + v1; umv = u1 - v1;
-    f[1][at(0, j)] = c.w[1] * c.rho1 * (1.0 + 3.0 * u1 + 4.5 * uu - uv);
-    f[5][at(0, j)] = c.w[5] * c.rho1 * (1.0 + 3.0 * upv + 4.5 * upv * upv - uv);
-    f[8][at(0, j)] = c.w[8] * c.rho1 * (1.0 + 3.0 * umv + 4.5 * umv * umv - uv);
-    m.u[at(0, j)] = u1;
-    m.v[at(0, j)] = v1;
-    m.rho[at(0, j)] = c.rho1;
+    ru = m.u[at(1, j)];
+    rv = m.v[at(1, j)];
+    rr = c.rho1;
+    w3 = west_eq(c, rr, ru, rv);
   } else if (wbc == 4) {
-    if (inner) {
-      f[1][at(0, j)] = f[3][at(1, j)];
-      f[8][at(0, j)] = f[6][at(1, j - 1)];
-      f[5][at(0, j)] = f[7][at(1, j + 1)];
-    }
+    if (inner) w3 = Three{f[3][at(1, j)], f[7][at(1, j + 1)], f[6][at(1, j - 1)]};
   }
-  // EAST
   if (ebc == 0) {
 #pragma unroll
-    for (int k = 0; k < 9; ++k) f[k][at(nx + 1, j)] = f[k][at(1, j)];
+    for (int k = 0; k < 9; ++k) fe[k] = f[k][at(1, j)];
   } else if (ebc == 3) {
     if (inner) {
-      const double ue = m.u[at(nx, j)], ve = m.v[at(nx, j)];
-      uu = ue * ue; vv = ve * ve; uv = 1.5 * (uu + vv); upv = ue + ve; umv = ue - ve;
-      f[3][at(nx + 1, j)] = c.w[3] * c.rho0 * (1.0 - 3.0 * ue + 4.5 * uu - uv);
-      f[6][at(nx + 1, j)] = c.w[6] * c.rho0 * (1.0 - 3.0 * umv + 4.5 * umv * umv - uv);
-      f[7][at(nx + 1, j)] = c.w[7] * c.rho0 * (1.0 - 3.0 * upv + 4.5 * upv * upv - uv);
-      m.u[at(nx + 1, j)] = ue;
-      m.v[at(nx + 1, j)] = ve;
-      m.rho[at(nx + 1, j)] = c.rho0;
+      eu = m.u[at(nx, j)];
+      ev = m.v[at(nx, j)];
+      e3 = east_eq(c, c.rho0, eu, ev);
     }
   } else if (ebc == 4) {
-    if (inner) {
-      f[3][at(nx + 1, j)] = f[1][at(nx, j)];
-      f[6][at(nx + 1, j)] = f[8][at(nx, j + 1)];
-      f[7][at(nx + 1, j)] = f[5][at(nx, j - 1)];
+    if (inner) e3 = Three{f[1][at(nx, j)], f[8][at(nx, j + 1)], f[5][at(nx, j - 1)]};
+  }
+  // ---- write
+  if (wbc == 0) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) f[k][at(0, j)] = fw[k];
+  } else if (wbc == 2 || wbc == 3 || inner) {
+    f[1][at(0, j)] = w3.a;
+    f[5][at(0, j)] = w3.b;
+    f[8][at(0, j)] = w3.d;
+    if (wbc == 1 || wbc == 3) {
+      m.u[at(0, j)] = ru;
+      m.v[at(0, j)] = rv;
+      m.rho[at(0, j)] = rr;
+    }
+  }
+  if (ebc == 0) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) f[k][at(nx + 1, j)] = fe[k];
+  } else if (inner) {
+    f[3][at(nx + 1, j)] = e3.a;
+    f[6][at(nx + 1, j)] = e3.b;
+    f[7][at(nx + 1, j)] = e3.d;
+    if (ebc == 3) {
+      m.u[at(nx + 1, j)] = eu;
+      m.v[at(nx + 1, j)] = ev;
+      m.rho[at(nx + 1, j)] = c.rho0;
     }
   }
 }
@@ -169,54 +198,73 @@ __device__ __forceinline__ void bc_f_ns(const Pops64& F, const Macro& m, const C
   auto at = [&](int ii, int jj) { return (int64_t)jj * P + ii; };
   const Strided2<double>* f = F.p;
   const bool inner = (i >= 1 && i <= nx);
-  // NORTH
+  // ---- read
+  double fn[9], fs[9];  // periodic
+  Three n3{}, s3{};     // directions 4, 7, 8 of the north, 2, 5, 6 of the south
+  double nr = 0.0, sr = 0.0;
   if (nbc == 0) {
 #pragma unroll
-    for (int k = 0; k < 9; ++k) f[k][at(i, ny + 1)] = f[k][at(i, 1)];
+    for (int k = 0; k < 9; ++k) fn[k] = f[k][at(i, 1)];
   } else if (nbc == 4) {
     if (inner) {
-      f[4][at(i, ny + 1)] = f[2][at(i, ny)];
-      f[7][at(i, ny + 1)] = f[5][at(i - 1, ny)];
-      f[8][at(i, ny + 1)] = f[6][at(i + 1, ny)];
-      m.rho[at(i, ny + 1)] = m.rho[at(i, ny)];
-      m.u[at(i, ny + 1)] = 0.0;
-      m.v[at(i, ny + 1)] = 0.0;
+      n3 = Three{f[2][at(i, ny)], f[5][at(i - 1, ny)], f[6][at(i + 1, ny)]};
+      nr = m.rho[at(i, ny)];
     }
-    if (i == 0) f[8][at(0, ny + 1)] = f[6][at(1, ny)];
+    if (i == 0) n3.d = f[6][at(1, ny)];
   } else if (nbc == 5) {
-    f[4][at(i, ny + 1)] = f[2][at(i, ny - 1)];
-    f[7][at(i, ny + 1)] = f[6][at(i, ny - 1)];
-    f[8][at(i, ny + 1)] = f[5][at(i, ny - 1)];
+    n3 = Three{f[2][at(i, ny - 1)], f[6][at(i, ny - 1)], f[5][at(i, ny - 1)]};
   } else if (nbc == 6) {
-    f[4][at(i, ny + 1)] = f[4][at(i, ny)];
-    f[7][at(i, ny + 1)] = f[7][at(i, ny)];
-    f[8][at(i, ny + 1)] = f[8][at(i, ny)];
+    n3 = Three{f[4][at(i, ny)], f[7][at(i, ny)], f[8][at(i, ny)]};
   } else if (nbc == 1) {
-    const double u0 = c.u0, v0 = c.v0;
-    const double uu = u0 * u0, vv = v0 * v0, uv = 1.5 * (uu + vv), upv = u0 + v0, umv = u0 - v0;
-    const double rn = m.rho[at(i, ny)];
-    f[4][at(i, ny + 1)] = c.w[4] * rn * (1.0 - 3.0 * v0 + 4.5 * vv - uv);
-    f[7][at(i, ny + 1)] = c.w[7] * rn * (1.0 - 3.0 * upv + 4.5 * upv * upv - uv);
-    f[8][at(i, ny + 1)] = c.w[8] * rn * (1.0 + 3.0 * umv + 4.5 * umv * umv - uv);
+    n3 = north_eq(c, m.rho[at(i, ny)], c.u0, c.v0);
   }
-  // SOUTH
   if (sbc == 0) {
 #pragma unroll
-    for (int k = 0; k < 9; ++k) f[k][at(i, 0)] = f[k][at(i, ny)];
+    for (int k = 0; k < 9; ++k) fs[k] = f[k][at(i, ny)];
   } else if (sbc == 4) {
     if (inner) {
-      f[2][at(i, 0)] = f[4][at(i, 1)];
-      f[5][at(i, 0)] = f[7][at(i + 1, 1)];
-      f[6][at(i, 0)] = f[8][at(i - 1, 1)];
-      m.rho[at(i, 0)] = m.rho[at(i, 1)];
-      m.u[at(i, 0)] = 0.0;
-      m.v[at(i, 0)] = 0.0;
+      s3 = Three{f[4][at(i, 1)], f[7][at(i + 1, 1)], f[8][at(i - 1, 1)]};
+      sr = m.rho[at(i, 1)];
     }
-    if (i == 0) f[5][at(0, 0)] = f[7][at(1, 1)];
+    if (i == 0) s3.b = f[7][at(1, 1)];
   } else if (sbc == 6) {
-    f[2][at(i, 0)] = f[2][at(i, 1)];
-    f[5][at(i, 0)] = f[5][at(i, 1)];
-    f[6][at(i, 0)] = f[6][at(i, 1)];
+    s3 = Three{f[2][at(i, 1)], f[5][at(i, 1)], f[6][at(i, 1)]};
+  }
+  // ---- write
+  const int64_t n = at(i, ny + 1), s = at(i, 0);
+  if (nbc == 0) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) f[k][n] = fn[k];
+  } else if (nbc == 4) {
+    if (inner) {
+      f[4][n] = n3.a;
+      f[7][n] = n3.b;
+      m.rho[n] = nr;
+      m.u[n] = 0.0;
+      m.v[n] = 0.0;
+    }
+    if (inner || i == 0) f[8][n] = n3.d;
+  } else {
+    f[4][n] = n3.a;
+    f[7][n] = n3.b;
+    f[8][n] = n3.d;
+  }
+  if (sbc == 0) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) f[k][s] = fs[k];
+  } else if (sbc == 4) {
+    if (inner) {
+      f[2][s] = s3.a;
+      f[6][s] = s3.d;
+      m.rho[s] = sr;
+      m.u[s] = 0.0;
+      m.v[s] = 0.0;
+    }
+    if (inner || i == 0) f[5][s] = s3.b;
+  } else {
+    f[2][s] = s3.a;
+    f[5][s] = s3.b;
+    f[6][s] = s3.d;
   }
 }
 
@@ -225,54 +273,57 @@ __device__ __forceinline__ void bc_f_ns(const Pops64& F, const Macro& m, const C
 __device__ __forceinline__ void bc_g_we(const Pops64& G, const Macro& m, const Consts& c,
                                         const Geom& gm, int j) {
   const int nx = gm.nx;
-  const int64_t P = gm.pitch;
-  auto at = [&](int ii, int jj) { return (int64_t)jj * P + ii; };
+  const int64_t w = (int64_t)j * gm.pitch, e = w + nx + 1;
   const Strided2<double>* g = G.p;
-  {
-    const double uw = m.u[at(0, j)], vw = m.v[at(0, j)];
-    const double uu = uw * uw, vv = vw * vw, uv = 1.5 * (uu + vv), upv = uw + vw, umv = uw - vw;
-    g[1][at(0, j)] = c.w[1] * c.tin * (1.0 + 3.0 * uw + 4.5 * uu - uv);
-    g[5][at(0, j)] = c.w[5] * c.tin * (1.0 + 3.0 * upv + 4.5 * upv * upv - uv);
-    g[8][at(0, j)] = c.w[8] * c.tin * (1.0 + 3.0 * umv + 4.5 * umv * umv - uv);
-    m.T[at(0, j)] = c.tin;
-  }
-  {
-    // the averaged T(Nx, j), or the cold-wall extension's fixed temperature
-    const double ue = m.u[at(nx + 1, j)], ve = m.v[at(nx + 1, j)];
-    const double te = c.east_cold ? c.t_cold : m.T[at(nx, j)];
-    const double uu = ue * ue, vv = ve * ve, uv = 1.5 * (uu + vv), upv = ue + ve, umv = ue - ve;
-    g[3][at(nx + 1, j)] = c.w[3] * te * (1.0 - 3.0 * ue + 4.5 * uu - uv);
-    g[6][at(nx + 1, j)] = c.w[6] * te * (1.0 - 3.0 * umv + 4.5 * umv * umv - uv);
-    g[7][at(nx + 1, j)] = c.w[7] * te * (1.0 - 3.0 * upv + 4.5 * upv * upv - uv);
-    m.T[at(nx + 1, j)] = te;
-  }
+  const double uw = m.u[w], vw = m.v[w], ue = m.u[e], ve = m.v[e];
+  // the averaged T(Nx, j), or the cold-wall extension's fixed temperature
+  const double te = c.east_cold ? c.t_cold : m.T[w + nx];
+  const Three w3 = west_eq(c, c.tin, uw, vw), e3 = east_eq(c, te, ue, ve);
+  g[1][w] = w3.a;
+  g[5][w] = w3.b;
+  g[8][w] = w3.d;
+  m.T[w] = c.tin;
+  g[3][e] = e3.a;
+  g[6][e] = e3.b;
+  g[7][e] = e3.d;
+  m.T[e] = te;
 }
 
 // North and south zero-gradient copies, column i = 0..Nx+1
 // (STEP_7/BC_g.f90:36-64), after bc_g_we.
 __device__ __forceinline__ void bc_g_ns(const Pops64& G, const Macro& m, double* phi,
                                         const Geom& gm, int i) {
-  const int ny = gm.ny;
   const int64_t P = gm.pitch;
-  const int64_t qn = (int64_t)ny * P + i, qn1 = (int64_t)(ny + 1) * P + i;
-  const int64_t q1 = P + i, q0 = i;
+  const int64_t qn = (int64_t)gm.ny * P + i, q1 = P + i;
+  double gn[9], gs[9];
 #pragma unroll
-  for (int k = 0; k < 9; ++k) G.p[k][qn1] = G.p[k][qn];
-  m.T[qn1] = m.T[qn];
-  phi[qn1] = phi[qn];
+  for (int k = 0; k < 9; ++k) {
+    gn[k] = G.p[k][qn];
+    gs[k] = G.p[k][q1];
+  }
+  const double tn = m.T[qn], ts = m.T[q1], pn = phi[qn], ps = phi[q1];
 #pragma unroll
-  for (int k = 0; k < 9; ++k) G.p[k][q0] = G.p[k][q1];
-  m.T[q0] = m.T[q1];
-  phi[q0] = phi[q1];
+  for (int k = 0; k < 9; ++k) {
+    G.p[k][qn + P] = gn[k];
+    G.p[k][i] = gs[k];
+  }
+  m.T[qn + P] = tn;
+  m.T[i] = ts;
+  phi[qn + P] = pn;
+  phi[i] = ps;
 }
 
-// BC_f and/or BC_g.  The sides depend on each other in the reference's order
-// (west and east, then north and south; f before g).  PHASE 0: all of it by one
-// workgroup, which waits between the four parts; 1..4: one part, one thread per
-// node, for lattices whose sides one workgroup would walk too slowly.  What
-// bounds a part is the latency of a launch or of a few dependent accesses, so
-// one launch of one workgroup beats four.
-constexpr int kBcThreads = 1024;
+// BC_f and/or BC_g in one launch.  The sides depend on each other in the
+// reference's order (west and east, then north and south; f before g), but
+// only in the columns 0, 1, Nx, Nx+1 and the rows 0, 1, Ny-1, Ny, Ny+1: the first
+// workgroup does these, waiting between the four parts; every other row of the
+// west and east and column of the north and south is a thread of its own
+// elsewhere, f before g.  On lattices of fewer than 8 rows or columns the first
+// workgroup does everything.
+// What bounds it: the latency of a launch and of a few dependent accesses.
+// Measured, us per step of a channel (this launch and k_general64): 2048 x 1024
+// 186 with one workgroup for all, 132 so; 1024 x 512 71 / 48; 64^2 13.3 / 12.8.
+constexpr int kBcThreads = 256;
 struct BcArgs {
   Pops64 F, G;
   Macro m;
@@ -281,23 +332,39 @@ struct BcArgs {
   Geom gm;
   Walls w;
   int do_f, do_g;
+  int small;
 };
-template <int PHASE>
 __global__ __launch_bounds__(kBcThreads) void k_bc(BcArgs a) {
   const int nx = a.gm.nx, ny = a.gm.ny;
-  const int t0 = blockIdx.x * blockDim.x + threadIdx.x;
-  const int step = PHASE == 0 ? kBcThreads : nx + ny + 4;  // (1..4: one node each)
-  if ((PHASE == 0 && a.do_f) || PHASE == 1)
-    for (int j = t0; j <= ny + 1; j += step) bc_f_we(a.F, a.m, a.c, a.gm, a.w, j);
-  if (PHASE == 0 && a.do_f) __syncthreads();
-  if ((PHASE == 0 && a.do_f) || PHASE == 2)
-    for (int i = t0; i <= nx + 1; i += step) bc_f_ns(a.F, a.m, a.c, a.gm, a.w, i);
-  if (PHASE == 0 && a.do_f && a.do_g) __syncthreads();
-  if ((PHASE == 0 && a.do_g) || PHASE == 3)
-    for (int j = t0 + 1; j <= ny; j += step) bc_g_we(a.G, a.m, a.c, a.gm, j);
-  if (PHASE == 0 && a.do_g) __syncthreads();
-  if ((PHASE == 0 && a.do_g) || PHASE == 4)
-    for (int i = t0; i <= nx + 1; i += step) bc_g_ns(a.G, a.m, a.phi, a.gm, i);
+  if (blockIdx.x > 0) {
+    int t = ((int)blockIdx.x - 1) * kBcThreads + (int)threadIdx.x;
+    if (t < ny - 3) {
+      const int j = t + 2;  // 2..Ny-2
+      if (a.do_f) bc_f_we(a.F, a.m, a.c, a.gm, a.w, j);
+      if (a.do_g) bc_g_we(a.G, a.m, a.c, a.gm, j);
+    } else if ((t -= ny - 3) < nx - 2) {
+      const int i = t + 2;  // 2..Nx-1
+      if (a.do_f) bc_f_ns(a.F, a.m, a.c, a.gm, a.w, i);
+      if (a.do_g) bc_g_ns(a.G, a.m, a.phi, a.gm, i);
+    }
+    return;
+  }
+  // rows and columns of the first workgroup
+  const int nr = a.small ? ny + 2 : 5, nc = a.small ? nx + 2 : 4;
+  auto row = [&](int e) { return a.small || e < 2 ? e : ny - 3 + e; };
+  auto col = [&](int e) { return a.small || e < 2 ? e : nx - 2 + e; };
+  if (a.do_f) {
+    for (int e = threadIdx.x; e < nr; e += kBcThreads) bc_f_we(a.F, a.m, a.c, a.gm, a.w, row(e));
+    __syncthreads();
+    for (int e = threadIdx.x; e < nc; e += kBcThreads) bc_f_ns(a.F, a.m, a.c, a.gm, a.w, col(e));
+    __syncthreads();
+  }
+  if (a.do_g) {
+    for (int e = threadIdx.x; e < nr; e += kBcThreads)
+      if (row(e) >= 1 && row(e) <= ny) bc_g_we(a.G, a.m, a.c, a.gm, row(e));
+    __syncthreads();
+    for (int e = threadIdx.x; e < nc; e += kBcThreads) bc_g_ns(a.G, a.m, a.phi, a.gm, col(e));
+  }
 }
 
 // ------------------------------------------------------------------ streaming
@@ -431,23 +498,12 @@ hipError_t launch_initialization(bgk_handle* h) {
 
 hipError_t launch_bc(bgk_handle* h, bool do_f, bool do_g) {
   const Geom& g = h->geom;
+  const bool small = g.nx < 8 || g.ny < 8;
   BcArgs a{pops(h->f[h->cur]), pops(h->g[h->cur]), macro_of(h), h->phi[h->pc], h->c, g,
            Walls{h->prm.west_bc, h->prm.east_bc, h->prm.north_bc, h->prm.south_bc},
-           do_f ? 1 : 0, do_g ? 1 : 0};
-  // one workgroup up to four rounds of its threads on a side
-  if (std::max(g.nx, g.ny) + 2 <= 4 * kBcThreads) {
-    hipLaunchKernelGGL(k_bc<0>, dim3(1), dim3(kBcThreads), 0, h->stream, a);
-    return hipGetLastError();
-  }
-  const dim3 we(blocks1d(g.ny + 2, 256)), ns(blocks1d(g.nx + 2, 256));
-  if (do_f) {
-    hipLaunchKernelGGL(k_bc<1>, we, dim3(256), 0, h->stream, a);
-    hipLaunchKernelGGL(k_bc<2>, ns, dim3(256), 0, h->stream, a);
-  }
-  if (do_g) {
-    hipLaunchKernelGGL(k_bc<3>, we, dim3(256), 0, h->stream, a);
-    hipLaunchKernelGGL(k_bc<4>, ns, dim3(256), 0, h->stream, a);
-  }
+           do_f ? 1 : 0, do_g ? 1 : 0, small ? 1 : 0};
+  const unsigned rest = small ? 0 : blocks1d(g.ny - 3 + g.nx - 2, kBcThreads);
+  hipLaunchKernelGGL(k_bc, dim3(1 + rest), dim3(kBcThreads), 0, h->stream, a);
   return hipGetLastError();
 }
 

@@ -24,6 +24,7 @@
 // 256^2 12.6 (9.4): below 2^17 nodes one step per launch stays (stream64).
 #include <algorithm>
 
+#include "bgk_pop64.h"
 #include "bgk_wave.h"
 
 namespace bgk {
@@ -65,59 +66,6 @@ struct Pend {
   // temperatures of the row and of the one south of it
   double o5, o6, gn[3], te_s, te_c;
 };
-
-struct Done {
-  double f[9], g[9], phi;
-  double T2, u2, v2;  // momentsPre, for the averages
-};
-
-// momentsPre .. collision of one node (STEP_7/momentsPre.f90:8-21,
-// phase_field.f90:24-52, forces.f90:18-26, collision.f90:14-150).
-template <bool STEP7>
-__device__ __forceinline__ Done node_step(const Consts& c, const double fp[9], const double gp[9],
-                                          const double tap[9]) {
-  Done o;
-  const double rho = fp[0] + fp[1] + fp[2] + fp[3] + fp[4] + fp[5] + fp[6] + fp[7] + fp[8];
-  double T = gp[0] + gp[1] + gp[2] + gp[3] + gp[4] + gp[5] + gp[6] + gp[7] + gp[8];
-  const double irho = 1.0 / rho;
-  double u = irho * (fp[1] - fp[3] + fp[5] - fp[6] - fp[7] + fp[8]);
-  double v = irho * (fp[2] - fp[4] + fp[5] + fp[6] - fp[7] - fp[8]);
-  o.T2 = T;
-  o.u2 = u;
-  o.v2 = v;
-  o.phi = phase_update(c, T, tap);
-  T = T - (c.dt_st * (o.phi - tap[0]) / 2.0);
-  double fy = buoyancy(c, rho, T, o.phi);
-  const double fx = -(u * (1.0 - o.phi) * 0.5);
-  fy = fy - v * (1.0 - o.phi) * 0.5;
-  u = u + fx / (c.omega_f * rho);
-  v = v + fy / (c.omega_f * rho);
-  regularised_bgk<STEP7>(c, c.omega_f, rho, u, v, fp, o.f);
-  regularised_bgk<STEP7>(c, omega_g_at(c, o.phi), T, u, v, gp, o.g);
-  return o;
-}
-
-struct Avg {
-  double rho, T, u, v;
-};
-// STEP_7/moments.f90:11-25
-__device__ __forceinline__ double averaged_T(const Done& o) {
-  const double* g = o.g;
-  const double tt = g[0] + g[1] + g[2] + g[3] + g[4] + g[5] + g[6] + g[7] + g[8];
-  return (tt + o.T2) * 0.5;
-}
-__device__ __forceinline__ Avg averaged(const Done& o) {
-  const double* f = o.f;
-  Avg a;
-  a.rho = f[0] + f[1] + f[2] + f[3] + f[4] + f[5] + f[6] + f[7] + f[8];
-  const double irho = 1.0 / a.rho;
-  const double tu = irho * (f[1] - f[3] + f[5] - f[6] - f[7] + f[8]);
-  const double tv = irho * (f[2] - f[4] + f[5] + f[6] - f[7] - f[8]);
-  a.T = averaged_T(o);
-  a.u = (tu + o.u2) * 0.5;
-  a.v = (tv + o.v2) * 0.5;
-  return a;
-}
 
 // Populations of row j already pulled: population k of node (i - cx_k, j -
 // cy_k).  off: byte offset of column i in a row of pairs.

@@ -213,7 +213,8 @@ int bgk_moments(bgk_handle* h);     /* STEP_7/moments.f90:8-27     */
  * streaming, momentsPre, phase_field, forces, collision, moments).  With
  * no-slip walls on all four sides (BC type 4, the only walls used by the
  * reference inputs UTIL/input.dat.0..3) this is one fused kernel per step;
- * other boundary types run the per-subroutine kernels (FP64 handles only).
+ * other boundary types run BC_f and BC_g in one launch and the rest fused in a
+ * second (FP64 handles only).
  * Afterwards f, g, rho, u, v, T and phi (halo included) hold what the
  * reference holds after the same steps; fp, gp, rho2, u2, v2, T2 and
  * phi_prec are scratch of the per-subroutine path and are left unspecified. */
