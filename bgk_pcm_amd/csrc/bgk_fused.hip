@@ -47,8 +47,14 @@ __global__ void k_teast_prologue(const double* __restrict__ T, double* __restric
   te[j] = T[(int64_t)j * gm.pitch + gm.nx];
 }
 
+// What bounds it on small lattices is latency: a launch every few us whose
+// waves make a dozen dependent memory accesses.  So a wave that holds a
+// boundary-adjacent node takes one path for all its lanes, with every load
+// (ghost velocities and halo values included) issued before the first use
+// (us per step: 256^2 9.4 with the ghosts' loads in branches, 7.6 so; 97 x 61 7.7
+// and 6.1).
 template <bool STEP7>
-__global__ __launch_bounds__(TILE_W) void k_fused64(Pairs64 A, Pairs64 B,
+__global__ __launch_bounds__(TILE_W) void k_fused64(Planes<double2> A, Planes<double2> B,
                                                      const double* __restrict__ pa,
                                                      double* __restrict__ pb,
                                                      const double* __restrict__ te_in,
@@ -63,49 +69,63 @@ __global__ __launch_bounds__(TILE_W) void k_fused64(Pairs64 A, Pairs64 B,
   const bool w_edge = (i == 1), e_edge = (i == nx), s_edge = (j == 1), n_edge = (j == ny);
   const bool edge = w_edge || e_edge || s_edge || n_edge;
 
-  // ---- streaming (STEP_7/streaming.f90:7-25) with the boundaries folded in
-  double fp[9], gp[9];
-  if (!edge) {
-#pragma unroll
-    for (int k = 0; k < 9; ++k) {
-      const double2 fg = stream_load(&A.p[k][q - CX[k] - (int64_t)CY[k] * P]);
-      fp[k] = fg.x;
-      gp[k] = fg.y;
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < 9; ++k) {
-      const int si = i - CX[k];
-      const int sj = j - CY[k];
-      if (si >= 1 && si <= nx && sj >= 1 && sj <= ny) {
-        fp[k] = A.p[k][(int64_t)sj * P + si].x;
-      } else if ((k == 6 && si == nx + 1 && sj == 0) || (k == 7 && si == nx + 1 && sj == ny + 1)) {
-        fp[k] = A.p[k][(int64_t)sj * P + si].x;  // never written by BC_f
-      } else {
-        fp[k] = A.p[OPP[k]][q].x;  // bounce-back
-      }
-      const int sjc = sj < 1 ? 1 : (sj > ny ? ny : sj);
-      if (si >= 1 && si <= nx) {
-        gp[k] = A.p[k][(int64_t)sjc * P + si].y;
-      } else if (si == 0) {
-        const int64_t h = (int64_t)sjc * P;
-        gp[k] = equilibrium_k(c, k, c.tin, m.u[h], m.v[h]);
-      } else {
-        const int64_t h = (int64_t)sjc * P + nx + 1;
-        gp[k] = equilibrium_k(c, k, east_T(c, te_in, sjc), m.u[h], m.v[h]);
-      }
-    }
-  }
-
-  // ---- momentsPre .. collision; phi_prec rows clamped per BC_g
+  // ---- phi_prec taps (STEP_7/phase_field.f90:27-45), rows clamped per BC_g
   const int64_t rn = (int64_t)(j < ny ? j + 1 : ny) * P;
   const int64_t rs = (int64_t)(j > 1 ? j - 1 : 1) * P;
   const int64_t r0 = (int64_t)j * P;
   const double tap[9] = {pa[q],          pa[r0 + i + 1], pa[rn + i],     pa[r0 + i - 1], pa[rs + i],
                          pa[rn + i + 1], pa[rn + i - 1], pa[rs + i - 1], pa[rs + i + 1]};
-  const Done o = node_step<STEP7>(c, fp, gp, tap);
+
+  // ---- streaming (STEP_7/streaming.f90:7-25) with the boundaries folded in
+  Row in;
+  double rho_was = 0.0, T_was = 0.0;  // of this node before the step (the halo)
+  double frozen6 = 0.0, frozen7 = 0.0;
+  if (!__any(edge)) {
 #pragma unroll
-  for (int k = 0; k < 9; ++k) stream_store(&B.p[k][q], o.f[k], o.g[k]);
+    for (int k = 0; k < 9; ++k) {
+      const double2 fg = stream_load(A.row(k, q - CX[k] - (int64_t)CY[k] * P));
+      in.f[k] = fg.x;
+      in.g[k] = fg.y;
+    }
+  } else {
+    using wave::as_scalar;
+    unsigned offs[3];
+    edge_offsets(i, nx, offs);
+    EdgeRow e;
+    load_pulled_edge(A, P, ny, offs, j, e);
+    rho_was = m.rho[q];
+    T_was = m.T[q];
+    frozen6 = as_scalar(&A.row(6, nx + 1)->x)[0];
+    frozen7 = as_scalar(&A.row(7, (int64_t)(ny + 1) * P + nx + 1)->x)[0];
+    // thermal ghosts in the rows below, beside and above (the row j is the
+    // workgroup's, so these are scalar loads)
+    const int rows[3] = {j > 1 ? j - 1 : 1, j, j < ny ? j + 1 : ny};
+    constexpr int KW[3] = {5, 1, 8}, KE[3] = {6, 3, 7};
+    double uw[3], vw[3], ue[3], ve[3], te[3];
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      const int64_t h = (int64_t)rows[s] * P;
+      uw[s] = as_scalar(m.u)[h];
+      vw[s] = as_scalar(m.v)[h];
+      ue[s] = as_scalar(m.u)[h + nx + 1];
+      ve[s] = as_scalar(m.v)[h + nx + 1];
+      te[s] = c.east_cold ? c.t_cold : as_scalar(te_in)[rows[s]];
+    }
+    wall_f(nx, ny, i, j, frozen6, frozen7, e);
+    in = e.r;
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      const double gw = equilibrium_k(c, KW[s], c.tin, uw[s], vw[s]);
+      const double ge = equilibrium_k(c, KE[s], te[s], ue[s], ve[s]);
+      in.g[KW[s]] = w_edge ? gw : in.g[KW[s]];
+      in.g[KE[s]] = e_edge ? ge : in.g[KE[s]];
+    }
+  }
+
+  // ---- momentsPre .. collision
+  const Done o = node_step<STEP7>(c, in.f, in.g, tap);
+#pragma unroll
+  for (int k = 0; k < 9; ++k) stream_store(B.row(k, q), o.f[k], o.g[k]);
   stream_store(&pb[q], o.phi);
 
   // ---- moments (STEP_7/moments.f90:11-25), where somebody reads them
@@ -114,23 +134,23 @@ __global__ __launch_bounds__(TILE_W) void k_fused64(Pairs64 A, Pairs64 B,
     if (edge) {
       // halo as BC_f / BC_g left it at the start of this step
       if (s_edge) {
-        m.rho[i] = m.rho[q];
-        m.T[i] = m.T[q];
+        m.rho[i] = rho_was;
+        m.T[i] = T_was;
         m.u[i] = 0.0;
         m.v[i] = 0.0;
-        pb[i] = pa[q];
+        pb[i] = tap[0];
       }
       if (n_edge) {
         const int64_t h = (int64_t)(ny + 1) * P + i;
-        m.rho[h] = m.rho[q];
-        m.T[h] = m.T[q];
+        m.rho[h] = rho_was;
+        m.T[h] = T_was;
         m.u[h] = 0.0;
         m.v[h] = 0.0;
-        pb[h] = pa[q];
+        pb[h] = tap[0];
       }
       if (w_edge) {
         m.T[r0] = c.tin;
-        pb[r0] = pa[r0];
+        pb[r0] = tap[3];
         if (s_edge) {
           m.T[0] = c.tin;
           pb[0] = pa[P];
@@ -144,18 +164,18 @@ __global__ __launch_bounds__(TILE_W) void k_fused64(Pairs64 A, Pairs64 B,
       if (e_edge) {
         const int64_t h = r0 + nx + 1;
         m.T[h] = east_T(c, te_in, j);
-        pb[h] = pa[h];
+        pb[h] = tap[1];
         te_out[j] = a.T;
         if (s_edge) {
           m.T[nx + 1] = east_T(c, te_in, 1);
           pb[nx + 1] = pa[P + nx + 1];
-          B.p[6][nx + 1].x = A.p[6][nx + 1].x;
+          B.row(6, nx + 1)->x = frozen6;
         }
         if (n_edge) {
           const int64_t hn = (int64_t)(ny + 1) * P + nx + 1;
           m.T[hn] = east_T(c, te_in, ny);
           pb[hn] = pa[(int64_t)ny * P + nx + 1];
-          B.p[7][hn].x = A.p[7][hn].x;
+          B.row(7, hn)->x = frozen7;
         }
       }
     }
@@ -239,12 +259,13 @@ hipError_t launch_fused_step64(bgk_handle* h, bool write_all) {
   const double* te_in = h->teast[h->te_cur];
   double* te_out = h->teast[1 - h->te_cur];
   const int a = h->cur, b = 1 - h->cur;
+  const Planes<double2> A = wave::planes_of<double2>(h->f[a]), B = wave::planes_of<double2>(h->f[b]);
   if (h->prm.rounding == BGK_ROUND_STEP7)
-    hipLaunchKernelGGL(k_fused64<true>, grd, blk, 0, h->stream, pairs(h->f[a]), pairs(h->f[b]), h->phi[h->pc], h->phi[1 - h->pc], te_in,
-                       te_out, m, h->c, g, tg, write_all ? 1 : 0);
+    hipLaunchKernelGGL(k_fused64<true>, grd, blk, 0, h->stream, A, B, h->phi[h->pc],
+                       h->phi[1 - h->pc], te_in, te_out, m, h->c, g, tg, write_all ? 1 : 0);
   else
-    hipLaunchKernelGGL(k_fused64<false>, grd, blk, 0, h->stream, pairs(h->f[a]), pairs(h->f[b]), h->phi[h->pc], h->phi[1 - h->pc], te_in,
-                       te_out, m, h->c, g, tg, write_all ? 1 : 0);
+    hipLaunchKernelGGL(k_fused64<false>, grd, blk, 0, h->stream, A, B, h->phi[h->pc],
+                       h->phi[1 - h->pc], te_in, te_out, m, h->c, g, tg, write_all ? 1 : 0);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) {
     h->cur = b;

@@ -4,9 +4,11 @@
 #ifndef BGK_POP64_H
 #define BGK_POP64_H
 
-#include "bgk_internal.h"
+#include "bgk_wave.h"
 
 namespace bgk {
+
+using wave::Planes;
 
 struct Done {
   double f[9], g[9], phi;
@@ -59,6 +61,53 @@ __device__ __forceinline__ Avg averaged(const Done& o) {
   a.u = (tu + o.u2) * 0.5;
   a.v = (tv + o.v2) * 0.5;
   return a;
+}
+
+// populations a row pulls
+struct Row {
+  double f[9], g[9];
+};
+
+// The populations of row j beside a wall, already pulled (population k of node
+// (i - cx_k, j - cy_k)).  Sources outside the lattice are taken from the nearest
+// column and row in it (right for g in the copied rows 0 and Ny+1); own: the
+// node's own f, for the bounce-back (wall_f).  Every lane makes the same loads,
+// all in flight at once.  offs: the byte offsets of columns i - 1, i, i + 1,
+// each within 1..Nx.
+struct EdgeRow {
+  Row r;
+  double own[9];
+};
+__device__ __forceinline__ void edge_offsets(int i, int nx, unsigned offs[3]) {
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+    offs[d] = (unsigned)min(max(i + d - 1, 1), nx) * (unsigned)sizeof(double2);
+}
+__device__ __forceinline__ void load_pulled_edge(const Planes<double2>& A, int64_t pitch, int ny,
+                                                 const unsigned offs[3], int j, EdgeRow& e) {
+#pragma unroll
+  for (int k = 0; k < 9; ++k) {
+    const int sj = min(max(j - CY[k], 1), ny);
+    const double2 v = wave::at(A.row(k, (int64_t)sj * pitch), offs[1 - CX[k]]);
+    e.r.f[k] = v.x;
+    e.r.g[k] = v.y;
+    if (k > 0) e.own[k] = wave::at(&A.row(k, (int64_t)j * pitch)->x, offs[1]);
+  }
+}
+
+// Bounce-back (BC_f type 4): a population whose source is a ghost is the node's
+// own opposite one, but for the two corner ghosts no BC_f branch writes.
+__device__ __forceinline__ void wall_f(int nx, int ny, int i, int j, double frozen6,
+                                       double frozen7, EdgeRow& e) {
+#pragma unroll
+  for (int k = 1; k < 9; ++k) {
+    const bool row = (CY[k] > 0 && j == 1) || (CY[k] < 0 && j == ny);
+    const bool col = (CX[k] > 0 && i == 1) || (CX[k] < 0 && i == nx);
+    double b = e.own[OPP[k]];
+    if (k == 6 && j == 1) b = i == nx ? frozen6 : b;
+    if (k == 7 && j == ny) b = i == nx ? frozen7 : b;
+    e.r.f[k] = row || col ? b : e.r.f[k];
+  }
 }
 
 }  // namespace bgk

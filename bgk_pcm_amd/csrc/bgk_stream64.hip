@@ -20,8 +20,8 @@
 // What bounds it: HBM (152 B per node and step, 304 with one step per launch);
 // a row costs its wave 1330 VALU instructions at two waves per SIMD, 75% of
 // its time at the memory rate.  Measured, us per step, against bgk_fused.hip:
-// 4096^2 552 (893), 2048^2 152 (228), 1003 x 777 34.9 (49), 512^2 18.1 (20.6),
-// 256^2 12.6 (9.4): below 2^17 nodes one step per launch stays (stream64).
+// 4096^2 552 (893), 2048^2 152 (228), 1003 x 777 34.9 (49), 512^2 18.1 (19.3),
+// 256^2 12.6 (7.6): below 2^18 nodes one step per launch stays (stream64).
 #include <algorithm>
 
 #include "bgk_pop64.h"
@@ -49,11 +49,6 @@ struct Args64 {
   WaveGrid g;
 };
 
-// populations a row pulls
-struct Row {
-  double f[9], g[9];
-};
-
 // A level's registers between two rows (levels 1 and up): of the row waiting
 // for its northern neighbours, the populations pulled from the south (2, 5,
 // 6) and from its own row (0, 1, 3); the southern share of the row after it;
@@ -75,42 +70,6 @@ __device__ __forceinline__ void load_pulled(const Args64& A, unsigned off, int j
     const double2 v = at(A.A.row(k, (int64_t)(j - CY[k]) * A.pitch - CX[k]), off);
     r.f[k] = v.x;
     r.g[k] = v.y;
-  }
-}
-
-// The same beside a wall.  Sources outside the lattice are taken from the
-// nearest column and row in it (right for g in the copied rows 0 and Ny+1);
-// own: the node's own f, for the bounce-back (wall_f).  offs: the byte offsets
-// of columns i - 1, i, i + 1, each within 1..Nx.
-struct EdgeRow {
-  Row r;
-  double own[9];
-};
-__device__ __forceinline__ void load_pulled_edge(const Args64& A, const unsigned offs[3], int j,
-                                                 EdgeRow& e) {
-#pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    const int sj = min(max(j - CY[k], 1), A.ny);
-    const double2 v = at(A.A.row(k, (int64_t)sj * A.pitch), offs[1 - CX[k]]);
-    e.r.f[k] = v.x;
-    e.r.g[k] = v.y;
-    if (k > 0) e.own[k] = at(&A.A.row(k, (int64_t)j * A.pitch)->x, offs[1]);
-  }
-}
-
-// Bounce-back (BC_f type 4) of level 0: a population whose source is a ghost
-// is the node's own opposite one, but for the two corner ghosts no BC_f branch
-// writes.
-__device__ __forceinline__ void wall_f(const Args64& A, int i, int j, double frozen6,
-                                       double frozen7, EdgeRow& e) {
-#pragma unroll
-  for (int k = 1; k < 9; ++k) {
-    const bool row = (CY[k] > 0 && j == 1) || (CY[k] < 0 && j == A.ny);
-    const bool col = (CX[k] > 0 && i == 1) || (CX[k] < 0 && i == A.nx);
-    double b = e.own[OPP[k]];
-    if (k == 6 && j == 1) b = i == A.nx ? frozen6 : b;
-    if (k == 7 && j == A.ny) b = i == A.nx ? frozen7 : b;
-    e.r.f[k] = row || col ? b : e.r.f[k];
   }
 }
 
@@ -359,9 +318,7 @@ __device__ __forceinline__ void strip_edge(const Args64& A, int j0, int j1, int 
   const bool ghost = i == 0 || i == nx + 1;
   const bool own_phi = own || (ghost && (i == 0 ? has_w : lane <= kLanes - T));
   unsigned offs[3];
-#pragma unroll
-  for (int d = 0; d < 3; ++d)
-    offs[d] = (unsigned)min(max(i + d - 1, 1), nx) * (unsigned)sizeof(double2);
+  edge_offsets(i, nx, offs);
   const unsigned offp = (unsigned)min(max(i, 0), nx + 1) * (unsigned)sizeof(double);
   const __amdgpu_buffer_rsrc_t te_out = strip_buffer(A.te_out, ny + 2);
   const scalar_ptr te_in = as_scalar(A.te_in);
@@ -373,7 +330,7 @@ __device__ __forceinline__ void strip_edge(const Args64& A, int j0, int j1, int 
   const int ra = max(1, j0 - (T - 1)), rb = j1 + (T - 1);  // rows of level 0
   auto phi_row = [&](int j) { return at(A.pa + (int64_t)min(max(j, 1), ny) * P, offp); };
   EdgeRow in;
-  load_pulled_edge(A, offs, ra, in);
+  load_pulled_edge(A.A, P, ny, offs, ra, in);
   const double ps = phi_row(ra - 1), pc = phi_row(ra);
   double pn = phi_row(ra + 1);
   double te_s = te_in[max(ra - 1, 1)], te_c = te_in[ra], te_n = te_in[min(ra + 1, ny)];
@@ -385,7 +342,7 @@ __device__ __forceinline__ void strip_edge(const Args64& A, int j0, int j1, int 
     if (r <= ny) {
       const double n3[3] = {from_west(pn), pn, from_east(pn)};
       const double tap0[9] = {c3[1], c3[2], n3[1], c3[0], s3[1], n3[2], n3[0], s3[0], s3[2]};
-      wall_f(A, i, r, frozen6, frozen7, in);
+      wall_f(nx, ny, i, r, frozen6, frozen7, in);
       wall_g(A, i, has_w, has_e, te_s, te_c, te_n, in.r.g);
       o = node_step<STEP7>(A.c, in.r.f, in.r.g, tap0);
       tav = averaged_T(o);
@@ -400,7 +357,7 @@ __device__ __forceinline__ void strip_edge(const Args64& A, int j0, int j1, int 
     te_c = te_n;
     te_n = te_in[min(r + 2, ny)];
     __builtin_amdgcn_sched_barrier(0);
-    load_pulled_edge(A, offs, min(r + 1, ny), in);
+    load_pulled_edge(A.A, P, ny, offs, min(r + 1, ny), in);
     pn = phi_row(r + 2);
     __builtin_amdgcn_sched_barrier(0);
     if (FINAL && T == 2 && r >= j0 && r <= j1 && own) halo(A, r, i, averaged(o), o.phi);
@@ -441,12 +398,12 @@ __global__ __launch_bounds__(kLanes, 2) void k_stream64(Args64 A) {
 
 }  // namespace
 
-// Lattices below 2^17 nodes stay in the caches, and the few waves they give
+// Lattices below 2^18 nodes stay in the caches, and the few waves they give
 // are bound by the latency of their rows; a handle whose ghost velocities were
 // uploaded takes the general kernel.
 bool stream64(const bgk_handle* h) {
   if (!h->ghost_uv || h->pop_variant == 1) return false;
-  return h->pop_variant > 1 || (int64_t)h->nx * h->ny >= (int64_t)1 << 17;
+  return h->pop_variant > 1 || (int64_t)h->nx * h->ny >= (int64_t)1 << 18;
 }
 
 hipError_t launch_stream64(bgk_handle* h, bool write_all) {
