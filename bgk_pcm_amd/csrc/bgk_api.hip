@@ -663,70 +663,84 @@ int bgk_diag_sums(bgk_handle* h, double out[4]) {
   return nonfinite_check(out, 2, "diag sums");
 }
 
-int bgk_gather(bgk_handle* h, int32_t field, int32_t n, const int32_t* i, const int32_t* j,
-               double* out) {
+int bgk_gather_fields(bgk_handle* h, int32_t nfields, const int32_t* fields, int32_t n,
+                      const int32_t* i, const int32_t* j, double* out) {
   int rc = check_handle(h);
   if (rc) return rc;
-  if (n < 0 || (n > 0 && (!i || !j || !out))) return fail(BGK_E_INVALID, "bad gather arguments");
+  if (nfields < 0 || (nfields > 0 && !fields) || n < 0 ||
+      (n > 0 && nfields > 0 && (!i || !j || !out)))
+    return fail(BGK_E_INVALID, "bad gather arguments");
   FieldRef r;
-  if ((rc = resolve(h, field, &r))) return rc;
+  for (int32_t f = 0; f < nfields; ++f)
+    if ((rc = resolve(h, fields[f], &r))) return rc;
   for (int32_t k = 0; k < n; ++k)
     if (i[k] < 0 || i[k] > h->nx + 1 || j[k] < 0 || j[k] > h->ny + 1)
       return fail(BGK_E_INVALID, "node (%d,%d) outside 0..%d x 0..%d", i[k], j[k], h->nx + 1,
                   h->ny + 1);
-  const double* plane = r.d64;
-  int stride = r.stride;
-  if (r.d32) {
-    HIP_TRY(bgk::launch_dev_to_f64(h, r.d32, 2, h->tmp, r.base, r.rho_table), "dev_to_f64");
-    plane = h->tmp;
-    stride = 1;
-  }
-  {
-    // through pinned memory, which the kernel reads and writes: the pairs
-    // behind the results
-    bgk::Staging s;
-    if (s.ptr()) {
-      const int64_t chunk = (int64_t)(bgk::Staging::bytes() / (2 * sizeof(double)));
-      double* const res = static_cast<double*>(s.ptr());
-      int32_t* const ij = reinterpret_cast<int32_t*>(res + chunk);
-      for (int64_t base = 0; base < n; base += chunk) {
-        const int m = (int)std::min<int64_t>(chunk, n - base);
-        for (int k = 0; k < m; ++k) {
-          ij[2 * k] = i[base + k];
-          ij[2 * k + 1] = j[base + k];
+  bgk::Staging s;
+  double* const pinned = static_cast<double*>(s.ptr());
+  // results and, behind them, the pairs: in pinned memory, which the kernel
+  // reads and writes, or (none to be had) in the handle's small buffer
+  const int64_t room = pinned ? (int64_t)(bgk::Staging::bytes() / sizeof(double)) : h->small_elems;
+  for (int32_t f0 = 0; f0 < nfields;) {
+    // FP32 deviations go through the staging plane, one field at a time
+    const double* planes[bgk::kGatherFields];
+    int strides[bgk::kGatherFields], nf = 0;
+    while (nf < bgk::kGatherFields && f0 + nf < nfields) {
+      FieldRef q;
+      if ((rc = resolve(h, fields[f0 + nf], &q))) return rc;
+      if (q.d32 && nf > 0) break;
+      if (q.d32)
+        HIP_TRY(bgk::launch_dev_to_f64(h, q.d32, 2, h->tmp, q.base, q.rho_table), "dev_to_f64");
+      planes[nf] = q.d32 ? h->tmp : q.d64;
+      strides[nf] = q.d32 ? 1 : q.stride;
+      ++nf;
+      if (q.d32) break;
+    }
+    const int64_t chunk = room / (nf + 1);
+    for (int64_t base = 0; base < n; base += chunk) {
+      const int m = (int)std::min<int64_t>(chunk, n - base);
+      double* const res = pinned ? pinned : h->small;
+      int32_t* ij = nullptr;
+      std::vector<int32_t> pairs;
+      if (m > bgk::kGatherInline) {
+        ij = reinterpret_cast<int32_t*>(res + chunk * nf);
+        int32_t* to = ij;
+        if (!pinned) {
+          try {
+            pairs.resize(2 * (size_t)m);
+          } catch (...) {
+            return fail(BGK_E_NOMEM, "host allocation");
+          }
+          to = pairs.data();
         }
-        HIP_TRY(bgk::launch_gather(h, plane, stride, m, ij, res), "gather");
-        HIP_TRY(hipStreamSynchronize(h->stream), "hipStreamSynchronize");
-        std::memcpy(out + base, res, (size_t)m * sizeof(double));
+        for (int k = 0; k < m; ++k) {
+          to[2 * k] = i[base + k];
+          to[2 * k + 1] = j[base + k];
+        }
+        if (!pinned)
+          HIP_TRY(hipMemcpyAsync(ij, to, pairs.size() * sizeof(int32_t), hipMemcpyHostToDevice,
+                                 h->stream),
+                  "hipMemcpyAsync(H2D)");
       }
-      return BGK_OK;
+      HIP_TRY(bgk::launch_gather(h, planes, strides, nf, m, i + base, j + base, ij, res), "gather");
+      for (int f = 0; f < nf && !pinned; ++f)
+        HIP_TRY(hipMemcpyAsync(out + (int64_t)(f0 + f) * n + base, res + (int64_t)f * m,
+                               (size_t)m * sizeof(double), hipMemcpyDeviceToHost, h->stream),
+                "hipMemcpyAsync(D2H)");
+      HIP_TRY(hipStreamSynchronize(h->stream), "hipStreamSynchronize");
+      for (int f = 0; f < nf && pinned; ++f)
+        std::memcpy(out + (int64_t)(f0 + f) * n + base, res + (int64_t)f * m,
+                    (size_t)m * sizeof(double));
     }
+    f0 += nf;
   }
-  // small buffer: first half outputs, second half (i,j) pairs
-  const int64_t chunk = h->small_elems / 2;
-  int32_t* ij_dev = reinterpret_cast<int32_t*>(h->small + chunk);
-  int32_t* pairs = new (std::nothrow) int32_t[2 * (size_t)std::min<int64_t>(chunk, n > 0 ? n : 1)];
-  if (!pairs) return fail(BGK_E_NOMEM, "host allocation");
-  for (int64_t base = 0; base < n; base += chunk) {
-    const int m = (int)std::min<int64_t>(chunk, n - base);
-    for (int k = 0; k < m; ++k) {
-      pairs[2 * k] = i[base + k];
-      pairs[2 * k + 1] = j[base + k];
-    }
-    hipError_t e = hipMemcpyAsync(ij_dev, pairs, (size_t)m * 2 * sizeof(int32_t),
-                                  hipMemcpyHostToDevice, h->stream);
-    if (e == hipSuccess) e = bgk::launch_gather(h, plane, stride, m, ij_dev, h->small);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(out + base, h->small, (size_t)m * sizeof(double), hipMemcpyDeviceToHost,
-                         h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (e != hipSuccess) {
-      delete[] pairs;
-      return hip_fail(e, "gather");
-    }
-  }
-  delete[] pairs;
   return BGK_OK;
+}
+
+int bgk_gather(bgk_handle* h, int32_t field, int32_t n, const int32_t* i, const int32_t* j,
+               double* out) {
+  return bgk_gather_fields(h, 1, &field, n, i, j, out);
 }
 
 int bgk_adj_setup_levels(bgk_handle* h, int32_t nsteps, int32_t seg_outer, int32_t seg_inner,

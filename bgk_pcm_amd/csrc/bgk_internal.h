@@ -150,8 +150,12 @@ hipError_t launch_initialization32(bgk_handle* h);
 hipError_t launch_field_sums(bgk_handle* h, double* out_dev);
 // diag sums (bgk_diag_sums layout)
 hipError_t launch_diag_sums(bgk_handle* h, double* out_dev);
-hipError_t launch_gather(bgk_handle* h, const double* plane, int stride, int n,
-                         const int32_t* ij_dev, double* out_dev);
+// values of nf planes at n nodes: (i[k], j[k]) for n <= kGatherInline and ij_dev
+// null, or the pairs at ij_dev; out_dev[f*n + k]
+constexpr int kGatherFields = 8, kGatherInline = 32;
+hipError_t launch_gather(bgk_handle* h, const double* const* planes, const int* strides, int nf,
+                         int n, const int32_t* i, const int32_t* j, const int32_t* ij_dev,
+                         double* out_dev);
 
 int reduce_partial_count(const bgk_handle* h);
 // field_check's sums over the interior of three caller-owned planes, with the

@@ -134,11 +134,24 @@ __global__ __launch_bounds__(RB) void k_final(const CSum* __restrict__ part, int
     for (int k = 0; k < nk; ++k) out[k] = acc[k].s + acc[k].c;
 }
 
-__global__ void k_gather(const double* __restrict__ plane, int stride, int64_t pitch, int n,
-                         const int32_t* __restrict__ ij, double* __restrict__ out) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+// Values of up to kGatherFields planes at n nodes: out[f*n + t].  Few nodes
+// (kGatherInline) come in the kernel's arguments instead of from memory, which
+// for a probe spares a read over the bus.  A launch and the wait for it are
+// all that a probe costs, so its five fields share one (97 x 61, a step and a
+// probe in turn, us of each pair: 98 with a launch and a wait per field, 24 so).
+struct GatherPlanes {
+  const double* p[kGatherFields];
+  int stride[kGatherFields];
+};
+struct GatherNodes {
+  int32_t ij[2 * kGatherInline];
+};
+__global__ void k_gather(GatherPlanes g, int64_t pitch, int n, const int32_t* __restrict__ ij,
+                         GatherNodes few, double* __restrict__ out) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x, f = blockIdx.y;
   if (t >= n) return;
-  out[t] = plane[((int64_t)ij[2 * t + 1] * pitch + ij[2 * t]) * stride];
+  const int i = ij ? ij[2 * t] : few.ij[2 * t], j = ij ? ij[2 * t + 1] : few.ij[2 * t + 1];
+  out[(int64_t)f * n + t] = g.p[f][((int64_t)j * pitch + i) * g.stride[f]];
 }
 
 inline int nparts(const Geom& g) { return g.ny < MAX_PARTS ? g.ny : MAX_PARTS; }
@@ -213,10 +226,22 @@ hipError_t launch_diag_sums(bgk_handle* h, double* out_dev) {
   return hipGetLastError();
 }
 
-hipError_t launch_gather(bgk_handle* h, const double* plane, int stride, int n,
-                         const int32_t* ij_dev, double* out_dev) {
-  hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream,
-                     plane, stride, h->geom.pitch, n, ij_dev, out_dev);
+hipError_t launch_gather(bgk_handle* h, const double* const* planes, const int* strides, int nf,
+                         int n, const int32_t* i, const int32_t* j, const int32_t* ij_dev,
+                         double* out_dev) {
+  GatherPlanes g{};
+  for (int f = 0; f < nf; ++f) {
+    g.p[f] = planes[f];
+    g.stride[f] = strides[f];
+  }
+  GatherNodes few{};
+  if (!ij_dev)
+    for (int k = 0; k < n; ++k) {
+      few.ij[2 * k] = i[k];
+      few.ij[2 * k + 1] = j[k];
+    }
+  hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256), (unsigned)nf), dim3(256), 0,
+                     h->stream, g, h->geom.pitch, n, ij_dev, few, out_dev);
   return hipGetLastError();
 }
 

@@ -126,14 +126,15 @@ module bgk_gpu
        type(c_ptr), value :: h
        real(c_double), intent(out) :: out(4)
      end function
-     integer(c_int) function c_bgk_gather(h, field, n, i, j, out) bind(C, name='bgk_gather')
+     integer(c_int) function c_bgk_gather_fields(h, nfields, fields, n, i, j, out) &
+         bind(C, name='bgk_gather_fields')
        import :: c_ptr, c_int, c_int32_t, c_double
        type(c_ptr), value :: h
-       integer(c_int32_t), value :: field, n
-       integer(c_int32_t), intent(in) :: i(*), j(*)
+       integer(c_int32_t), value :: nfields, n
+       integer(c_int32_t), intent(in) :: fields(*), i(*), j(*)
        real(c_double), intent(out) :: out(*)
      end function
-     integer(c_int) function c_bgk_set_extensions(h, e) bind(C, name='bgk_set_extensions')
+    integer(c_int) function c_bgk_set_extensions(h, e) bind(C, name='bgk_set_extensions')
        import :: c_ptr, c_int, bgk_ext_t
        type(c_ptr), value :: h
        type(bgk_ext_t), intent(in) :: e
@@ -332,10 +333,8 @@ contains
     integer(c_int32_t), intent(in) :: ii(n), jj(n)
     real(c_double), intent(out) :: vals(n, 5)
     integer(c_int32_t), parameter :: ids(5) = [F_U, F_V, F_RHO, F_T, F_PHI]
-    integer :: k
-    do k = 1, 5
-       call check(c_bgk_gather(handle, ids(k), int(n, c_int32_t), ii, jj, vals(:, k)), 'bgk_gather')
-    end do
+    call check(c_bgk_gather_fields(handle, 5_c_int32_t, ids, int(n, c_int32_t), ii, jj, vals), &
+         'bgk_gather_fields')
   end subroutine gather5
 
   ! STEP_7/field_check.f90:11-24 -> fort.64

@@ -34,6 +34,8 @@ FIELD_NAMES = (
     + ["rho", "u", "v", "T", "rho2", "u2", "v2", "T2", "phi", "phi_prec"]
 )
 FIELD_ID = {n: k for k, n in enumerate(FIELD_NAMES)}
+# the fields of the reference's probe and profiles, in their order
+_PROFILE = np.array([FIELD_ID[f] for f in ("u", "v", "rho", "T", "phi")], dtype=np.int32)
 
 ERRORS = {0: "BGK_OK", -1: "BGK_E_INVALID", -2: "BGK_E_HIP", -3: "BGK_E_NOMEM",
           -4: "BGK_E_UNSUPPORTED", -5: "BGK_E_NODEVICE"}
@@ -96,6 +98,7 @@ SIGNATURES = {
     "bgk_mass_check": [_H, _D],
     "bgk_diag_sums": [_H, _D],
     "bgk_gather": [_H, ctypes.c_int32, ctypes.c_int32, _I32P, _I32P, _D],
+    "bgk_gather_fields": [_H, ctypes.c_int32, _I32P, ctypes.c_int32, _I32P, _I32P, _D],
     "bgk_synchronize": [_H],
     "bgk_get_info": [_H, ctypes.POINTER(BgkInfoC)],
     "bgk_adj_setup": [_H, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _I32P, _I32P],
@@ -327,22 +330,29 @@ class Lattice:
                                     jj.ctypes.data_as(_I32P), out.ctypes.data_as(_D)))
         return out
 
+    def _profile(self, i: np.ndarray, j: np.ndarray) -> np.ndarray:
+        """u, v, rho, T, phi at the nodes (i, j): (nodes, 5), in one call."""
+        n = int(i.size)
+        out = np.empty((len(_PROFILE), n), dtype=np.float64)
+        _check(self._lib.bgk_gather_fields(self._h, len(_PROFILE), _PROFILE.ctypes.data_as(_I32P),
+                                           n, i.ctypes.data_as(_I32P), j.ctypes.data_as(_I32P),
+                                           out.ctypes.data_as(_D)))
+        return out.T
+
     def probe(self) -> list:
         """u, v, rho, T, phi at (Nx/2, Ny/2) (STEP_7/probe.f90:7-15)."""
-        i, j = [self.nx // 2], [self.ny // 2]
-        return [float(self.gather(f, i, j)[0]) for f in ("u", "v", "rho", "T", "phi")]
+        ij = np.array([self.nx // 2, self.ny // 2], dtype=np.int32)
+        return [float(x) for x in self._profile(ij[:1], ij[1:])[0]]
 
     def prof_x(self) -> np.ndarray:
         """Rows i=1..Nx of u, v, rho, T, phi at j=Ny/2 (STEP_7/prof_x.f90:7-17)."""
-        i = np.arange(1, self.nx + 1)
-        j = np.full_like(i, self.ny // 2)
-        return np.stack([self.gather(f, i, j) for f in ("u", "v", "rho", "T", "phi")], axis=1)
+        i = np.arange(1, self.nx + 1, dtype=np.int32)
+        return np.ascontiguousarray(self._profile(i, np.full_like(i, self.ny // 2)))
 
     def prof_y(self) -> np.ndarray:
         """Columns j=1..Ny of u, v, rho, T, phi at i=Nx/2 (STEP_7/prof_y.f90:7-17)."""
-        j = np.arange(1, self.ny + 1)
-        i = np.full_like(j, self.nx // 2)
-        return np.stack([self.gather(f, i, j) for f in ("u", "v", "rho", "T", "phi")], axis=1)
+        j = np.arange(1, self.ny + 1, dtype=np.int32)
+        return np.ascontiguousarray(self._profile(np.full_like(j, self.nx // 2), j))
 
     # ---- runtime
     def set_stream(self, stream_ptr: int | None) -> None:

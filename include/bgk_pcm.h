@@ -260,6 +260,11 @@ int bgk_diag_sums(bgk_handle* h, double out[4]);
 int bgk_gather(bgk_handle* h, int32_t field, int32_t n, const int32_t* i,
                const int32_t* j, double* out);
 
+/* The same of several fields at once: out[f*n + k] = fields[f] at node k (one
+ * launch and one wait where nfields bgk_gather calls make as many each). */
+int bgk_gather_fields(bgk_handle* h, int32_t nfields, const int32_t* fields, int32_t n,
+                      const int32_t* i, const int32_t* j, double* out);
+
 /* Wait for all queued work of the handle. */
 int bgk_synchronize(bgk_handle* h);
 

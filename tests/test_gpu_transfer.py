@@ -42,6 +42,29 @@ def test_gather_of_more_nodes_than_a_buffer():
                 assert np.array_equal(lat.gather(f, i, j), lat.download(f)[j, i]), (prec, f)
 
 
+def test_gather_of_several_fields():
+    """More fields than a launch takes, FP32 deviations among them, and node
+    counts on either side of what the launch's arguments hold."""
+    names = ["T", "f5", "u", "phi", "g0", "v", "rho", "f1", "g8", "T", "phi_prec"]
+    ids = np.array([FIELD_ID[f] for f in names], dtype=np.int32)
+    r = np.random.default_rng(2)
+    P32, PD = ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_double)
+    for prec in (0, FP32_DEV):
+        with Lattice(Params(nx=50, ny=40, precision=prec), **EXT) as lat:
+            lat.step(3)
+            for n in (0, 1, 32, 33, 400):
+                i = r.integers(0, 52, n).astype(np.int32)
+                j = r.integers(0, 42, n).astype(np.int32)
+                out = np.empty((len(names), n))
+                rc = lat._lib.bgk_gather_fields(lat._h, len(names), ids.ctypes.data_as(P32), n,
+                                                i.ctypes.data_as(P32), j.ctypes.data_as(P32),
+                                                out.ctypes.data_as(PD))
+                assert rc == 0
+                for k, f in enumerate(names):
+                    assert np.array_equal(out[k], lat.download(f)[j, i]), (prec, n, f)
+            assert np.array_equal(lat.prof_x()[24], np.array(lat.probe()))
+
+
 def test_two_threads_with_a_handle_each():
     bad = []
 
