@@ -1149,39 +1149,42 @@ hipError_t adj_forward(bgk_handle* h, double* probe_T_host) {
   if (e != hipSuccess) return e;
   size_t next_chain = 0;
   const int lvl1 = x->seg1 > 0 ? x->seg1 : x->seg;
-  for (int n = 0; n < x->nsteps;) {
-    const int a = h->cur, b = 1 - h->cur;
-    StatePtrs in{h->ma[a], h->mb[a], h->mc[a], h->phi[h->pc], h->teast[h->te_cur]};
-    StatePtrs out{h->ma[b], h->mb[b], h->mc[b], h->phi[1 - h->pc], h->teast[1 - h->te_cur]};
+  // the state before step 0: the handle's own, kept as a copy
+  StatePtrs in{h->ma[h->cur], h->mb[h->cur], h->mc[h->cur], h->phi[h->pc], h->teast[h->te_cur]};
+  const StatePtrs& first = x->nsnap > 0 ? x->snap[0] : x->ckpt[0];
+  e = copy_state(h, first, in.a, in.b, in.c, in.phi, in.te);
+  for (int n = 0; e == hipSuccess && n < x->nsteps;) {
+    // the next state to keep, if any: the launch that reaches it writes it in
+    // its place, and the one after reads it there, so no state but the first
+    // is copied (2048^2, FP32, 12 states kept of 48 steps: 11 copies of 84 us
+    // less in 4 ms)
+    int stop = x->nsteps;
     const StatePtrs* keep = nullptr;
     if (x->nsnap > 0) {
-      if (n == 0) {
-        keep = &x->snap[0];
-      } else if (next_chain < x->chain.size() && x->chain[next_chain] == n) {
+      if (next_chain < x->chain.size()) {
+        stop = x->chain[next_chain];
         keep = &x->snap[next_chain + 1];
-        ++next_chain;
       }
-    } else if (n % lvl1 == 0) {
-      keep = &x->ckpt[(size_t)(n / lvl1)];
-    }
-    if (keep) {
-      e = copy_state(h, *keep, in.a, in.b, in.c, in.phi, in.te);
-      if (e != hipSuccess) return e;
-    }
-    // steps to the next state to keep
-    int stop = x->nsteps;
-    if (x->nsnap > 0) {
-      if (next_chain < x->chain.size()) stop = std::min(stop, x->chain[next_chain]);
-    } else {
-      stop = std::min(stop, (n / lvl1 + 1) * lvl1);
+    } else if ((n / lvl1 + 1) * lvl1 < x->nsteps) {
+      stop = (n / lvl1 + 1) * lvl1;
+      keep = &x->ckpt[(size_t)(stop / lvl1)];
     }
     const int T = mom_next_steps(h, stop - n);
+    const int b = 1 - h->cur;
+    const StatePtrs own{h->ma[b], h->mb[b], h->mc[b], h->phi[1 - h->pc], h->teast[1 - h->te_cur]};
+    const bool kept = keep && n + T == stop;
+    const StatePtrs out = kept ? *keep : own;
     e = fwd_steps(h, T, in, out, x->np > 0 ? x->probe_T + (size_t)n * x->np : nullptr,
                   x->probe_idx, x->np, mom_write_all(h, T, x->nsteps - n - T), nullptr);
     if (e != hipSuccess) return e;
-    h->cur = b;
-    h->pc = 1 - h->pc;
-    h->te_cur = 1 - h->te_cur;
+    if (kept) {
+      if (x->nsnap > 0) ++next_chain;
+    } else {
+      h->cur = b;
+      h->pc = 1 - h->pc;
+      h->te_cur = 1 - h->te_cur;
+    }
+    in = out;
     n += T;
   }
   if (x->np > 0)
