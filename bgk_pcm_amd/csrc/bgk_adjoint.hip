@@ -18,8 +18,8 @@
 // pulled from it, and turns it into the adjoint of its own stored moments
 // through the derivative of the population rebuild.  The node update is
 // reversed by hand (core_backward below), on values recomputed with the
-// same core_forward the forward kernels run: the adjoint of step n reads
-// only the state before step n.
+// same node update the forward kernels run (core_from_sums, bgk_mom.h): the
+// adjoint of step n reads only the state before step n.
 //
 // Checkpointing, binomial (bgk_adj_setup_binomial): the optimal schedule for
 // a number of state slots (see rev_cost below).  Levels (bgk_adj_setup,
@@ -33,14 +33,18 @@
 #include <algorithm>
 #include <cstring>
 #include <new>
+#include <type_traits>
 #include <vector>
 
-#include "bgk_mom.h"
+#include "bgk_level.h"
+
+// (the adjoint's arithmetic need not be the same in two instantiations)
+#pragma clang fp contract(fast)
 
 namespace bgk {
 namespace {
 
-using namespace mom;
+using namespace level;
 
 // one stored state: moment planes, phi, east-wall column
 struct StatePtrs {
@@ -51,131 +55,34 @@ struct StatePtrs {
   double* te;
 };
 
-// adjoint planes of one step (structure of arrays, node q at [q]), stored
-// in the state's precision R (the arithmetic is FP64 either way)
+// Adjoint of one step as stored and computed, in the state's precision: node q
+// at [q] of
+//   v[0] (rho, jx, jy, dT)  v[1] (gxx, gyy, gxy, kp)  v[2] (km, pc)
+// and, unless omega_f = 1, v[2] (km, pc, fxx, fyy)  v[3] fxy.
 struct AdjPlanes {
-  void* v[13];  // rho jx jy fxx fyy fxy dT gxx gyy gxy kp km pc
+  void* v[4];
 };
-template <typename R>
-__device__ __forceinline__ double plane_at(const AdjPlanes& L, int p, int64_t q) {
-  return (double)static_cast<const R*>(L.v[p])[q];
-}
-template <typename R>
-__device__ __forceinline__ void plane_set(const AdjPlanes& L, int p, int64_t q, double x) {
-  static_cast<R*>(L.v[p])[q] = (R)x;
-}
-enum { L_RHO, L_JX, L_JY, L_FXX, L_FYY, L_FXY, L_DT, L_GXX, L_GYY, L_GXY, L_KP, L_KM, L_PC };
 
 struct AdjArgs {
   // the state before step n (the inputs of step n); the state after it, whose
   // moments the gather of step n+1's pulls differentiates at, is recomputed
-  // from it in the kernel (core = 1) or is this state itself (core = 0)
+  // from it in the kernel, or is this state itself (the launch for the
+  // initial state)
   StatePtrs sprev;
-  const double* uh;  // macroscopic u, v planes: their halo columns are the ghost velocities
-  const double* vh;
-  AdjPlanes next;    // adjoint of step n+1 (read)
-  AdjPlanes cur;     // adjoint of step n (written)
-  int has_next;      // 0 at the last step: no step n+1
-  int core;          // 0: only the gather (the initial state)
+  AdjPlanes next;  // adjoint of step n+1 (read)
+  AdjPlanes cur;   // adjoint of step n (written)
+  int has_next;    // 0 at the last step: no step n+1
   const int* probe_idx;
   const double* seeds;  // dL/dT at the probes after step n (null: none)
   double* partial;      // 3 per workgroup: dL/dSt, dL/dk_ratio, dL/dt_hot (accumulated)
   Consts c;
-  ConstsF cf;  // FP32 copies for the FP32 kernel
-  Geom gm;
+  ConstsF cf;    // FP32 copies for the FP32 kernel
+  double gd[9];  // d (thermal ghost of direction k) / dT
+  int nx, ny;
+  int64_t pitch;
   int interf;
-  int ntx, nty;  // tiles across and down
+  WaveGrid g;
 };
-
-// The workgroup's window in LDS: a tile of BX x BY nodes and a one-node
-// halo, with the adjoint planes of step n+1 (those read at neighbours: not
-// L_PC, and with omega_f = 1 (EQF) not the second moments of f, whose
-// adjoints are (1 - omega_f) times finite values, exact zeros, and are
-// neither stored nor read) and the state before step n (moments and phi).
-// Every read of a node's update lies in its 3 x 3 neighbourhood, so each
-// value comes from HBM once per tile instead of from L2 for every neighbour.
-// Tiles of 64 x 8 nodes (one workgroup of 8 waves) with FP32 moments, 64 x 4
-// (4 waves) with FP64 moments.  The window holds 68 B per node with FP32
-// moments and omega_f = 1 (45 KB at 64 x 8: three workgroups per CU, 6
-// waves per SIMD, 72 VGPRs), 92 B with the general FP32 layout (61 KB: 4
-// waves per SIMD), 136 B and 168 B with FP64 moments (64 x 4: 3 and 2 waves
-// per SIMD).  Measured at 8192^2 (FP32, omega_f = 1, XCD bands of 8-tile
-// groups) per launch: 64 x 8 2.05 ms, 64 x 12 (two workgroups of 12 waves)
-// 2.07 ms, 64 x 4 (six of 4 waves) 2.19 ms.  Per wave: 765 VALU
-// instructions, and HBM reads of 1.17x the algorithmic bytes (the halo
-// rows and columns are L2 hits, see tile_of).
-constexpr int BX = 64, WX = BX + 2;
-template <typename R, bool EQF>
-constexpr int tile_rows() {
-  return sizeof(R) == sizeof(float) ? 8 : 4;
-}
-
-// Window types of the state's FP64 members (rho, T - T_crit and phi): the
-// FP32 kernel evaluates in FP32, so its window holds them rounded once, in
-// 12 bytes instead of 24.
-template <typename R>
-struct WinT {
-  using A2 = double2;
-  using P = double;
-  static __device__ __forceinline__ A2 a2(const double2 v) { return v; }
-};
-template <>
-struct WinT<float> {
-  using A2 = float2;
-  using P = float;
-  static __device__ __forceinline__ A2 a2(const double2 v) {
-    return make_float2((float)v.x, (float)v.y);
-  }
-};
-
-template <bool EQF>
-struct LSlots {
-  static constexpr int N = EQF ? 9 : 12;
-  // plane staged in LDS slot s
-  static constexpr int plane[12] = {L_RHO, L_JX, L_JY, L_DT, L_GXX, L_GYY,
-                                    L_GXY, L_KP, L_KM, L_FXX, L_FYY, L_FXY};
-  enum { RHO, JX, JY, DT, GXX, GYY, GXY, KP, KM, FXX, FYY, FXY };
-};
-
-template <typename R, bool EQF>
-struct Win {
-  static constexpr int WY = tile_rows<R, EQF>() + 2;
-  R lam[LSlots<EQF>::N][WY][WX];  // as stored: every read widens exactly
-  typename WinT<R>::A2 a[WY][WX];
-  typename Vec<R>::V4 b[WY][WX];
-  typename CType<R, EQF>::T c[WY][WX];
-  typename WinT<R>::P phi[WY][WX];
-};
-
-// Adjoint of population k as pulled by the node at window (x, y), from that
-// node's adjoint of its pulled moments (PullSums is linear in the
-// populations).
-template <typename R, bool EQF>
-__device__ __forceinline__ R lam_f(const Win<R, EQF>& W, int k, int x, int y) {
-  using S = LSlots<EQF>;
-  R r = W.lam[S::RHO][y][x];
-  if constexpr (EQF) {
-    if (CX[k] != 0) r += CX[k] > 0 ? W.lam[S::JX][y][x] : -W.lam[S::JX][y][x];
-    if (CY[k] != 0) r += CY[k] > 0 ? W.lam[S::JY][y][x] : -W.lam[S::JY][y][x];
-  } else {
-    if (CX[k] != 0)
-      r += (CX[k] > 0 ? W.lam[S::JX][y][x] : -W.lam[S::JX][y][x]) + W.lam[S::FXX][y][x];
-    if (CY[k] != 0)
-      r += (CY[k] > 0 ? W.lam[S::JY][y][x] : -W.lam[S::JY][y][x]) + W.lam[S::FYY][y][x];
-    if (CX[k] * CY[k] != 0)
-      r += CX[k] * CY[k] > 0 ? W.lam[S::FXY][y][x] : -W.lam[S::FXY][y][x];
-  }
-  return r;
-}
-template <typename R, bool EQF>
-__device__ __forceinline__ R lam_g(const Win<R, EQF>& W, int k, int x, int y) {
-  using S = LSlots<EQF>;
-  R r = W.lam[S::DT][y][x];
-  if (CX[k] != 0) r += W.lam[S::GXX][y][x];
-  if (CY[k] != 0) r += W.lam[S::GYY][y][x];
-  if (CX[k] * CY[k] != 0) r += CX[k] * CY[k] > 0 ? W.lam[S::GXY][y][x] : -W.lam[S::GXY][y][x];
-  return r;
-}
 
 // Stored moments of a node (EQF: Pf = 0), or their adjoints, in the
 // arithmetic type A.
@@ -184,9 +91,9 @@ struct Mom {
   A rho, th, u, v, pf[3], pg[3];
 };
 
-// The moments a forward step stores for a node (bgk_fused_mom.hip's
-// update_node), widened back to FP64: rho and T - T_crit as computed, u, v
-// and the scaled non-equilibrium moments rounded to the storage type R.
+// The moments a forward step stores for a node, widened back to A: rho and T -
+// T_crit as computed, u, v and the scaled non-equilibrium moments rounded to
+// the storage type R.
 template <typename R, bool EQF, typename A, typename C>
 __device__ __forceinline__ Mom<A> stored_mom(const C& c, const CoreT<A>& o) {
   Mom<A> m;
@@ -209,62 +116,175 @@ __device__ __forceinline__ Mom<A> stored_mom(const C& c, const CoreT<A>& o) {
   return m;
 }
 
-// Moments of a node held in the window (the state before the step).
-template <typename R, bool EQF, typename A, typename A2>
-__device__ __forceinline__ Mom<A> win_mom(const A2& a, const typename Vec<R>::V4& b,
-                                          const typename CType<R, EQF>::T& cc) {
-  Mom<A> m;
-  m.rho = (A)a.x;
-  m.th = (A)a.y;
-  m.u = (A)b.x;
-  m.v = (A)b.y;
-  if constexpr (EQF) {
-    m.pf[0] = m.pf[1] = m.pf[2] = A(0);
-    m.pg[0] = (A)b.z;
-    m.pg[1] = (A)b.w;
-    m.pg[2] = (A)cc;
-  } else {
-    m.pf[0] = (A)b.z;
-    m.pf[1] = (A)b.w;
-    m.pf[2] = (A)cc.x;
-    m.pg[0] = (A)cc.y;
-    m.pg[1] = (A)cc.z;
-    m.pg[2] = (A)cc.w;
-  }
-  return m;
-}
-
 // Weighted moments sum_k w_k c_k^n a_k (n = 0, 1, 2) of a vector over the
 // nine directions.
 template <typename A>
 struct WMom {
   A m0, mx, my, mxx, myy, mxy;
 };
+
+// The share of the three directions with c_y = 1 (or -1) in them: c the value
+// of the axis direction, e and w those of the diagonals with c_x = 1 and -1.
 template <typename A>
-__device__ __forceinline__ WMom<A> wmoments(const A a[9]) {
-  const A s13 = a[1] + a[3], s24 = a[2] + a[4];
-  const A sd = (a[5] + a[6]) + (a[7] + a[8]);
-  WMom<A> m;
-  m.m0 = A(kW[0]) * a[0] + A(kW[1]) * (s13 + s24) + A(kW[5]) * sd;
-  m.mx = A(kW[1]) * (a[1] - a[3]) + A(kW[5]) * ((a[5] + a[8]) - (a[6] + a[7]));
-  m.my = A(kW[1]) * (a[2] - a[4]) + A(kW[5]) * ((a[5] + a[6]) - (a[7] + a[8]));
-  m.mxx = A(kW[1]) * s13 + A(kW[5]) * sd;
-  m.myy = A(kW[1]) * s24 + A(kW[5]) * sd;
-  m.mxy = A(kW[5]) * ((a[5] + a[7]) - (a[6] + a[8]));
-  return m;
+__device__ __forceinline__ TripleT<A> weighted(A c, A e, A w) {
+  const A p = A(kW[5]) * (e + w);
+  return TripleT<A>{A(kW[1]) * c + p, p, A(kW[5]) * (e - w)};
+}
+template <typename A>
+__device__ __forceinline__ void add_north(WMom<A>& m, const TripleT<A>& t) {
+  m.m0 += t.n;
+  m.mx += t.d;
+  m.my += t.n;
+  m.mxx += t.p;
+  m.myy += t.n;
+  m.mxy += t.d;
+}
+template <typename A>
+__device__ __forceinline__ void add_south(WMom<A>& m, const TripleT<A>& t) {
+  m.m0 += t.n;
+  m.mx += t.d;
+  m.my -= t.n;
+  m.mxx += t.p;
+  m.myy += t.n;
+  m.mxy -= t.d;
+}
+// c_y = 0: s the southern share, a0, e, w the values of directions 0, 1, 3
+template <typename A>
+__device__ __forceinline__ WMom<A> centre(const TripleT<A>& s, A a0, A e, A w) {
+  const A p = A(kW[1]) * (e + w);
+  return WMom<A>{A(kW[0]) * a0 + p + s.n, A(kW[1]) * (e - w) + s.d, -s.n, p + s.p, s.n, -s.d};
 }
 
-// Accumulate into lm the adjoint of the node's moments from the adjoints
-// lf[k], lg[k] of its nine populations f_k and gd_k (the transposed rebuild
-// Jacobian).  Population k is w_k rho (1 + p_k) + c_k H_k : Pf for f and
-// w_k (dT + T p_k) + c_k H_k : Pg for gd, with p_k = 3 cu + 9/2 cu^2 -
-// 3/2 |u|^2, cu = c_k . u, c_k = w_k / (2 cs^4) and H_k = c_k c_k - cs^2 I;
-// its derivatives are polynomials in c_k, so the sums over k reduce to the
-// weighted moments of lf and lg.
+// The adjoints of a step's pulled sums and taps at a node.
 template <typename A>
-__device__ __forceinline__ void rebuild_adjoint(const Mom<A>& m, const A lf[9], const A lg[9],
-                                                Mom<A>* lm) {
-  const WMom<A> F = wmoments<A>(lf), G = wmoments<A>(lg);
+struct Lam {
+  A rho, jx, jy, fxx, fyy, fxy, dT, gxx, gyy, gxy, kp, km, pc;
+};
+
+// Registers of the gather between two rows: what the row awaiting its northern
+// neighbours has so far, and the southern share of the row after it.  te: the
+// adjoint of the east wall's temperature (column Nx).
+template <typename A>
+struct AdjLevel {
+  WMom<A> F, G;
+  A kp, km, te, pc;
+  TripleT<A> sf, sg;
+  A skp, skm, ste;
+};
+
+// Reverse of step n+1's pulls.  Population k as pulled by node x has the adjoint
+// (rho + c j + c c : f)(x), which belongs to node x - c_k: feed row j (1..Ny, or
+// Ny+1: nothing more comes) of these, one node per lane; gives row j - 1's
+// weighted moments F, G over its nine populations, the sums over the nine
+// nodes that read its phi, and tin, row j's adjoint of the west wall's
+// temperature.
+//
+// Boundaries (feed in bgk_level.h): a direction pulled from a ghost was the
+// node's own opposite population (not the two frozen corners); rows 0 and
+// Ny+1 of g and phi were rows 1 and Ny; the ghosts of columns 0 and Nx+1 are
+// thermal equilibria (gd their derivative).  Lanes outside 1..Nx carry zeros.
+template <bool EQF, bool EDGE, typename A>
+__device__ __forceinline__ void feed_adjoint(AdjLevel<A>& L, const Lam<A>& x, int j, int ny, int i,
+                                             int nx, bool has_w, bool has_e, const A gd[9],
+                                             AdjLevel<A>* out, A* tin) {
+  *out = L;
+  *tin = A(0);
+  if (EDGE && j > ny) return;
+  A fx = x.rho, fy = x.rho, fp = x.rho, fm = x.rho;
+  if constexpr (!EQF) {
+    fx += x.fxx;
+    fy += x.fyy;
+    const A d = fx + x.fyy;
+    fp = d + x.fxy;
+    fm = d - x.fxy;
+  }
+  const A jp = x.jx + x.jy, jm = x.jx - x.jy;
+  const A f1 = fx + x.jx, f3 = fx - x.jx, f2 = fy + x.jy, f4 = fy - x.jy;
+  const A f5 = fp + jp, f7 = fp - jp, f8 = fm + jm, f6 = fm - jm;
+  const A g1 = x.dT + x.gxx, g2 = x.dT + x.gyy, gs = g1 + x.gyy;
+  const A g5 = gs + x.gxy, g6 = gs - x.gxy;  // directions 5 and 7, 6 and 8
+  const A rkp = (from_west(x.kp) + from_east(x.kp)) + x.kp;
+  const A rkm = (from_west(x.km) + from_east(x.km)) + x.km;
+  const A g5w = from_west(g5), g5e = from_east(g5), g6w = from_west(g6), g6e = from_east(g6);
+  // row j - 1 pulled from here with directions 4, 7, 8: its 2, 5, 6
+  const TripleT<A> nf = weighted(f2, from_east(f5), from_west(f6));
+  const TripleT<A> ng = weighted(g2, g5e, g6w);
+  add_north(out->F, nf);
+  add_north(out->G, ng);
+  out->kp += rkp;
+  out->km += rkm;
+  // and row j + 1
+  const TripleT<A> uf = weighted(f4, from_east(f8), from_west(f7));
+  const TripleT<A> ug = weighted(g2, g6e, g5w);
+  if (EDGE && has_e) out->te += gd[6] * g6;
+  if (EDGE && j == 1) {
+    L.sf = weighted(f2, i == nx ? A(0) : f6, f5);
+    L.sg = TripleT<A>{A(0), A(0), A(0)};
+    L.skp = rkp;
+    L.skm = rkm;
+    L.ste = A(0);
+  }
+  L.F = centre(L.sf, x.rho, from_east(f1), from_west(f3));
+  L.G = centre(L.sg, x.dT, from_east(g1), from_west(g1));
+  L.kp = L.skp + rkp;
+  L.km = L.skm + rkm;
+  L.pc = x.pc;
+  if (EDGE) {
+    L.te = L.ste + gd[3] * g1;
+    if (j == 1) {
+      add_north(L.G, ng);
+      L.te += gd[6] * g6;
+    }
+    if (j == ny) {
+      add_north(L.F, weighted(f4, i == nx ? A(0) : f7, f8));
+      add_south(L.G, ug);
+      L.kp += rkp;
+      L.km += rkm;
+      L.te += gd[7] * g5;
+    }
+    if (has_w) {  // column 1: directions 1, 5, 8 were its own 3, 7, 6
+      const bool on = i == 1;
+      const A a = on ? A(kW[1]) * f1 : A(0);
+      const A b = on && j != 1 ? A(kW[5]) * f5 : A(0);
+      const A d = on && j != ny ? A(kW[5]) * f8 : A(0);
+      L.F.m0 += a + b + d;
+      L.F.mx -= a + b + d;
+      L.F.my += d - b;
+      L.F.mxx += a + b + d;
+      L.F.myy += b + d;
+      L.F.mxy += b - d;
+      if (on) *tin = gd[1] * g1 + gd[5] * g5 + gd[8] * g6;
+    }
+    if (has_e) {  // column Nx: directions 3, 6, 7 were its own 1, 8, 5
+      const bool on = i == nx;
+      const A a = on ? A(kW[1]) * f3 : A(0);
+      const A b = on && j != 1 ? A(kW[5]) * f6 : A(0);
+      const A d = on && j != ny ? A(kW[5]) * f7 : A(0);
+      L.F.m0 += a + b + d;
+      L.F.mx += a + b + d;
+      L.F.my += d - b;
+      L.F.mxx += a + b + d;
+      L.F.myy += b + d;
+      L.F.mxy += d - b;
+    }
+    L.ste = gd[7] * g5;
+  }
+  L.sf = uf;
+  L.sg = ug;
+  L.skp = rkp;
+  L.skm = rkm;
+}
+
+// Accumulate into lm the adjoint of the node's moments from the weighted
+// moments F, G of the adjoints of its nine populations f_k and gd_k (the
+// transposed rebuild Jacobian).  Population k is w_k rho (1 + p_k) + c_k H_k :
+// Pf for f and w_k (dT + T p_k) + c_k H_k : Pg for gd, with p_k = 3 cu + 9/2
+// cu^2 - 3/2 |u|^2, cu = c_k . u, c_k = w_k / (2 cs^4) and H_k = c_k c_k - cs^2
+// I; its derivatives are polynomials in c_k, so the sums over k reduce to the
+// weighted moments.
+template <typename A>
+__device__ __forceinline__ void rebuild_adjoint(const Mom<A>& m, const WMom<A>& F,
+                                                const WMom<A>& G, Mom<A>* lm) {
   const A u = m.u, v = m.v, uu = u * u, vv = v * v, uv2 = A(2) * u * v;
   const A c0 = A(1) - A(1.5) * (uu + vv);
   // sum_k w_k a_k (1 + p_k)
@@ -289,86 +309,39 @@ __device__ __forceinline__ void rebuild_adjoint(const Mom<A>& m, const A lf[9], 
   lm->pg[2] += A(9) * G.mxy;
 }
 
-// d ghost_gdev / dT for direction k at velocity (u, v)
-template <typename A>
-__device__ __forceinline__ A ghost_dT(int k, A u, A v) {
-  return A(kW[k]) * (A(1) + eq_poly_t<A>(k, u, v));
-}
-
-// Pulled sums and taps of step n at node (i, j), window (ox, oy), from the
-// state before the step, with the boundary folding of the forward kernels
-// (mom_edge_nodes).  EDGE = false: the node and its eight neighbours are
-// interior nodes (no boundary tests).
-template <typename R, bool EQF, typename A, bool EDGE>
-__device__ __forceinline__ void pull_step(const AdjArgs& a, const Win<R, EQF>& W, int i, int j,
-                                          int ox, int oy, PullSumsT<A>* S, A tap[9]) {
-  const int nx = a.gm.nx, ny = a.gm.ny;
-  const int64_t P = a.gm.pitch;
-  pull_zero(*S);
-#pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    const int si = i - CX[k], sj = j - CY[k];
-    const int sjc = !EDGE ? sj : (sj < 1 ? 1 : (sj > ny ? ny : sj));
-    const int wx = ox - CX[k], wy = oy + (sjc - j);
-    A fk = A(0), gk;
-    if (!EDGE || (si >= 1 && si <= nx)) {
-      rebuild<R, EQF, A, typename WinT<R>::A2>(k, W.a[wy][wx], W.b[wy][wx], W.c[wy][wx], &fk,
-                                               &gk);
-    } else {
-      const int64_t h = (int64_t)sjc * P + si;
-      gk = ghost_gdev<A>(k, (A)(si == 0 ? a.c.tin : east_T(a.c, a.sprev.te, sjc)),
-                         (A)a.uh[h], (A)a.vh[h]);
-    }
-    if (EDGE && (si < 1 || si > nx || sj < 1 || sj > ny)) {
-      if (k == 6 && si == nx + 1 && sj == 0)
-        fk = (A)a.c.frozen6;
-      else if (k == 7 && si == nx + 1 && sj == ny + 1)
-        fk = (A)a.c.frozen7;
-      else
-        fk = rebuild_f<R, EQF, A, typename WinT<R>::A2>(OPP[k], W.a[oy][ox], W.b[oy][ox],
-                                                        W.c[oy][ox]);
-    }
-    pull_add(*S, k, fk, gk);
-  }
-  const int yn = oy + (!EDGE || j < ny ? 1 : 0), ys = oy - (!EDGE || j > 1 ? 1 : 0);
-  tap[0] = (A)W.phi[oy][ox];
-  tap[1] = (A)W.phi[oy][ox + 1];
-  tap[2] = (A)W.phi[yn][ox];
-  tap[3] = (A)W.phi[oy][ox - 1];
-  tap[4] = (A)W.phi[ys][ox];
-  tap[5] = (A)W.phi[yn][ox + 1];
-  tap[6] = (A)W.phi[yn][ox - 1];
-  tap[7] = (A)W.phi[ys][ox - 1];
-  tap[8] = (A)W.phi[ys][ox + 1];
-}
-
 // Reverse of core_forward (bgk_mom.h) and of the state it stores.  lo: the
 // adjoint of the node's stored moments after the step (rho, T - T_crit, u,
 // v, Pf, Pg) and of its phi; ldT2 an extra adjoint on the pulled T (the
 // averaged T of moments.f90 seeds half of its adjoint here).  Returns the
-// adjoints of the pulled sums in lS, of the tap sums in lkp, lkm and of the
-// centre tap (direct terms) in lpc; adds parameter adjoints to g[3].
-template <typename A, typename C>
+// adjoints of the pulled sums, of the tap sums and of the centre tap (direct
+// terms) in lS; gives the parameter adjoints of the Stefan number and k_ratio
+// in g.  EQF: (1 - omega_f) = 0, the second moments of f carry none.
+template <bool EQF, typename A, typename C>
 __device__ __forceinline__ void core_backward(const C& c, const PullSumsT<A>& S,
-                                              const A tap[9], const CoreT<A>& o, const Mom<A>& lo,
-                                              A lphi_o, A ldT2_in, PullSumsT<A>* lS, A* lkp,
-                                              A* lkm, A* lpc, A g[3]) {
+                                              const CoreT<A>& o, const Mom<A>& lo, A lphi_o,
+                                              A ldT2_in, Lam<A>* lS, A g[2]) {
   A lrho = lo.rho, lu = lo.u, lv = lo.v, lphi = lphi_o;
   A ldT2 = ldT2_in;
   // Pg = (1 - omega_g) Qg, Pf = (1 - omega_f) Qf
-  const A omg1 = A(1) - o.omega_g, omf1 = A(1) - (A)c.omega_f;
+  const A omg1 = A(1) - o.omega_g;
   const A lqgxx = omg1 * lo.pg[0], lqgyy = omg1 * lo.pg[1], lqgxy = omg1 * lo.pg[2];
   const A lomg = -(o.qgxx * lo.pg[0] + o.qgyy * lo.pg[1] + o.qgxy * lo.pg[2]);
-  const A lqfxx = omf1 * lo.pf[0], lqfyy = omf1 * lo.pf[1], lqfxy = omf1 * lo.pf[2];
   // Qg = S_g - cs2 dT2 - T u u
   ldT2 += -A(kCs2) * (lqgxx + lqgyy);
   A lT = -(o.u * o.u * lqgxx + o.v * o.v * lqgyy + o.u * o.v * lqgxy);
   lu += -A(2) * o.T * o.u * lqgxx - o.T * o.v * lqgxy;
   lv += -A(2) * o.T * o.v * lqgyy - o.T * o.u * lqgxy;
-  // Qf = S_f - cs2 rho - rho u u
-  lrho += -(A(kCs2) + o.u * o.u) * lqfxx - (A(kCs2) + o.v * o.v) * lqfyy - o.u * o.v * lqfxy;
-  lu += -A(2) * o.rho * o.u * lqfxx - o.rho * o.v * lqfxy;
-  lv += -A(2) * o.rho * o.v * lqfyy - o.rho * o.u * lqfxy;
+  if constexpr (!EQF) {
+    // Qf = S_f - cs2 rho - rho u u
+    const A omf1 = A(1) - (A)c.omega_f;
+    const A lqfxx = omf1 * lo.pf[0], lqfyy = omf1 * lo.pf[1], lqfxy = omf1 * lo.pf[2];
+    lrho += -(A(kCs2) + o.u * o.u) * lqfxx - (A(kCs2) + o.v * o.v) * lqfyy - o.u * o.v * lqfxy;
+    lu += -A(2) * o.rho * o.u * lqfxx - o.rho * o.v * lqfxy;
+    lv += -A(2) * o.rho * o.v * lqfyy - o.rho * o.u * lqfxy;
+    lS->fxx = lqfxx;
+    lS->fyy = lqfyy;
+    lS->fxy = lqfxy;
+  }
   // omega_g(phi, k_ratio) = 1 / (1/2 + alpha/cs2), alpha = alpha_l (fl +
   // k_ratio (1 - fl)): the k_ratio derivative is taken at k_ratio = 1 too,
   // where the forward uses the constant omega_g (the same value)
@@ -376,7 +349,7 @@ __device__ __forceinline__ void core_backward(const C& c, const PullSumsT<A>& S,
     const A fl = A(0.5) * (A(1) + o.phi);
     const A domg_dalpha = -o.omega_g * o.omega_g * A(3);  // 1/cs2
     lphi += lomg * domg_dalpha * (A)c.alpha_l * (A(1) - (A)c.k_ratio) * A(0.5);
-    g[1] += lomg * domg_dalpha * (A)c.alpha_l * (A(1) - fl);
+    g[1] = lomg * domg_dalpha * (A)c.alpha_l * (A(1) - fl);
   }
   // u = u2 + fx s, v = v2 + fy s, s = irho / omega_f
   const A s = o.irho * (A)c.inv_omega_f;
@@ -402,27 +375,24 @@ __device__ __forceinline__ void core_backward(const C& c, const PullSumsT<A>& S,
   lphi += -(A)c.dt_st * A(0.5) * ldT;
   A lpcv = (A)c.dt_st * A(0.5) * ldT;
   // dt_st = delta_T / St
-  g[0] += (-(o.phi - o.pc) * A(0.5) * ldT) * (-(A)c.dt_st * (A)c.inv_stefan);
+  g[0] = (-(o.phi - o.pc) * A(0.5) * ldT) * (-(A)c.dt_st * (A)c.inv_stefan);
   // phi = pc + 0.5 kpr (1 - pc) - 0.5 kmr (1 + pc), kpr = kp/8 rp, kmr = km/8 rm
   const A rp = A(1) - o.rm;
   const A kpr = o.kp_sum * A(0.125) * rp, kmr = o.km_sum * A(0.125) * o.rm;
   const A lkpr = A(0.5) * (A(1) - o.pc) * lphi, lkmr = -A(0.5) * (A(1) + o.pc) * lphi;
   lpcv += lphi * (A(1) - A(0.5) * kpr - A(0.5) * kmr);
-  *lkp = rp * A(0.125) * lkpr;
-  *lkm = o.rm * A(0.125) * lkmr;
+  lS->kp = rp * A(0.125) * lkpr;
+  lS->km = o.rm * A(0.125) * lkmr;
   const A lrm = o.km_sum * A(0.125) * lkmr - o.kp_sum * A(0.125) * lkpr;
   // rm = 1/(1 + exp((dT2 + crit_shift) * 2/T_width))
   ldT2 += -o.rm * rp * (A)c.two_over_tw * lrm;
-  *lpc = lpcv;
+  lS->pc = lpcv;
   // u2 = jx irho, v2 = jy irho, irho = 1/rho
   lS->jx = o.irho * lu2;
   lS->jy = o.irho * lv2;
   lirho += S.jx * lu2 + S.jy * lv2;
   lrho += -o.irho * o.irho * lirho;
   lS->rho = lrho;
-  lS->fxx = lqfxx;
-  lS->fyy = lqfyy;
-  lS->fxy = lqfxy;
   lS->dT = ldT2;
   lS->gxx = lqgxx;
   lS->gyy = lqgyy;
@@ -441,273 +411,280 @@ struct ConstsOf<float> {
   static __device__ __forceinline__ const ConstsF& of(const AdjArgs& a) { return a.cf; }
 };
 
-// The adjoint of step n at node (i, j), window (ox, oy); the parameter
-// adjoints are added to g.  EDGE = false for the tiles whose nodes and their
-// neighbours are all interior nodes: no boundary terms and no tests.
-// Arithmetic in the storage precision: FP64 for FP64 moments, FP32 for FP32
-// moments (the Jacobians evaluated in FP32: the kernel is bound by its
-// arithmetic).
-template <typename R, bool EQF, bool EDGE>
-__device__ __forceinline__ void adjoint_node(const AdjArgs& a, const Win<R, EQF>& W, int i, int j,
-                                             int ox, int oy, R g[3]) {
-  using A = R;
-  const int nx = a.gm.nx, ny = a.gm.ny;
-  const int64_t P = a.gm.pitch;
-  const int64_t q = (int64_t)j * P + i;
-  // this node's state after step n: recomputed from the window (the same
-  // core_forward the forward kernels run), or the state itself for the
-  // initial-state launch
-  Mom<A> m;
-  A ph;
-  PullSumsT<A> S;
-  A tap[9];
-  CoreT<A> o;
-  if (a.core) {
-    pull_step<R, EQF, A, EDGE>(a, W, i, j, ox, oy, &S, tap);
-    o = core_forward_t<A>(ConstsOf<A>::of(a), S, tap);
-    m = stored_mom<R, EQF, A>(ConstsOf<A>::of(a), o);
-    ph = o.phi;
-  } else {
-    m = win_mom<R, EQF, A, typename WinT<R>::A2>(W.a[oy][ox], W.b[oy][ox], W.c[oy][ox]);
-    ph = (A)W.phi[oy][ox];
-  }
-  Mom<A> lm = {};
-  A lphi = A(0);
-  A lTrep = A(0);
-  if (a.has_next) {
-    using S = LSlots<EQF>;
-    // ---- reverse of step n+1's pulls from this node: the adjoints of its
-    // nine populations, then through the rebuild to its moments
-    A lf[9], lg[9];
-#pragma unroll
-    for (int k = 0; k < 9; ++k) {
-      const int xi = i + CX[k], xj = j + CY[k];
-      if (!EDGE || (xi >= 1 && xi <= nx && xj >= 1 && xj <= ny)) {
-        lf[k] = lam_f(W, k, ox + CX[k], oy + CY[k]);
-        lg[k] = lam_g(W, k, ox + CX[k], oy + CY[k]);
-      } else {
-        lf[k] = lg[k] = A(0);
-      }
-    }
-    if constexpr (EDGE) {
-      // this node's own pull of direction k from a ghost: bounce-back of
-      // its opposite population (not for the two frozen corner ghosts)
-#pragma unroll
-      for (int k = 0; k < 9; ++k) {
-        const int si = i - CX[k], sj = j - CY[k];
-        if (si < 1 || si > nx || sj < 1 || sj > ny) {
-          const bool frozen = (k == 6 && si == nx + 1 && sj == 0) ||
-                              (k == 7 && si == nx + 1 && sj == ny + 1);
-          if (!frozen) lf[OPP[k]] += lam_f(W, k, ox, oy);
-        }
-      }
-      // ghost rows of g: row 0 is a copy of row 1, row Ny+1 of row Ny
-      if (j == 1) {
-#pragma unroll
-        for (int k = 0; k < 9; ++k)
-          if (CY[k] > 0) {
-            const int xi = i + CX[k];
-            if (xi >= 1 && xi <= nx) lg[k] += lam_g(W, k, ox + CX[k], oy);
-          }
-      }
-      if (j == ny) {
-#pragma unroll
-        for (int k = 0; k < 9; ++k)
-          if (CY[k] < 0) {
-            const int xi = i + CX[k];
-            if (xi >= 1 && xi <= nx) lg[k] += lam_g(W, k, ox + CX[k], oy);
-          }
-      }
-    }
-    rebuild_adjoint<A>(m, lf, lg, &lm);
-    // east ghost: equilibrium at this node's averaged T of step n (not
-    // with the cold-wall extension: then a constant)
-    if (EDGE && i == nx && !a.c.east_cold) {
-      for (int xj = j - 1; xj <= j + 1; ++xj) {
-        if (xj < 1 || xj > ny) continue;
-#pragma unroll
-        for (int k = 0; k < 9; ++k) {
-          if (CX[k] >= 0) continue;  // directions 3, 6, 7 pull from column Nx+1
-          const int sj = xj - CY[k];
-          const int sjc = sj < 1 ? 1 : (sj > ny ? ny : sj);
-          if (sjc != j) continue;
-          const int64_t h = (int64_t)j * P + nx + 1;
-          lTrep += ghost_dT<A>(k, (A)a.uh[h], (A)a.vh[h]) * lam_g(W, k, ox, oy + (xj - j));
-        }
-      }
-    }
-    // ---- phi of step n as a tap of step n+1 (C, E, N, W, S, NE, NW, SW, SE)
-    constexpr int DX[9] = {0, 1, 0, -1, 0, 1, -1, -1, 1};
-    constexpr int DY[9] = {0, 0, 1, 0, -1, 1, 1, -1, -1};
-    A skp = A(0), skm = A(0);
-#pragma unroll
-    for (int t = 0; t < 9; ++t) {
-      // nodes x whose tap t reads this node: x = y - d, and in rows 1 / Ny
-      // also those whose tap t reads the ghost row copied from this node
-      const int xi = i - DX[t], xj = j - DY[t];
-      if (!EDGE || (xi >= 1 && xi <= nx && xj >= 1 && xj <= ny)) {
-        const int wx = ox - DX[t], wy = oy - DY[t];
-        skp += W.lam[S::KP][wy][wx];
-        skm += W.lam[S::KM][wy][wx];
-      }
-      if (EDGE && ((j == 1 && DY[t] < 0) || (j == ny && DY[t] > 0))) {
-        if (xi >= 1 && xi <= nx) {
-          const int wx = ox - DX[t];
-          skp += W.lam[S::KP][oy][wx];
-          skm += W.lam[S::KM][oy][wx];
-        }
-      }
-    }
-    lphi = A(0.5) * (A(1) + ph) * skp - A(0.5) * (A(1) - ph) * skm;
-    lphi += (A)plane_at<R>(a.next, L_PC, q);
-  }
-  if (a.core) {
-    // ---- loss seed at a probe node (averaged T after step n); column 0
-    // of the index plane flags the rows that hold probes, so the other
-    // rows skip the per-node index load
-    if (a.seeds && a.probe_idx[(int64_t)j * P] >= 0) {
-      const int p = a.probe_idx[q];
-      if (p >= 0) lTrep += (A)a.seeds[p];
-    }
-    // averaged T = T_crit + (dT + dT2)/2: half on the stored dT, half on dT2
-    lm.th += A(0.5) * lTrep;
-    // ---- reverse of step n at this node
-    PullSumsT<A> lS;
-    A lkp, lkm, lpc;
-    core_backward<A>(ConstsOf<A>::of(a), S, tap, o, lm, lphi, A(0.5) * lTrep, &lS, &lkp, &lkm,
-                     &lpc, g);
-    const AdjPlanes& v = a.cur;
-    plane_set<R>(v, L_RHO, q, lS.rho);
-    plane_set<R>(v, L_JX, q, lS.jx);
-    plane_set<R>(v, L_JY, q, lS.jy);
-    if constexpr (!EQF) {
-      plane_set<R>(v, L_FXX, q, lS.fxx);
-      plane_set<R>(v, L_FYY, q, lS.fyy);
-      plane_set<R>(v, L_FXY, q, lS.fxy);
-    }
-    plane_set<R>(v, L_DT, q, lS.dT);
-    plane_set<R>(v, L_GXX, q, lS.gxx);
-    plane_set<R>(v, L_GYY, q, lS.gyy);
-    plane_set<R>(v, L_GXY, q, lS.gxy);
-    plane_set<R>(v, L_KP, q, lkp);
-    plane_set<R>(v, L_KM, q, lkm);
-    plane_set<R>(v, L_PC, q, lpc);
-  }
-  // this node's pulls from the west ghost (column 1): equilibria at the
-  // hot-wall temperature (left for last: no register holds the sum while
-  // the rest of the node is reversed)
-  if (EDGE && a.has_next && i == 1) {
-#pragma unroll
-    for (int k = 0; k < 9; ++k)
-      if (CX[k] == 1) {
-        const int sj = j - CY[k];
-        const int sjc = sj < 1 ? 1 : (sj > ny ? ny : sj);
-        const int64_t h = (int64_t)sjc * P;
-        g[2] += ghost_dT<A>(k, (A)a.uh[h], (A)a.vh[h]) * lam_g(W, k, ox, oy);
-      }
-  }
-  if (!a.core && i <= a.interf) {
-    // initial state: T = t_hot in the liquid strip (initialization.f90:15-26)
-    g[2] += lm.th;
-  }
-}
-
-// Tile order.  gfx950 dispatches workgroup b to XCD b % 8 and each XCD has
-// its own L2.  XCD x takes the x-th of eight horizontal bands of tile rows
-// and walks it in groups of kGroup tile columns, row by row within a group:
-// the cache lines of a window's halo (the 4- or 8-byte columns left and right
-// of the tile and the rows above and below it) were then fetched into the
-// same L2 by a tile a few places earlier on the same XCD, instead of by
-// another XCD.  Returns false for the padding workgroups of the shorter bands.
-constexpr int kGroup = 8;
-__device__ __forceinline__ bool tile_of(int ntx, int nty, int b, int* tx, int* ty) {
-  const int x = b % NXCD, s = b / NXCD;
-  const int r0 = (int)((int64_t)x * nty / NXCD), r1 = (int)((int64_t)(x + 1) * nty / NXCD);
-  const int rows = r1 - r0;
-  if (s >= rows * ntx) return false;
-  const int g = s / (kGroup * rows);
-  const int r = s - g * kGroup * rows;
-  const int gw = ntx - g * kGroup < kGroup ? ntx - g * kGroup : kGroup;
-  *ty = r0 + r / gw;
-  *tx = g * kGroup + r % gw;
-  return true;
-}
-inline int tile_grid(int ntx, int nty) { return NXCD * ((nty + NXCD - 1) / NXCD) * ntx; }
-
-// Waves per SIMD that the LDS of a CU (160 KiB) holds for k_adjoint: the
-// register budget asked of the compiler (more registers would not raise the
-// occupancy).
-template <typename R, bool EQF>
+// The kernel walks as the forward kernels do (bgk_wave.h): a wave owns 62
+// columns and goes up a strip of rows, the columns beside a node come by lane
+// shifts, the rows below and above it as sums kept in registers: step n's
+// pulled sums and taps (feed, bgk_level.h) and the gather of step n+1's
+// adjoints (feed_adjoint).  Every node is read from HBM once but for a strip's
+// two rows and a wave's two columns of its neighbours.  The adjoints lie in
+// planes of four values, so that a row is seven loads and three stores, and the
+// next row's loads are issued as soon as this one's values are taken.
+//
+// Registers decide: FP32 162 (omega_f = 1) and 174, held to two waves per SIMD
+// (three: the same with omega_f = 1, 4% slower with 20 bytes spilled without;
+// four: twice the time, spilled); FP64 more than 256, so one wave per SIMD (two:
+// 46 spilled, twice the time).  Bound by HBM from 2048^2 up; below, by the
+// latency of one row after another in a few waves.
+// Measured against tiles of 64 x 8 and 64 x 4 nodes with a window of everything
+// in LDS (765 VALU instructions per wave, the populations rebuilt for every
+// pull), us per launch, before -> now: FP32 moments with omega_f = 1 2048^2 139 ->
+// 120, 8192^2 2085 -> 1804 (4.6 TB/s of the 124 bytes per node that a launch
+// cannot do without), general 2048^2 193 -> 153; FP64 moments with omega_f = 1
+// 512^2 27.6 -> 18.9, 4096^2 1210 -> 775 (4.8 TB/s of 224 bytes), general 512^2
+// 30.5 -> 21.9, 4096^2 1380 -> 1031.
+constexpr int kAdjCols = kLanes - 2;
+template <typename R>
 constexpr int adj_waves() {
-  constexpr int waves_per_wg = BX * tile_rows<R, EQF>() / 64;
-  constexpr int lds = (int)sizeof(Win<R, EQF>) + 3 * 8 * waves_per_wg;
-  constexpr int w = (160 * 1024 / lds) * waves_per_wg / 4;
-  return w > 8 ? 8 : (w < 1 ? 1 : w);
+  return sizeof(R) == 4 ? 2 : 1;
+}
+// FP64 adjoints are stored through the caches: small lattices find them there
+// (gradient at 512^2, 300 steps: 9.4 ms for 9.8; 4096^2, 24 steps: 27.4 for
+// 29.3); FP32 ones past them (2048^2, 48 steps: 9.2 ms for 9.3).
+template <typename R>
+constexpr int adj_store() {
+  return sizeof(R) == 4 ? kNonTemporal : 0;
+}
+// The initial phi of the ghost columns 0 and Nx+1, which no step changes
+// (STEP_7/initialization.f90:15-26: liquid for i <= Nx/40).
+constexpr double kPhiWest = 1.0, kPhiEast = -1.0;
+
+template <typename R>
+struct V2Of;
+template <>
+struct V2Of<double> {
+  using T = double2;
+};
+template <>
+struct V2Of<float> {
+  using T = float2;
+};
+
+// A row as loaded: the state before the step and the adjoint of the step after.
+template <typename R, bool EQF>
+struct AdjRow {
+  using V4 = typename Vec<R>::V4;
+  using C = typename CType<R, EQF>::T;
+  using L2 = typename std::conditional<EQF, typename V2Of<R>::T, V4>::type;
+  double2 a;
+  V4 b;
+  C c;
+  double phi;
+  V4 l0, l1;
+  L2 l2;
+  R l3;
+
+  __device__ __forceinline__ void load_state(const AdjArgs& A, int j, unsigned ic) {
+    const int64_t q = (int64_t)j * A.pitch;
+    a = at(A.sprev.a + q, ic * (unsigned)sizeof(double2));
+    b = at(static_cast<const V4*>(A.sprev.b) + q, ic * (unsigned)sizeof(V4));
+    c = at(static_cast<const C*>(A.sprev.c) + q, ic * (unsigned)sizeof(C));
+    phi = at(A.sprev.phi + q, ic * (unsigned)sizeof(double));
+  }
+  __device__ __forceinline__ void load_lam(const AdjArgs& A, int j, unsigned ic) {
+    const int64_t q = (int64_t)j * A.pitch;
+    l0 = at(static_cast<const V4*>(A.next.v[0]) + q, ic * (unsigned)sizeof(V4));
+    l1 = at(static_cast<const V4*>(A.next.v[1]) + q, ic * (unsigned)sizeof(V4));
+    l2 = at(static_cast<const L2*>(A.next.v[2]) + q, ic * (unsigned)sizeof(L2));
+    if constexpr (!EQF) l3 = at(static_cast<const R*>(A.next.v[3]) + q, ic * (unsigned)sizeof(R));
+  }
+  __device__ __forceinline__ Mom<R> state(R* ph) const {
+    Mom<R> m;
+    if constexpr (sizeof(R) == 4) {
+      m.rho = (R)a.x;
+      m.th = (R)a.y;
+      *ph = (R)phi;
+    } else {
+      m.rho = taken(a.x);
+      m.th = taken(a.y);
+      *ph = taken(phi);
+    }
+    m.u = taken(b.x);
+    m.v = taken(b.y);
+    if constexpr (EQF) {
+      m.pf[0] = m.pf[1] = m.pf[2] = R(0);
+      m.pg[0] = taken(b.z);
+      m.pg[1] = taken(b.w);
+      m.pg[2] = taken(c);
+    } else {
+      m.pf[0] = taken(b.z);
+      m.pf[1] = taken(b.w);
+      m.pf[2] = taken(c.x);
+      m.pg[0] = taken(c.y);
+      m.pg[1] = taken(c.z);
+      m.pg[2] = taken(c.w);
+    }
+    return m;
+  }
+  // (zeros where there is no step after, and outside the lattice)
+  __device__ __forceinline__ Lam<R> lam(bool live) const {
+    Lam<R> x;
+    const auto get = [&](R y) __attribute__((always_inline)) { return live ? taken(y) : R(0); };
+    x.rho = get(l0.x);
+    x.jx = get(l0.y);
+    x.jy = get(l0.z);
+    x.dT = get(l0.w);
+    x.gxx = get(l1.x);
+    x.gyy = get(l1.y);
+    x.gxy = get(l1.z);
+    x.kp = get(l1.w);
+    x.km = get(l2.x);
+    x.pc = get(l2.y);
+    if constexpr (EQF) {
+      x.fxx = x.fyy = x.fxy = R(0);
+    } else {
+      x.fxx = get(l2.z);
+      x.fyy = get(l2.w);
+      x.fxy = get(l3);
+    }
+    return x;
+  }
+};
+
+// Stores of row j (lanes that must not store: column kPastStrip).
+template <typename R, bool EQF>
+__device__ __forceinline__ void store_adjoint(const AdjArgs& A, int j, int i, const Lam<R>& x) {
+  using Row = AdjRow<R, EQF>;
+  const int64_t q = (int64_t)j * A.pitch;
+  const int n = (int)A.pitch;
+  buffer_put<adj_store<R>()>(strip_buffer(static_cast<typename Row::V4*>(A.cur.v[0]) + q, n), i,
+             make4<R>(x.rho, x.jx, x.jy, x.dT));
+  buffer_put<adj_store<R>()>(strip_buffer(static_cast<typename Row::V4*>(A.cur.v[1]) + q, n), i,
+             make4<R>(x.gxx, x.gyy, x.gxy, x.kp));
+  const auto b2 = strip_buffer(static_cast<typename Row::L2*>(A.cur.v[2]) + q, n);
+  if constexpr (EQF) {
+    typename Row::L2 y;
+    y.x = x.km;
+    y.y = x.pc;
+    buffer_put<adj_store<R>()>(b2, i, y);
+  } else {
+    buffer_put<adj_store<R>()>(b2, i, make4<R>(x.km, x.pc, x.fxx, x.fyy));
+    buffer_put<adj_store<R>()>(strip_buffer(static_cast<R*>(A.cur.v[3]) + q, n), i, x.fxy);
+  }
 }
 
-template <typename R, bool EQF>
-__global__ __launch_bounds__((BX * tile_rows<R, EQF>()), (adj_waves<R, EQF>())) void k_adjoint(
-    AdjArgs a) {
-  constexpr int BY = tile_rows<R, EQF>(), WY = BY + 2;
-  const int nx = a.gm.nx, ny = a.gm.ny;
-  const int64_t P = a.gm.pitch;
-  int tx, ty;
-  if (!tile_of(a.ntx, a.nty, (int)blockIdx.x, &tx, &ty)) return;  // whole workgroup
-  const int i0 = tx * BX + 1, j0 = ty * BY + 1;
-  const int ox = threadIdx.x + 1, oy = threadIdx.y + 1;  // this node in the window
-  const int i = i0 + threadIdx.x, j = j0 + threadIdx.y;
-  // ---- the window: rows j0-1 .. j0+BY, columns i0-1 .. i0+BX, clamped to
-  // the planes' extent (clamped entries are never read: every read below is
-  // guarded as in the global form)
-  __shared__ Win<R, EQF> W;
-  {
-    using S = LSlots<EQF>;
-    for (int e = threadIdx.y * BX + threadIdx.x; e < WX * WY; e += BX * BY) {
-      const int ex = e % WX, ey = e / WX;
-      int xi = i0 - 1 + ex, xj = j0 - 1 + ey;
-      xi = xi > nx + 1 ? nx + 1 : xi;
-      xj = xj > ny + 1 ? ny + 1 : xj;
-      const int64_t x = (int64_t)xj * P + xi;
-      if (a.has_next)
+// One wave's strip, rows j0..j1.  EDGE: the wave or the strip touches a wall.
+// INIT: the share of the initial state, sprev itself (nothing is stored).  g: this
+// lane's parameter adjoints, summed in FP64.
+template <typename R, bool EQF, bool EDGE, bool INIT>
+__device__ __forceinline__ void adjoint_strip(const AdjArgs& A, int j0, int j1, int i, bool has_w,
+                                              bool has_e, double g[3]) {
+  const auto& c = ConstsOf<R>::of(A);
+  const int nx = A.nx, ny = A.ny, lane = (int)threadIdx.x;
+  const unsigned ic = (unsigned)(i < 0 ? 0 : (i > nx + 1 ? nx + 1 : i));  // column loaded
+  const bool ghost = EDGE && (i == 0 || i == nx + 1);
+  const bool own = lane >= 1 && lane < kLanes - 1 && i <= nx;  // columns this wave stores
+  const bool live = A.has_next && (!EDGE || (i >= 1 && i <= nx));
+  R gd[9];
 #pragma unroll
-        for (int sl = 0; sl < S::N; ++sl) W.lam[sl][ey][ex] = plane_at<R>(a.next, S::plane[sl], x);
-      W.a[ey][ex] = WinT<R>::a2(a.sprev.a[x]);
-      W.b[ey][ex] = b_at<R, EQF>(a.sprev.b, x);
-      W.c[ey][ex] = c_at<R, EQF>(a.sprev.c, x);
-      W.phi[ey][ex] = (typename WinT<R>::P)a.sprev.phi[x];
+  for (int k = 0; k < 9; ++k) gd[k] = (R)A.gd[k];
+
+  // rows of the strip that hold a probe (column 0 of the probe index plane is
+  // >= 0 there; at most kMaxRows rows)
+  uint64_t probes = 0;
+  if (!INIT && A.seeds)
+    probes = __ballot(j0 + lane <= j1 &&
+                      A.probe_idx[(int64_t)min(j0 + lane, j1) * A.pitch] >= 0);
+
+  LevelT<R> S = LevelT<R>{};
+  AdjLevel<R> L = AdjLevel<R>{};
+  R u_was = R(0), v_was = R(0);  // INIT: the completed row's velocity
+  const int ra = EDGE ? max(1, j0 - 1) : j0 - 1, rb = j1 + 1;
+  AdjRow<R, EQF> row;
+  row.load_lam(A, ra, ic);
+  row.load_state(A, ra, ic);
+  const scalar_ptr te_in = as_scalar(A.sprev.te);
+  double te_row = EDGE ? te_in[ra] : 0.0;
+  __builtin_amdgcn_s_waitcnt(kWaitLoads);
+  auto feed_row = [&](int r) __attribute__((always_inline)) {
+    const Lam<R> x = row.lam(live);
+    __builtin_amdgcn_sched_barrier(0);
+    row.load_lam(A, min(r + 1, ny), ic);
+    const int jc = r - 1;  // row completed
+    const bool on = own && jc >= j0 && jc <= j1;
+    // ---- step n+1's pulls reversed
+    AdjLevel<R> G;
+    R tin;
+    feed_adjoint<EQF, EDGE>(L, x, r, ny, i, nx, has_w, has_e, gd, &G, &tin);
+    if (EDGE && r >= j0 && r <= j1 && own) g[2] += (double)tin;
+    __builtin_amdgcn_sched_barrier(0);
+    R phi;
+    Mom<R> m = row.state(&phi);
+    __builtin_amdgcn_sched_barrier(0);
+    row.load_state(A, min(r + 1, ny), ic);
+    Mom<R> lm = {};
+    if constexpr (INIT) {
+      Mom<R> was = {};
+      was.u = u_was;
+      was.v = v_was;
+      rebuild_adjoint<R>(was, G.F, G.G, &lm);
+      // T = t_hot in the liquid strip (initialization.f90:15-26)
+      if (on && i <= A.interf) g[2] += (double)lm.th;
+      u_was = m.u;
+      v_was = m.v;
+      return;
     }
-  }
-  __syncthreads();
-  // parameter adjoints of this thread's node, in the arithmetic type (FP32
-  // terms are summed in FP32 over the 64 nodes of a wave, in FP64 beyond)
-  R g[3] = {R(0), R(0), R(0)};
-  // tiles whose nodes all have four interior neighbours skip every
-  // boundary test (a workgroup-uniform branch)
-  const bool edge = !(i0 > 1 && i0 + BX <= nx && j0 > 1 && j0 + BY <= ny);
-  if (i <= nx && j <= ny) {
-    if (edge)
-      adjoint_node<R, EQF, true>(a, W, i, j, ox, oy, g);
-    else
-      adjoint_node<R, EQF, false>(a, W, i, j, ox, oy, g);
-  }
-  // ---- parameter adjoints: workgroup sum into this workgroup's own slot
-  // (butterfly within each wave, then the waves in order: deterministic)
-  constexpr int NW = BX * BY / 64;
-  __shared__ double red[3][NW];
-  const int t = threadIdx.y * BX + threadIdx.x;
+    // ---- step n's pulled sums and taps
+    if (EDGE) {
+      const double te = A.c.east_cold ? A.c.t_cold : te_row;
+      te_row = te_in[min(r + 1, ny)];
+      if (ghost) {  // no flow populations, the wall's T and velocity
+        m.rho = m.pf[0] = m.pf[1] = m.pf[2] = m.pg[0] = m.pg[1] = m.pg[2] = R(0);
+        m.th = (R)((i == 0 ? A.c.tin : te) - kTcrit);
+        m.u = (R)A.c.u0;
+        m.v = (R)A.c.v0;
+        phi = i == 0 ? R(kPhiWest) : R(kPhiEast);
+      }
+    }
+    R f[9], gp[9];
+    populations<!EQF>(m.rho, m.rho, m.u, m.v, m.pf[0], m.pf[1], m.pf[2], f);
+    populations<true>(m.th, R(kTcrit) + m.th, m.u, m.v, m.pg[0], m.pg[1], m.pg[2], gp);
+    PullSumsT<R> P;
+    R st, st2, pc;
+    feed<EDGE>(S, f, gp, phi, r, ny, i, nx, has_w, has_e, (R)A.c.frozen6, (R)A.c.frozen7, &P, &st,
+               &st2, &pc);
+    __builtin_amdgcn_sched_barrier(0);
+    const CoreT<R> o = core_from_sums<R>(c, P, st, st2, pc);
+    // ---- the adjoint of the state after step n
+    rebuild_adjoint<R>(stored_mom<R, EQF, R>(c, o), G.F, G.G, &lm);
+    const R lphi = R(0.5) * (R(1) + o.phi) * G.kp - R(0.5) * (R(1) - o.phi) * G.km + G.pc;
+    // averaged T = T_crit + (dT + dT2)/2: its adjoint half on the stored dT,
+    // half on dT2.  The east ghosts of step n+1 are equilibria at this node's
+    // (not with the cold-wall extension: then a constant)
+    R lt = EDGE && i == nx && !A.c.east_cold ? G.te : R(0);
+    if (jc >= j0 && ((probes >> (jc - j0)) & 1) && on) {
+      const int p = A.probe_idx[(int64_t)jc * A.pitch + i];
+      if (p >= 0) lt += (R)A.seeds[p];
+    }
+    lm.th += R(0.5) * lt;
+    // ---- reverse of step n at this node
+    Lam<R> out;
+    R gp2[2];
+    core_backward<EQF, R>(c, P, o, lm, lphi, R(0.5) * lt, &out, gp2);
+    store_adjoint<R, EQF>(A, min(max(jc, j0), j1), on ? i : kPastStrip, out);
+    g[0] += on ? (double)gp2[0] : 0.0;
+    g[1] += on ? (double)gp2[1] : 0.0;
+  };
+  for (int r = ra; r <= rb; ++r) feed_row(r);
+}
+
+template <typename R, bool EQF, bool INIT>
+__global__ __launch_bounds__(kLanes, (adj_waves<R>())) void k_adjoint(AdjArgs A) {
+  int seg, j0, j1;
+  bool edge;
+  if (!wave_tile(A.g, A.ny, &seg, &j0, &j1, &edge)) return;
+  const int i0 = seg * kAdjCols + 1;
+  const int i = i0 - 1 + (int)threadIdx.x;
+  double g[3] = {0.0, 0.0, 0.0};
+  if (edge)
+    adjoint_strip<R, EQF, true, INIT>(A, j0, j1, i, i0 == 1, i0 + kAdjCols >= A.nx, g);
+  else
+    adjoint_strip<R, EQF, false, INIT>(A, j0, j1, i, false, false, g);
+  // parameter adjoints: butterfly over the wave, then this workgroup's own
+  // slot (deterministic)
 #pragma unroll
-  for (int c = 0; c < 3; ++c)
-    for (int m = 32; m > 0; m >>= 1) g[c] += __shfl_xor(g[c], m, 64);
-  if ((t & 63) == 0)
-    for (int c = 0; c < 3; ++c) red[c][t >> 6] = (double)g[c];
-  __syncthreads();
-  if (t == 0) {
-    const int64_t b = (int64_t)ty * a.ntx + tx;
-    for (int c = 0; c < 3; ++c) {
-      double sum = 0.0;
-      for (int w = 0; w < NW; ++w) sum += red[c][w];
-      a.partial[3 * b + c] += sum;
-    }
+  for (int k = 0; k < 3; ++k) {
+    for (int m = 32; m > 0; m >>= 1) g[k] += __shfl_xor(g[k], m, 64);
+    if (threadIdx.x == 0) A.partial[3 * (int64_t)blockIdx.x + k] += g[k];
   }
 }
 
@@ -893,11 +870,13 @@ size_t c_bytes(const bgk_handle* h) {
   if (h->mom_eqf) return f64 ? sizeof(double) : sizeof(float);
   return f64 ? sizeof(double4) : sizeof(float4);
 }
-// rows of the adjoint kernel's tile for the handle's instantiation
-int tile_rows_of(const bgk_handle* h) {
+// the adjoint kernel's work split: strips of at most 32 rows with FP32 moments
+// (2048^2 and 4096^2 with 16 / 32 / 64: 9.3 / 9.2 / 9.5 and 17.3 / 17.3 / 17.4
+// ms), 16 with FP64 (4096^2 with 8 / 16 / 32 / 64: 29.3 / 29.3 / 29.2 / 29.6)
+WaveGrid adj_grid(const bgk_handle* h) {
   const bool f64 = h->prm.precision == BGK_FP64_MOM;
-  if (h->mom_eqf) return f64 ? tile_rows<double, true>() : tile_rows<float, true>();
-  return f64 ? tile_rows<double, false>() : tile_rows<float, false>();
+  return make_wave_grid(h->nx, h->ny, kAdjCols, 1, 2, 1.4, f64 ? 16 : 32, h->n_cu, h->strip_rows,
+                        f64 ? adj_waves<double>() : adj_waves<float>());
 }
 
 struct Bump {
@@ -936,11 +915,13 @@ void carve_state(Bump& b, const bgk_handle* h, StatePtrs* s) {
 size_t carve_fixed(bgk_handle* h, AdjCtx* a, Bump& b) {
   const size_t n = (size_t)h->plane_elems;
   const size_t before = b.off;
-  for (int l = 0; l < 2; ++l)
-    for (int v = 0; v < 13; ++v) {
-      const bool zero = h->mom_eqf && (v == L_FXX || v == L_FYY || v == L_FXY);
-      a->lam[l].v[v] = zero ? nullptr : b.plane<char>(n, lam_bytes(h));
-    }
+  for (int l = 0; l < 2; ++l) {
+    const size_t e = lam_bytes(h);
+    a->lam[l].v[0] = b.plane<char>(n, 4 * e);
+    a->lam[l].v[1] = b.plane<char>(n, 4 * e);
+    a->lam[l].v[2] = b.plane<char>(n, (h->mom_eqf ? 2 : 4) * e);
+    a->lam[l].v[3] = h->mom_eqf ? nullptr : b.plane<char>(n, e);
+  }
   a->probe_idx = b.plane<int>(n);
   a->probe_ij = b.take<int>(2 * (size_t)std::max(a->np, 1));
   a->probe_T = b.take<double>((size_t)a->nsteps * std::max(a->np, 1));
@@ -999,38 +980,44 @@ hipError_t copy_state(bgk_handle* h, const StatePtrs& dst, const double2* a, con
   return e;
 }
 
+template <typename R, bool EQF>
+void run_adjoint(bgk_handle* h, const AdjArgs& a, int core) {
+  const dim3 grd((unsigned)a.g.nwg);
+  if (core)
+    hipLaunchKernelGGL((k_adjoint<R, EQF, false>), grd, dim3(kLanes), 0, h->stream, a);
+  else
+    hipLaunchKernelGGL((k_adjoint<R, EQF, true>), grd, dim3(kLanes), 0, h->stream, a);
+}
+
 // adjoint of the step from state `sprev` (core = 1), or the initial state's
 // share (core = 0, sprev = the initial state)
 hipError_t launch_adjoint(bgk_handle* h, AdjCtx* x, const StatePtrs& sprev, int lam_next,
                           int has_next, int core, const double* seeds) {
   AdjArgs a;
   a.sprev = sprev;
-  a.uh = h->u;
-  a.vh = h->v;
   a.next = x->lam[lam_next];
   a.cur = x->lam[1 - lam_next];
   a.has_next = has_next;
-  a.core = core;
   a.probe_idx = x->probe_idx;
   a.seeds = seeds;
   a.partial = x->partial;
   a.c = h->c;
   a.cf = consts_f(h->c);
-  a.gm = h->geom;
+  const double u = h->c.u0, v = h->c.v0;
+  for (int k = 0; k < 9; ++k) {
+    const double cu = CX[k] * u + CY[k] * v;
+    a.gd[k] = kW[k] * (1.0 + 3.0 * cu + 4.5 * cu * cu - 1.5 * (u * u + v * v));
+  }
+  a.nx = h->nx;
+  a.ny = h->ny;
+  a.pitch = h->pitch;
   a.interf = h->nx / 40;
-  const int by = tile_rows_of(h);
-  a.ntx = (h->nx + BX - 1) / BX;
-  a.nty = (h->ny + by - 1) / by;
-  const dim3 grd((unsigned)tile_grid(a.ntx, a.nty));
+  a.g = adj_grid(h);
   const bool f64 = h->prm.precision == BGK_FP64_MOM;
-  if (h->mom_eqf && f64)
-    hipLaunchKernelGGL((k_adjoint<double, true>), grd, dim3(BX, by), 0, h->stream, a);
-  else if (h->mom_eqf)
-    hipLaunchKernelGGL((k_adjoint<float, true>), grd, dim3(BX, by), 0, h->stream, a);
-  else if (f64)
-    hipLaunchKernelGGL((k_adjoint<double, false>), grd, dim3(BX, by), 0, h->stream, a);
+  if (h->mom_eqf)
+    f64 ? run_adjoint<double, true>(h, a, core) : run_adjoint<float, true>(h, a, core);
   else
-    hipLaunchKernelGGL((k_adjoint<float, false>), grd, dim3(BX, by), 0, h->stream, a);
+    f64 ? run_adjoint<double, false>(h, a, core) : run_adjoint<float, false>(h, a, core);
   return hipGetLastError();
 }
 
@@ -1069,8 +1056,7 @@ int64_t adj_bytes(bgk_handle* h, int nsteps, int np, int nsnap) {
   x.nsteps = nsteps;
   x.np = np;
   x.nsnap = nsnap;
-  const int by = tile_rows_of(h);
-  x.nblk = (int)(((h->nx + BX - 1) / BX) * ((h->ny + by - 1) / by));
+  x.nblk = adj_grid(h).nwg;
   return (int64_t)carve_ctx(h, &x, nullptr);
 }
 
@@ -1094,8 +1080,7 @@ hipError_t adj_setup(bgk_handle* h, int nsteps, int seg_outer, int seg, int nsna
     // (the first checkpoint of an outer segment is the outer checkpoint)
     x->nckpt2 = seg_outer > 0 ? (std::min(seg_outer, nsteps) + seg - 1) / seg - 1 : 0;
   }
-  const int by = tile_rows_of(h);
-  x->nblk = (int)(((h->nx + BX - 1) / BX) * ((h->ny + by - 1) / by));
+  x->nblk = adj_grid(h).nwg;
   x->bytes = carve_ctx(h, x, nullptr);
   hipError_t e = hipMalloc(&x->pool, x->bytes);
   if (e != hipSuccess) {

@@ -1,6 +1,7 @@
 // bgk_level.h -- one level of the wave-streaming kernels whose node update needs
 // its pulled populations only through their moments: moment storage
-// (bgk_stream_mom.hip) and FP32 populations (bgk_stream32.hip).
+// (bgk_stream_mom.hip), FP32 populations (bgk_stream32.hip) and the adjoint
+// (bgk_adjoint.hip).  A: double, or float for the adjoint of the FP32 step.
 //
 // A row's populations are formed once, in the lane of their node, and enter the
 // pulled sums of the rows below, beside and above it as three numbers per
@@ -26,64 +27,67 @@ using namespace wave;
 // rho for f; m0 = T - T_crit, m = T for g, whose populations are the
 // deviations g_k - w_k T_crit.  With Q = 9/2 (m u u + P), E = m0 - tr Q / 3:
 // p_k = w_k (E + c c : Q + 3 c . j).
-template <bool HAVE_P>
-__device__ __forceinline__ void populations(double m0, double m, double u, double v, double pxx,
-                                            double pyy, double pxy, double p[9]) {
-  const double jx = m * u, jy = m * v;
-  double qxx, qyy, qxy;
+template <bool HAVE_P, typename A>
+__device__ __forceinline__ void populations(A m0, A m, A u, A v, A pxx, A pyy, A pxy, A p[9]) {
+  const A jx = m * u, jy = m * v;
+  A qxx, qyy, qxy;
   if constexpr (HAVE_P) {
-    qxx = 4.5 * fma(jx, u, pxx);
-    qyy = 4.5 * fma(jy, v, pyy);
-    qxy = 9.0 * fma(jx, v, pxy);
+    qxx = A(4.5) * fma(jx, u, pxx);
+    qyy = A(4.5) * fma(jy, v, pyy);
+    qxy = A(9.0) * fma(jx, v, pxy);
   } else {
-    qxx = 4.5 * (jx * u);
-    qyy = 4.5 * (jy * v);
-    qxy = 9.0 * (jx * v);
+    qxx = A(4.5) * (jx * u);
+    qyy = A(4.5) * (jy * v);
+    qxy = A(9.0) * (jx * v);
   }
-  const double s = qxx + qyy;
-  const double e = fma(s, -1.0 / 3.0, m0);
-  const double ax = (e + qxx) * (1.0 / 9.0), ay = (e + qyy) * (1.0 / 9.0), d = e + s;
-  const double dp = (d + qxy) * (1.0 / 36.0), dm = (d - qxy) * (1.0 / 36.0);
-  const double jp = jx + jy, jm = jx - jy;
-  p[0] = e * (4.0 / 9.0);
-  p[1] = fma(jx, 1.0 / 3.0, ax);
-  p[3] = fma(jx, -1.0 / 3.0, ax);
-  p[2] = fma(jy, 1.0 / 3.0, ay);
-  p[4] = fma(jy, -1.0 / 3.0, ay);
-  p[5] = fma(jp, 1.0 / 12.0, dp);
-  p[7] = fma(jp, -1.0 / 12.0, dp);
-  p[8] = fma(jm, 1.0 / 12.0, dm);
-  p[6] = fma(jm, -1.0 / 12.0, dm);
+  const A s = qxx + qyy;
+  const A e = fma(s, A(-1.0 / 3.0), m0);
+  const A ax = (e + qxx) * A(1.0 / 9.0), ay = (e + qyy) * A(1.0 / 9.0), d = e + s;
+  const A dp = (d + qxy) * A(1.0 / 36.0), dm = (d - qxy) * A(1.0 / 36.0);
+  const A jp = jx + jy, jm = jx - jy;
+  p[0] = e * A(4.0 / 9.0);
+  p[1] = fma(jx, A(1.0 / 3.0), ax);
+  p[3] = fma(jx, A(-1.0 / 3.0), ax);
+  p[2] = fma(jy, A(1.0 / 3.0), ay);
+  p[4] = fma(jy, A(-1.0 / 3.0), ay);
+  p[5] = fma(jp, A(1.0 / 12.0), dp);
+  p[7] = fma(jp, A(-1.0 / 12.0), dp);
+  p[8] = fma(jm, A(1.0 / 12.0), dm);
+  p[6] = fma(jm, A(-1.0 / 12.0), dm);
 }
 
 // What three neighbouring source nodes of one row give to a node's pulled
 // sums: their total, the total of the two diagonals, and the difference
 // (eastward - westward) of the diagonals.
-struct Triple {
-  double n, p, d;
+template <typename A>
+struct TripleT {
+  A n, p, d;
 };
-__device__ __forceinline__ Triple triple(double c, double w, double e) {
-  const double p = w + e;
-  return Triple{c + p, p, w - e};
+template <typename A>
+__device__ __forceinline__ TripleT<A> triple(A c, A w, A e) {
+  const A p = w + e;
+  return TripleT<A>{c + p, p, w - e};
 }
 
 // Registers of one level between two rows.
-struct Level {
+template <typename A>
+struct LevelT {
   // row awaiting its northern neighbours: pulled sums so far, phi sums of
   // its own and the southern row, its centre tap
-  PullSums s;
-  double t1, t2, pc;
+  PullSumsT<A> s;
+  A t1, t2, pc;
   // the southern share of the row after it
-  Triple sf, sg;
-  double n1, n2;
+  TripleT<A> sf, sg;
+  A n1, n2;
 };
+using Level = LevelT<double>;
 
 struct Updated {
   double rho, dT, u, v, pfxx, pfyy, pfxy, pgxx, pgyy, pgxy, phi;  // stored
   double dT2, u2, v2;                                              // before the forces
 };
 
-// momentsPre .. collision of one node (see core_forward_t in bgk_mom.h for
+// momentsPre .. collision of one node (see core_from_sums in bgk_mom.h for
 // the citations), on explicit fused multiply-adds; st, st2: sums of the nine
 // phi_prec taps and of their squares, pc the centre tap.
 struct StepC {
@@ -152,22 +156,22 @@ __device__ __forceinline__ Updated update(const StepC& c, const PullSums& S, dou
 // (their f vanish) and the wall's temperature and velocity (their g are the
 // thermal ghosts); bounce-back adds a node's own opposite populations; rows 0
 // and Ny+1 of g and phi are rows 1 and Ny.
-template <bool EDGE>
-__device__ __forceinline__ void feed(Level& L, const double f[9], const double g[9], double phi, int j, int ny, int i, int nx,
-                                     bool has_w, bool has_e, double frozen6, double frozen7,
-                                     PullSums* S, double* st, double* st2, double* pc) {
+template <bool EDGE, typename A>
+__device__ __forceinline__ void feed(LevelT<A>& L, const A f[9], const A g[9], A phi, int j, int ny,
+                                     int i, int nx, bool has_w, bool has_e, A frozen6, A frozen7,
+                                     PullSumsT<A>* S, A* st, A* st2, A* pc) {
   *S = L.s;
   *st = L.t1;
   *st2 = L.t2;
   *pc = L.pc;
   if (EDGE && j > ny) return;
   // row sums of the phi taps
-  const double pw = from_west(phi), pe = from_east(phi);
-  const double r1 = (pw + pe) + phi;
-  const double r2 = fma(phi, phi, fma(pw, pw, pe * pe));
+  const A pw = from_west(phi), pe = from_east(phi);
+  const A r1 = (pw + pe) + phi;
+  const A r2 = fma(phi, phi, fma(pw, pw, pe * pe));
   // northern sources of row j - 1
-  const Triple nf = triple(f[4], from_west(f[8]), from_east(f[7]));
-  const Triple ng = triple(g[4], from_west(g[8]), from_east(g[7]));
+  const TripleT<A> nf = triple(f[4], from_west(f[8]), from_east(f[7]));
+  const TripleT<A> ng = triple(g[4], from_west(g[8]), from_east(g[7]));
   S->rho += nf.n;
   S->jx += nf.d;
   S->jy -= nf.n;
@@ -181,10 +185,10 @@ __device__ __forceinline__ void feed(Level& L, const double f[9], const double g
   *st += r1;
   *st2 += r2;
   // southern sources of row j + 1
-  const Triple sf = triple(f[2], from_west(f[5]), from_east(f[6]));
-  const Triple sg = triple(g[2], from_west(g[5]), from_east(g[6]));
+  const TripleT<A> sf = triple(f[2], from_west(f[5]), from_east(f[6]));
+  const TripleT<A> sg = triple(g[2], from_west(g[5]), from_east(g[6]));
   if (EDGE && j == 1) {  // row 0: bounce-back, copied g and phi
-    const double f6 = i == nx ? frozen6 : f[8];
+    const A f6 = i == nx ? frozen6 : f[8];
     L.sf = triple(f[4], f[7], f6);
     L.sg = sg;
     L.n1 = r1;
@@ -192,8 +196,8 @@ __device__ __forceinline__ void feed(Level& L, const double f[9], const double g
   }
   // row j: southern share, then its own row's sources
   {
-    const Triple cf = triple(f[0], from_west(f[1]), from_east(f[3]));
-    const Triple cg = triple(g[0], from_west(g[1]), from_east(g[3]));
+    const TripleT<A> cf = triple(f[0], from_west(f[1]), from_east(f[3]));
+    const TripleT<A> cg = triple(g[0], from_west(g[1]), from_east(g[3]));
     L.s.rho = L.sf.n + cf.n;
     L.s.jx = L.sf.d + cf.d;
     L.s.jy = L.sf.n;
@@ -210,7 +214,7 @@ __device__ __forceinline__ void feed(Level& L, const double f[9], const double g
   }
   if (EDGE) {
     if (j == ny) {  // row Ny+1: bounce-back, copied g and phi
-      const Triple v = triple(f[2], f[6], i == nx ? frozen7 : f[5]);
+      const TripleT<A> v = triple(f[2], f[6], i == nx ? frozen7 : f[5]);
       L.s.rho += v.n;
       L.s.jx += v.d;
       L.s.jy -= v.n;
@@ -226,9 +230,9 @@ __device__ __forceinline__ void feed(Level& L, const double f[9], const double g
     }
     if (has_w) {  // column 1: directions 1, 5, 8 bounce back
       const bool on = i == 1;
-      const double a = on ? f[3] : 0.0;
-      const double b = on && j != 1 ? f[7] : 0.0;
-      const double d = on && j != ny ? f[6] : 0.0;
+      const A a = on ? f[3] : A(0);
+      const A b = on && j != 1 ? f[7] : A(0);
+      const A d = on && j != ny ? f[6] : A(0);
       L.s.rho += a + b + d;
       L.s.jx += a + b + d;
       L.s.jy += b - d;
@@ -238,9 +242,9 @@ __device__ __forceinline__ void feed(Level& L, const double f[9], const double g
     }
     if (has_e) {  // column Nx: directions 3, 6, 7 bounce back
       const bool on = i == nx;
-      const double a = on ? f[1] : 0.0;
-      const double b = on && j != 1 ? f[8] : 0.0;
-      const double d = on && j != ny ? f[5] : 0.0;
+      const A a = on ? f[1] : A(0);
+      const A b = on && j != 1 ? f[8] : A(0);
+      const A d = on && j != ny ? f[5] : A(0);
       L.s.rho += a + b + d;
       L.s.jx -= a + b + d;
       L.s.jy += b - d;

@@ -106,28 +106,20 @@ __device__ __forceinline__ typename CType<R, EQF>::T c_stream(const void* c, int
     return nt_load4<R>(static_cast<const typename Vec<R>::V4*>(c) + q);
 }
 
-// The helpers below take the arithmetic type A: double for the forward
-// kernels (and the FP64-moment adjoint), float for the adjoint of the FP32
-// moment step, which evaluates its Jacobians in FP32.
-
 // P_k(u,v): the equilibrium polynomial of direction k minus its leading 1.
-template <typename A>
-__device__ __forceinline__ A eq_poly_t(int k, A u, A v) {
-  const A uv = A(1.5) * (u * u + v * v);
+__device__ __forceinline__ double eq_poly(int k, double u, double v) {
+  const double uv = 1.5 * (u * u + v * v);
   switch (k) {
     case 0: return -uv;
-    case 1: return A(3) * u + A(4.5) * (u * u) - uv;
-    case 2: return A(3) * v + A(4.5) * (v * v) - uv;
-    case 3: return -A(3) * u + A(4.5) * (u * u) - uv;
-    case 4: return -A(3) * v + A(4.5) * (v * v) - uv;
-    case 5: { const A s = u + v; return A(3) * s + A(4.5) * (s * s) - uv; }
-    case 6: { const A s = u - v; return -A(3) * s + A(4.5) * (s * s) - uv; }
-    case 7: { const A s = u + v; return -A(3) * s + A(4.5) * (s * s) - uv; }
-    default: { const A s = u - v; return A(3) * s + A(4.5) * (s * s) - uv; }
+    case 1: return 3.0 * u + 4.5 * (u * u) - uv;
+    case 2: return 3.0 * v + 4.5 * (v * v) - uv;
+    case 3: return -3.0 * u + 4.5 * (u * u) - uv;
+    case 4: return -3.0 * v + 4.5 * (v * v) - uv;
+    case 5: { const double s = u + v; return 3.0 * s + 4.5 * (s * s) - uv; }
+    case 6: { const double s = u - v; return -3.0 * s + 4.5 * (s * s) - uv; }
+    case 7: { const double s = u + v; return -3.0 * s + 4.5 * (s * s) - uv; }
+    default: { const double s = u - v; return 3.0 * s + 4.5 * (s * s) - uv; }
   }
-}
-__device__ __forceinline__ double eq_poly(int k, double u, double v) {
-  return eq_poly_t<double>(k, u, v);
 }
 
 // H_k : P for P = (pxx, pyy, pxy), H_k = c_k c_k - cs2 I, in the storage
@@ -148,43 +140,44 @@ __device__ __forceinline__ R h_k(int k, R pxx, R pyy, R pxy) {
 }
 
 // Population k of a node from its moments: f_k and gd_k = g_k - w_k*T_crit.
-template <typename R, bool EQF, typename A = double, typename A2 = double2>
-__device__ __forceinline__ void rebuild(int k, const A2 a, const typename Vec<R>::V4 b,
-                                        const typename CType<R, EQF>::T cc, A* fk, A* gdk) {
-  const A p = eq_poly_t<A>(k, (A)b.x, (A)b.y);
-  const A ax = (A)a.x, ay = (A)a.y;
+template <typename R, bool EQF>
+__device__ __forceinline__ void rebuild(int k, const double2 a, const typename Vec<R>::V4 b,
+                                        const typename CType<R, EQF>::T cc, double* fk, double* gdk) {
+  const double p = eq_poly(k, (double)b.x, (double)b.y);
+  const double ax = a.x, ay = a.y;
   if constexpr (EQF) {
-    const A hg = (A)h_k<R>(k, b.z, b.w, cc);
-    *fk = A(kW[k]) * ax * (A(1) + p);
-    *gdk = A(kW[k]) * (ay + (A(kTcrit) + ay) * p) + A(coef_of(k)) * hg;
+    const double hg = (double)h_k<R>(k, b.z, b.w, cc);
+    *fk = kW[k] * ax * (1.0 + p);
+    *gdk = kW[k] * (ay + (kTcrit + ay) * p) + coef_of(k) * hg;
   } else {
-    const A hf = (A)h_k<R>(k, b.z, b.w, cc.x);
-    const A hg = (A)h_k<R>(k, cc.y, cc.z, cc.w);
-    *fk = A(kW[k]) * ax * (A(1) + p) + A(coef_of(k)) * hf;
-    *gdk = A(kW[k]) * (ay + (A(kTcrit) + ay) * p) + A(coef_of(k)) * hg;
+    const double hf = (double)h_k<R>(k, b.z, b.w, cc.x);
+    const double hg = (double)h_k<R>(k, cc.y, cc.z, cc.w);
+    *fk = kW[k] * ax * (1.0 + p) + coef_of(k) * hf;
+    *gdk = kW[k] * (ay + (kTcrit + ay) * p) + coef_of(k) * hg;
   }
 }
 
-template <typename R, bool EQF, typename A = double, typename A2 = double2>
-__device__ __forceinline__ A rebuild_f(int k, const A2 a, const typename Vec<R>::V4 b,
+template <typename R, bool EQF>
+__device__ __forceinline__ double rebuild_f(int k, const double2 a, const typename Vec<R>::V4 b,
                                        const typename CType<R, EQF>::T cc) {
-  const A p = eq_poly_t<A>(k, (A)b.x, (A)b.y);
+  const double p = eq_poly(k, (double)b.x, (double)b.y);
   if constexpr (EQF) {
-    return A(kW[k]) * (A)a.x * (A(1) + p);
+    return kW[k] * a.x * (1.0 + p);
   } else {
-    const A hf = (A)h_k<R>(k, b.z, b.w, cc.x);
-    return A(kW[k]) * (A)a.x * (A(1) + p) + A(coef_of(k)) * hf;
+    const double hf = (double)h_k<R>(k, b.z, b.w, cc.x);
+    return kW[k] * a.x * (1.0 + p) + coef_of(k) * hf;
   }
 }
 
 // Equilibrium deviation of a boundary ghost, g_k - w_k*T_crit.
-template <typename A = double>
-__device__ __forceinline__ A ghost_gdev(int k, A T, A u, A v) {
-  return A(kW[k]) * (T - A(kTcrit)) + A(kW[k]) * T * eq_poly_t<A>(k, u, v);
+__device__ __forceinline__ double ghost_gdev(int k, double T, double u, double v) {
+  return kW[k] * (T - kTcrit) + kW[k] * T * eq_poly(k, u, v);
 }
 
 // Moments of the pulled populations of a node: zeroth, first and second
 // moments of f, and of gd = g - w*T_crit (its first moment is not needed).
+// A: the arithmetic type, double but for the adjoint of the FP32 moment step,
+// which evaluates its Jacobians in FP32.
 template <typename A>
 struct PullSumsT {
   A rho, jx, jy, fxx, fyy, fxy;
@@ -192,15 +185,13 @@ struct PullSumsT {
 };
 using PullSums = PullSumsT<double>;
 
-template <typename A>
-__device__ __forceinline__ void pull_zero(PullSumsT<A>& S) {
-  S.rho = S.jx = S.jy = S.fxx = S.fyy = S.fxy = A(0);
-  S.dT = S.gxx = S.gyy = S.gxy = A(0);
+__device__ __forceinline__ void pull_zero(PullSums& S) {
+  S.rho = S.jx = S.jy = S.fxx = S.fyy = S.fxy = 0.0;
+  S.dT = S.gxx = S.gyy = S.gxy = 0.0;
 }
 
 // Add population k (f_k, gd_k) to the sums.
-template <typename A>
-__device__ __forceinline__ void pull_add(PullSumsT<A>& S, int k, A fk, A gk) {
+__device__ __forceinline__ void pull_add(PullSums& S, int k, double fk, double gk) {
   S.rho += fk;
   S.dT += gk;
   if (CX[k] != 0) {
@@ -295,9 +286,10 @@ __device__ __forceinline__ A omega_g_of(const C& c, A phi) {
   return rcp_nr(A(0.5) + alpha * A(3));  // 1/(1/2 + alpha/cs2)
 }
 
+// st, st2: sums of the nine phi_prec taps and of their squares, pc the centre tap.
 template <typename A, typename C>
-__device__ __forceinline__ CoreT<A> core_forward_t(const C& c, const PullSumsT<A>& S,
-                                                   const A tap[9]) {
+__device__ __forceinline__ CoreT<A> core_from_sums(const C& c, const PullSumsT<A>& S, A st, A st2,
+                                                   A pc) {
   CoreT<A> o;
   o.rho = S.rho;
   o.dT2 = S.dT;
@@ -306,17 +298,11 @@ __device__ __forceinline__ CoreT<A> core_forward_t(const C& c, const PullSumsT<A
   o.v2 = S.jy * o.irho;
 
   // sum_m ((1 +/- t_m)/2)^2 = (9 +/- 2 sum t + sum t^2) / 4
-  A st = tap[0], st2 = tap[0] * tap[0];
-#pragma unroll
-  for (int m = 1; m < 9; ++m) {
-    st = st + tap[m];
-    st2 = fma(tap[m], tap[m], st2);
-  }
   const A kp = A(0.25) * ((A(9) + st2) + A(2) * st);
   const A km = A(0.25) * ((A(9) + st2) - A(2) * st);
   o.kp_sum = kp;
   o.km_sum = km;
-  o.pc = tap[0];
+  o.pc = pc;
   // Both reaction terms vanish exactly when kp = 0 (all taps -1) or pc = 1,
   // and km = 0 (all taps +1) or pc = -1: phi = pc whatever the rates, which
   // are then not evaluated (rm = 1/2 keeps every product below finite; the
@@ -350,7 +336,13 @@ __device__ __forceinline__ CoreT<A> core_forward_t(const C& c, const PullSumsT<A
 
 __device__ __forceinline__ Core core_forward(const Consts& c, const PullSums& S,
                                              const double tap[9]) {
-  return core_forward_t<double, Consts>(c, S, tap);
+  double st = tap[0], st2 = tap[0] * tap[0];
+#pragma unroll
+  for (int m = 1; m < 9; ++m) {
+    st = st + tap[m];
+    st2 = fma(tap[m], tap[m], st2);
+  }
+  return core_from_sums<double, Consts>(c, S, st, st2, tap[0]);
 }
 
 // Averaged moments of STEP_7/moments.f90:11-25 from the stored state: sum_k

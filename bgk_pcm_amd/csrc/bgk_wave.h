@@ -43,6 +43,14 @@ __device__ __forceinline__ double from_east(double x) {
                                                             0xf, 0xf, true);
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
+__device__ __forceinline__ float from_west(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x),
+                                                               kDppShr1, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float from_east(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x),
+                                                               kDppShl1, 0xf, 0xf, true));
+}
 
 // Buffer descriptor of n elements at p (wave-uniform), and a store of one
 // element at offset q that the hardware drops where q >= n.  kPastStrip times
@@ -55,25 +63,25 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t strip_buffer(E* p, int n) {
   return __builtin_amdgcn_make_buffer_rsrc(p, 0, n * (int)sizeof(E), 0x00020000);
 }
 constexpr int kNonTemporal = 2;
-template <typename E>
+template <int HOW = kNonTemporal, typename E>
 __device__ __forceinline__ void buffer_put(__amdgpu_buffer_rsrc_t r, int q, const E& x) {
   typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
   const int off = (int)((unsigned)q * (unsigned)sizeof(E));
   if constexpr (sizeof(E) == 4) {
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x), r, off, 0, kNonTemporal);
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x), r, off, 0, HOW);
   } else if constexpr (sizeof(E) == 8) {
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), r, off, 0, kNonTemporal);
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), r, off, 0, HOW);
   } else if constexpr (sizeof(E) == 16) {
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, off, 0, kNonTemporal);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, off, 0, HOW);
   } else {
     static_assert(sizeof(E) == 32, "element size");
     struct Two {
       u32x4 lo, hi;
     };
     const Two t = __builtin_bit_cast(Two, x);
-    __builtin_amdgcn_raw_buffer_store_b128(t.lo, r, off, 0, kNonTemporal);
-    __builtin_amdgcn_raw_buffer_store_b128(t.hi, r, off + 16, 0, kNonTemporal);
+    __builtin_amdgcn_raw_buffer_store_b128(t.lo, r, off, 0, HOW);
+    __builtin_amdgcn_raw_buffer_store_b128(t.hi, r, off + 16, 0, HOW);
   }
 }
 
@@ -89,6 +97,11 @@ __device__ __forceinline__ E at(const E* base, unsigned off) {
 __device__ __forceinline__ double taken(double x) {
   double y;
   asm("v_mov_b64 %0, %1" : "=v"(y) : "v"(x));
+  return y;
+}
+__device__ __forceinline__ float taken(float x) {
+  float y;
+  asm("v_mov_b32 %0, %1" : "=v"(y) : "v"(x));
   return y;
 }
 
@@ -188,11 +201,12 @@ inline WaveGrid split_waves(int nx, int ny, int cols, int T, int extra, double s
 
 // The strip height, 1..most, by a model of the launch.  Up to one wave per SIMD
 // (4 n_cu) all run at once at full speed; two waves on a SIMD slow each other
-// by 1.2 to 1.6 (measured, large to small lattices); beyond 8 n_cu waves the
-// launch takes its work at that rate, plus half a strip for the last waves.
-// Taller strips repeat fewer rows.  rows_override > 0 fixes the height.
+// by 1.2 to 1.6 (measured, large to small lattices); beyond 8 n_cu waves (4
+// n_cu where the registers hold one wave, `deep` = 1) the launch takes its work
+// at that rate, plus half a strip for the last waves.  Taller strips repeat
+// fewer rows.  rows_override > 0 fixes the height.
 inline WaveGrid make_wave_grid(int nx, int ny, int cols, int T, int extra, double slow, int most,
-                               int n_cu, int rows_override) {
+                               int n_cu, int rows_override, int deep = 2) {
   // (offsets within a strip stay below kMaxStrip elements)
   most = std::max(1, std::min({most, ny, kMaxRows, (int)(kMaxStrip / (int64_t)(nx + 256))}));
   if (rows_override > 0)
@@ -201,15 +215,16 @@ inline WaveGrid make_wave_grid(int nx, int ny, int cols, int T, int extra, doubl
   double cost = -1.0;
   for (int h = 1; h <= most; ++h) {
     const WaveGrid g = split_waves(nx, ny, cols, T, extra, slow, h);
-    const double inner = g.nseg - g.ne, slots = 8.0 * n_cu;
+    const double inner = g.nseg - g.ne, slots = 4.0 * deep * n_cu;
+    const double shared = deep > 1 ? 1.35 : 1.0;
     const double waves = g.nedge + inner * g.nmid;
     const double te = slow * (std::max(g.re, inner > 0 ? g.ra : 0) + extra);
     const double longest = std::max(te, g.nmid > 0 ? (double)(h + extra) : 0.0);
     const double work = slow * ((double)g.ne * g.nse * (g.re + extra) + 2 * inner * (g.ra + extra)) +
                         inner * g.nmid * (h + extra);
-    const double c = waves <= 0.5 * slots ? longest
-                     : waves <= slots     ? 1.35 * longest
-                                          : 1.35 * (work / slots + 0.5 * longest);
+    const double c = waves <= 4.0 * n_cu ? longest
+                     : waves <= slots      ? shared * longest
+                                           : shared * (work / slots + 0.5 * longest);
     if (cost < 0.0 || c < cost) {
       cost = c;
       best = g;
