@@ -84,6 +84,30 @@ __device__ __forceinline__ void stream_store(double* p, double x) {
   __builtin_nontemporal_store(x, p);
 }
 
+// The same, or through the caches.
+template <bool CACHED, typename P2>
+__device__ __forceinline__ P2 load_pair(const P2* p) {
+  return CACHED ? *p : stream_load(p);
+}
+template <bool CACHED, typename P2, typename E>
+__device__ __forceinline__ void store_pair(P2* p, E x, E y) {
+  if constexpr (CACHED) {
+    P2 v;
+    v.x = x;
+    v.y = y;
+    *p = v;
+  } else {
+    stream_store(p, x, y);
+  }
+}
+template <bool CACHED>
+__device__ __forceinline__ void store_one(double* p, double x) {
+  if constexpr (CACHED)
+    *p = x;
+  else
+    stream_store(p, x);
+}
+
 // Pair views of the same planes (used by the fused kernels).
 struct Pairs64 {
   double2* p[9];
@@ -163,28 +187,42 @@ __device__ __forceinline__ double east_T(const Consts& c, const double* te, int 
   return c.east_cold ? c.t_cold : te[j];
 }
 
-// XCD-aware tiling of the fused kernels.  The lattice interior is cut into
-// tiles of one row j and TILE_W consecutive columns.  gfx950 dispatches
-// workgroup b to XCD b % 8, and each XCD has its own L2; a pull reads one
-// cache line past each end of its row segment, which the neighbouring
-// segment of the same row also reads.  So all segments of a row go to one
-// XCD (workgroup b serves row (b/8 / nseg)*8 + b%8 + 1, segment b/8 % nseg):
-// the shared lines are L2 hits, and at any moment the eight XCDs stream
-// eight neighbouring rows.  Workgroups past the last row return at once.
+// XCD-aware tiling of the one-step population kernels.  The lattice interior is
+// cut into tiles of one row j and TILE_W consecutive columns.  gfx950 dispatches
+// workgroup b to XCD b % 8, and each XCD has its own L2.  All segments of a row
+// go to one XCD (a pull reads one cache line past each end of its segment, which
+// the neighbouring segment reads too), and the rows either
+//  * in eight bands, row by row within each: a row's populations are then read
+//    by the XCD that wrote them, and pulled from the rows above and below within
+//    it; for lattices whose two states fit the 256 MB last-level cache; or
+//  * in turn, so that at any moment the eight XCDs stream eight neighbouring
+//    rows of memory.
+// FP64, us per step in turn / in bands: 256^2 7.5 / 6.6, 128 x 512 8.7 / 7.7,
+// 512^2 19.2 / 17.5, 2048^2 226 / 242.
+// Workgroups past the last row return at once.
 constexpr int NXCD = 8;
 constexpr int TILE_W = 256;
 
 struct TileGrid {
-  int nseg;        // tiles per row
-  int64_t ntiles;  // nseg * ny
-  int64_t per;     // workgroups per XCD: ceil(ny/8) * nseg
+  int nseg;     // tiles per row
+  int band;     // rows per XCD (0: in turn)
+  int64_t per;  // workgroups per XCD: ceil(ny/8) * nseg
+  bool cached;  // loads and stores through the caches, see make_tile_grid
 };
 
-inline TileGrid make_tile_grid(const Geom& g) {
+// node_bytes: read and written per node and step.  Lattices in bands of more than
+// 2^16 nodes go through the caches: the planes written past them (nt) are
+// fetched from further away in the next step (FP64, us per step past / through:
+// 384^2 12.5 / 10.8, 512^2 17.6 / 13.9, 1003 x 777 48.7 / 39.5; 256^2 6.6 / 6.9,
+// 2048^2 242 / 252).
+inline TileGrid make_tile_grid(const Geom& g, int node_bytes) {
+  const int64_t nodes = (int64_t)g.nx * g.ny;
+  const int rows = (g.ny + NXCD - 1) / NXCD;
   TileGrid t;
   t.nseg = (g.nx + TILE_W - 1) / TILE_W;
-  t.ntiles = (int64_t)t.nseg * g.ny;
-  t.per = (int64_t)((g.ny + NXCD - 1) / NXCD) * t.nseg;
+  t.band = nodes * node_bytes <= (int64_t)256 << 20 ? rows : 0;
+  t.per = (int64_t)rows * t.nseg;
+  t.cached = t.band > 0 && nodes > (int64_t)1 << 16;
   return t;
 }
 
@@ -192,7 +230,8 @@ inline TileGrid make_tile_grid(const Geom& g) {
 __device__ __forceinline__ bool tile_node(const TileGrid& t, const Geom& g, int* i, int* j) {
   const int64_t b = blockIdx.x;
   const int64_t k = b / NXCD;
-  *j = (int)((k / t.nseg) * NXCD + (b % NXCD)) + 1;
+  const int x = (int)(b % NXCD), row = (int)(k / t.nseg);
+  *j = (t.band > 0 ? x * t.band + row : row * NXCD + x) + 1;
   if (*j > g.ny) return false;
   *i = (int)(k % t.nseg) * TILE_W + (int)threadIdx.x + 1;
   return *i <= g.nx;

@@ -41,6 +41,8 @@ inline Pairs64 pairs(double* const* fplanes) {
   return r;
 }
 
+constexpr int kNodeBytes = 2 * (18 + 1) * (int)sizeof(double);  // populations and phi
+
 __global__ void k_teast_prologue(const double* __restrict__ T, double* __restrict__ te, Geom gm) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j > gm.ny + 1) return;
@@ -51,9 +53,9 @@ __global__ void k_teast_prologue(const double* __restrict__ T, double* __restric
 // waves make a dozen dependent memory accesses.  So a wave that holds a
 // boundary-adjacent node takes one path for all its lanes, with every load
 // (ghost velocities and halo values included) issued before the first use
-// (us per step: 256^2 9.4 with the ghosts' loads in branches, 7.6 so; 97 x 61 7.7
-// and 6.1).
-template <bool STEP7>
+// (us per step: 256^2 9.4 with the ghosts' loads in branches, 7.6 so; with rows in
+// bands, make_tile_grid, 6.4; 97 x 61 7.7, 6.1 and 5.7).
+template <bool STEP7, bool CACHED>
 __global__ __launch_bounds__(TILE_W) void k_fused64(Planes<double2> A, Planes<double2> B,
                                                      const double* __restrict__ pa,
                                                      double* __restrict__ pb,
@@ -83,7 +85,7 @@ __global__ __launch_bounds__(TILE_W) void k_fused64(Planes<double2> A, Planes<do
   if (!__any(edge)) {
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
-      const double2 fg = stream_load(A.row(k, q - CX[k] - (int64_t)CY[k] * P));
+      const double2 fg = load_pair<CACHED>(A.row(k, q - CX[k] - (int64_t)CY[k] * P));
       in.f[k] = fg.x;
       in.g[k] = fg.y;
     }
@@ -125,8 +127,8 @@ __global__ __launch_bounds__(TILE_W) void k_fused64(Planes<double2> A, Planes<do
   // ---- momentsPre .. collision
   const Done o = node_step<STEP7>(c, in.f, in.g, tap);
 #pragma unroll
-  for (int k = 0; k < 9; ++k) stream_store(B.row(k, q), o.f[k], o.g[k]);
-  stream_store(&pb[q], o.phi);
+  for (int k = 0; k < 9; ++k) store_pair<CACHED>(B.row(k, q), o.f[k], o.g[k]);
+  store_one<CACHED>(&pb[q], o.phi);
 
   // ---- moments (STEP_7/moments.f90:11-25), where somebody reads them
   if (edge || write_all) {
@@ -191,8 +193,8 @@ __global__ __launch_bounds__(TILE_W) void k_fused64(Planes<double2> A, Planes<do
 // tiles copy the ghosts, of which a boundary type may leave some unwritten, to
 // the next step's planes.  304 B per node as k_fused64, where the eight
 // subroutines move about 1.1 KB in ten launches (1024 x 512 channel, us per
-// step: 149 by subroutines, 48 in two launches).
-template <bool STEP7>
+// step: 149 by subroutines, 48 in two launches, 38 with rows in bands).
+template <bool STEP7, bool CACHED>
 __global__ __launch_bounds__(TILE_W) void k_general64(Pairs64 A, Pairs64 B,
                                                       const double* __restrict__ pa,
                                                       double* __restrict__ pb, Macro m, Consts c,
@@ -218,7 +220,7 @@ __global__ __launch_bounds__(TILE_W) void k_general64(Pairs64 A, Pairs64 B,
   double fp[9], gp[9];
 #pragma unroll
   for (int k = 0; k < 9; ++k) {
-    const double2 fg = stream_load(&A.p[k][q - CX[k] - (int64_t)CY[k] * P]);
+    const double2 fg = load_pair<CACHED>(&A.p[k][q - CX[k] - (int64_t)CY[k] * P]);
     fp[k] = fg.x;
     gp[k] = fg.y;
   }
@@ -226,8 +228,8 @@ __global__ __launch_bounds__(TILE_W) void k_general64(Pairs64 A, Pairs64 B,
                          pa[q + 1 + P], pa[q - 1 + P], pa[q - 1 - P], pa[q + 1 - P]};
   const Done o = node_step<STEP7>(c, fp, gp, tap);
 #pragma unroll
-  for (int k = 0; k < 9; ++k) stream_store(&B.p[k][q], o.f[k], o.g[k]);
-  stream_store(&pb[q], o.phi);
+  for (int k = 0; k < 9; ++k) store_pair<CACHED>(&B.p[k][q], o.f[k], o.g[k]);
+  store_one<CACHED>(&pb[q], o.phi);
   // BC_f and BC_g read the moments of the boundary-adjacent nodes
   if (write_all || i == 1 || i == nx || j == 1 || j == ny) {
     const Avg a = averaged(o);
@@ -252,7 +254,7 @@ hipError_t launch_teast_prologue(bgk_handle* h) {
 
 hipError_t launch_fused_step64(bgk_handle* h, bool write_all) {
   const Geom& g = h->geom;
-  const TileGrid tg = make_tile_grid(g);
+  const TileGrid tg = make_tile_grid(g, kNodeBytes);
   dim3 blk(TILE_W);
   dim3 grd((unsigned)(tg.per * NXCD));
   Macro m{h->rho, h->u, h->v, h->T};
@@ -260,12 +262,11 @@ hipError_t launch_fused_step64(bgk_handle* h, bool write_all) {
   double* te_out = h->teast[1 - h->te_cur];
   const int a = h->cur, b = 1 - h->cur;
   const Planes<double2> A = wave::planes_of<double2>(h->f[a]), B = wave::planes_of<double2>(h->f[b]);
-  if (h->prm.rounding == BGK_ROUND_STEP7)
-    hipLaunchKernelGGL(k_fused64<true>, grd, blk, 0, h->stream, A, B, h->phi[h->pc],
-                       h->phi[1 - h->pc], te_in, te_out, m, h->c, g, tg, write_all ? 1 : 0);
-  else
-    hipLaunchKernelGGL(k_fused64<false>, grd, blk, 0, h->stream, A, B, h->phi[h->pc],
-                       h->phi[1 - h->pc], te_in, te_out, m, h->c, g, tg, write_all ? 1 : 0);
+  const bool s7 = h->prm.rounding == BGK_ROUND_STEP7;
+  const auto k = s7 ? (tg.cached ? k_fused64<true, true> : k_fused64<true, false>)
+                    : (tg.cached ? k_fused64<false, true> : k_fused64<false, false>);
+  hipLaunchKernelGGL(k, grd, blk, 0, h->stream, A, B, h->phi[h->pc], h->phi[1 - h->pc], te_in,
+                     te_out, m, h->c, g, tg, write_all ? 1 : 0);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) {
     h->cur = b;
@@ -279,19 +280,16 @@ hipError_t launch_general_step64(bgk_handle* h, bool write_all) {
   hipError_t e = launch_bc(h, true, true);
   if (e != hipSuccess) return e;
   const Geom& g = h->geom;
-  const TileGrid tg = make_tile_grid(g);
+  const TileGrid tg = make_tile_grid(g, kNodeBytes);
   const int64_t ghosts = 2 * ((int64_t)g.nx + 2) + 2 * (int64_t)g.ny;
   const dim3 grd((unsigned)(tg.per * NXCD + (ghosts + TILE_W - 1) / TILE_W));
   Macro m{h->rho, h->u, h->v, h->T};
   const int a = h->cur, b = 1 - h->cur;
-  if (h->prm.rounding == BGK_ROUND_STEP7)
-    hipLaunchKernelGGL(k_general64<true>, grd, dim3(TILE_W), 0, h->stream, pairs(h->f[a]),
-                       pairs(h->f[b]), h->phi[h->pc], h->phi[1 - h->pc], m, h->c, g, tg,
-                       write_all ? 1 : 0);
-  else
-    hipLaunchKernelGGL(k_general64<false>, grd, dim3(TILE_W), 0, h->stream, pairs(h->f[a]),
-                       pairs(h->f[b]), h->phi[h->pc], h->phi[1 - h->pc], m, h->c, g, tg,
-                       write_all ? 1 : 0);
+  const bool s7 = h->prm.rounding == BGK_ROUND_STEP7;
+  const auto k = s7 ? (tg.cached ? k_general64<true, true> : k_general64<true, false>)
+                    : (tg.cached ? k_general64<false, true> : k_general64<false, false>);
+  hipLaunchKernelGGL(k, grd, dim3(TILE_W), 0, h->stream, pairs(h->f[a]), pairs(h->f[b]),
+                     h->phi[h->pc], h->phi[1 - h->pc], m, h->c, g, tg, write_all ? 1 : 0);
   e = hipGetLastError();
   if (e == hipSuccess) {
     h->cur = b;

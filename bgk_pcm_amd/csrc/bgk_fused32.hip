@@ -216,7 +216,7 @@ __device__ __forceinline__ double rho_ref(const double* __restrict__ tab, int S,
   return rs + (0.5 * (1.0 + phi)) * (tab[S + j] - rs);
 }
 
-template <typename RC>
+template <typename RC, bool CACHED>
 __global__ __launch_bounds__(TILE_W) void k_fused32(Pairs32 A, Pairs32 B,
                                                      const double* __restrict__ pa,
                                                      double* __restrict__ pb,
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(TILE_W) void k_fused32(Pairs32 A, Pairs32 B,
   if (!edge) {
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
-      const float2 fg = stream_load(&A.p[k][q - CX[k] - (int64_t)CY[k] * P]);
+      const float2 fg = load_pair<CACHED>(&A.p[k][q - CX[k] - (int64_t)CY[k] * P]);
       const double sh = k == 0 ? 0.0 : rho_ref(tab, S, j - CY[k], tap[OPP[k]]) - r0;
       df[k] = (double)fg.x + kW[k] * sh;
       dg[k] = (double)fg.y;
@@ -290,9 +290,9 @@ __global__ __launch_bounds__(TILE_W) void k_fused32(Pairs32 A, Pairs32 B,
 #pragma unroll
   for (int k = 0; k < 9; ++k) {
     fs[k] = (float)(fd[k] + kW[k] * dr);
-    stream_store(&B.p[k][q], fs[k], gs[k]);
+    store_pair<CACHED>(&B.p[k][q], fs[k], gs[k]);
   }
-  stream_store(&pb[q], o.phi);
+  store_one<CACHED>(&pb[q], o.phi);
 
   if (!(edge || write_all)) return;
   // ---- moments of the stored state (STEP_7/moments.f90:11-25)
@@ -549,7 +549,7 @@ hipError_t launch_fused_steps32(bgk_handle* h, int nsteps) {
 
 hipError_t launch_fused_step32(bgk_handle* h, bool write_all) {
   const Geom& g = h->geom;
-  const TileGrid tg = make_tile_grid(g);
+  const TileGrid tg = make_tile_grid(g, 2 * (18 * (int)sizeof(float) + (int)sizeof(double)));
   dim3 blk(TILE_W);
   dim3 grd((unsigned)(tg.per * NXCD));
   Macro m{h->rho, h->u, h->v, h->T};
@@ -557,14 +557,12 @@ hipError_t launch_fused_step32(bgk_handle* h, bool write_all) {
   double* te_out = h->teast[1 - h->te_cur];
   const int a = h->cur, b = 1 - h->cur;
   const double* tab = h->rref[h->rc];
-  if (h->prm.fp32_collision)
-    hipLaunchKernelGGL(k_fused32<float>, grd, blk, 0, h->stream, pairs32(h->f32[a]),
-                       pairs32(h->f32[b]), h->phi[h->pc], h->phi[1 - h->pc], te_in, te_out, m,
-                       h->c, g, tg, tab, write_all ? 1 : 0);
-  else
-    hipLaunchKernelGGL(k_fused32<double>, grd, blk, 0, h->stream, pairs32(h->f32[a]),
-                       pairs32(h->f32[b]), h->phi[h->pc], h->phi[1 - h->pc], te_in, te_out, m,
-                       h->c, g, tg, tab, write_all ? 1 : 0);
+  const auto k = h->prm.fp32_collision
+                     ? (tg.cached ? k_fused32<float, true> : k_fused32<float, false>)
+                     : (tg.cached ? k_fused32<double, true> : k_fused32<double, false>);
+  hipLaunchKernelGGL(k, grd, blk, 0, h->stream, pairs32(h->f32[a]), pairs32(h->f32[b]),
+                     h->phi[h->pc], h->phi[1 - h->pc], te_in, te_out, m, h->c, g, tg, tab,
+                     write_all ? 1 : 0);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) {
     h->cur = b;

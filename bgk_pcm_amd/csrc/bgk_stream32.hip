@@ -280,8 +280,8 @@ __global__ __launch_bounds__(kLanes, 2) void k_stream32(Args32 A) {
 }  // namespace
 
 // Measured, us per step, two steps per launch against k_fused32: 4096^2 354
-// (472), 2048^2 91 (135), 1003 x 777 25.4 (38.4), 512^2 19.6 (16.8), 256^2 16
-// (10).  FP32 collision arithmetic and uploaded ghost velocities are the
+// (472), 2048^2 91 (135), 1003 x 777 25.4 (27.9), 724^2 22.2 (23.1), 512^2
+// 19.6 (14.6).  FP32 collision arithmetic and uploaded ghost velocities are the
 // general kernel's.
 bool stream32(const bgk_handle* h) {
   if (!h->ghost_uv || h->prm.fp32_collision || h->pop_variant == 1) return false;

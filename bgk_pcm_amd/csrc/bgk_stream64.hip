@@ -20,8 +20,8 @@
 // What bounds it: HBM (152 B per node and step, 304 with one step per launch);
 // a row costs its wave 1330 VALU instructions at two waves per SIMD, 75% of
 // its time at the memory rate.  Measured, us per step, against bgk_fused.hip:
-// 4096^2 552 (893), 2048^2 152 (228), 1003 x 777 34.9 (49), 512^2 18.1 (19.3),
-// 256^2 12.6 (7.6): below 2^18 nodes one step per launch stays (stream64).
+// 4096^2 552 (893), 2048^2 152 (228), 1003 x 777 34.9 (38.5), 724^2 27.6
+// (26.6), 512^2 18.1 (13.9): below 2^19 nodes one step per launch (stream64).
 #include <algorithm>
 
 #include "bgk_pop64.h"
@@ -398,12 +398,12 @@ __global__ __launch_bounds__(kLanes, 2) void k_stream64(Args64 A) {
 
 }  // namespace
 
-// Lattices below 2^18 nodes stay in the caches, and the few waves they give
-// are bound by the latency of their rows; a handle whose ghost velocities were
+// Below 2^19 nodes one step per launch is faster (it stays in the caches, and the
+// few waves of this kernel are bound by the latency of their rows); a handle whose ghost velocities were
 // uploaded takes the general kernel.
 bool stream64(const bgk_handle* h) {
   if (!h->ghost_uv || h->pop_variant == 1) return false;
-  return h->pop_variant > 1 || (int64_t)h->nx * h->ny >= (int64_t)1 << 18;
+  return h->pop_variant > 1 || (int64_t)h->nx * h->ny >= (int64_t)1 << 19;
 }
 
 hipError_t launch_stream64(bgk_handle* h, bool write_all) {
