@@ -442,7 +442,7 @@ constexpr int adj_waves() {
 // 29.3); FP32 ones past them (2048^2, 48 steps: 9.2 ms for 9.3).
 template <typename R>
 constexpr int adj_store() {
-  return sizeof(R) == 4 ? kNonTemporal : 0;
+  return sizeof(R) == 4 ? kNonTemporal : kCached;
 }
 // The initial phi of the ghost columns 0 and Nx+1, which no step changes
 // (STEP_7/initialization.f90:15-26: liquid for i <= Nx/40).

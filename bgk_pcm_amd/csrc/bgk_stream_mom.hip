@@ -89,7 +89,7 @@ constexpr double kPhiWest = 1.0, kPhiEast = -1.0;
 
 // Stores of a strip's nodes through buffer descriptors: a lane that must not
 // store gives an offset past the strip.
-template <typename R, bool EQF>
+template <typename R, bool EQF, int HOW>
 struct StoreMom {
   using V4 = typename Vec<R>::V4;
   using C = typename CType<R, EQF>::T;
@@ -102,15 +102,15 @@ struct StoreMom {
   }
   __device__ __forceinline__ void store(int q, bool on, bool on_phi, const Updated& o) const {
     const int qa = on ? q : kPastStrip;
-    buffer_put(a, qa, make_double2(o.rho, o.dT));
+    buffer_put<HOW>(a, qa, make_double2(o.rho, o.dT));
     if constexpr (EQF) {
-      buffer_put(b, qa, make4<R>((R)o.u, (R)o.v, (R)o.pgxx, (R)o.pgyy));
-      buffer_put(c, qa, (R)o.pgxy);
+      buffer_put<HOW>(b, qa, make4<R>((R)o.u, (R)o.v, (R)o.pgxx, (R)o.pgyy));
+      buffer_put<HOW>(c, qa, (R)o.pgxy);
     } else {
-      buffer_put(b, qa, make4<R>((R)o.u, (R)o.v, (R)o.pfxx, (R)o.pfyy));
-      buffer_put(c, qa, make4<R>((R)o.pfxy, (R)o.pgxx, (R)o.pgyy, (R)o.pgxy));
+      buffer_put<HOW>(b, qa, make4<R>((R)o.u, (R)o.v, (R)o.pfxx, (R)o.pfyy));
+      buffer_put<HOW>(c, qa, make4<R>((R)o.pfxy, (R)o.pgxx, (R)o.pgyy, (R)o.pgxy));
     }
-    buffer_put(phi, on_phi ? q : kPastStrip, o.phi);
+    buffer_put<HOW>(phi, on_phi ? q : kPastStrip, o.phi);
   }
 };
 
@@ -206,7 +206,7 @@ enum { kPlain, kProbes, kFinal };
 // the hardware drops, so that the wait for a row's loads (issued two rows
 // ahead) never has to cover stores issued since.  With conditional stores the
 // compiler's waits did, and a row cost 2.2 us of store latency on top.
-template <int T, typename R, bool EQF, bool EDGE, int MODE>
+template <int T, typename R, bool EQF, bool EDGE, int MODE, int HOW>
 __device__ __forceinline__ void stream_strip(const StreamArgs& A, int i0, int j0, int j1, int i,
                                              bool has_w, bool has_e) {
   const int nx = A.nx, ny = A.ny;
@@ -218,7 +218,7 @@ __device__ __forceinline__ void stream_strip(const StreamArgs& A, int i0, int j0
   // phi also in the ghost columns next to an owned column
   const bool own_phi = own || (ghost && (i == 0 ? has_w : lane <= kLanes - T));
   const int64_t qs = (int64_t)j0 * P;  // first node of the strip
-  const StoreMom<R, EQF> out(A.out, A.pb, qs, (j1 - j0 + 1) * (int)P);
+  const StoreMom<R, EQF, HOW> out(A.out, A.pb, qs, (j1 - j0 + 1) * (int)P);
 
   // rows of the strip that hold a probe (the flags in column 0 of the probe
   // index plane; at most kMaxRows rows)
@@ -300,7 +300,7 @@ __device__ __forceinline__ void stream_strip(const StreamArgs& A, int i0, int j0
   }
 }
 
-template <int T, typename R, bool EQF, int MODE>
+template <int T, typename R, bool EQF, int MODE, int HOW>
 __global__ __launch_bounds__(kLanes, 2) void k_stream_mom(StreamArgs A) {
   int seg, j0, j1;
   bool edge;
@@ -308,9 +308,10 @@ __global__ __launch_bounds__(kLanes, 2) void k_stream_mom(StreamArgs A) {
   const int i0 = seg * (kLanes - 2 * T) + 1;
   const int i = i0 - T + (int)threadIdx.x;
   if (edge)
-    stream_strip<T, R, EQF, true, MODE>(A, i0, j0, j1, i, i0 - T <= 1, i0 - T + kLanes - 1 >= A.nx);
+    stream_strip<T, R, EQF, true, MODE, HOW>(A, i0, j0, j1, i, i0 - T <= 1,
+                                             i0 - T + kLanes - 1 >= A.nx);
   else
-    stream_strip<T, R, EQF, false, MODE>(A, i0, j0, j1, i, false, false);
+    stream_strip<T, R, EQF, false, MODE, HOW>(A, i0, j0, j1, i, false, false);
 }
 
 template <int T, typename R, bool EQF>
@@ -345,12 +346,21 @@ hipError_t launch_t(bgk_handle* h, const MomStep& st) {
   constexpr int most = sizeof(R) == sizeof(float) ? 64 : 16;
   a.g = make_wave_grid(h->nx, h->ny, kLanes - 2 * T, T, 2 * T, 1.4, most, h->n_cu, h->strip_rows);
   const dim3 grd((unsigned)a.g.nwg);
-  if (st.write_all)
-    hipLaunchKernelGGL((k_stream_mom<T, R, EQF, kFinal>), grd, dim3(kLanes), 0, h->stream, a);
-  else if (st.probe_out)
-    hipLaunchKernelGGL((k_stream_mom<T, R, EQF, kProbes>), grd, dim3(kLanes), 0, h->stream, a);
-  else
-    hipLaunchKernelGGL((k_stream_mom<T, R, EQF, kPlain>), grd, dim3(kLanes), 0, h->stream, a);
+  // Where the states read and written fit the 256 MB last-level cache but not the
+  // L2s, the next launch finds more of what went through the caches than of what
+  // went past them (us per step past / through: FP64 moments 724^2, 88 MB, 14.9 /
+  // 13.2, 1003 x 777 19.9 / 16.1, 1200^2, 242 MB, 32.5 / 26.7, 1300^2, 284 MB, 36.8
+  // / 37.0, 512^2, 44 MB, 8.9 / 9.2; FP32 moments 1448^2, 224 MB, 30.9 / 29.2, 860^2,
+  // 79 MB, 15.1 / 15.2).
+  const int64_t mb = (int64_t)h->nx * h->ny * 2 *
+                     (int64_t)(sizeof(double2) + sizeof(typename Vec<R>::V4) +
+                               sizeof(typename CType<R, EQF>::T) + sizeof(double)) >> 20;
+  const bool cached = mb >= (sizeof(R) == sizeof(float) ? 96 : 64) && mb < 256;
+  const auto k = st.write_all   ? k_stream_mom<T, R, EQF, kFinal, kNonTemporal>
+                 : st.probe_out ? k_stream_mom<T, R, EQF, kProbes, kNonTemporal>
+                 : cached       ? k_stream_mom<T, R, EQF, kPlain, kCached>
+                                : k_stream_mom<T, R, EQF, kPlain, kNonTemporal>;
+  hipLaunchKernelGGL(k, grd, dim3(kLanes), 0, h->stream, a);
   return hipGetLastError();
 }
 

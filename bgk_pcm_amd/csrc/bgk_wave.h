@@ -62,7 +62,7 @@ template <typename E>
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t strip_buffer(E* p, int n) {
   return __builtin_amdgcn_make_buffer_rsrc(p, 0, n * (int)sizeof(E), 0x00020000);
 }
-constexpr int kNonTemporal = 2;
+constexpr int kCached = 0, kNonTemporal = 2;
 template <int HOW = kNonTemporal, typename E>
 __device__ __forceinline__ void buffer_put(__amdgpu_buffer_rsrc_t r, int q, const E& x) {
   typedef unsigned u32x2 __attribute__((ext_vector_type(2)));

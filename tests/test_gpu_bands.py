@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 
 from bgk_pcm_amd.lattice import Lattice
-from bgk_pcm_amd.params import FP32_DEV, FP64, ROUND_CLEAN, ROUND_STEP7, Params
+from bgk_pcm_amd.params import FP32_DEV, FP32_MOM, FP64, FP64_MOM, ROUND_CLEAN, ROUND_STEP7, Params
 from golden_io import compare_state
 from oracle_py import Oracle
 from test_gpu_parity import POPS, STATE, compare_interior, gpu_state
@@ -58,3 +58,21 @@ def test_fp32_step_follows_fp64(monkeypatch, nx, ny, single):
         err = np.abs(got[f] - want[f]).max() / scale
         print(nx, ny, f, err, flush=True)
         assert err <= (1e-4 if single else 1e-6), (f, err)
+
+
+@pytest.mark.parametrize("precision,nx,ny", [(FP64_MOM, 645, 640), (FP32_MOM, 1003, 941),
+                                             (FP32_MOM, 1290, 1003)])
+@pytest.mark.parametrize("tau_f", [1.0, 0.8])
+def test_moment_stores_through_the_caches(precision, nx, ny, tau_f):
+    """Sizes whose plain launches store through the caches: the bits of single
+    steps, each the last launch of its call, which stores past them."""
+    p = Params(nx=nx, ny=ny, length=float(ny), grav=1e-3, rounding=ROUND_CLEAN, tau_f=tau_f,
+               precision=precision)
+    out = []
+    for split in ([11], [1] * 11):
+        with Lattice(p, k_ratio=1.5, noise_amp=1e-3, noise_seed=3) as lat:
+            for n in split:
+                lat.step(n)
+            out.append({f: lat.download(f) for f in FIELDS})
+    for f in FIELDS:
+        assert np.array_equal(out[0][f], out[1][f]), f
