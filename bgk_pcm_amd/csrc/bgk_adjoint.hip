@@ -1021,9 +1021,23 @@ hipError_t launch_adjoint(bgk_handle* h, AdjCtx* x, const StatePtrs& sprev, int 
   return hipGetLastError();
 }
 
-// T forward steps from state `in` to state `out` (explicit buffers) in one launch
-hipError_t fwd_steps(bgk_handle* h, int T, const StatePtrs& in, const StatePtrs& out,
-                     double* probe_out, const int* probe_idx, int np, bool write_all,
+// Whether two steps with the state between them kept go in one launch.  Measured,
+// ms per gradient of 60 steps (segments of 20), backward pass, two launches / one:
+// FP32 moments 512^2 1.70 / 1.71, 1024^2 4.20 / 3.96, 2048^2 15.5 / 14.1, FP64
+// 512^2 2.26 / 2.35, 724^2 3.53 / 3.61, 1024^2 7.49 / 7.19, 2048^2 26.7 / 24.7; with
+// omega_f = 1 FP32 512^2 1.55 / 1.56, 724^2 2.15 / 2.07, 2048^2 12.5 / 11.4, FP64 724^2
+// 2.98 / 2.71, 2048^2 20.1 / 18.4.  (BGK_MOM_VARIANT of 2 or 3: at any size.)
+bool keeps_between(const bgk_handle* h) {
+  if (mom_most_steps(h) < 2) return false;
+  const bool f64 = h->prm.precision == BGK_FP64_MOM;
+  const int64_t least = (int64_t)1 << (f64 && !h->mom_eqf ? 20 : 19);
+  return h->mom_variant > 0 || (int64_t)h->nx * h->ny >= least;
+}
+
+// T forward steps from state `in` to state `out` (explicit buffers) in one launch;
+// T = 2 with `mid`: the state between them too
+hipError_t fwd_steps(bgk_handle* h, int T, const StatePtrs& in, const StatePtrs* mid,
+                     const StatePtrs& out, double* probe_out, const int* probe_idx, int np, bool write_all,
                      double* const* macro) {
   mom::MomStep st;
   st.in = mom::MomIn{in.a, in.b, in.c};
@@ -1037,6 +1051,11 @@ hipError_t fwd_steps(bgk_handle* h, int T, const StatePtrs& in, const StatePtrs&
   st.probe_out = probe_out;
   st.probe_np = np;
   for (int m = 0; m < 4; ++m) st.macro[m] = macro ? macro[m] : nullptr;
+  if (mid) {
+    st.mid = mom::MomOut{mid->a, mid->b, mid->c};
+    st.phi_mid = mid->phi;
+    st.te_mid = mid->te;
+  }
   return launch_mom_steps(h, st, T);
 }
 
@@ -1138,32 +1157,39 @@ hipError_t adj_forward(bgk_handle* h, double* probe_T_host) {
   StatePtrs in{h->ma[h->cur], h->mb[h->cur], h->mc[h->cur], h->phi[h->pc], h->teast[h->te_cur]};
   const StatePtrs& first = x->nsnap > 0 ? x->snap[0] : x->ckpt[0];
   e = copy_state(h, first, in.a, in.b, in.c, in.phi, in.te);
-  for (int n = 0; e == hipSuccess && n < x->nsteps;) {
-    // the next state to keep, if any: the launch that reaches it writes it in
-    // its place, and the one after reads it there, so no state but the first
-    // is copied (2048^2, FP32, 12 states kept of 48 steps: 11 copies of 84 us
-    // less in 4 ms)
-    int stop = x->nsteps;
-    const StatePtrs* keep = nullptr;
+  // the first state after n that is kept (its step in *stop), null: none is
+  auto next_kept = [&](int n, size_t chain, int* stop) -> const StatePtrs* {
+    *stop = x->nsteps;
     if (x->nsnap > 0) {
-      if (next_chain < x->chain.size()) {
-        stop = x->chain[next_chain];
-        keep = &x->snap[next_chain + 1];
-      }
-    } else if ((n / lvl1 + 1) * lvl1 < x->nsteps) {
-      stop = (n / lvl1 + 1) * lvl1;
-      keep = &x->ckpt[(size_t)(stop / lvl1)];
+      if (chain >= x->chain.size()) return nullptr;
+      *stop = x->chain[chain];
+      return &x->snap[chain + 1];
     }
-    const int T = mom_next_steps(h, stop - n);
+    if ((n / lvl1 + 1) * lvl1 >= x->nsteps) return nullptr;
+    *stop = (n / lvl1 + 1) * lvl1;
+    return &x->ckpt[(size_t)(*stop / lvl1)];
+  };
+  for (int n = 0; e == hipSuccess && n < x->nsteps;) {
+    // the launch that reaches a state that is kept writes it in its place, and
+    // the one after reads it there, so no state but the first is copied (2048^2,
+    // FP32, 12 states kept of 48 steps: 11 copies of 84 us less in 4 ms)
+    int stop;
+    const StatePtrs *keep = next_kept(n, next_chain, &stop), *mid = nullptr;
+    int T = mom_next_steps(h, stop - n);
+    if (keep && stop == n + 1 && n + 4 <= x->nsteps && keeps_between(h)) {
+      mid = keep;
+      keep = next_kept(n + 1, ++next_chain, &stop);
+      T = 2;
+    }
     const int b = 1 - h->cur;
     const StatePtrs own{h->ma[b], h->mb[b], h->mc[b], h->phi[1 - h->pc], h->teast[1 - h->te_cur]};
     const bool kept = keep && n + T == stop;
     const StatePtrs out = kept ? *keep : own;
-    e = fwd_steps(h, T, in, out, x->np > 0 ? x->probe_T + (size_t)n * x->np : nullptr,
+    e = fwd_steps(h, T, in, mid, out, x->np > 0 ? x->probe_T + (size_t)n * x->np : nullptr,
                   x->probe_idx, x->np, mom_write_all(h, T, x->nsteps - n - T), nullptr);
     if (e != hipSuccess) return e;
     if (kept) {
-      if (x->nsnap > 0) ++next_chain;
+      ++next_chain;
     } else {
       h->cur = b;
       h->pc = 1 - h->pc;
@@ -1208,25 +1234,32 @@ hipError_t adj_backward(bgk_handle* h, const double* seeds_host, double grad[3])
     has_next = true;
     return e == hipSuccess;
   };
-  auto steps = [&](int T, const StatePtrs& in, const StatePtrs& out) {
+  auto steps = [&](int T, const StatePtrs& in, const StatePtrs* mid, const StatePtrs& out) {
     x->recomputed += T;
-    e = fwd_steps(h, T, in, out, nullptr, nullptr, 0, false, x->macro);
+    e = fwd_steps(h, T, in, mid, out, nullptr, nullptr, 0, false, x->macro);
     return e == hipSuccess;
   };
-  auto step = [&](const StatePtrs& in, const StatePtrs& out) { return steps(1, in, out); };
+  const bool pairs = keeps_between(h);
+  auto step = [&](const StatePtrs& in, const StatePtrs& out) {
+    return steps(1, in, nullptr, out);
+  };
   // from state `src` on by n steps to state `dst`, through two scratch states,
-  // of which `dst` may be one
-  auto run = [&](const StatePtrs& src, int n, const StatePtrs& dst, const StatePtrs* scratch) {
+  // of which `dst` may be one, and `src` the one that the first launch does not
+  // write: launch m writes scratch (first_scratch + m) & 1, the one before last
+  // not `dst`
+  auto first_scratch = [&](int n, const StatePtrs& dst, const StatePtrs* scratch) {
     int launches = 0;
     for (int left = n; left > 0; ++launches) left -= mom_next_steps(h, left);
-    // launch m writes scratch (k + m) & 1: the one before last not `dst`
-    int k = (&dst == &scratch[0] ? 1 : 0) ^ (launches & 1);
+    return (&dst == &scratch[0] ? 1 : 0) ^ (launches & 1);
+  };
+  auto run = [&](const StatePtrs& src, int n, const StatePtrs& dst, const StatePtrs* scratch) {
+    int k = first_scratch(n, dst, scratch);
     const StatePtrs* in = &src;
     for (int left = n; left > 0; k ^= 1) {
       const int T = mom_next_steps(h, left);
       left -= T;
       const StatePtrs* out = left == 0 ? &dst : &scratch[k];
-      if (!steps(T, *in, *out)) return false;
+      if (!steps(T, *in, nullptr, *out)) return false;
       in = out;
     }
     return true;
@@ -1234,10 +1267,34 @@ hipError_t adj_backward(bgk_handle* h, const double* seeds_host, double grad[3])
   if (x->nsnap > 0) {
     // binomial schedule: slots >= 0 are snapshots, -1 and -2 the work states
     auto at = [&](int sl) -> const StatePtrs& { return sl >= 0 ? x->snap[(size_t)sl] : x->work[-1 - sl]; };
-    auto advance = [&](int src, int from, int to, int dst) {
-      return run(at(src), to - from, at(dst), x->work);
+    // an advance by one step waits for the next one from the state it gives,
+    // to share its first launch
+    const StatePtrs *one_src = nullptr, *one_dst = nullptr;
+    auto flush = [&]() {
+      if (!one_src) return true;
+      const StatePtrs* src = one_src;
+      one_src = nullptr;
+      return step(*src, *one_dst);
     };
-    auto adjoint = [&](int n, int sl) { return adjoint_step(n, at(sl)); };
+    auto advance = [&](int src, int from, int to, int dst) {
+      const StatePtrs *s = &at(src), *d = &at(dst);
+      const int n = to - from;
+      if (one_src && one_dst == s) {
+        const StatePtrs* o = n == 1 ? d : &x->work[1 - first_scratch(n - 1, *d, x->work)];
+        const StatePtrs* from0 = one_src;
+        one_src = nullptr;
+        if (!steps(2, *from0, s, *o)) return false;
+        return n == 1 || run(*o, n - 1, *d, x->work);
+      }
+      if (!flush()) return false;
+      if (n == 1 && pairs && src >= 0 && dst >= 0) {
+        one_src = s;
+        one_dst = d;
+        return true;
+      }
+      return run(*s, n, *d, x->work);
+    };
+    auto adjoint = [&](int n, int sl) { return flush() && adjoint_step(n, at(sl)); };
     int right = x->nsteps;
     for (int k = (int)x->chain.size(); k >= 0 && e == hipSuccess; --k) {
       const int a = k == 0 ? 0 : x->chain[(size_t)k - 1];
@@ -1251,7 +1308,11 @@ hipError_t adj_backward(bgk_handle* h, const double* seeds_host, double grad[3])
     // state of the segment (state n0 is `start` itself), then reverse them
     auto inner = [&](const StatePtrs& start, int n0, int n1) {
       auto st = [&](int n) -> const StatePtrs& { return n == n0 ? start : x->slot[n - n0]; };
-      for (int n = n0 + 1; n < n1 && e == hipSuccess; ++n) step(st(n - 1), st(n));
+      for (int n = n0 + 1; n < n1 && e == hipSuccess;) {
+        const bool two = pairs && n + 1 < n1;
+        two ? steps(2, st(n - 1), &st(n), st(n + 1)) : step(st(n - 1), st(n));
+        n += two ? 2 : 1;
+      }
       for (int n = n1; n > n0 && e == hipSuccess; --n) adjoint_step(n, st(n - 1));
     };
     if (x->seg1 == 0) {

@@ -372,6 +372,11 @@ struct MomStep {
   const int* probe_idx;
   double* probe_out;
   int probe_np;
+  // two steps, not the last of a call: the state between them, where it is
+  // kept (mid.a null: it is not)
+  MomOut mid{};
+  double* phi_mid = nullptr;
+  double* te_mid = nullptr;
 };
 
 }  // namespace mom
@@ -381,6 +386,7 @@ struct MomStep {
 hipError_t launch_mom_steps(bgk_handle* h, const mom::MomStep& st, int T);
 hipError_t launch_mom_stream(bgk_handle* h, const mom::MomStep& st, int T);
 int mom_next_steps(const bgk_handle* h, int left);
+int mom_most_steps(const bgk_handle* h);
 bool mom_write_all(const bgk_handle* h, int T, int left);
 }  // namespace bgk
 

@@ -131,6 +131,8 @@ struct StreamArgs {
   const int* probe_idx;
   double* probe_out;
   int probe_np;
+  MomOut mid;  // kKeep, kKeepProbes
+  double *phi_mid, *te_mid;
 };
 
 // What the last launch of a call adds for row jc (1..Ny) completed by level t
@@ -197,8 +199,11 @@ __device__ __forceinline__ void record(const StreamArgs& A, int t, int jc, int i
 
 // What a launch observes besides the state: nothing, probes, or probes and the
 // end of a call (separate instantiations: the probe test alone costs the
-// plain loop 40 VGPRs).
-enum { kPlain, kProbes, kFinal };
+// plain loop 40 VGPRs).  The adjoint's runs keep some states: a launch of two
+// steps that stores the one between them too costs less than two launches where
+// HBM bounds them (2048^2, FP32 moments with omega_f = 1: 142 us, two launches 2 x
+// 92; see keeps_between in bgk_adjoint.hip).
+enum { kPlain, kProbes, kFinal, kKeep, kKeepProbes };
 
 // One wave's strip.  EDGE: the wave or the strip touches a wall.  But for the
 // last launch of a call the loop holds one path for its loads
@@ -219,11 +224,13 @@ __device__ __forceinline__ void stream_strip(const StreamArgs& A, int i0, int j0
   const bool own_phi = own || (ghost && (i == 0 ? has_w : lane <= kLanes - T));
   const int64_t qs = (int64_t)j0 * P;  // first node of the strip
   const StoreMom<R, EQF, HOW> out(A.out, A.pb, qs, (j1 - j0 + 1) * (int)P);
+  constexpr bool KEEP = MODE == kKeep || MODE == kKeepProbes;
+  constexpr bool PROBES = MODE != kPlain && MODE != kKeep;
 
   // rows of the strip that hold a probe (the flags in column 0 of the probe
   // index plane; at most kMaxRows rows)
   uint64_t probes = 0;
-  if (MODE != kPlain && A.probe_out)
+  if (PROBES && A.probe_out)
     probes = __ballot(j0 + lane <= j1 && A.probe_idx[(int64_t)min(j0 + lane, j1) * P] >= 0);
 
   Level L[T];
@@ -270,9 +277,19 @@ __device__ __forceinline__ void stream_strip(const StreamArgs& A, int i0, int j0
       o = update<R, EQF>(A.c, S, st, st2, pc);
       tav = kTcrit + (o.dT + o.dT2) * 0.5;
       const int jd = j - 1 - j0;  // (rows outside the strip are its neighbours')
-      if (MODE != kPlain && jd >= 0 && jd < kMaxRows && ((probes >> jd) & 1) && own)
+      if (PROBES && jd >= 0 && jd < kMaxRows && ((probes >> jd) & 1) && own)
         record(A, t, j - 1, i, tav);
       if (MODE == kFinal && jd >= 0 && j - 1 <= j1 && own) finish<T>(A, t, j - 1, i, o, tav);
+      if (KEEP && t == 0) {
+        const bool mine = jd >= 0 && j - 1 <= j1;
+        Updated k = o;
+        if (EDGE && ghost) k.phi = i == 0 ? kPhiWest : kPhiEast;
+        const StoreMom<R, EQF, HOW> mid(A.mid, A.phi_mid, qs, (j1 - j0 + 1) * (int)P);
+        mid.store(jd * (int)P + i, mine && own, mine && own_phi, k);
+        if (EDGE)
+          buffer_put(strip_buffer(A.te_mid, ny + 2), mine && own && i == nx ? j - 1 : kPastStrip,
+                     tav);
+      }
       if (t < T - 1) {
         nd.rho = o.rho;
         nd.th = o.dT;
@@ -338,6 +355,9 @@ hipError_t launch_t(bgk_handle* h, const MomStep& st) {
   a.probe_idx = st.probe_idx;
   a.probe_out = st.probe_out;
   a.probe_np = st.probe_np;
+  a.mid = st.mid;
+  a.phi_mid = st.phi_mid;
+  a.te_mid = st.te_mid;
   // Strips of at most 64 rows with FP32 moments, 16 with FP64; a row beside a
   // wall counts 1.4 (measured at 1.2 / 1.6 / 2.2, us per step: 512^2 8.9 / 9.5
   // / 10.9, 1003 x 777 15.2 / 15.3 / 17.4, 4096^2 210 / 202 / 209; all strips
@@ -356,6 +376,14 @@ hipError_t launch_t(bgk_handle* h, const MomStep& st) {
                      (int64_t)(sizeof(double2) + sizeof(typename Vec<R>::V4) +
                                sizeof(typename CType<R, EQF>::T) + sizeof(double)) >> 20;
   const bool cached = mb >= (sizeof(R) == sizeof(float) ? 96 : 64) && mb < 256;
+  if constexpr (T == 2) {
+    if (st.mid.a) {
+      const auto k = st.probe_out ? k_stream_mom<T, R, EQF, kKeepProbes, kNonTemporal>
+                                  : k_stream_mom<T, R, EQF, kKeep, kNonTemporal>;
+      hipLaunchKernelGGL(k, grd, dim3(kLanes), 0, h->stream, a);
+      return hipGetLastError();
+    }
+  }
   const auto k = st.write_all   ? k_stream_mom<T, R, EQF, kFinal, kNonTemporal>
                  : st.probe_out ? k_stream_mom<T, R, EQF, kProbes, kNonTemporal>
                  : cached       ? k_stream_mom<T, R, EQF, kPlain, kCached>

@@ -50,3 +50,36 @@ def test_gradient_at_the_edges_of_the_split(nx, ny, tau_f):
             g = lat.adj_backward(2.0 * (rec - 280.0) / rec.size)
         print("precision", prec, g, flush=True)
         np.testing.assert_allclose(g, g_ref, rtol=rtol, atol=of_largest * largest)
+
+
+@pytest.mark.parametrize("precision", [FP64_MOM, FP32_MOM])
+@pytest.mark.parametrize("tau_f", [1.0, 0.8])
+@pytest.mark.parametrize("nx,ny", [(1, 3), (59, 4), (61, 9), (64, 33)])
+def test_schedules_that_keep_the_state_between_two_steps(monkeypatch, nx, ny, precision, tau_f):
+    """Launches of two steps that store the state between them: the record and the
+    gradient have the bits of one step per launch, whatever is kept."""
+    p = Params(nx=nx, ny=ny, length=float(max(nx, ny)), grav=2e-3, rounding=ROUND_CLEAN,
+               tau_f=tau_f, precision=precision, stefan_number=0.1)
+    pi = sorted({1, min(nx, 61), nx})
+    pj = [1 + (3 * k) % ny for k in range(len(pi))]
+    for nsteps in (1, 2, 3, 4, 5, 23):
+        want = None
+        for variant, kind, n in [(1, "seg", nsteps), (2, "seg", nsteps), (2, "seg", 1),
+                                 (2, "seg", min(4, nsteps)), (2, "seg", min(7, nsteps)),
+                                 (2, "states", 1), (2, "states", 2), (2, "states", 3),
+                                 (2, "states", 5), (2, "states", 9)]:
+            monkeypatch.setenv("BGK_MOM_VARIANT", str(variant))
+            with Lattice(p, initialize=False, t_hot=283.5, k_ratio=1.3) as lat:
+                lat.initialization()
+                if kind == "seg":
+                    lat.adj_setup(nsteps, n, pi, pj)
+                else:
+                    lat.adj_setup_binomial(nsteps, n, pi, pj)
+                rec = lat.adj_forward()
+                T = lat.download("T")
+                g = lat.adj_backward(2.0 * (rec - 280.0) / rec.size)
+            want = want or (rec, g, T)
+            case = (nsteps, variant, kind, n)
+            assert np.array_equal(rec, want[0]), case
+            assert np.array_equal(T, want[2]), case
+            assert np.array_equal(g, want[1]), case
