@@ -17,21 +17,22 @@ the GPU to its working clocks) followed by its W warm-up and K timed steps.
 Printed JSON line (one):
   value          MLUPS of the moment-storage step = Nx*Ny*K/t/1e6 over the K
                  timed steps (one bgk_step call after W warm-up steps)
-  roofline       algorithmic HBM bytes per launch (112 B per lattice update:
-                 48 B of moments read + written, phi FP64 read + written)
-                 over the fused kernel's time per launch, measured with HIP
-                 events on the stream the kernel runs on as the difference of
-                 a 400- and a 200-step call (which cancels the last launch of
-                 a call, that also writes every macroscopic field), median of
-                 three; vs 8 TB/s.  last_launch_extra_ms: a one-step call
-                 less a plain launch (median of five)
-  fp32_population the fused step with FP32 population storage (f -
-                 w*rho_ref(row, phi), g - w*T_crit; 160 B per update), same
-                 workload and measurements (the kernel's time per launch on
-                 a handle that does not re-base its reference density;
+  roofline       algorithmic HBM bytes per launch (112 B per node: 48 B of
+                 moments read + written, phi FP64 read + written, once for
+                 the steps_per_launch steps that a launch advances) over the
+                 kernel's time per launch, measured with HIP events on the
+                 stream the kernel runs on as the difference of a 400- and a
+                 200-step call (which cancels the last launch of a call, that
+                 also writes every macroscopic field), median of three; vs 8
+                 TB/s.  last_launch_extra_ms: a call of one launch less a
+                 plain launch (median of five)
+  fp32_population the step with FP32 population storage (f - w*rho_ref(row,
+                 phi), g - w*T_crit; 160 B per node), same workload and
+                 measurements (the kernel's time per launch on a handle that
+                 does not re-base its reference density;
                  ms_per_launch_with_rebase with the re-basing every 500
                  steps amortized)
-  fp64           the FP64 fused kernel (304 B per update), likewise
+  fp64           the FP64 population step (304 B per node), likewise
   fp32_error     relative max-norm error (per field, liquid fraction for
                  phi) after 5000, 10000 and 20000 steps of the FP32 moment
                  and FP32 population storages, of the FP64 moment storage and
@@ -85,10 +86,13 @@ sys.path.insert(0, str(ROOT))
 
 HBM_PEAK_GBS = 8000.0
 METRIC = "MLUPS (D2Q9 f+g) on 1 MI355X: FP32-store vs FP64 at <=1e-5 error; % HBM peak"
-# algorithmic HBM bytes per lattice update: state read + written, phi
-# (FP64) read + written
-BYTES_PER_LUP = {"mom_eq": 36 * 2 + 8 * 2, "mom": 48 * 2 + 8 * 2,
+# algorithmic HBM bytes per node and launch: state read + written, phi (FP64)
+# read + written
+BYTES_PER_NODE = {"mom_eq": 36 * 2 + 8 * 2, "mom": 48 * 2 + 8 * 2,
                  "fp32": 18 * 4 * 2 + 8 * 2, "fp64": 18 * 8 * 2 + 8 * 2}
+# kernels of launches of one and of several steps
+KERNELS = {"mom_eq": ("k_fused_mom", "k_stream_mom"), "mom": ("k_fused_mom", "k_stream_mom"),
+           "fp32": ("k_fused32", "k_stream32"), "fp64": ("k_fused64", "k_stream64")}
 FIELDS = ("rho", "u", "v", "T", "phi")
 BOUND = 1e-5
 
@@ -187,23 +191,31 @@ def call_ms(lat, stream, n: int) -> float:
     return e0.elapsed_time(e1)
 
 
-def per_launch(lat, stream, m: int = 200, reps: int = 3):
-    """(kernel ms per launch, extra ms of a call's last launch): a call of n
-    steps costs a prologue, n - 1 plain launches and a last launch that also
-    writes every macroscopic field, so T(2m) - T(m) = m plain launches
-    (median over reps); the extra is the median time of one-step calls less
-    one plain launch."""
+def steps_per_launch(kind: str, nodes: int) -> int:
+    """Steps a plain launch advances (the library's rules for the storages that
+    are measured here)."""
+    if kind == "mom_eq":
+        return 1 if nodes > 1 << 25 else 2
+    return 2 if kind == "mom" or nodes >= 1 << 19 else 1
+
+
+def per_launch(lat, stream, t: int, m: int = 200, reps: int = 3):
+    """(kernel ms per launch of t steps, extra ms of a call's last launch): a
+    call of n steps costs a prologue, n/t - 1 plain launches and a last launch
+    that also writes every macroscopic field, so T(2m) - T(m) = m/t plain
+    launches (median over reps); the extra is the median time of one-launch
+    calls less one plain launch."""
     k = []
     for _ in range(reps):
         t1 = call_ms(lat, stream, m)
         t2 = call_ms(lat, stream, 2 * m)
-        k.append((t2 - t1) / m)
+        k.append((t2 - t1) * t / m)
     kms = statistics.median(k)
-    one = statistics.median(call_ms(lat, stream, 1) for _ in range(5))
+    one = statistics.median(call_ms(lat, stream, t) for _ in range(5))
     return kms, one - kms
 
 
-def measure(p, stream, steps, warmup, kind, kernel, ext=None):
+def measure(p, stream, steps, warmup, kind, ext=None):
     """MLUPS over `steps` timed steps (wall clock, one bgk_step call after
     `warmup` steps), and the roofline figures of the fused kernel from HIP
     events on its stream.  The per-launch timing runs first: its thousands
@@ -212,6 +224,7 @@ def measure(p, stream, steps, warmup, kind, kernel, ext=None):
     next calls take)."""
     from bgk_pcm_amd.lattice import Lattice
     lups = p.nx * p.ny
+    t = steps_per_launch(kind, lups)
     more = {}
     if kind == "fp32":
         # FP32 populations re-base their reference density every 500 steps
@@ -223,7 +236,7 @@ def measure(p, stream, steps, warmup, kind, kernel, ext=None):
         try:
             with Lattice(p, **(ext or {})) as lat:
                 lat.set_stream(stream.cuda_stream)
-                kms, extra = per_launch(lat, stream)
+                kms, extra = per_launch(lat, stream, t)
         finally:
             if old is None:
                 del os.environ["BGK_REBASE_EVERY"]
@@ -234,10 +247,10 @@ def measure(p, stream, steps, warmup, kind, kernel, ext=None):
         if kind == "fp32":
             # calls of 500 and 1000 steps hold one and two re-basings: the
             # time per step with the re-basing amortized
-            kr, _ = per_launch(lat, stream, m=500, reps=1)
+            kr, _ = per_launch(lat, stream, t, m=500, reps=1)
             more["ms_per_launch_with_rebase"] = round(kr, 5)
         else:
-            kms, extra = per_launch(lat, stream)
+            kms, extra = per_launch(lat, stream, t)
         lat.step(warmup)
         lat.synchronize()
         t0 = time.perf_counter()
@@ -245,14 +258,20 @@ def measure(p, stream, steps, warmup, kind, kernel, ext=None):
         lat.synchronize()
         wall = (time.perf_counter() - t0) * 1e3 / steps
         lat.field_check()  # raises on a non-finite field
-    nbytes = BYTES_PER_LUP[kind] * lups
+    nbytes = BYTES_PER_NODE[kind] * lups
     ach = nbytes / (kms * 1e-3) / 1e9
     return {"mlups": round(lups / (wall * 1e-3) / 1e6, 1), "ms_per_step": round(wall, 5),
-            "kernel": kernel, "kernel_ms": round(kms, 5),
+            "kernel": KERNELS[kind][t > 1], "steps_per_launch": t,
+            "kernel_ms": round(kms, 5),
             "last_launch_extra_ms": round(extra, 5),
             "achieved_gbs": round(ach, 1), "frac": round(ach / HBM_PEAK_GBS, 4),
-            "bytes_per_lup": BYTES_PER_LUP[kind], "algorithmic_bytes_per_launch": nbytes,
+            "bytes_per_lup": BYTES_PER_NODE[kind] / t, "algorithmic_bytes_per_launch": nbytes,
             "traffic": traffic_from_profile(p.nx, p.ny, kind), **more}
+
+
+def per_step(m):
+    """Kernel ms per step of a measurement."""
+    return m["kernel_ms"] / m["steps_per_launch"]
 
 
 def rel_errors(a, b):
@@ -348,7 +367,7 @@ def cpu_baseline(p, steps: int):
 def traffic_from_profile(nx: int, ny: int, kind: str):
     """HBM bytes per launch measured with rocprofv3 counters, when a
     summary for this kernel and lattice is committed under profiles/."""
-    f = ROOT / "profiles" / f"fused_{kind}_{nx}x{ny}_hbm_traffic.json"
+    f = ROOT / "profiles" / f"step_{kind}_{nx}x{ny}_hbm_traffic.json"
     if not f.exists():
         return None
     try:
@@ -534,7 +553,7 @@ def main():
     if args.error_steps > 0 and not args.headline_only:
         err = errors(w, args.error_steps)
     progress("timed steps")
-    mm = measure(pm, stream, args.steps, args.warmup, mom_kind, "k_fused_mom", ext)
+    mm = measure(pm, stream, args.steps, args.warmup, mom_kind, ext)
     res = {
         "metric": METRIC,
         "value": mm["mlups"],
@@ -570,23 +589,23 @@ def main():
             "frac": mm["frac"],
             "traffic": mm["traffic"],
             "kernel": mm["kernel"],
+            "steps_per_launch": mm["steps_per_launch"],
             "kernel_ms": mm["kernel_ms"],
             "last_launch_extra_ms": mm["last_launch_extra_ms"],
             "bytes_per_lup": mm["bytes_per_lup"],
             "algorithmic_bytes_per_launch": mm["algorithmic_bytes_per_launch"],
         },
     }
-    res["fp32_population"] = measure(pp, stream, args.steps, args.warmup, "fp32", "k_fused32",
-                                     ext)
+    res["fp32_population"] = measure(pp, stream, args.steps, args.warmup, "fp32", ext)
     if not args.no_fp64:
         res["fp64"] = measure(p.replace(precision=FP64), stream, max(args.steps // 2, 1),
-                              args.warmup, "fp64", "k_fused64", ext)
+                              args.warmup, "fp64", ext)
         res["mom_over_fp64"] = round(res["value"] / res["fp64"]["mlups"], 3)
         res["fp32_population_over_fp64"] = round(
             res["fp32_population"]["mlups"] / res["fp64"]["mlups"], 3)
-        res["mom_over_fp64_kernel"] = round(res["fp64"]["kernel_ms"] / mm["kernel_ms"], 3)
+        res["mom_over_fp64_kernel"] = round(per_step(res["fp64"]) / per_step(mm), 3)
         res["fp32_population_over_fp64_kernel"] = round(
-            res["fp64"]["kernel_ms"] / res["fp32_population"]["kernel_ms"], 3)
+            per_step(res["fp64"]) / per_step(res["fp32_population"]), 3)
     if err is not None:
         res["fp32_error"] = err
     if args.layout_probe > 0:
@@ -598,7 +617,7 @@ def main():
     # one GPU's share of the 8192^2 lattice over 8 GPUs (design-only sharding)
     ps = configs.cavity(8192, 1e7, stefan_number=p.stefan_number, rounding=p.rounding,
                         precision=FP32_MOM, **configs.PR002).replace(ny=1026)
-    res["slab"] = dict(measure(ps, stream, args.steps, args.warmup, mom_kind, "k_fused_mom", ext),
+    res["slab"] = dict(measure(ps, stream, args.steps, args.warmup, mom_kind, ext),
                        workload="8192 x 1026: one GPU's rows of 8192^2 on 8 GPUs + 2 halo rows")
     if not args.no_adjoint:
         progress("adjoint 512^2")
