@@ -747,7 +747,6 @@ struct AdjCtx {
   int* probe_ij = nullptr;
   double* probe_T = nullptr;  // nsteps x np
   double* seeds = nullptr;    // nsteps x np
-  double* macro[4] = {};      // scratch macroscopic planes for recomputed steps
   double* partial = nullptr;
   double* out3 = nullptr;
   int nblk = 0;
@@ -926,7 +925,6 @@ size_t carve_fixed(bgk_handle* h, AdjCtx* a, Bump& b) {
   a->probe_ij = b.take<int>(2 * (size_t)std::max(a->np, 1));
   a->probe_T = b.take<double>((size_t)a->nsteps * std::max(a->np, 1));
   a->seeds = b.take<double>((size_t)a->nsteps * std::max(a->np, 1));
-  for (int m = 0; m < 4; ++m) a->macro[m] = b.plane<double>(n);
   a->partial = b.take<double>(3 * (size_t)a->nblk);
   a->out3 = b.take<double>(3);
   return b.off - before;
@@ -1028,7 +1026,7 @@ hipError_t launch_adjoint(bgk_handle* h, AdjCtx* x, const StatePtrs& sprev, int 
 // omega_f = 1 FP32 512^2 1.55 / 1.56, 724^2 2.15 / 2.07, 2048^2 12.5 / 11.4, FP64 724^2
 // 2.98 / 2.71, 2048^2 20.1 / 18.4.  (BGK_MOM_VARIANT of 2 or 3: at any size.)
 bool keeps_between(const bgk_handle* h) {
-  if (mom_most_steps(h) < 2) return false;
+  if (mom_most_steps(h, true) < 2) return false;
   const bool f64 = h->prm.precision == BGK_FP64_MOM;
   const int64_t least = (int64_t)1 << (f64 && !h->mom_eqf ? 20 : 19);
   return h->mom_variant > 0 || (int64_t)h->nx * h->ny >= least;
@@ -1037,8 +1035,8 @@ bool keeps_between(const bgk_handle* h) {
 // T forward steps from state `in` to state `out` (explicit buffers) in one launch;
 // T = 2 with `mid`: the state between them too
 hipError_t fwd_steps(bgk_handle* h, int T, const StatePtrs& in, const StatePtrs* mid,
-                     const StatePtrs& out, double* probe_out, const int* probe_idx, int np, bool write_all,
-                     double* const* macro) {
+                     const StatePtrs& out, double* probe_out, const int* probe_idx, int np,
+                     bool write_all) {
   mom::MomStep st;
   st.in = mom::MomIn{in.a, in.b, in.c};
   st.out = mom::MomOut{out.a, out.b, out.c};
@@ -1050,7 +1048,7 @@ hipError_t fwd_steps(bgk_handle* h, int T, const StatePtrs& in, const StatePtrs*
   st.probe_idx = probe_idx;
   st.probe_out = probe_out;
   st.probe_np = np;
-  for (int m = 0; m < 4; ++m) st.macro[m] = macro ? macro[m] : nullptr;
+  st.adjoint = true;
   if (mid) {
     st.mid = mom::MomOut{mid->a, mid->b, mid->c};
     st.phi_mid = mid->phi;
@@ -1140,16 +1138,8 @@ void adj_invalidate(bgk_handle* h) {
 hipError_t adj_forward(bgk_handle* h, double* probe_T_host) {
   AdjCtx* x = h->adj;
   x->forward_done = false;
-  // halo velocities of the recorded run for the recomputed steps (the
-  // ghost columns of u, v are constant over a run: they are the ones the
-  // state holds now)
-  hipError_t e = hipMemcpyAsync(x->macro[1], h->u, (size_t)h->plane_elems * sizeof(double),
-                                hipMemcpyDeviceToDevice, h->stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(x->macro[2], h->v, (size_t)h->plane_elems * sizeof(double),
-                       hipMemcpyDeviceToDevice, h->stream);
   // east column of the initial state (T(Nx, :) as the first BC_g reads it)
-  if (e == hipSuccess) e = launch_teast_prologue(h);
+  hipError_t e = launch_teast_prologue(h);
   if (e != hipSuccess) return e;
   size_t next_chain = 0;
   const int lvl1 = x->seg1 > 0 ? x->seg1 : x->seg;
@@ -1175,7 +1165,7 @@ hipError_t adj_forward(bgk_handle* h, double* probe_T_host) {
     // FP32, 12 states kept of 48 steps: 11 copies of 84 us less in 4 ms)
     int stop;
     const StatePtrs *keep = next_kept(n, next_chain, &stop), *mid = nullptr;
-    int T = mom_next_steps(h, stop - n);
+    int T = mom_next_steps(h, stop - n, true);
     if (keep && stop == n + 1 && n + 4 <= x->nsteps && keeps_between(h)) {
       mid = keep;
       keep = next_kept(n + 1, ++next_chain, &stop);
@@ -1186,7 +1176,7 @@ hipError_t adj_forward(bgk_handle* h, double* probe_T_host) {
     const bool kept = keep && n + T == stop;
     const StatePtrs out = kept ? *keep : own;
     e = fwd_steps(h, T, in, mid, out, x->np > 0 ? x->probe_T + (size_t)n * x->np : nullptr,
-                  x->probe_idx, x->np, mom_write_all(h, T, x->nsteps - n - T), nullptr);
+                  x->probe_idx, x->np, mom_write_all(h, T, x->nsteps - n - T, true));
     if (e != hipSuccess) return e;
     if (kept) {
       ++next_chain;
@@ -1236,7 +1226,7 @@ hipError_t adj_backward(bgk_handle* h, const double* seeds_host, double grad[3])
   };
   auto steps = [&](int T, const StatePtrs& in, const StatePtrs* mid, const StatePtrs& out) {
     x->recomputed += T;
-    e = fwd_steps(h, T, in, mid, out, nullptr, nullptr, 0, false, x->macro);
+    e = fwd_steps(h, T, in, mid, out, nullptr, nullptr, 0, false);
     return e == hipSuccess;
   };
   const bool pairs = keeps_between(h);
@@ -1249,14 +1239,14 @@ hipError_t adj_backward(bgk_handle* h, const double* seeds_host, double grad[3])
   // not `dst`
   auto first_scratch = [&](int n, const StatePtrs& dst, const StatePtrs* scratch) {
     int launches = 0;
-    for (int left = n; left > 0; ++launches) left -= mom_next_steps(h, left);
+    for (int left = n; left > 0; ++launches) left -= mom_next_steps(h, left, true);
     return (&dst == &scratch[0] ? 1 : 0) ^ (launches & 1);
   };
   auto run = [&](const StatePtrs& src, int n, const StatePtrs& dst, const StatePtrs* scratch) {
     int k = first_scratch(n, dst, scratch);
     const StatePtrs* in = &src;
     for (int left = n; left > 0; k ^= 1) {
-      const int T = mom_next_steps(h, left);
+      const int T = mom_next_steps(h, left, true);
       left -= T;
       const StatePtrs* out = left == 0 ? &dst : &scratch[k];
       if (!steps(T, *in, nullptr, *out)) return false;

@@ -83,9 +83,7 @@ __device__ __forceinline__ void put(Ring<W, NS, R, EQF>& L, int r, int s, const 
 template <typename R, bool EQF>
 __device__ __forceinline__ NodeOut update_node(const Consts& c, const PullSums& S,
                                                const double tap[9], const MomOut& out,
-                                               double* __restrict__ pb, int64_t q,
-                                               const int* __restrict__ probe_idx,
-                                               double* __restrict__ probe_out) {
+                                               double* __restrict__ pb, int64_t q) {
   const Core o = core_forward(c, S, tap);
   const R us = (R)o.u, vs = (R)o.v;
   const R pgxx = (R)((1.0 - o.omega_g) * o.qgxx);
@@ -107,10 +105,6 @@ __device__ __forceinline__ NodeOut update_node(const Consts& c, const PullSums& 
   r.Tav = kTcrit + (o.dT + o.dT2) * 0.5;
   r.uav = ((double)us + o.u2) * 0.5;
   r.vav = ((double)vs + o.v2) * 0.5;
-  if (probe_out) {
-    const int p = probe_idx[q];
-    if (p >= 0) probe_out[p] = r.Tav;
-  }
   return r;
 }
 
@@ -123,8 +117,7 @@ __device__ __forceinline__ void mom_interior(const MomIn& in, const MomOut& out,
                                              const double* __restrict__ pa,
                                              double* __restrict__ pb, const Macro& m,
                                              const Consts& c, const Geom& gm, const StripGrid& sg,
-                                             int write_all, const int* __restrict__ probe_idx,
-                                             double* __restrict__ probe_out) {
+                                             int write_all) {
   __shared__ Ring<W, NS, R, EQF> L;
   const int nx = gm.nx, ny = gm.ny;
   const int64_t P = gm.pitch;
@@ -145,14 +138,6 @@ __device__ __forceinline__ void mom_interior(const MomIn& in, const MomOut& out,
   for (int jj = j0 - 1; jj <= j0 + 1; ++jj) {
     put(L, slot(jj), t + 1, load_node<R, EQF>(in, pa, gm, i, clampj(jj)));
     if (t < 2) put(L, slot(jj), hslot, load_node<R, EQF>(in, pa, gm, hcol, clampj(jj)));
-  }
-  // rows j0 .. j0+63 of the strip that hold a probe (the flag in column 0
-  // of the probe index plane): one load per lane here instead of a load and
-  // its wait in every row
-  uint64_t pmask = 0;
-  if (probe_out) {
-    const int jr = min(j0 + (t & 63), j1);
-    pmask = __ballot(probe_idx[(int64_t)jr * P] >= 0);
   }
   __syncthreads();
 
@@ -181,10 +166,7 @@ __device__ __forceinline__ void mom_interior(const MomIn& in, const MomOut& out,
       const double tap[9] = {L.phi[rC][s],     L.phi[rC][s + 1], L.phi[rN][s],
                              L.phi[rC][s - 1], L.phi[rS][s],     L.phi[rN][s + 1],
                              L.phi[rN][s - 1], L.phi[rS][s - 1], L.phi[rS][s + 1]};
-      const bool prow = probe_out && (j - j0 < 64 ? ((pmask >> (j - j0)) & 1) != 0
-                                                   : probe_idx[(int64_t)j * P] >= 0);
-      double* const po = prow ? probe_out : nullptr;
-      const NodeOut o = update_node<R, EQF>(c, S, tap, out, pb, q, probe_idx, po);
+      const NodeOut o = update_node<R, EQF>(c, S, tap, out, pb, q);
       if (write_all) {
         m.rho[q] = o.rho;
         m.T[q] = o.Tav;
@@ -213,9 +195,7 @@ __device__ __forceinline__ void mom_edge_nodes(const MomIn& in, const MomOut& ou
                                                double* __restrict__ pb,
                                                const double* __restrict__ te_in,
                                                double* __restrict__ te_out, const Macro& m,
-                                               const Consts& c, const Geom& gm, int e,
-                                               const int* __restrict__ probe_idx,
-                                               double* __restrict__ probe_out) {
+                                               const Consts& c, const Geom& gm, int e) {
   const int nx = gm.nx, ny = gm.ny;
   const int64_t P = gm.pitch;
   int i, j;
@@ -256,7 +236,7 @@ __device__ __forceinline__ void mom_edge_nodes(const MomIn& in, const MomOut& ou
   pull_zero(S);
 #pragma unroll
   for (int k = 0; k < 9; ++k) pull_add(S, k, f[k], gd[k]);
-  const NodeOut o = update_node<R, EQF>(c, S, tap, out, pb, q, probe_idx, probe_out);
+  const NodeOut o = update_node<R, EQF>(c, S, tap, out, pb, q);
 
   // ---- halo bookkeeping: BC_f N/S rows (rho copied, u = v = 0), BC_g
   // T and phi ghosts, the east column's averaged T for the next step
@@ -314,14 +294,13 @@ template <int W, int NS, typename R, bool EQF>
 __global__ __launch_bounds__(W) void k_fused_mom(
     MomIn in, MomOut out, const double* __restrict__ pa, double* __restrict__ pb,
     const double* __restrict__ te_in, double* __restrict__ te_out, Macro m, Consts c, Geom gm,
-    StripGrid sg, int write_all, const int* __restrict__ probe_idx,
-    double* __restrict__ probe_out) {
+    StripGrid sg, int write_all) {
   if ((int)blockIdx.x >= sg.nmain) {
     const int e = ((int)blockIdx.x - sg.nmain) * W + (int)threadIdx.x;
-    mom_edge_nodes<R, EQF>(in, out, pa, pb, te_in, te_out, m, c, gm, e, probe_idx, probe_out);
+    mom_edge_nodes<R, EQF>(in, out, pa, pb, te_in, te_out, m, c, gm, e);
     return;
   }
-  mom_interior<W, NS, R, EQF>(in, out, pa, pb, m, c, gm, sg, write_all, probe_idx, probe_out);
+  mom_interior<W, NS, R, EQF>(in, out, pa, pb, m, c, gm, sg, write_all);
 }
 
 // STEP_7/initialization.f90:15-152 for a moment handle: the initial
@@ -360,10 +339,9 @@ hipError_t launch_ring(bgk_handle* h, const MomStep& st) {
   const int nedge = edge_count(h->nx, h->ny);
   const int64_t nwg = (int64_t)sg.nmain + (nedge + W - 1) / W;
   Macro m{h->rho, h->u, h->v, h->T};
-  if (st.macro[0]) m = Macro{st.macro[0], st.macro[1], st.macro[2], st.macro[3]};
   hipLaunchKernelGGL((k_fused_mom<W, NS, float, EQF>), dim3((unsigned)nwg), dim3(W), 0, h->stream,
                      st.in, st.out, st.pa, st.pb, st.te_in, st.te_out, m, h->c, h->geom, sg,
-                     st.write_all ? 1 : 0, st.probe_idx, st.probe_out);
+                     st.write_all ? 1 : 0);
   return hipGetLastError();
 }
 
@@ -393,22 +371,23 @@ void launch_init(bgk_handle* h, const MomOut& st, dim3 grd) {
 // 4096^2 188 against 239 us per step, 2048^2 62 against 64, smaller lattices
 // lose).  FP32 moments with omega_f = 1 take one step per launch beyond 2^25
 // nodes: there the cost of the adjoint is held to three plain forward steps,
-// and its own kernel, at 50% of the memory rate, cannot follow a forward step
-// of half the time.
-int mom_most_steps(const bgk_handle* h) {
+// and its own kernel, at 58% of the memory rate, cannot follow a forward step
+// of half the time (8192^2: 1.80 ms; the forward step 1.13, or 0.69 with two per
+// launch).  The adjoint's own forward runs (`adjoint`) take two.
+int mom_most_steps(const bgk_handle* h, bool adjoint) {
   const bool f64 = h->prm.precision == BGK_FP64_MOM;
   const int64_t nodes = (int64_t)h->nx * h->ny;
   if (h->mom_variant >= 4) return 1;
   if (h->mom_variant > 0) return h->mom_variant == 3 && !(f64 && h->mom_eqf) ? 2 : h->mom_variant;
-  if (!f64 && h->mom_eqf && nodes > (int64_t)1 << 25) return 1;
+  if (!adjoint && !f64 && h->mom_eqf && nodes > (int64_t)1 << 25) return 1;
   return f64 && h->mom_eqf && nodes >= (int64_t)1 << 21 ? 3 : 2;
 }
 
 // Of `left` steps, how many the next launch takes: an odd rest first, so that
 // a call ends with a launch of several steps (which knows the state before
 // the last one, for the halo).
-int mom_next_steps(const bgk_handle* h, int left) {
-  const int most = mom_most_steps(h);
+int mom_next_steps(const bgk_handle* h, int left, bool adjoint) {
+  const int most = mom_most_steps(h, adjoint);
   return left % most ? left % most : most;
 }
 
@@ -416,12 +395,12 @@ int mom_next_steps(const bgk_handle* h, int left) {
 // a call; and the one before a last launch of one step, which takes the halo
 // from them, unless it is a ring launch (these keep the boundary nodes
 // current).
-bool mom_write_all(const bgk_handle* h, int T, int left) {
-  return left == 0 || (left == 1 && !(T == 1 && ring_step(h)));
+bool mom_write_all(const bgk_handle* h, int T, int left, bool adjoint) {
+  return left == 0 || (left == 1 && !(T == 1 && !adjoint && ring_step(h)));
 }
 
 hipError_t launch_mom_steps(bgk_handle* h, const MomStep& st, int T) {
-  if (T > 1 || !ring_step(h)) return launch_mom_stream(h, st, T);
+  if (T > 1 || st.adjoint || !ring_step(h)) return launch_mom_stream(h, st, T);
   // Ring tiling (workgroup width / ring rows), measured at 4096^2: omega_f = 1
   // (36-byte nodes, 64-row strips) 512/4 57.2 GLUPS, 512/3 53.1, 256/4 53.9;
   // general layout (48 bytes, 32-row strips) 512/3 45.9, 512/4 45.6
@@ -444,7 +423,6 @@ hipError_t launch_fused_steps_mom(bgk_handle* h, int nsteps) {
     st.probe_idx = nullptr;
     st.probe_out = nullptr;
     st.probe_np = 0;
-    for (int k = 0; k < 4; ++k) st.macro[k] = nullptr;
     const hipError_t e = launch_mom_steps(h, st, T);
     if (e != hipSuccess) return e;
     h->cur = b;

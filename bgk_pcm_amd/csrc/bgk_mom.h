@@ -358,10 +358,11 @@ struct NodeOut {
 // of the launch to probe_out[t*probe_np + probe_idx]; probe_idx in column 0 of
 // a row is >= 0 when the row holds a probe).  write_all: the macroscopic
 // fields of every node and the halo.  One-step launches of the ring kernel
-// write those of the boundary nodes in any case, to the handle's planes or to
-// `macro` (whose halo columns of u, v must hold the ghost velocities).
+// write those of the boundary nodes in any case, and record no probes: the
+// adjoint's runs keep to the streaming kernel, whose steps have the same bits
+// however a run is split.
 struct MomStep {
-  double* macro[4];
+  bool adjoint = false;
   MomIn in;
   MomOut out;
   const double* pa;
@@ -385,9 +386,9 @@ struct MomStep {
 // streaming kernel's share of them (bgk_stream_mom.hip)
 hipError_t launch_mom_steps(bgk_handle* h, const mom::MomStep& st, int T);
 hipError_t launch_mom_stream(bgk_handle* h, const mom::MomStep& st, int T);
-int mom_next_steps(const bgk_handle* h, int left);
-int mom_most_steps(const bgk_handle* h);
-bool mom_write_all(const bgk_handle* h, int T, int left);
+int mom_next_steps(const bgk_handle* h, int left, bool adjoint = false);
+int mom_most_steps(const bgk_handle* h, bool adjoint = false);
+bool mom_write_all(const bgk_handle* h, int T, int left, bool adjoint = false);
 }  // namespace bgk
 
 #endif  // BGK_MOM_H
