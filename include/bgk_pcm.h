@@ -212,7 +212,7 @@ int bgk_moments(bgk_handle* h);     /* STEP_7/moments.f90:8-27     */
 /* nsteps iterations of the block STEP_7/main.f90:60-69 (BC_f, BC_g,
  * streaming, momentsPre, phase_field, forces, collision, moments).  With
  * no-slip walls on all four sides (BC type 4, the only walls used by the
- * reference inputs UTIL/input.dat.0..3) this is one fused kernel per step;
+ * reference inputs UTIL/input.dat.0..3) a launch fuses one whole step, or two;
  * other boundary types run BC_f and BC_g in one launch and the rest fused in a
  * second (FP64 handles only).
  * Afterwards f, g, rho, u, v, T and phi (halo included) hold what the
