@@ -182,7 +182,8 @@ __device__ __forceinline__ void strip32(const Args32& A, int j0, int j1, int i, 
     rl[d] = tab[ny + 2 + j];
   }
   __builtin_amdgcn_s_waitcnt(kWaitLoads);
-  for (int r = ra; r <= rb; ++r) {
+  // full: levels that have completed a row of use; level `full` is only fed
+  auto feed_row = [&](int r, int full) __attribute__((always_inline)) {
     Pops p;
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
@@ -200,7 +201,7 @@ __device__ __forceinline__ void strip32(const Args32& A, int j0, int j1, int i, 
     Updated o;
     double tav = 0.0, rr = 0.0;
 #pragma unroll
-    for (int t = 0; t < T; ++t) {
+    for (int t = 0; t < T && t <= full; ++t) {
       const int j = r - t;  // row fed to level t
       if (j < j0 - (T - t) || (EDGE && (j < 1 || j > ny + 1))) continue;
       if (EDGE && j <= ny) {
@@ -220,6 +221,7 @@ __device__ __forceinline__ void strip32(const Args32& A, int j0, int j1, int i, 
       double st, st2, pc;
       feed<EDGE>(L[t], p.f, p.g, phi, j, ny, i, nx, has_w, has_e, frozen6, frozen7, &S, &st, &st2,
                  &pc);
+      if (t == full) break;
       o = update<double, false>(A.c, S, st, st2, pc);
       const int jc = j - 1;
       phi = o.phi;
@@ -233,22 +235,24 @@ __device__ __forceinline__ void strip32(const Args32& A, int j0, int j1, int i, 
       }
       if (t < T - 1) decode(rr, p);
     }
-    const int jc = r - T;  // row completed by the last level
-    const bool on = jc >= j0;
-    const int64_t qr = (int64_t)jc * P;
-    const int qa = on && jc <= j1 && own ? i : kPastStrip;
+    if (full == T) {
+      const int jc = r - T;  // row completed by the last level
+      const bool on = jc >= j0;
+      const int64_t qr = (int64_t)jc * P;
+      const int qa = on && jc <= j1 && own ? i : kPastStrip;
 #pragma unroll
-    for (int k = 0; k < 9; ++k)
-      buffer_put(strip_buffer(A.B.row(k, qr), (int)P), qa, make_float2(p.fs[k], p.gs[k]));
-    buffer_put(strip_buffer(A.pb + qr, (int)P), on && jc <= j1 && own_phi ? i : kPastStrip, phi);
-    if (EDGE) buffer_put(te_out, on && jc <= j1 && own && i == nx ? jc : kPastStrip, tav);
-    if (FINAL && on && jc <= j1 && own) {
-      const int64_t qg = (int64_t)jc * P + i;
-      const Avg a = averaged(p, o, rr);
-      A.m.rho[qg] = a.rho;
-      A.m.T[qg] = a.T;
-      A.m.u[qg] = a.u;
-      A.m.v[qg] = a.v;
+      for (int k = 0; k < 9; ++k)
+        buffer_put(strip_buffer(A.B.row(k, qr), (int)P), qa, make_float2(p.fs[k], p.gs[k]));
+      buffer_put(strip_buffer(A.pb + qr, (int)P), on && jc <= j1 && own_phi ? i : kPastStrip, phi);
+      if (EDGE) buffer_put(te_out, on && jc <= j1 && own && i == nx ? jc : kPastStrip, tav);
+      if (FINAL && on && jc <= j1 && own) {
+        const int64_t qg = (int64_t)jc * P + i;
+        const Avg a = averaged(p, o, rr);
+        A.m.rho[qg] = a.rho;
+        A.m.T[qg] = a.T;
+        A.m.u[qg] = a.u;
+        A.m.v[qg] = a.v;
+      }
     }
 #pragma unroll
     for (int d = T; d > 0; --d) {
@@ -257,7 +261,18 @@ __device__ __forceinline__ void strip32(const Args32& A, int j0, int j1, int i, 
     }
     rs[0] = rsn;
     rl[0] = rln;
+  };
+  // (as in bgk_stream_mom.hip; us per step: 1003 x 777 25.7 -> 23.9, 1448^2 52.5 ->
+  // 49.8, 2048^2 90.6 -> 90.4, 4096^2 341.7 -> 338.7)
+  int r = ra;
+  if constexpr (!EDGE && !FINAL) {
+#pragma unroll
+    for (int t = 0; t < T; ++t, r += 2) {
+      feed_row(r, t);
+      feed_row(r + 1, t);
+    }
   }
+  for (; r <= rb; ++r) feed_row(r, T);
   if (EDGE && own && i == nx) {
     if (j0 == 1) A.B.row(6, nx + 1)->x = fr6;
     if (j1 == ny) A.B.row(7, (int64_t)(ny + 1) * P + nx + 1)->x = fr7;
@@ -280,7 +295,7 @@ __global__ __launch_bounds__(kLanes, 2) void k_stream32(Args32 A) {
 }  // namespace
 
 // Measured, us per step, two steps per launch against k_fused32: 4096^2 354
-// (472), 2048^2 91 (135), 1003 x 777 25.4 (27.9), 724^2 22.2 (23.1), 512^2
+// (472), 2048^2 90 (135), 1003 x 777 23.9 (27.9), 724^2 22.2 (23.1), 512^2
 // 19.6 (14.6).  FP32 collision arithmetic and uploaded ghost velocities are the
 // general kernel's.
 bool stream32(const bgk_handle* h) {
