@@ -35,9 +35,9 @@
 // The FP32 rounding of ft/gt done by STEP_7 (implicit REAL) is not modelled.
 //
 // Tiling: one node per thread in the XCD-aware row tiles of bgk_device.h;
-// the 9-point phi_prec stencil comes through the L2.  Each phi row is then
-// fetched into three XCDs' L2s (rows are interleaved over the XCDs), which
-// the HBM counters show as 1.23x the algorithmic reads; staging phi in LDS
+// the 9-point phi_prec stencil comes through the L2.  Where the rows go to the
+// XCDs in turn, each phi row is then fetched into three XCDs' L2s, which the
+// HBM counters show as 1.23x the algorithmic reads; staging phi in LDS
 // removes that but costs more than it saves, measured at 4096^2 per step:
 // these row tiles 0.472 ms; a row-strip kernel with phi in an LDS ring, as
 // the moment kernel has, 0.61 ms (its barrier per row exposes the latency

@@ -1,10 +1,10 @@
-// bgk_strip.h -- row-strip tiling shared by the moment kernel
-// (bgk_fused_mom.hip) and the FP32-population kernel (bgk_fused32.hip).
+// bgk_strip.h -- row-strip tiling of the moment ring kernel
+// (bgk_fused_mom.hip).
 //
 // A workgroup owns W consecutive columns of a strip of consecutive rows and
-// walks the strip row by row, keeping a few rows of phi (and, for moment
-// storage, of the moments) in an LDS ring, so every row of those fields is
-// read from HBM once per step plus the strip's two boundary rows.  gfx950
+// walks the strip row by row, keeping a few rows of the moments and of phi in
+// an LDS ring, so every row is read from HBM once per step plus the strip's
+// two boundary rows.  gfx950
 // dispatches workgroup b to XCD b % 8 and each XCD has its own L2: all
 // column segments of a strip go to one XCD (the cache line a segment reads
 // past its ends is then an L2 hit) and the eight XCDs work on eight
