@@ -1167,6 +1167,7 @@ hipError_t adj_forward(bgk_handle* h, double* probe_T_host) {
     *stop = (n / lvl1 + 1) * lvl1;
     return &x->ckpt[(size_t)(*stop / lvl1)];
   };
+  const int cur0 = h->cur;
   for (int n = 0; e == hipSuccess && n < x->nsteps;) {
     // the launch that reaches a state that is kept writes it in its place, and
     // the one after reads it there, so no state but the first is copied (2048^2,
@@ -1196,7 +1197,15 @@ hipError_t adj_forward(bgk_handle* h, double* probe_T_host) {
     in = out;
     n += T;
   }
-  if (x->np > 0)
+  if (e == hipSuccess && h->recorded && (h->cur ^ cur0) != (x->nsteps & 1)) {
+    const int b = 1 - h->cur;
+    const StatePtrs own{h->ma[b], h->mb[b], h->mc[b], h->phi[1 - h->pc], h->teast[1 - h->te_cur]};
+    e = copy_state(h, own, in.a, in.b, in.c, in.phi, in.te);
+    h->cur = b;
+    h->pc = 1 - h->pc;
+    h->te_cur = 1 - h->te_cur;
+  }
+  if (e == hipSuccess && x->np > 0)
     e = hipMemcpyAsync(probe_T_host, x->probe_T, (size_t)x->nsteps * x->np * sizeof(double),
                        hipMemcpyDeviceToHost, h->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(h->stream);

@@ -243,7 +243,7 @@ __global__ __launch_bounds__(TILE_W) void k_general64(Pairs64 A, Pairs64 B,
 }  // namespace
 
 hipError_t launch_teast_prologue(bgk_handle* h) {
-  if (h->te_ok) return hipSuccess;
+  if (h->te_ok && !h->recorded) return hipSuccess;
   const Geom& g = h->geom;
   hipLaunchKernelGGL(k_teast_prologue, dim3((unsigned)((g.ny + 2 + 255) / 256)), dim3(256), 0,
                      h->stream, h->T, h->teast[h->te_cur], g);

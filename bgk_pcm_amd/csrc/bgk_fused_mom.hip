@@ -408,8 +408,12 @@ hipError_t launch_mom_steps(bgk_handle* h, const MomStep& st, int T) {
 }
 
 hipError_t launch_fused_steps_mom(bgk_handle* h, int nsteps) {
+  // With a graph (recorded) the launches have the parity of the steps: what does
+  // not fill whole ones, two of them where `most` is even, goes step by step.
+  const int most = mom_most_steps(h), group = most % 2 == 0 ? 2 * most : most;
+  const int whole = nsteps / group * group;
   for (int left = nsteps; left > 0;) {
-    const int T = mom_next_steps(h, left);
+    const int T = !h->recorded ? mom_next_steps(h, left) : left > whole ? 1 : most;
     left -= T;
     const int a = h->cur, b = 1 - h->cur;
     MomStep st;

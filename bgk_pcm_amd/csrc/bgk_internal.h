@@ -72,6 +72,7 @@ struct bgk_handle {
   bool te_ok;
   // the ghost columns of u and v hold the initial velocities (no upload since)
   bool ghost_uv;
+  bool recorded;  // see recorded()
   // FP32 population handles: solid and liquid reference densities of rows
   // 0..Ny+1 ([0, Ny+2) and [Ny+2, 2(Ny+2)) of rref[rc]; the other is the
   // next table) the f members are stored against, and the re-basing cadence
@@ -92,6 +93,21 @@ struct bgk_handle {
 
 namespace bgk {
 
+// Whether a HIP graph records, or has recorded, calls of this handle.  Replays
+// start from the buffers the recording did, after whatever calls came since:
+// from then on no call takes a decision by what the host knows of the device's
+// state, and the buffers (cur, pc, te_cur) change with every step of the cavity
+// and with nothing else, so that the handle is back in the recording's after any
+// even number of steps, recorded or not.
+inline bool recorded(bgk_handle* h) {
+  if (!h->recorded) {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    h->recorded =
+        hipStreamIsCapturing(h->stream, &s) == hipSuccess && s != hipStreamCaptureStatusNone;
+  }
+  return h->recorded;
+}
+
 // ---- per-subroutine kernels (bgk_stage.hip), FP64 handles
 hipError_t launch_initialization(bgk_handle* h);
 // BC_f and / or BC_g; the entry points of one each
@@ -104,10 +120,13 @@ hipError_t launch_phase_field(bgk_handle* h);
 hipError_t launch_forces(bgk_handle* h);
 hipError_t launch_collision(bgk_handle* h);
 hipError_t launch_moments(bgk_handle* h);
+// a step by these, in the reference's order
+hipError_t launch_stages64(bgk_handle* h);
 
 // ---- fused step (bgk_fused.hip / bgk_fused32.hip)
 // Make teast[te_cur] hold the averaged T(Nx, :) before the first fused step of
-// a call: a launch only where something but the fused step wrote T since.
+// a call: a launch only where something but the fused step wrote T since (or a
+// graph may have, see recorded).
 hipError_t launch_teast_prologue(bgk_handle* h);
 // One fused FP64 step from buffer cur to 1-cur; write_all: write the
 // moments of every node (else only the boundary-adjacent ones).

@@ -525,10 +525,16 @@ hipError_t launch_moments_pre(bgk_handle* h) {
 hipError_t launch_phase_field(bgk_handle* h) {
   const Geom& g = h->geom;
   const dim3 grd((unsigned)((g.nx + 2 + TX - 1) / TX), (unsigned)((g.ny + 2 + TY - 1) / TY));
-  hipLaunchKernelGGL(k_phase_field, grd, dim3(TX, TY), 0, h->stream, h->phi[1 - h->pc],
-                     h->phi[h->pc], h->T, h->c, g);
+  const bool copy = h->recorded;  // (the exchange would change the buffers)
+  if (copy) {
+    const hipError_t e = launch_copy64(h, h->phi[h->pc], 1, h->phi[1 - h->pc], 1);
+    if (e != hipSuccess) return e;
+  }
+  const int to = copy ? h->pc : 1 - h->pc;
+  hipLaunchKernelGGL(k_phase_field, grd, dim3(TX, TY), 0, h->stream, h->phi[to], h->phi[1 - to],
+                     h->T, h->c, g);
   const hipError_t e = hipGetLastError();
-  if (e == hipSuccess) h->pc = 1 - h->pc;
+  if (e == hipSuccess) h->pc = to;
   return e;
 }
 
@@ -554,6 +560,15 @@ hipError_t launch_moments(bgk_handle* h) {
   hipLaunchKernelGGL(k_moments, interior_grid(h->geom), dim3(TX, TY), 0, h->stream,
                      pairs(h->f[h->cur]), macro_of(h), h->geom);
   return hipGetLastError();
+}
+
+hipError_t launch_stages64(bgk_handle* h) {
+  for (const auto launch : {launch_bc_f, launch_bc_g, launch_streaming, launch_moments_pre,
+                            launch_phase_field, launch_forces, launch_collision, launch_moments}) {
+    const hipError_t e = launch(h);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace bgk

@@ -299,7 +299,7 @@ __global__ __launch_bounds__(kLanes, 2) void k_stream32(Args32 A) {
 // 19.6 (14.6).  FP32 collision arithmetic and uploaded ghost velocities are the
 // general kernel's.
 bool stream32(const bgk_handle* h) {
-  if (!h->ghost_uv || h->prm.fp32_collision || h->pop_variant == 1) return false;
+  if (!h->ghost_uv || h->recorded || h->prm.fp32_collision || h->pop_variant == 1) return false;
   return h->pop_variant > 1 || (int64_t)h->nx * h->ny >= (int64_t)1 << 19;
 }
 

@@ -402,7 +402,7 @@ __global__ __launch_bounds__(kLanes, 2) void k_stream64(Args64 A) {
 // few waves of this kernel are bound by the latency of their rows); a handle whose ghost velocities were
 // uploaded takes the general kernel.
 bool stream64(const bgk_handle* h) {
-  if (!h->ghost_uv || h->pop_variant == 1) return false;
+  if (!h->ghost_uv || h->recorded || h->pop_variant == 1) return false;
   return h->pop_variant > 1 || (int64_t)h->nx * h->ny >= (int64_t)1 << 19;
 }
 
