@@ -309,7 +309,7 @@ __device__ __forceinline__ void rebuild_adjoint(const Mom<A>& m, const WMom<A>& 
   lm->pg[2] += A(9) * G.mxy;
 }
 
-// Reverse of core_forward (bgk_mom.h) and of the state it stores.  lo: the
+// Reverse of core_from_sums (bgk_mom.h) and of the state it stores.  lo: the
 // adjoint of the node's stored moments after the step (rho, T - T_crit, u,
 // v, Pf, Pg) and of its phi; ldT2 an extra adjoint on the pulled T (the
 // averaged T of moments.f90 seeds half of its adjoint here).  Returns the

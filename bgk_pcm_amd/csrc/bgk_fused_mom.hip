@@ -14,27 +14,31 @@
 // their own relative precision.
 //
 // Tiling: a workgroup owns W columns and a strip of consecutive rows, and
-// walks the strip row by row.  Row j+2 is fetched from HBM while row j is
-// computed; rows j-1..j+2 live in an LDS ring, so every node's moments and
-// phi are read from HBM once per step (plus the strip's two boundary rows
-// and the two halo columns).  phi_prec's 9-point stencil comes from the
-// same ring.  The boundary-adjacent nodes run in extra workgroups of the
-// same launch with BC_f (no-slip) and BC_g folded in as in bgk_fused.hip:
-// ghost rows of g and phi are the clamped rows, own opposite populations
-// for bounce-back, the two frozen corner ghosts as constants.
+// walks the strip row by row.  Row r + 1 is fetched from HBM while row r, in
+// LDS, is fed to the sums of the rows below, beside and above it (feed_three in
+// bgk_level.h; the LDS holds two rows, for one barrier a row), so every node's
+// moments and phi are read from HBM once per step (plus the strip's two
+// boundary rows and the two halo columns).  The boundary-adjacent nodes run in
+// extra workgroups of the same launch with BC_f (no-slip) and BC_g folded in as
+// in bgk_fused.hip: ghost rows of g and phi are the clamped rows, own opposite
+// populations for bounce-back, the two frozen corner ghosts as constants.  The
+// operations and their order are the streaming kernel's, so a step has the same
+// bits in either (4096^2, us per step: 364, and 286 with omega_f = 1; rebuilding
+// nine upstream nodes' populations at every node, in an order of its own, 362
+// and 290).
 //
 // Arithmetic is FP64 throughout.  STEP_7's FP32 temporaries (ft, gt) cannot
 // be represented by moments, so this path follows the clean rounding policy;
 // beta follows bgk_params.rounding as everywhere.
 #include <algorithm>
 
-#include "bgk_mom.h"
+#include "bgk_level.h"
 #include "bgk_strip.h"
 
 namespace bgk {
 namespace {
 
-using namespace mom;
+using namespace level;
 
 constexpr int TX = 64, TY = 4;  // block of the initialization kernel
 
@@ -42,13 +46,13 @@ struct Macro {
   double *rho, *u, *v, *T;
 };
 
-// LDS ring of NS rows of W + 2 nodes (W columns and the two halo columns).
-template <int W, int NS, typename R, bool EQF>
+// LDS ring of two rows of W + 2 nodes (W columns and the two halo columns).
+template <int W, typename R, bool EQF>
 struct Ring {
-  double2 a[NS][W + 2];
-  typename Vec<R>::V4 b[NS][W + 2];
-  typename CType<R, EQF>::T c[NS][W + 2];
-  double phi[NS][W + 2];
+  double2 a[2][W + 2];
+  typename Vec<R>::V4 b[2][W + 2];
+  typename CType<R, EQF>::T c[2][W + 2];
+  double phi[2][W + 2];
 };
 
 template <typename R, bool EQF>
@@ -69,58 +73,73 @@ __device__ __forceinline__ Node<R, EQF> load_node(const MomIn& in, const double*
   return n;
 }
 
-template <int W, int NS, typename R, bool EQF>
-__device__ __forceinline__ void put(Ring<W, NS, R, EQF>& L, int r, int s, const Node<R, EQF>& n) {
+template <int W, typename R, bool EQF>
+__device__ __forceinline__ void put(Ring<W, R, EQF>& L, int r, int s, const Node<R, EQF>& n) {
   L.a[r][s] = n.a;
   L.b[r][s] = n.b;
   L.c[r][s] = n.c;
   L.phi[r][s] = n.phi;
 }
 
-// Node update from its pulled moments and phi_prec taps (C, E, N, W, S, NE,
-// NW, SW, SE); stores the node's moments and phi, and T (averaged as
-// STEP_7/moments.f90:11-25) at a probe node.  Returns the averaged moments.
 template <typename R, bool EQF>
-__device__ __forceinline__ NodeOut update_node(const Consts& c, const PullSums& S,
-                                               const double tap[9], const MomOut& out,
-                                               double* __restrict__ pb, int64_t q) {
-  const Core o = core_forward(c, S, tap);
-  const R us = (R)o.u, vs = (R)o.v;
-  const R pgxx = (R)((1.0 - o.omega_g) * o.qgxx);
-  const R pgyy = (R)((1.0 - o.omega_g) * o.qgyy);
-  const R pgxy = (R)((1.0 - o.omega_g) * o.qgxy);
-  stream_store(out.a + q, o.rho, o.dT);
-  using V4 = typename Vec<R>::V4;
+__device__ __forceinline__ Pops populations_of(const double2& a, const typename Vec<R>::V4& b,
+                                               const typename CType<R, EQF>::T& c) {
+  const double u = (double)b.x, v = (double)b.y;
+  Pops p;
   if constexpr (EQF) {
-    nt_store4<R>(static_cast<V4*>(out.b) + q, us, vs, pgxx, pgyy);
-    __builtin_nontemporal_store(pgxy, static_cast<R*>(out.c) + q);
+    populations<false>(a.x, a.x, u, v, 0.0, 0.0, 0.0, p.f);
+    populations<true>(a.y, kTcrit + a.y, u, v, (double)b.z, (double)b.w, (double)c, p.g);
   } else {
-    const double omf1 = 1.0 - c.omega_f;
-    nt_store4<R>(static_cast<V4*>(out.b) + q, us, vs, (R)(omf1 * o.qfxx), (R)(omf1 * o.qfyy));
-    nt_store4<R>(static_cast<V4*>(out.c) + q, (R)(omf1 * o.qfxy), pgxx, pgyy, pgxy);
+    populations<true>(a.x, a.x, u, v, (double)b.z, (double)b.w, (double)c.x, p.f);
+    populations<true>(a.y, kTcrit + a.y, u, v, (double)c.y, (double)c.z, (double)c.w, p.g);
   }
-  stream_store(&pb[q], o.phi);
-  NodeOut r;
-  r.rho = o.rho;
-  r.Tav = kTcrit + (o.dT + o.dT2) * 0.5;
-  r.uav = ((double)us + o.u2) * 0.5;
-  r.vav = ((double)vs + o.v2) * 0.5;
-  return r;
+  return p;
 }
 
-// Interior nodes (1 < i < Nx, 1 < j < Ny) by row strips through the LDS
-// ring.  W columns per workgroup, NS rows in the ring (4: one barrier per
-// row; 3: two, for less LDS).  Workgroups from sg.nmain on serve the
-// boundary-adjacent nodes (mom_edge_nodes).
-template <int W, int NS, typename R, bool EQF>
+// Node update from its pulled moments and phi_prec sums; stores the node's
+// moments and phi.
+template <typename R, bool EQF>
+__device__ __forceinline__ Updated update_node(const StepC& c, const PullSums& S, double st,
+                                               double st2, double pc, const MomOut& out,
+                                               double* __restrict__ pb, int64_t q) {
+  const Updated o = update<R, EQF>(c, S, st, st2, pc);
+  using V4 = typename Vec<R>::V4;
+  stream_store(out.a + q, o.rho, o.dT);
+  if constexpr (EQF) {
+    nt_store4<R>(static_cast<V4*>(out.b) + q, (R)o.u, (R)o.v, (R)o.pgxx, (R)o.pgyy);
+    __builtin_nontemporal_store((R)o.pgxy, static_cast<R*>(out.c) + q);
+  } else {
+    nt_store4<R>(static_cast<V4*>(out.b) + q, (R)o.u, (R)o.v, (R)o.pfxx, (R)o.pfyy);
+    nt_store4<R>(static_cast<V4*>(out.c) + q, (R)o.pfxy, (R)o.pgxx, (R)o.pgyy, (R)o.pgxy);
+  }
+  stream_store(&pb[q], o.phi);
+  return o;
+}
+
+// The averaged moments after the step (STEP_7/moments.f90:11-25).
+__device__ __forceinline__ double averaged_T(const Updated& o) {
+  return kTcrit + (o.dT + o.dT2) * 0.5;
+}
+__device__ __forceinline__ void put_macro(const Macro& m, int64_t q, const Updated& o) {
+  m.rho[q] = o.rho;
+  m.T[q] = averaged_T(o);
+  m.u[q] = (o.u + o.u2) * 0.5;
+  m.v[q] = (o.v + o.v2) * 0.5;
+}
+
+// Interior nodes (1 < i < Nx, 1 < j < Ny) by row strips, W columns per workgroup.
+// A thread feeds its column's node and the two beside it, row after row, to the
+// sums of bgk_level.h, so that a row is needed in LDS only while it is fed.
+// Workgroups from sg.nmain on serve the boundary-adjacent nodes
+// (mom_edge_nodes).
+template <int W, typename R, bool EQF>
 __device__ __forceinline__ void mom_interior(const MomIn& in, const MomOut& out,
                                              const double* __restrict__ pa,
                                              double* __restrict__ pb, const Macro& m,
-                                             const Consts& c, const Geom& gm, const StripGrid& sg,
+                                             const StepC& c, const Geom& gm, const StripGrid& sg,
                                              int write_all) {
-  __shared__ Ring<W, NS, R, EQF> L;
+  __shared__ Ring<W, R, EQF> L;
   const int nx = gm.nx, ny = gm.ny;
-  const int64_t P = gm.pitch;
   int strip, seg;
   if (!strip_of(sg, (int)blockIdx.x, &strip, &seg)) return;  // whole workgroup
   const int j0 = strip * sg.rows + 1;
@@ -132,54 +151,31 @@ __device__ __forceinline__ void mom_interior(const MomIn& in, const MomOut& out,
   const int hcol = (t == 0) ? i0 - 1 : i0 + W;
   const int hslot = (t == 0) ? 0 : W + 1;
   auto clampj = [ny](int jj) { return jj < 1 ? 1 : (jj > ny ? ny : jj); };
-  auto slot = [j0](int jj) { return (jj - j0 + 1) % NS; };
   const bool col_in = (i > 1 && i < nx);
-
-  for (int jj = j0 - 1; jj <= j0 + 1; ++jj) {
-    put(L, slot(jj), t + 1, load_node<R, EQF>(in, pa, gm, i, clampj(jj)));
-    if (t < 2) put(L, slot(jj), hslot, load_node<R, EQF>(in, pa, gm, hcol, clampj(jj)));
-  }
-  __syncthreads();
-
-  for (int j = j0; j <= j1; ++j) {
-    const bool pre = (j + 2 <= j1 + 1);
-    Node<R, EQF> nn, nh;
-    if (pre) {
-      nn = load_node<R, EQF>(in, pa, gm, i, clampj(j + 2));
-      if (t < 2) nh = load_node<R, EQF>(in, pa, gm, hcol, clampj(j + 2));
+  Level S = Level{};
+  Node<R, EQF> nn = load_node<R, EQF>(in, pa, gm, i, clampj(j0 - 1)), nh;
+  if (t < 2) nh = load_node<R, EQF>(in, pa, gm, hcol, clampj(j0 - 1));
+  for (int r = j0 - 1; r <= j1 + 1; ++r) {  // row fed
+    const int b = r & 1;
+    put(L, b, t + 1, nn);
+    if (t < 2) put(L, b, hslot, nh);
+    __syncthreads();  // (row r + 1 overwrites row r - 1, which nobody reads any more)
+    if (r <= j1) {
+      nn = load_node<R, EQF>(in, pa, gm, i, clampj(r + 1));
+      if (t < 2) nh = load_node<R, EQF>(in, pa, gm, hcol, clampj(r + 1));
     }
-    if (col_in && j > 1 && j < ny) {
-      const int rS = slot(j - 1), rC = slot(j), rN = slot(j + 1);
-      const int s = t + 1;
-      const int64_t q = (int64_t)j * P + i;
-      // ---- streaming: rebuild population k of node (i - cx_k, j - cy_k)
-      PullSums S;
-      pull_zero(S);
-#pragma unroll
-      for (int k = 0; k < 9; ++k) {
-        const int r = CY[k] > 0 ? rS : (CY[k] < 0 ? rN : rC);
-        const int ss = s - CX[k];
-        double fk, gk;
-        rebuild<R, EQF>(k, L.a[r][ss], L.b[r][ss], L.c[r][ss], &fk, &gk);
-        pull_add(S, k, fk, gk);
-      }
-      const double tap[9] = {L.phi[rC][s],     L.phi[rC][s + 1], L.phi[rN][s],
-                             L.phi[rC][s - 1], L.phi[rS][s],     L.phi[rN][s + 1],
-                             L.phi[rN][s - 1], L.phi[rS][s - 1], L.phi[rS][s + 1]};
-      const NodeOut o = update_node<R, EQF>(c, S, tap, out, pb, q);
-      if (write_all) {
-        m.rho[q] = o.rho;
-        m.T[q] = o.Tav;
-        m.u[q] = o.uav;
-        m.v[q] = o.vav;
-      }
+    const Pops w = populations_of<R, EQF>(L.a[b][t], L.b[b][t], L.c[b][t]);
+    const Pops c0 = populations_of<R, EQF>(L.a[b][t + 1], L.b[b][t + 1], L.c[b][t + 1]);
+    const Pops e = populations_of<R, EQF>(L.a[b][t + 2], L.b[b][t + 2], L.c[b][t + 2]);
+    PullSums P;
+    double st, st2, pc;
+    feed_three(S, w, c0, e, L.phi[b][t], L.phi[b][t + 1], L.phi[b][t + 2], &P, &st, &st2, &pc);
+    const int j = r - 1;  // row completed
+    if (j >= j0 && col_in && j > 1 && j < ny) {
+      const int64_t q = (int64_t)j * gm.pitch + i;
+      const Updated o = update_node<R, EQF>(c, P, st, st2, pc, out, pb, q);
+      if (write_all) put_macro(m, q, o);
     }
-    if constexpr (NS == 3) __syncthreads();  // row j+2 overwrites row j-1
-    if (pre) {
-      put(L, slot(j + 2), t + 1, nn);
-      if (t < 2) put(L, slot(j + 2), hslot, nh);
-    }
-    __syncthreads();
   }
 }
 
@@ -195,36 +191,31 @@ __device__ __forceinline__ void mom_edge_nodes(const MomIn& in, const MomOut& ou
                                                double* __restrict__ pb,
                                                const double* __restrict__ te_in,
                                                double* __restrict__ te_out, const Macro& m,
-                                               const Consts& c, const Geom& gm, int e) {
+                                               const Consts& c, const StepC& sc, const Geom& gm,
+                                               int e) {
   const int nx = gm.nx, ny = gm.ny;
   const int64_t P = gm.pitch;
   int i, j;
   if (!edge_node(e, nx, ny, &i, &j)) return;
   const int64_t q = (int64_t)j * P + i;
-  const double2 oa = in.a[q];
-  const typename Vec<R>::V4 ob = b_at<R, EQF>(in.b, q);
-  const typename CType<R, EQF>::T oc = c_at<R, EQF>(in.c, q);
-  double f[9], gd[9];
+  const Pops own = populations_of<R, EQF>(in.a[q], b_at<R, EQF>(in.b, q), c_at<R, EQF>(in.c, q));
+  double f[9], g[9];
 #pragma unroll
   for (int k = 0; k < 9; ++k) {
     const int si = i - CX[k], sj = j - CY[k];
     const int sjc = sj < 1 ? 1 : (sj > ny ? ny : sj);
     if (si >= 1 && si <= nx) {
-      // interior source column: rebuild from the node (si, sjc); for a ghost
-      // row this is the N/S copy of g, and f is replaced below
       const int64_t h = (int64_t)sjc * P + si;
-      rebuild<R, EQF>(k, in.a[h], b_at<R, EQF>(in.b, h), c_at<R, EQF>(in.c, h), &f[k], &gd[k]);
-    } else {
-      const int64_t h = (int64_t)sjc * P + si;
-      gd[k] = ghost_gdev(k, si == 0 ? c.tin : east_T(c, te_in, sjc), m.u[h], m.v[h]);
-    }
-    if (si < 1 || si > nx || sj < 1 || sj > ny) {
-      if (k == 6 && si == nx + 1 && sj == 0)
-        f[k] = c.frozen6;
-      else if (k == 7 && si == nx + 1 && sj == ny + 1)
-        f[k] = c.frozen7;
-      else
-        f[k] = rebuild_f<R, EQF>(OPP[k], oa, ob, oc);
+      const Pops p =
+          populations_of<R, EQF>(in.a[h], b_at<R, EQF>(in.b, h), c_at<R, EQF>(in.c, h));
+      f[k] = p.f[k];
+      g[k] = p.g[k];
+    } else {  // no flow populations, the wall's T and velocity
+      const double th = (si == 0 ? c.tin : east_T(c, te_in, sjc)) - kTcrit;
+      double p[9];
+      populations<true>(th, kTcrit + th, c.u0, c.v0, 0.0, 0.0, 0.0, p);
+      f[k] = 0.0;
+      g[k] = p[k];
     }
   }
   const int64_t rn = (int64_t)(j < ny ? j + 1 : ny) * P;
@@ -232,11 +223,10 @@ __device__ __forceinline__ void mom_edge_nodes(const MomIn& in, const MomOut& ou
   const int64_t r0 = (int64_t)j * P;
   const double tap[9] = {pa[q],          pa[r0 + i + 1], pa[rn + i],     pa[r0 + i - 1], pa[rs + i],
                          pa[rn + i + 1], pa[rn + i - 1], pa[rs + i - 1], pa[rs + i + 1]};
-  PullSums S;
-  pull_zero(S);
-#pragma unroll
-  for (int k = 0; k < 9; ++k) pull_add(S, k, f[k], gd[k]);
-  const NodeOut o = update_node<R, EQF>(c, S, tap, out, pb, q);
+  const PullSums S = pulled_sums(f, g, own.f, i, j, nx, ny, c.frozen6, c.frozen7);
+  double st, st2;
+  tap_sums(tap, &st, &st2);
+  const Updated o = update_node<R, EQF>(sc, S, st, st2, tap[0], out, pb, q);
 
   // ---- halo bookkeeping: BC_f N/S rows (rho copied, u = v = 0), BC_g
   // T and phi ghosts, the east column's averaged T for the next step
@@ -273,7 +263,7 @@ __device__ __forceinline__ void mom_edge_nodes(const MomIn& in, const MomOut& ou
     const int64_t h = r0 + nx + 1;
     m.T[h] = east_T(c, te_in, j);
     pb[h] = pa[h];
-    te_out[j] = o.Tav;
+    te_out[j] = averaged_T(o);
     if (s_edge) {
       m.T[nx + 1] = east_T(c, te_in, 1);
       pb[nx + 1] = pa[P + nx + 1];
@@ -284,23 +274,20 @@ __device__ __forceinline__ void mom_edge_nodes(const MomIn& in, const MomOut& ou
       pb[hn] = pa[(int64_t)ny * P + nx + 1];
     }
   }
-  m.rho[q] = o.rho;
-  m.T[q] = o.Tav;
-  m.u[q] = o.uav;
-  m.v[q] = o.vav;
+  put_macro(m, q, o);
 }
 
-template <int W, int NS, typename R, bool EQF>
+template <int W, typename R, bool EQF>
 __global__ __launch_bounds__(W) void k_fused_mom(
     MomIn in, MomOut out, const double* __restrict__ pa, double* __restrict__ pb,
-    const double* __restrict__ te_in, double* __restrict__ te_out, Macro m, Consts c, Geom gm,
-    StripGrid sg, int write_all) {
+    const double* __restrict__ te_in, double* __restrict__ te_out, Macro m, Consts c, StepC sc,
+    Geom gm, StripGrid sg, int write_all) {
   if ((int)blockIdx.x >= sg.nmain) {
     const int e = ((int)blockIdx.x - sg.nmain) * W + (int)threadIdx.x;
-    mom_edge_nodes<R, EQF>(in, out, pa, pb, te_in, te_out, m, c, gm, e);
+    mom_edge_nodes<R, EQF>(in, out, pa, pb, te_in, te_out, m, c, sc, gm, e);
     return;
   }
-  mom_interior<W, NS, R, EQF>(in, out, pa, pb, m, c, gm, sg, write_all);
+  mom_interior<W, R, EQF>(in, out, pa, pb, m, sc, gm, sg, write_all);
 }
 
 // STEP_7/initialization.f90:15-152 for a moment handle: the initial
@@ -324,12 +311,12 @@ __global__ void k_initialization_mom(MomOut st, Macro m, double* phi, double* ph
   phip[q] = s0.phi;
 }
 
-template <int W, int NS, bool EQF>
+template <int W, typename R, bool EQF>
 hipError_t launch_ring(bgk_handle* h, const MomStep& st) {
   // resident workgroups per CU of this instantiation (LDS and registers)
   static const int per_cu = [] {
     int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_fused_mom<W, NS, float, EQF>, W, 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_fused_mom<W, R, EQF>, W, 0) !=
         hipSuccess)
       n = 0;
     return n;
@@ -339,17 +326,16 @@ hipError_t launch_ring(bgk_handle* h, const MomStep& st) {
   const int nedge = edge_count(h->nx, h->ny);
   const int64_t nwg = (int64_t)sg.nmain + (nedge + W - 1) / W;
   Macro m{h->rho, h->u, h->v, h->T};
-  hipLaunchKernelGGL((k_fused_mom<W, NS, float, EQF>), dim3((unsigned)nwg), dim3(W), 0, h->stream,
-                     st.in, st.out, st.pa, st.pb, st.te_in, st.te_out, m, h->c, h->geom, sg,
-                     st.write_all ? 1 : 0);
+  hipLaunchKernelGGL((k_fused_mom<W, R, EQF>), dim3((unsigned)nwg), dim3(W), 0, h->stream,
+                     st.in, st.out, st.pa, st.pb, st.te_in, st.te_out, m, h->c,
+                     step_constants(h->c), h->geom, sg, st.write_all ? 1 : 0);
   return hipGetLastError();
 }
 
 // Whether one step alone goes through the ring kernel.  Measured per step on
 // MI355X, ring against the streaming kernel with T = 1, FP32 moments: 4096^2
-// 362 / 394 us (omega_f = 1: 290 / 329), 2048^2 107 / 104 (89 / 84), 512^2
-// 20.2 / 11.8 (17.6 / 10.4); FP64 moments are faster or within 4% with the
-// streaming kernel at every size.
+// 364 / 416 us (omega_f = 1: 286 / 343), 2048^2 103 / 106 (85 / 87), 512^2
+// 20.2 / 11.8 (17.6 / 10.4).
 bool ring_step(const bgk_handle* h) {
   if (h->prm.precision != BGK_FP32_MOM) return false;
   if (h->mom_variant != 0) return h->mom_variant >= 4;
@@ -401,10 +387,7 @@ bool mom_write_all(const bgk_handle* h, int T, int left, bool adjoint) {
 
 hipError_t launch_mom_steps(bgk_handle* h, const MomStep& st, int T) {
   if (T > 1 || st.adjoint || !ring_step(h)) return launch_mom_stream(h, st, T);
-  // Ring tiling (workgroup width / ring rows), measured at 4096^2: omega_f = 1
-  // (36-byte nodes, 64-row strips) 512/4 57.2 GLUPS, 512/3 53.1, 256/4 53.9;
-  // general layout (48 bytes, 32-row strips) 512/3 45.9, 512/4 45.6
-  return h->mom_eqf ? launch_ring<512, 4, true>(h, st) : launch_ring<512, 3, false>(h, st);
+  return h->mom_eqf ? launch_ring<512, float, true>(h, st) : launch_ring<512, float, false>(h, st);
 }
 
 hipError_t launch_fused_steps_mom(bgk_handle* h, int nsteps) {

@@ -69,6 +69,24 @@ __device__ __forceinline__ TripleT<A> triple(A c, A w, A e) {
   return TripleT<A>{c + p, p, w - e};
 }
 
+// The pulled sums of a node from the row below (sf, sg) and its own (cf, cg).
+template <typename A>
+__device__ __forceinline__ PullSumsT<A> row_sums(const TripleT<A>& sf, const TripleT<A>& cf,
+                                                 const TripleT<A>& sg, const TripleT<A>& cg) {
+  PullSumsT<A> s;
+  s.rho = sf.n + cf.n;
+  s.jx = sf.d + cf.d;
+  s.jy = sf.n;
+  s.fxx = sf.p + cf.p;
+  s.fyy = sf.n;
+  s.fxy = sf.d;
+  s.dT = sg.n + cg.n;
+  s.gxx = sg.p + cg.p;
+  s.gyy = sg.n;
+  s.gxy = sg.d;
+  return s;
+}
+
 // Registers of one level between two rows.
 template <typename A>
 struct LevelT {
@@ -198,16 +216,7 @@ __device__ __forceinline__ void feed(LevelT<A>& L, const A f[9], const A g[9], A
   {
     const TripleT<A> cf = triple(f[0], from_west(f[1]), from_east(f[3]));
     const TripleT<A> cg = triple(g[0], from_west(g[1]), from_east(g[3]));
-    L.s.rho = L.sf.n + cf.n;
-    L.s.jx = L.sf.d + cf.d;
-    L.s.jy = L.sf.n;
-    L.s.fxx = L.sf.p + cf.p;
-    L.s.fyy = L.sf.n;
-    L.s.fxy = L.sf.d;
-    L.s.dT = L.sg.n + cg.n;
-    L.s.gxx = L.sg.p + cg.p;
-    L.s.gyy = L.sg.n;
-    L.s.gxy = L.sg.d;
+    L.s = row_sums(L.sf, cf, L.sg, cg);
     L.t1 = L.n1 + r1;
     L.t2 = L.n2 + r2;
     L.pc = phi;
@@ -257,6 +266,106 @@ __device__ __forceinline__ void feed(LevelT<A>& L, const A f[9], const A g[9], A
   L.sg = sg;
   L.n1 = r1;
   L.n2 = r2;
+}
+
+// Moments of a node as the rebuild of its populations takes them.
+struct NodeD {
+  double rho, th, u, v, pfxx, pfyy, pfxy, pgxx, pgyy, pgxy, phi;
+};
+
+// `feed` away from the walls, where the neighbours' populations and phi come from
+// elsewhere than the lanes beside: w, c, e of the columns i - 1, i, i + 1.  The same
+// operations, so the same bits.
+struct Pops {
+  double f[9], g[9];
+};
+__device__ __forceinline__ void feed_three(Level& L, const Pops& w, const Pops& c, const Pops& e,
+                                           double pw, double p, double pe, PullSums* S, double* st,
+                                           double* st2, double* pc) {
+  const TripleT<double> nf = triple(c.f[4], w.f[8], e.f[7]), ng = triple(c.g[4], w.g[8], e.g[7]);
+  const TripleT<double> cf = triple(c.f[0], w.f[1], e.f[3]), cg = triple(c.g[0], w.g[1], e.g[3]);
+  const double r1 = (pw + pe) + p, r2 = fma(p, p, fma(pw, pw, pe * pe));
+  *S = L.s;
+  S->rho += nf.n;
+  S->jx += nf.d;
+  S->jy -= nf.n;
+  S->fxx += nf.p;
+  S->fyy += nf.n;
+  S->fxy -= nf.d;
+  S->dT += ng.n;
+  S->gxx += ng.p;
+  S->gyy += ng.n;
+  S->gxy -= ng.d;
+  *st = L.t1 + r1;
+  *st2 = L.t2 + r2;
+  *pc = L.pc;
+  L.s = row_sums(L.sf, cf, L.sg, cg);
+  L.t1 = L.n1 + r1;
+  L.t2 = L.n2 + r2;
+  L.pc = p;
+  L.sf = triple(c.f[2], w.f[5], e.f[6]);
+  L.sg = triple(c.g[2], w.g[5], e.g[6]);
+  L.n1 = r1;
+  L.n2 = r2;
+}
+
+// The sums that `feed` completes for a node (i, j) beside a wall, from its nine
+// sources at once and in the same order.  f, g: population k of node (i - cx_k, j -
+// cy_k); rows 0 and Ny+1 are rows 1 and Ny, the ghost columns carry f = 0 and the
+// wall's g.  own: the node's own f.
+__device__ __forceinline__ PullSums pulled_sums(const double f[9], const double g[9],
+                                                const double own[9], int i, int j, int nx, int ny,
+                                                double frozen6, double frozen7) {
+  using Triple = TripleT<double>;
+  const bool south = j == 1, north = j == ny;
+  const Triple sf = south ? triple(own[4], own[7], i == nx ? frozen6 : own[8])
+                          : triple(f[2], f[5], f[6]);
+  const Triple nf = north ? triple(own[2], own[6], i == nx ? frozen7 : own[5])
+                          : triple(f[4], f[8], f[7]);
+  const Triple ng = triple(g[4], g[8], g[7]);
+  PullSums s = row_sums(sf, triple(f[0], f[1], f[3]), triple(g[2], g[5], g[6]),
+                        triple(g[0], g[1], g[3]));
+  const auto add_north = [&]() __attribute__((always_inline)) {
+    s.rho += nf.n;
+    s.jx += nf.d;
+    s.jy -= nf.n;
+    s.fxx += nf.p;
+    s.fyy += nf.n;
+    s.fxy -= nf.d;
+    s.dT += ng.n;
+    s.gxx += ng.p;
+    s.gyy += ng.n;
+    s.gxy -= ng.d;
+  };
+  if (north) add_north();
+  if (i == 1) {
+    const double a = own[3], b = south ? 0.0 : own[7], d = north ? 0.0 : own[6];
+    s.rho += a + b + d;
+    s.jx += a + b + d;
+    s.jy += b - d;
+    s.fxx += a + b + d;
+    s.fyy += b + d;
+    s.fxy += b - d;
+  }
+  if (i == nx) {
+    const double a = own[1], b = south ? 0.0 : own[8], d = north ? 0.0 : own[5];
+    s.rho += a + b + d;
+    s.jx -= a + b + d;
+    s.jy += b - d;
+    s.fxx += a + b + d;
+    s.fyy += b + d;
+    s.fxy += d - b;
+  }
+  if (!north) add_north();
+  return s;
+}
+
+// The phi sums that `feed` completes: taps C, E, N, W, S, NE, NW, SW, SE.
+__device__ __forceinline__ void tap_sums(const double t[9], double* st, double* st2) {
+  const auto sum = [](double w, double c, double e) { return (w + e) + c; };
+  const auto square = [](double w, double c, double e) { return fma(c, c, fma(w, w, e * e)); };
+  *st = (sum(t[7], t[4], t[8]) + sum(t[3], t[0], t[1])) + sum(t[6], t[2], t[5]);
+  *st2 = (square(t[7], t[4], t[8]) + square(t[3], t[0], t[1])) + square(t[6], t[2], t[5]);
 }
 
 inline StepC step_constants(const Consts& c) {

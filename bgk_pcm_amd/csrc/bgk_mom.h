@@ -106,74 +106,6 @@ __device__ __forceinline__ typename CType<R, EQF>::T c_stream(const void* c, int
     return nt_load4<R>(static_cast<const typename Vec<R>::V4*>(c) + q);
 }
 
-// P_k(u,v): the equilibrium polynomial of direction k minus its leading 1.
-__device__ __forceinline__ double eq_poly(int k, double u, double v) {
-  const double uv = 1.5 * (u * u + v * v);
-  switch (k) {
-    case 0: return -uv;
-    case 1: return 3.0 * u + 4.5 * (u * u) - uv;
-    case 2: return 3.0 * v + 4.5 * (v * v) - uv;
-    case 3: return -3.0 * u + 4.5 * (u * u) - uv;
-    case 4: return -3.0 * v + 4.5 * (v * v) - uv;
-    case 5: { const double s = u + v; return 3.0 * s + 4.5 * (s * s) - uv; }
-    case 6: { const double s = u - v; return -3.0 * s + 4.5 * (s * s) - uv; }
-    case 7: { const double s = u + v; return -3.0 * s + 4.5 * (s * s) - uv; }
-    default: { const double s = u - v; return 3.0 * s + 4.5 * (s * s) - uv; }
-  }
-}
-
-// H_k : P for P = (pxx, pyy, pxy), H_k = c_k c_k - cs2 I, in the storage
-// precision (FP32 operands keep their relative precision in FP32).
-template <typename R>
-__device__ __forceinline__ R h_k(int k, R pxx, R pyy, R pxy) {
-  constexpr R A = R(-1) / R(3), B = R(2) / R(3);
-  switch (k) {
-    case 0: return A * (pxx + pyy);
-    case 1:
-    case 3: return B * pxx + A * pyy;
-    case 2:
-    case 4: return A * pxx + B * pyy;
-    case 5:
-    case 7: return B * (pxx + pyy) + R(2) * pxy;
-    default: return B * (pxx + pyy) - R(2) * pxy;
-  }
-}
-
-// Population k of a node from its moments: f_k and gd_k = g_k - w_k*T_crit.
-template <typename R, bool EQF>
-__device__ __forceinline__ void rebuild(int k, const double2 a, const typename Vec<R>::V4 b,
-                                        const typename CType<R, EQF>::T cc, double* fk, double* gdk) {
-  const double p = eq_poly(k, (double)b.x, (double)b.y);
-  const double ax = a.x, ay = a.y;
-  if constexpr (EQF) {
-    const double hg = (double)h_k<R>(k, b.z, b.w, cc);
-    *fk = kW[k] * ax * (1.0 + p);
-    *gdk = kW[k] * (ay + (kTcrit + ay) * p) + coef_of(k) * hg;
-  } else {
-    const double hf = (double)h_k<R>(k, b.z, b.w, cc.x);
-    const double hg = (double)h_k<R>(k, cc.y, cc.z, cc.w);
-    *fk = kW[k] * ax * (1.0 + p) + coef_of(k) * hf;
-    *gdk = kW[k] * (ay + (kTcrit + ay) * p) + coef_of(k) * hg;
-  }
-}
-
-template <typename R, bool EQF>
-__device__ __forceinline__ double rebuild_f(int k, const double2 a, const typename Vec<R>::V4 b,
-                                       const typename CType<R, EQF>::T cc) {
-  const double p = eq_poly(k, (double)b.x, (double)b.y);
-  if constexpr (EQF) {
-    return kW[k] * a.x * (1.0 + p);
-  } else {
-    const double hf = (double)h_k<R>(k, b.z, b.w, cc.x);
-    return kW[k] * a.x * (1.0 + p) + coef_of(k) * hf;
-  }
-}
-
-// Equilibrium deviation of a boundary ghost, g_k - w_k*T_crit.
-__device__ __forceinline__ double ghost_gdev(int k, double T, double u, double v) {
-  return kW[k] * (T - kTcrit) + kW[k] * T * eq_poly(k, u, v);
-}
-
 // Moments of the pulled populations of a node: zeroth, first and second
 // moments of f, and of gd = g - w*T_crit (its first moment is not needed).
 // A: the arithmetic type, double but for the adjoint of the FP32 moment step,
@@ -184,34 +116,6 @@ struct PullSumsT {
   A dT, gxx, gyy, gxy;
 };
 using PullSums = PullSumsT<double>;
-
-__device__ __forceinline__ void pull_zero(PullSums& S) {
-  S.rho = S.jx = S.jy = S.fxx = S.fyy = S.fxy = 0.0;
-  S.dT = S.gxx = S.gyy = S.gxy = 0.0;
-}
-
-// Add population k (f_k, gd_k) to the sums.
-__device__ __forceinline__ void pull_add(PullSums& S, int k, double fk, double gk) {
-  S.rho += fk;
-  S.dT += gk;
-  if (CX[k] != 0) {
-    S.jx += CX[k] > 0 ? fk : -fk;
-    S.fxx += fk;
-    S.gxx += gk;
-  }
-  if (CY[k] != 0) {
-    S.jy += CY[k] > 0 ? fk : -fk;
-    S.fyy += fk;
-    S.gyy += gk;
-  }
-  if (CX[k] * CY[k] > 0) {
-    S.fxy += fk;
-    S.gxy += gk;
-  } else if (CX[k] * CY[k] < 0) {
-    S.fxy -= fk;
-    S.gxy -= gk;
-  }
-}
 
 // The node update in moment form: momentsPre (STEP_7/momentsPre.f90:8-21),
 // phase field (phase_field.f90:24-52, reaction rates in closed form),
@@ -243,7 +147,6 @@ struct CoreT {
   A qfxx, qfyy, qfxy;             // Pi_f^neq
   A qgxx, qgyy, qgxy;             // Pi_g^neq
 };
-using Core = CoreT<double>;
 
 // 1/d as the hardware estimate refined by two Newton steps (r <- r + r (1 -
 // d r), each doubling the correct bits): within an ulp or two of the IEEE
@@ -333,24 +236,6 @@ __device__ __forceinline__ CoreT<A> core_from_sums(const C& c, const PullSumsT<A
   o.qgxy = S.gxy - o.T * o.u * o.v;
   return o;
 }
-
-__device__ __forceinline__ Core core_forward(const Consts& c, const PullSums& S,
-                                             const double tap[9]) {
-  double st = tap[0], st2 = tap[0] * tap[0];
-#pragma unroll
-  for (int m = 1; m < 9; ++m) {
-    st = st + tap[m];
-    st2 = fma(tap[m], tap[m], st2);
-  }
-  return core_from_sums<double, Consts>(c, S, st, st2, tap[0]);
-}
-
-// Averaged moments of STEP_7/moments.f90:11-25 from the stored state: sum_k
-// f_k = rho, sum_k g_k = T and sum_k c_k f_k / rho = u exactly for the
-// rebuilt populations.
-struct NodeOut {
-  double rho, Tav, uav, vav;
-};
 
 // One launch of T moment-storage steps: state and phi in and out, the
 // east-wall temperature column before and after, an optional probe record (T

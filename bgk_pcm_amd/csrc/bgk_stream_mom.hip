@@ -34,11 +34,6 @@ struct Macro {
   double *rho, *u, *v, *T;
 };
 
-// Moments of a node as the rebuild of its populations takes them.
-struct NodeD {
-  double rho, th, u, v, pfxx, pfyy, pfxy, pgxx, pgyy, pgxy, phi;
-};
-
 // A row as loaded: converted only when it is fed.
 template <typename R, bool EQF>
 struct Raw {
