@@ -1,6 +1,6 @@
 // bgk_fused_mom.hip -- moment storage: the choice of kernel and of the steps
 // per launch, the initialization, and the ring kernel, one step per launch
-// through LDS, which large FP32-moment lattices take for a step alone (see
+// through LDS, which large lattices take for a step alone (see
 // ring_step; every other launch is bgk_stream_mom.hip's).
 //
 // The node state is the ten moments of bgk_mom.h (rho, T - T_crit in FP64;
@@ -332,14 +332,43 @@ hipError_t launch_ring(bgk_handle* h, const MomStep& st) {
   return hipGetLastError();
 }
 
-// Whether one step alone goes through the ring kernel.  Measured per step on
-// MI355X, ring against the streaming kernel with T = 1, FP32 moments: 4096^2
-// 364 / 416 us (omega_f = 1: 286 / 343), 2048^2 103 / 106 (85 / 87), 512^2
-// 20.2 / 11.8 (17.6 / 10.4).
+template <int W, typename R>
+hipError_t launch_ring_layout(bgk_handle* h, const MomStep& st) {
+  return h->mom_eqf ? launch_ring<W, R, true>(h, st) : launch_ring<W, R, false>(h, st);
+}
+
+// Width of the ring kernel's workgroups: the widest that adds at most a quarter to
+// the columns, or the narrowest that adds at most half; 0: none.  (The wider, the
+// longer the contiguous pieces of a row; FP64 rows wider than 256 do not fit
+// the LDS of a resident workgroup twice.)
+int ring_width(const bgk_handle* h) {
+  const auto columns = [h](int w) { return ((int64_t)h->nx + w - 1) / w * w; };
+  for (int w = h->prm.precision == BGK_FP32_MOM ? 512 : 256; w >= 128; w /= 2)
+    if (4 * columns(w) <= 5 * (int64_t)h->nx) return w;
+  return 2 * columns(128) <= 3 * (int64_t)h->nx ? 128 : 0;
+}
+
+// Whether one step alone goes through the ring kernel: its loads go past the caches,
+// which leaves these to the macroscopic fields that a call's last step writes,
+// and its rows are longer pieces than a wave's.  Measured, us per call of one
+// step, streaming kernel with T = 1 / ring:
+//              FP32 moments  omega_f = 1  FP64 moments  omega_f = 1
+//   1700^2        85 / 84       71 / 73     151 / 133     105 / 96
+//   1850^2       108 / 97       86 / 81     176 / 151     135 / 113
+//   2048^2       146 / 107     121 / 89     211 / 172     165 / 129
+//   4096^2       551 / 510     475 / 427    812 / 767     631 / 587
+//   90 x 40000   157 / 125     136 / 105    215 / 186     170 / 140
+//   130 x 40000  234 / 208     208 / 189    319 / 369     254 / 279  (width 0)
+//   512 x 1500    30 / 37       25 / 35      42 / 44       32 / 35
+//   250 x 2200    31 / 24       28 / 22      37 / 31       31 / 26
+//   128 x 8000    47 / 39       42 / 35      66 / 55       54 / 43
+//   120 x 6000    29 / 28       27 / 27      38 / 41       31 / 33
+//   250 x 1000    15 / 19       14 / 18      17 / 23       15 / 20
+// (of few columns a wave's last segment is a large share).
 bool ring_step(const bgk_handle* h) {
-  if (h->prm.precision != BGK_FP32_MOM) return false;
   if (h->mom_variant != 0) return h->mom_variant >= 4;
-  return (int64_t)h->nx * h->ny >= (int64_t)1 << 23;
+  const int64_t least = h->nx <= 384 ? (int64_t)1 << 19 : (int64_t)3 << 20;
+  return (int64_t)h->nx * h->ny >= least && ring_width(h) > 0;
 }
 
 template <typename R, bool EQF>
@@ -387,7 +416,12 @@ bool mom_write_all(const bgk_handle* h, int T, int left, bool adjoint) {
 
 hipError_t launch_mom_steps(bgk_handle* h, const MomStep& st, int T) {
   if (T > 1 || st.adjoint || !ring_step(h)) return launch_mom_stream(h, st, T);
-  return h->mom_eqf ? launch_ring<512, float, true>(h, st) : launch_ring<512, float, false>(h, st);
+  const int w = ring_width(h);
+  if (h->prm.precision == BGK_FP64_MOM)
+    return w == 256 ? launch_ring_layout<256, double>(h, st) : launch_ring_layout<128, double>(h, st);
+  return w == 512   ? launch_ring_layout<512, float>(h, st)
+         : w == 256 ? launch_ring_layout<256, float>(h, st)
+                    : launch_ring_layout<128, float>(h, st);
 }
 
 hipError_t launch_fused_steps_mom(bgk_handle* h, int nsteps) {

@@ -60,11 +60,12 @@ inline int edge_count(int nx, int ny) {
 
 // Row strips of about `target` rows, and at least one workgroup per slot
 // of the device (slots = CUs x resident workgroups per CU) on small
-// lattices, down to 2 rows per strip.  The strip count is chosen, where one
-// exists within a factor two, as a multiple of 8 (the XCDs) whose workgroups
-// fill whole rounds of the device: measured at 4096^2 with the moment
-// kernel, 64-row strips (512 workgroups) run at 57 GLUPS and 96-row strips
-// (43 strips, 1.5 rounds) at 43.  rows_override > 0 fixes the strip height.
+// lattices, down to 2 rows per strip.  Of the strip counts from that to twice
+// as many (multiples of 8, the XCDs) the one whose rounds of the device take
+// the fewest rows, a strip's two extra ones included: measured with the moment
+// kernel, one step alone, FP32 moments with omega_f = 1: 2896^2 in 288
+// workgroups (two rounds, the second nearly empty) 284 us, in 480 212.
+// rows_override > 0 fixes the strip height.
 inline StripGrid make_strip_grid(int nx, int ny, int w, int target, int slots,
                                  int rows_override) {
   StripGrid s;
@@ -75,12 +76,17 @@ inline StripGrid make_strip_grid(int nx, int ny, int w, int target, int slots,
     int want = std::max(1, (ny + target - 1) / target);
     if (slots > 0) want = std::max(want, (slots + s.nseg - 1) / s.nseg);
     want = std::min(want, std::max(1, (ny + 1) / 2));
-    int pick = (want + NXCD - 1) / NXCD * NXCD;
-    for (int n = pick; n <= 2 * want && n <= ny; n += NXCD)
-      if (slots > 0 && ((int64_t)n * s.nseg) % slots == 0) {
+    const int least = (want + NXCD - 1) / NXCD * NXCD;
+    int pick = least;
+    int64_t cost = -1;
+    for (int n = least; n == least || (n <= 2 * want && n <= ny); n += NXCD) {
+      const int64_t rounds = slots > 0 ? ((int64_t)n * s.nseg + slots - 1) / slots : 1;
+      const int64_t c = rounds * ((ny + n - 1) / n + 2);
+      if (cost < 0 || c < cost) {
+        cost = c;
         pick = n;
-        break;
       }
+    }
     s.rows = std::max(1, (ny + pick - 1) / pick);
   }
   s.nstrip = (ny + s.rows - 1) / s.rows;

@@ -2,8 +2,8 @@
 one thread per node through the LDS ring (BGK_MOM_VARIANT=4), one wave per strip
 (1: one step per launch, 2: two), mixed as the rule does on large lattices, and in a
 gradient's forward run.  Exact, fields and halo: every one of them writes out the same
-operations in the same order.  Widths on either side of the ring's 256 and 512
-columns, with segments and strips that touch no wall, and ring strips of 1 to 3 rows.
+operations in the same order.  Widths on either side of the ring's 128, 256 and
+512 columns, with segments and strips that touch no wall, and ring strips of 1 to 3 rows.
 """
 import numpy as np
 import pytest
@@ -15,8 +15,8 @@ pytestmark = pytest.mark.gpu
 
 FIELDS = ("rho", "u", "v", "T", "phi")
 EXT = dict(k_ratio=1.5, noise_amp=1e-3, noise_seed=11)
-SHAPES = [(1, 1), (1, 9), (9, 1), (2, 3), (61, 7), (130, 5), (256, 6), (513, 9), (1100, 9),
-          (1537, 5)]
+SHAPES = [(1, 1), (1, 9), (9, 1), (2, 3), (61, 7), (130, 5), (256, 6), (513, 9), (300, 9), (700, 5),
+          (1100, 9), (1537, 5)]
 
 
 def params(nx, ny, precision, tau_f):
@@ -47,7 +47,8 @@ def test_ring_and_stream(monkeypatch, nx, ny, precision, tau_f, cold, rows):
             assert np.array_equal(got[f], want[f]), (variant, split, f)
 
 
-@pytest.mark.parametrize("nx,ny,precision", [(4100, 2050, FP32_MOM), (2900, 2899, FP64_MOM)])
+@pytest.mark.parametrize("nx,ny,precision", [(4100, 2050, FP32_MOM), (2900, 2899, FP64_MOM),
+                                             (250, 2200, FP64_MOM), (130, 30000, FP32_MOM)])
 @pytest.mark.parametrize("tau_f", [1.0, 0.8])
 def test_splits_of_a_run_on_a_large_lattice(nx, ny, precision, tau_f):
     want = None
