@@ -44,9 +44,9 @@
 // of the population loads); 64 x 4 and 64 x 8 tiles with a phi window in
 // LDS, walked in XCD bands, 0.605 and 0.623 ms (a plane's rows are then
 // streamed in 512-byte pieces instead of 2 KB).  Same folding of BC_f/BC_g and the same
-// halo bookkeeping as the FP64 kernel (bgk_fused.hip).  Runs on larger lattices
-// take two steps per launch instead (bgk_stream32.hip); this kernel does one,
-// and the FP32-collision form.
+// halo bookkeeping as the FP64 kernel (bgk_fused.hip).  Larger lattices take the
+// kernels of bgk_stream32.hip instead (sums32); this one serves the others, and the
+// FP32-collision form.
 #include "bgk_internal.h"
 
 namespace bgk {
@@ -531,7 +531,7 @@ hipError_t launch_rephase32(bgk_handle* h, const double* phi_new) {
 // A run of steps: two per launch where stream32 allows and the re-basing leaves
 // room (which step a re-basing precedes does not depend on how a run is
 // split).  The last launch of a call knows the state before its last step, for
-// the halo: two steps, or one of k_fused32 after another one of it.
+// the halo: two steps, or one after another one.
 hipError_t launch_fused_steps32(bgk_handle* h, int nsteps) {
   for (int left = nsteps; left > 0;) {
     if (h->rebase_every > 0 && h->since_rebase >= h->rebase_every) {
@@ -541,7 +541,9 @@ hipError_t launch_fused_steps32(bgk_handle* h, int nsteps) {
     const bool room = h->rebase_every == 0 || h->since_rebase + kSteps32 <= h->rebase_every;
     const bool many = left % kSteps32 == 0 && room && stream32(h);
     left -= many ? kSteps32 : 1;
-    const hipError_t e = many ? launch_stream32(h, left == 0) : launch_fused_step32(h, left == 0);
+    const hipError_t e = many        ? launch_stream32(h, left == 0)
+                         : sums32(h) ? launch_step32(h, left == 0)
+                                     : launch_fused_step32(h, left == 0);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

@@ -223,7 +223,7 @@ __device__ __forceinline__ void mom_edge_nodes(const MomIn& in, const MomOut& ou
   const int64_t r0 = (int64_t)j * P;
   const double tap[9] = {pa[q],          pa[r0 + i + 1], pa[rn + i],     pa[r0 + i - 1], pa[rs + i],
                          pa[rn + i + 1], pa[rn + i - 1], pa[rs + i - 1], pa[rs + i + 1]};
-  const PullSums S = pulled_sums(f, g, own.f, i, j, nx, ny, c.frozen6, c.frozen7);
+  const PullSums S = pulled_sums<true>(f, g, own.f, i, j, nx, ny, c.frozen6, c.frozen7);
   double st, st2;
   tap_sums(tap, &st, &st2);
   const Updated o = update_node<R, EQF>(sc, S, st, st2, tap[0], out, pb, q);

@@ -139,10 +139,13 @@ bool stream64(const bgk_handle* h);
 hipError_t launch_stream64(bgk_handle* h, bool write_all);
 hipError_t launch_fused_step32(bgk_handle* h, bool write_all);
 // nsteps steps of an FP32 population handle; kSteps32 of them in one launch
-// (bgk_stream32.hip), where stream32(h)
+// (bgk_stream32.hip), where stream32(h).  sums32(h): with that kernel's arithmetic,
+// a step alone too (launch_step32), whatever launches a run is cut into
 hipError_t launch_fused_steps32(bgk_handle* h, int nsteps);
 constexpr int kSteps32 = 2;
+bool sums32(const bgk_handle* h);
 bool stream32(const bgk_handle* h);
+hipError_t launch_step32(bgk_handle* h, bool write_all);
 hipError_t launch_stream32(bgk_handle* h, bool write_all);
 // nsteps moment steps
 hipError_t launch_fused_steps_mom(bgk_handle* h, int nsteps);

@@ -309,15 +309,16 @@ __device__ __forceinline__ void feed_three(Level& L, const Pops& w, const Pops& 
   L.n2 = r2;
 }
 
-// The sums that `feed` completes for a node (i, j) beside a wall, from its nine
-// sources at once and in the same order.  f, g: population k of node (i - cx_k, j -
-// cy_k); rows 0 and Ny+1 are rows 1 and Ny, the ghost columns carry f = 0 and the
-// wall's g.  own: the node's own f.
+// The sums that `feed` completes for a node (i, j), from its nine sources at once
+// and in the same order.  f, g: population k of node (i - cx_k, j - cy_k); rows 0
+// and Ny+1 are rows 1 and Ny, the ghost columns carry f = 0 and the wall's g.
+// own: the node's own f.  EDGE: the node may be beside a wall.
+template <bool EDGE>
 __device__ __forceinline__ PullSums pulled_sums(const double f[9], const double g[9],
                                                 const double own[9], int i, int j, int nx, int ny,
                                                 double frozen6, double frozen7) {
   using Triple = TripleT<double>;
-  const bool south = j == 1, north = j == ny;
+  const bool south = EDGE && j == 1, north = EDGE && j == ny;
   const Triple sf = south ? triple(own[4], own[7], i == nx ? frozen6 : own[8])
                           : triple(f[2], f[5], f[6]);
   const Triple nf = north ? triple(own[2], own[6], i == nx ? frozen7 : own[5])
@@ -338,7 +339,7 @@ __device__ __forceinline__ PullSums pulled_sums(const double f[9], const double 
     s.gxy -= ng.d;
   };
   if (north) add_north();
-  if (i == 1) {
+  if (EDGE && i == 1) {
     const double a = own[3], b = south ? 0.0 : own[7], d = north ? 0.0 : own[6];
     s.rho += a + b + d;
     s.jx += a + b + d;
@@ -347,7 +348,7 @@ __device__ __forceinline__ PullSums pulled_sums(const double f[9], const double 
     s.fyy += b + d;
     s.fxy += b - d;
   }
-  if (i == nx) {
+  if (EDGE && i == nx) {
     const double a = own[1], b = south ? 0.0 : own[8], d = north ? 0.0 : own[5];
     s.rho += a + b + d;
     s.jx -= a + b + d;

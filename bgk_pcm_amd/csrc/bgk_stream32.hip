@@ -1,4 +1,6 @@
-// bgk_stream32.hip -- T time steps with FP32 population storage in one launch.
+// bgk_stream32.hip -- T time steps with FP32 population storage in one launch, and
+// a step alone with the same arithmetic (k_step32), so that a run does not depend on
+// how it is split.
 //
 // Storage and reference densities as in bgk_fused32.hip (f_k - w_k rho_ref and
 // g_k - w_k T_crit in FP32); the walk and the node update are those of
@@ -58,7 +60,7 @@ __device__ __forceinline__ void load_raw(const Args32& A, unsigned off, unsigned
 
 // Populations as a launch hands them on: what the planes hold and what they
 // stand for.
-struct Pops {
+struct Stored {
   float fs[9], gs[9];
   double f[9], g[9];
 };
@@ -69,7 +71,7 @@ __device__ __forceinline__ double ref_density(double rs, double rl, double phi) 
   return fma(fma(0.5, phi, 0.5), rl - rs, rs);
 }
 
-__device__ __forceinline__ void encode(const Updated& o, double rr, Pops& p) {
+__device__ __forceinline__ void encode(const Updated& o, double rr, Stored& p) {
   populations<true>(o.rho, o.rho, o.u, o.v, o.pfxx, o.pfyy, o.pfxy, p.f);
   populations<true>(o.dT, kTcrit + o.dT, o.u, o.v, o.pgxx, o.pgyy, o.pgxy, p.g);
 #pragma unroll
@@ -78,7 +80,7 @@ __device__ __forceinline__ void encode(const Updated& o, double rr, Pops& p) {
     p.gs[k] = (float)p.g[k];
   }
 }
-__device__ __forceinline__ void decode(double rr, Pops& p) {
+__device__ __forceinline__ void decode(double rr, Stored& p) {
 #pragma unroll
   for (int k = 0; k < 9; ++k) {
     p.f[k] = fma(kW[k], rr, (double)p.fs[k]);
@@ -87,7 +89,7 @@ __device__ __forceinline__ void decode(double rr, Pops& p) {
 }
 
 // Averaged moments of the stored state (STEP_7/moments.f90:11-25).
-__device__ __forceinline__ double averaged_T(const Pops& p, const Updated& o) {
+__device__ __forceinline__ double averaged_T(const Stored& p, const Updated& o) {
   double s = (double)p.gs[0];
 #pragma unroll
   for (int k = 1; k < 9; ++k) s += (double)p.gs[k];
@@ -96,7 +98,7 @@ __device__ __forceinline__ double averaged_T(const Pops& p, const Updated& o) {
 struct Avg {
   double rho, T, u, v;
 };
-__device__ __forceinline__ Avg averaged(const Pops& p, const Updated& o, double rr) {
+__device__ __forceinline__ Avg averaged(const Stored& p, const Updated& o, double rr) {
   double a[9];
 #pragma unroll
   for (int k = 0; k < 9; ++k) a[k] = (double)p.fs[k];
@@ -184,7 +186,7 @@ __device__ __forceinline__ void strip32(const Args32& A, int j0, int j1, int i, 
   __builtin_amdgcn_s_waitcnt(kWaitLoads);
   // full: levels that have completed a row of use; level `full` is only fed
   auto feed_row = [&](int r, int full) __attribute__((always_inline)) {
-    Pops p;
+    Stored p;
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
       p.fs[k] = raw.p[k].x;
@@ -292,19 +294,103 @@ __global__ __launch_bounds__(kLanes, 2) void k_stream32(Args32 A) {
     strip32<T, false, FINAL>(A, j0, j1, i, false, false);
 }
 
-}  // namespace
-
-// Measured, us per step, two steps per launch against k_fused32: 4096^2 354
-// (472), 2048^2 90 (135), 1003 x 777 23.9 (27.9), 724^2 22.2 (23.1), 512^2
-// 19.6 (14.6).  FP32 collision arithmetic and uploaded ghost velocities are the
-// general kernel's.
-bool stream32(const bgk_handle* h) {
-  if (!h->ghost_uv || h->recorded || h->prm.fp32_collision || h->pop_variant == 1) return false;
-  return h->pop_variant > 1 || (int64_t)h->nx * h->ny >= (int64_t)1 << 19;
+// One step, one node per thread in the tiles of bgk_device.h, with the arithmetic
+// of the walk: an odd step has the bits it has within a launch of two.  A wave with
+// a boundary-adjacent node takes one path for all its lanes: ghost columns carry
+// no flow populations and the wall's equilibria (at the ghost velocities of m.u
+// and m.v), and every lane makes the same loads, from the nearest nodes inside.
+// Bound by HBM; past the caches three waves per SIMD instead of the four that the
+// registers allow disturb each other less (4096^2, us per call of one step: 586 /
+// 559; cached, 727^2, 19.0 / 19.7).  Against k_fused32: 4096^2 578 -> 559, 2048^2
+// 151 -> 133, 1003 x 777 30.2 -> 25.4.
+template <bool CACHED>
+__global__ __launch_bounds__(TILE_W) __attribute__((amdgpu_waves_per_eu(2, CACHED ? 4 : 3)))
+void k_step32(Args32 A, TileGrid tg, int write_all) {
+  const int nx = A.nx, ny = A.ny;
+  const int64_t P = A.pitch;
+  int i, j;
+  if (!tile_node(tg, Geom{nx, ny, P}, &i, &j)) return;
+  const bool edge = i == 1 || i == nx || j == 1 || j == ny;
+  const int row[3] = {max(j - 1, 1), j, min(j + 1, ny)};  // south, own, north
+  const int64_t q = (int64_t)j * P + i;
+  const double* const ps = A.pa + ((int64_t)row[0] * P + i);
+  const double* const pc = A.pa + q;
+  const double* const pn = A.pa + ((int64_t)row[2] * P + i);
+  // taps C, E, N, W, S, NE, NW, SW, SE: of direction OPP[k] at population k's source
+  const double tap[9] = {pc[0], pc[1], pn[0], pc[-1], ps[0], pn[1], pn[-1], ps[-1], ps[1]};
+  const scalar_ptr tab = as_scalar(A.tab);
+  double rs[3], rl[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    rs[d] = tab[row[d]];
+    rl[d] = tab[ny + 2 + row[d]];
+  }
+  double f[9], g[9], own[9] = {}, rho_was = 0.0, T_was = 0.0;
+  float fr6 = 0.0f, fr7 = 0.0f;
+  PullSums S;
+  if (!__any(edge)) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      const float2 v = load_pair<CACHED>(A.A.row(k, q - CX[k] - (int64_t)CY[k] * P));
+      f[k] = fma(kW[k], ref_density(rs[1 - CY[k]], rl[1 - CY[k]], tap[OPP[k]]), (double)v.x);
+      g[k] = (double)v.y;
+    }
+    S = pulled_sums<false>(f, g, f, i, j, nx, ny, 0.0, 0.0);
+  } else {
+    const double r1 = ref_density(rs[1], rl[1], tap[0]);
+    fr6 = A.A.row(6, nx + 1)->x;
+    fr7 = A.A.row(7, (int64_t)(ny + 1) * P + nx + 1)->x;
+    rho_was = A.m.rho[q];
+    T_was = A.m.T[q];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const int64_t h = (int64_t)row[d] * P;
+      const double t = A.east_cold ? A.t_cold : as_scalar(A.te_in)[row[d]];
+      double gw[9], ge[9];
+      populations<false>(A.tin - kTcrit, A.tin, A.m.u[h], A.m.v[h], 0.0, 0.0, 0.0, gw);
+      populations<false>(t - kTcrit, t, A.m.u[h + nx + 1], A.m.v[h + nx + 1], 0.0, 0.0, 0.0, ge);
+#pragma unroll
+      for (int k = 0; k < 9; ++k) {
+        if (1 - CY[k] != d) continue;
+        const int si = i - CX[k];
+        const float2 v = *A.A.row(k, h + min(max(si, 1), nx));
+        const double x = fma(kW[k], ref_density(rs[d], rl[d], tap[OPP[k]]), (double)v.x);
+        f[k] = si >= 1 && si <= nx ? x : 0.0;
+        g[k] = si < 1 ? gw[k] : si > nx ? ge[k] : (double)v.y;
+        if (k > 0) own[k] = fma(kW[k], r1, (double)A.A.row(k, q)->x);
+      }
+    }
+    S = pulled_sums<true>(f, g, own, i, j, nx, ny, fma(kW[6], A.rho0, (double)fr6),
+                          fma(kW[7], A.rho0, (double)fr7));
+  }
+  double st, st2;
+  tap_sums(tap, &st, &st2);
+  const Updated o = update<double, false>(A.c, S, st, st2, tap[0]);
+  const double rr = ref_density(rs[1], rl[1], o.phi);
+  Stored p;
+  encode(o, rr, p);
+#pragma unroll
+  for (int k = 0; k < 9; ++k) store_pair<CACHED>(A.B.row(k, q), p.fs[k], p.gs[k]);
+  store_one<CACHED>(&A.pb[q], o.phi);
+  if (!(edge || write_all)) return;
+  const Avg a = averaged(p, o, rr);
+  if (edge) {
+    halo(A, j, i, rho_was, T_was, tap[0]);
+    if (i == 1) A.pb[q - 1] = tap[3];
+    if (i == nx) {
+      A.pb[q + 1] = tap[1];
+      A.te_out[j] = a.T;
+      if (j == 1) A.B.row(6, nx + 1)->x = fr6;
+      if (j == ny) A.B.row(7, (int64_t)(ny + 1) * P + nx + 1)->x = fr7;
+    }
+  }
+  A.m.rho[q] = a.rho;
+  A.m.T[q] = a.T;
+  A.m.u[q] = a.u;
+  A.m.v[q] = a.v;
 }
 
-hipError_t launch_stream32(bgk_handle* h, bool write_all) {
-  constexpr int T = kSteps32;
+Args32 args32(const bgk_handle* h) {
   Args32 a;
   const int ca = h->cur, cb = 1 - h->cur;
   a.A = planes_of<float2>(h->f32[ca]);
@@ -325,6 +411,41 @@ hipError_t launch_stream32(bgk_handle* h, bool write_all) {
   a.nx = h->nx;
   a.ny = h->ny;
   a.pitch = h->pitch;
+  return a;
+}
+
+void advanced(bgk_handle* h, int steps) {
+  h->cur = 1 - h->cur;
+  h->pc = 1 - h->pc;
+  h->te_cur = 1 - h->te_cur;
+  h->since_rebase += steps;
+}
+
+}  // namespace
+
+// Measured, us per step, two steps per launch against k_fused32: 4096^2 354
+// (472), 2048^2 90 (135), 1003 x 777 23.9 (27.9), 724^2 22.2 (23.1), 512^2
+// 19.6 (14.6).  FP32 collision arithmetic is the general kernel's.
+bool sums32(const bgk_handle* h) {
+  if (h->prm.fp32_collision || h->pop_variant == 1) return false;
+  return h->pop_variant > 1 || (int64_t)h->nx * h->ny >= (int64_t)1 << 19;
+}
+// (the ghost velocities are the initial ones in strip32)
+bool stream32(const bgk_handle* h) { return sums32(h) && h->ghost_uv && !h->recorded; }
+
+hipError_t launch_step32(bgk_handle* h, bool write_all) {
+  const TileGrid tg = make_tile_grid(h->geom, 2 * (18 * (int)sizeof(float) + (int)sizeof(double)));
+  const auto k = tg.cached ? k_step32<true> : k_step32<false>;
+  hipLaunchKernelGGL(k, dim3((unsigned)(tg.per * NXCD)), dim3(TILE_W), 0, h->stream, args32(h), tg,
+                     write_all ? 1 : 0);
+  const hipError_t e = hipGetLastError();
+  if (e == hipSuccess) advanced(h, 1);
+  return e;
+}
+
+hipError_t launch_stream32(bgk_handle* h, bool write_all) {
+  constexpr int T = kSteps32;
+  Args32 a = args32(h);
   // at most 16 rows per strip (measured at 8 / 16 / 24 / 48, us per step: 4096^2
   // 361 / 352 / 352 / 352, 2048^2 103 / 100 / 107 / 118)
   a.g = make_wave_grid(h->nx, h->ny, kLanes - 2 * T, T, 2 * T, 1.4, 16, h->n_cu, h->strip_rows);
@@ -334,12 +455,7 @@ hipError_t launch_stream32(bgk_handle* h, bool write_all) {
   else
     hipLaunchKernelGGL((k_stream32<T, false>), grd, dim3(kLanes), 0, h->stream, a);
   const hipError_t e = hipGetLastError();
-  if (e == hipSuccess) {
-    h->cur = cb;
-    h->pc = 1 - h->pc;
-    h->te_cur = 1 - h->te_cur;
-    h->since_rebase += T;
-  }
+  if (e == hipSuccess) advanced(h, T);
   return e;
 }
 
