@@ -14,7 +14,6 @@
 #include <cstring>
 #include <future>
 #include <mutex>
-#include <vector>
 
 #include "bgk_internal.h"
 
@@ -25,7 +24,8 @@ constexpr size_t kChunk = (size_t)4 << 20;
 constexpr int kMaxBuffers = 8;
 
 std::mutex g_mu;
-std::vector<void*> g_free;  // idle buffers of kChunk bytes
+void* g_idle[kMaxBuffers];  // buffers of kChunk bytes (no container: nothing here throws)
+int g_nidle = 0;
 int g_users = 0;            // handles alive
 
 // rows r0 .. r0 + gridDim.y - 1 of a plane, nx + 2 values each
@@ -40,11 +40,7 @@ __global__ void k_pack(const double* __restrict__ src, int stride, int64_t pitch
 void* take() {
   {
     std::lock_guard<std::mutex> lock(g_mu);
-    if (!g_free.empty()) {
-      void* p = g_free.back();
-      g_free.pop_back();
-      return p;
-    }
+    if (g_nidle > 0) return g_idle[--g_nidle];
   }
   void* p = nullptr;
   if (hipHostMalloc(&p, kChunk, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
@@ -58,8 +54,8 @@ void give(void* p) {
   if (!p) return;
   {
     std::lock_guard<std::mutex> lock(g_mu);
-    if (g_users > 0 && (int)g_free.size() < kMaxBuffers) {
-      g_free.push_back(p);
+    if (g_users > 0 && g_nidle < kMaxBuffers) {
+      g_idle[g_nidle++] = p;
       return;
     }
   }
@@ -92,12 +88,14 @@ void staging_open() {
 }
 
 void staging_close() {
-  std::vector<void*> idle;
+  void* idle[kMaxBuffers];
+  int n = 0;
   {
     std::lock_guard<std::mutex> lock(g_mu);
-    if (--g_users == 0) idle.swap(g_free);
+    if (--g_users == 0)
+      while (g_nidle > 0) idle[n++] = g_idle[--g_nidle];
   }
-  for (void* p : idle) (void)hipHostFree(p);
+  while (n > 0) (void)hipHostFree(idle[--n]);
 }
 
 Staging::Staging() : p_(take()) {}
