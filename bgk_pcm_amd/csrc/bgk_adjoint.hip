@@ -473,15 +473,16 @@ struct AdjRow {
   L2 l2;
   R l3;
 
-  __device__ __forceinline__ void load_state(const AdjArgs& A, int j, unsigned ic) {
-    const int64_t q = (int64_t)j * A.pitch;
+  // columns counted from ib
+  __device__ __forceinline__ void load_state(const AdjArgs& A, int j, int ib, unsigned ic) {
+    const int64_t q = (int64_t)j * A.pitch + ib;
     a = at(A.sprev.a + q, ic * (unsigned)sizeof(double2));
     b = at(static_cast<const V4*>(A.sprev.b) + q, ic * (unsigned)sizeof(V4));
     c = at(static_cast<const C*>(A.sprev.c) + q, ic * (unsigned)sizeof(C));
     phi = at(A.sprev.phi + q, ic * (unsigned)sizeof(double));
   }
-  __device__ __forceinline__ void load_lam(const AdjArgs& A, int j, unsigned ic) {
-    const int64_t q = (int64_t)j * A.pitch;
+  __device__ __forceinline__ void load_lam(const AdjArgs& A, int j, int ib, unsigned ic) {
+    const int64_t q = (int64_t)j * A.pitch + ib;
     l0 = at(static_cast<const V4*>(A.next.v[0]) + q, ic * (unsigned)sizeof(V4));
     l1 = at(static_cast<const V4*>(A.next.v[1]) + q, ic * (unsigned)sizeof(V4));
     l2 = at(static_cast<const L2*>(A.next.v[2]) + q, ic * (unsigned)sizeof(L2));
@@ -540,12 +541,12 @@ struct AdjRow {
   }
 };
 
-// Stores of row j (lanes that must not store: column kPastStrip).
+// Stores of row j at column i of n from ib on (lanes that must not store: kPastStrip).
 template <typename R, bool EQF>
-__device__ __forceinline__ void store_adjoint(const AdjArgs& A, int j, int i, const Lam<R>& x) {
+__device__ __forceinline__ void store_adjoint(const AdjArgs& A, int j, int ib, int n, int i,
+                                              const Lam<R>& x) {
   using Row = AdjRow<R, EQF>;
-  const int64_t q = (int64_t)j * A.pitch;
-  const int n = (int)A.pitch;
+  const int64_t q = (int64_t)j * A.pitch + ib;
   buffer_put<adj_store<R>()>(strip_buffer(static_cast<typename Row::V4*>(A.cur.v[0]) + q, n), i,
              make4<R>(x.rho, x.jx, x.jy, x.dT));
   buffer_put<adj_store<R>()>(strip_buffer(static_cast<typename Row::V4*>(A.cur.v[1]) + q, n), i,
@@ -564,13 +565,16 @@ __device__ __forceinline__ void store_adjoint(const AdjArgs& A, int j, int i, co
 
 // One wave's strip, rows j0..j1.  EDGE: the wave or the strip touches a wall.
 // INIT: the share of the initial state, sprev itself (nothing is stored).  g: this
-// lane's parameter adjoints, summed in FP64.
-template <typename R, bool EQF, bool EDGE, bool INIT>
-__device__ __forceinline__ void adjoint_strip(const AdjArgs& A, int j0, int j1, int i, bool has_w,
-                                              bool has_e, double g[3]) {
+// lane's parameter adjoints, summed in FP64.  WIDE: a row is more than a 32-bit byte
+// offset reaches, so columns are counted from the wave's first one (at every width
+// 2% slower with FP64 moments).
+template <typename R, bool EQF, bool EDGE, bool INIT, bool WIDE>
+__device__ __forceinline__ void adjoint_strip(const AdjArgs& A, int j0, int j1, int i0, int i,
+                                              bool has_w, bool has_e, double g[3]) {
   const auto& c = ConstsOf<R>::of(A);
   const int nx = A.nx, ny = A.ny, lane = (int)threadIdx.x;
-  const unsigned ic = (unsigned)(i < 0 ? 0 : (i > nx + 1 ? nx + 1 : i));  // column loaded
+  const int ib = WIDE ? i0 - 1 : 0;
+  const unsigned ic = (unsigned)((i < 0 ? 0 : (i > nx + 1 ? nx + 1 : i)) - ib);  // column loaded
   const bool ghost = EDGE && (i == 0 || i == nx + 1);
   const bool own = lane >= 1 && lane < kLanes - 1 && i <= nx;  // columns this wave stores
   const bool live = A.has_next && (!EDGE || (i >= 1 && i <= nx));
@@ -590,15 +594,15 @@ __device__ __forceinline__ void adjoint_strip(const AdjArgs& A, int j0, int j1, 
   R u_was = R(0), v_was = R(0);  // INIT: the completed row's velocity
   const int ra = EDGE ? max(1, j0 - 1) : j0 - 1, rb = j1 + 1;
   AdjRow<R, EQF> row;
-  row.load_lam(A, ra, ic);
-  row.load_state(A, ra, ic);
+  row.load_lam(A, ra, ib, ic);
+  row.load_state(A, ra, ib, ic);
   const scalar_ptr te_in = as_scalar(A.sprev.te);
   double te_row = EDGE ? te_in[ra] : 0.0;
   __builtin_amdgcn_s_waitcnt(kWaitLoads);
   auto feed_row = [&](int r, auto feed_only) __attribute__((always_inline)) {
     const Lam<R> x = row.lam(live);
     __builtin_amdgcn_sched_barrier(0);
-    row.load_lam(A, min(r + 1, ny), ic);
+    row.load_lam(A, min(r + 1, ny), ib, ic);
     const int jc = r - 1;  // row completed
     const bool on = own && jc >= j0 && jc <= j1;
     // ---- step n+1's pulls reversed
@@ -610,7 +614,7 @@ __device__ __forceinline__ void adjoint_strip(const AdjArgs& A, int j0, int j1, 
     R phi;
     Mom<R> m = row.state(&phi);
     __builtin_amdgcn_sched_barrier(0);
-    row.load_state(A, min(r + 1, ny), ic);
+    row.load_state(A, min(r + 1, ny), ib, ic);
     Mom<R> lm = {};
     if constexpr (INIT) {
       Mom<R> was = {};
@@ -661,7 +665,8 @@ __device__ __forceinline__ void adjoint_strip(const AdjArgs& A, int j0, int j1, 
     Lam<R> out;
     R gp2[2];
     core_backward<EQF, R>(c, P, o, lm, lphi, R(0.5) * lt, &out, gp2);
-    store_adjoint<R, EQF>(A, min(max(jc, j0), j1), on ? i : kPastStrip, out);
+    store_adjoint<R, EQF>(A, min(max(jc, j0), j1), ib, WIDE ? kLanes : (int)A.pitch,
+                          on ? i - ib : kPastStrip, out);
     g[0] += on ? (double)gp2[0] : 0.0;
     g[1] += on ? (double)gp2[1] : 0.0;
   };
@@ -675,7 +680,7 @@ __device__ __forceinline__ void adjoint_strip(const AdjArgs& A, int j0, int j1, 
   for (; r <= rb; ++r) feed_row(r, std::false_type{});
 }
 
-template <typename R, bool EQF, bool INIT>
+template <typename R, bool EQF, bool INIT, bool WIDE>
 __global__ __launch_bounds__(kLanes, (adj_waves<R>())) void k_adjoint(AdjArgs A) {
   int seg, j0, j1;
   bool edge;
@@ -684,9 +689,9 @@ __global__ __launch_bounds__(kLanes, (adj_waves<R>())) void k_adjoint(AdjArgs A)
   const int i = i0 - 1 + (int)threadIdx.x;
   double g[3] = {0.0, 0.0, 0.0};
   if (edge)
-    adjoint_strip<R, EQF, true, INIT>(A, j0, j1, i, i0 == 1, i0 + kAdjCols >= A.nx, g);
+    adjoint_strip<R, EQF, true, INIT, WIDE>(A, j0, j1, i0, i, i0 == 1, i0 + kAdjCols >= A.nx, g);
   else
-    adjoint_strip<R, EQF, false, INIT>(A, j0, j1, i, false, false, g);
+    adjoint_strip<R, EQF, false, INIT, WIDE>(A, j0, j1, i0, i, false, false, g);
   // parameter adjoints: butterfly over the wave, then this workgroup's own
   // slot (deterministic)
 #pragma unroll
@@ -988,11 +993,10 @@ hipError_t copy_state(bgk_handle* h, const StatePtrs& dst, const double2* a, con
 
 template <typename R, bool EQF>
 void run_adjoint(bgk_handle* h, const AdjArgs& a, int core) {
-  const dim3 grd((unsigned)a.g.nwg);
-  if (core)
-    hipLaunchKernelGGL((k_adjoint<R, EQF, false>), grd, dim3(kLanes), 0, h->stream, a);
-  else
-    hipLaunchKernelGGL((k_adjoint<R, EQF, true>), grd, dim3(kLanes), 0, h->stream, a);
+  const bool wide = wide_rows(h);
+  const auto k = core ? (wide ? k_adjoint<R, EQF, false, true> : k_adjoint<R, EQF, false, false>)
+                      : (wide ? k_adjoint<R, EQF, true, true> : k_adjoint<R, EQF, true, false>);
+  hipLaunchKernelGGL(k, dim3((unsigned)a.g.nwg), dim3(kLanes), 0, h->stream, a);
 }
 
 // adjoint of the step from state `sprev` (core = 1), or the initial state's

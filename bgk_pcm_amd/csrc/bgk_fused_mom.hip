@@ -392,7 +392,7 @@ void launch_init(bgk_handle* h, const MomOut& st, dim3 grd) {
 int mom_most_steps(const bgk_handle* h, bool adjoint) {
   const bool f64 = h->prm.precision == BGK_FP64_MOM;
   const int64_t nodes = (int64_t)h->nx * h->ny;
-  if (h->mom_variant >= 4) return 1;
+  if (h->mom_variant >= 4 || wave::wide_rows(h)) return 1;
   if (h->mom_variant > 0) return h->mom_variant == 3 && !(f64 && h->mom_eqf) ? 2 : h->mom_variant;
   if (!adjoint && !f64 && h->mom_eqf && nodes > (int64_t)1 << 25) return 1;
   return f64 && h->mom_eqf && nodes >= (int64_t)1 << 21 ? 3 : 2;

@@ -241,12 +241,12 @@ __device__ __forceinline__ void strip32(const Args32& A, int j0, int j1, int i, 
       const int jc = r - T;  // row completed by the last level
       const bool on = jc >= j0;
       const int64_t qr = (int64_t)jc * P;
-      const int qa = on && jc <= j1 && own ? i : kPastStrip;
+      const int qa = on && jc <= j1 && own ? i : kPastRow;
 #pragma unroll
       for (int k = 0; k < 9; ++k)
-        buffer_put(strip_buffer(A.B.row(k, qr), (int)P), qa, make_float2(p.fs[k], p.gs[k]));
-      buffer_put(strip_buffer(A.pb + qr, (int)P), on && jc <= j1 && own_phi ? i : kPastStrip, phi);
-      if (EDGE) buffer_put(te_out, on && jc <= j1 && own && i == nx ? jc : kPastStrip, tav);
+        buffer_put(row_buffer(A.B.row(k, qr), P), qa, make_float2(p.fs[k], p.gs[k]));
+      buffer_put(row_buffer(A.pb + qr, P), on && jc <= j1 && own_phi ? i : kPastRow, phi);
+      if (EDGE) buffer_put(te_out, on && jc <= j1 && own && i == nx ? jc : kPastRow, tav);
       if (FINAL && on && jc <= j1 && own) {
         const int64_t qg = (int64_t)jc * P + i;
         const Avg a = averaged(p, o, rr);

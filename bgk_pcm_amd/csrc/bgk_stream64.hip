@@ -247,11 +247,11 @@ struct Store64 {
                                              bool own, bool own_phi, const Done& o) {
     const bool on = jc >= j0 && jc <= j1;
     const int64_t qr = (int64_t)jc * A.pitch;
-    const int qa = on && own ? i : kPastStrip;
+    const int qa = on && own ? i : kPastRow;
 #pragma unroll
     for (int k = 0; k < 9; ++k)
-      buffer_put(strip_buffer(A.B.row(k, qr), (int)A.pitch), qa, make_double2(o.f[k], o.g[k]));
-    buffer_put(strip_buffer(A.pb + qr, (int)A.pitch), on && own_phi ? i : kPastStrip, o.phi);
+      buffer_put(row_buffer(A.B.row(k, qr), A.pitch), qa, make_double2(o.f[k], o.g[k]));
+    buffer_put(row_buffer(A.pb + qr, A.pitch), on && own_phi ? i : kPastRow, o.phi);
     if (FINAL && on && own) {
       const Avg a = averaged(o);
       const int64_t qg = qr + i;
@@ -375,7 +375,7 @@ __device__ __forceinline__ void strip_edge(const Args64& A, int j0, int j1, int 
     }
     const int jc = r - (T - 1);  // row completed by the last level
     Store64<FINAL>::put(A, jc, j0, j1, i, own, own_phi, o);
-    buffer_put(te_out, jc >= j0 && jc <= j1 && own && i == nx ? jc : kPastStrip, tav);
+    buffer_put(te_out, jc >= j0 && jc <= j1 && own && i == nx ? jc : kPastRow, tav);
   }
   if (own && i == nx) {
     if (j0 == 1) A.B.row(6, nx + 1)->x = frozen6;

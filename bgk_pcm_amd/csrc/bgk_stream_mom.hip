@@ -83,19 +83,27 @@ __device__ __forceinline__ NodeD widen(const Raw<R, EQF>& r) {
 constexpr double kPhiWest = 1.0, kPhiEast = -1.0;
 
 // Stores of a strip's nodes through buffer descriptors: a lane that must not
-// store gives an offset past the strip.
-template <typename R, bool EQF, int HOW>
+// store gives an offset past the strip.  WIDE: a strip is one row, described from
+// the wave's first column ib on (wide_rows).
+template <typename R, bool EQF, int HOW, bool WIDE>
 struct StoreMom {
   using V4 = typename Vec<R>::V4;
   using C = typename CType<R, EQF>::T;
   __amdgpu_buffer_rsrc_t a, b, c, phi;
-  __device__ __forceinline__ StoreMom(const MomOut& out, double* pb, int64_t qs, int n) {
+  int ib;
+  __device__ __forceinline__ StoreMom(const MomOut& out, double* pb, int64_t qs, int n, int first)
+      : ib(first) {
+    if constexpr (WIDE) {
+      qs += ib;
+      n = kLanes;
+    }
     a = strip_buffer(out.a + qs, n);
     b = strip_buffer(static_cast<V4*>(out.b) + qs, n);
     c = strip_buffer(static_cast<C*>(out.c) + qs, n);
     phi = strip_buffer(pb + qs, n);
   }
   __device__ __forceinline__ void store(int q, bool on, bool on_phi, const Updated& o) const {
+    if constexpr (WIDE) q -= ib;
     const int qa = on ? q : kPastStrip;
     buffer_put<HOW>(a, qa, make_double2(o.rho, o.dT));
     if constexpr (EQF) {
@@ -206,7 +214,7 @@ enum { kPlain, kProbes, kFinal, kKeep, kKeepProbes };
 // the hardware drops, so that the wait for a row's loads (issued two rows
 // ahead) never has to cover stores issued since.  With conditional stores the
 // compiler's waits did, and a row cost 2.2 us of store latency on top.
-template <int T, typename R, bool EQF, bool EDGE, int MODE, int HOW>
+template <int T, typename R, bool EQF, bool EDGE, int MODE, int HOW, bool WIDE>
 __device__ __forceinline__ void stream_strip(const StreamArgs& A, int i0, int j0, int j1, int i,
                                              bool has_w, bool has_e) {
   const int nx = A.nx, ny = A.ny;
@@ -218,7 +226,7 @@ __device__ __forceinline__ void stream_strip(const StreamArgs& A, int i0, int j0
   // phi also in the ghost columns next to an owned column
   const bool own_phi = own || (ghost && (i == 0 ? has_w : lane <= kLanes - T));
   const int64_t qs = (int64_t)j0 * P;  // first node of the strip
-  const StoreMom<R, EQF, HOW> out(A.out, A.pb, qs, (j1 - j0 + 1) * (int)P);
+  const StoreMom<R, EQF, HOW, WIDE> out(A.out, A.pb, qs, (j1 - j0 + 1) * (int)P, i0 - T);
   constexpr bool KEEP = MODE == kKeep || MODE == kKeepProbes;
   constexpr bool PROBES = MODE != kPlain && MODE != kKeep;
 
@@ -281,7 +289,7 @@ __device__ __forceinline__ void stream_strip(const StreamArgs& A, int i0, int j0
         const bool mine = jd >= 0 && j - 1 <= j1;
         Updated k = o;
         if (EDGE && ghost) k.phi = i == 0 ? kPhiWest : kPhiEast;
-        const StoreMom<R, EQF, HOW> mid(A.mid, A.phi_mid, qs, (j1 - j0 + 1) * (int)P);
+        const StoreMom<R, EQF, HOW, WIDE> mid(A.mid, A.phi_mid, qs, (j1 - j0 + 1) * (int)P, i0 - T);
         mid.store(jd * (int)P + i, mine && own, mine && own_phi, k);
         if (EDGE)
           buffer_put(strip_buffer(A.te_mid, ny + 2), mine && own && i == nx ? j - 1 : kPastStrip,
@@ -302,7 +310,7 @@ __device__ __forceinline__ void stream_strip(const StreamArgs& A, int i0, int j0
       }
     }
     const int jc = r - T;  // row completed by the last level
-    const bool on = jc >= j0;
+    const bool on = jc >= j0 && (!WIDE || jc <= j1);
     const int qo = (jc - j0) * (int)P + i;
     if (EDGE && ghost) o.phi = i == 0 ? kPhiWest : kPhiEast;
     out.store(qo, on && own, on && own_phi, o);
@@ -329,7 +337,7 @@ __device__ __forceinline__ void stream_strip(const StreamArgs& A, int i0, int j0
   }
 }
 
-template <int T, typename R, bool EQF, int MODE, int HOW>
+template <int T, typename R, bool EQF, int MODE, int HOW, bool WIDE = false>
 __global__ __launch_bounds__(kLanes, 2) void k_stream_mom(StreamArgs A) {
   int seg, j0, j1;
   bool edge;
@@ -337,10 +345,10 @@ __global__ __launch_bounds__(kLanes, 2) void k_stream_mom(StreamArgs A) {
   const int i0 = seg * (kLanes - 2 * T) + 1;
   const int i = i0 - T + (int)threadIdx.x;
   if (edge)
-    stream_strip<T, R, EQF, true, MODE, HOW>(A, i0, j0, j1, i, i0 - T <= 1,
-                                             i0 - T + kLanes - 1 >= A.nx);
+    stream_strip<T, R, EQF, true, MODE, HOW, WIDE>(A, i0, j0, j1, i, i0 - T <= 1,
+                                                   i0 - T + kLanes - 1 >= A.nx);
   else
-    stream_strip<T, R, EQF, false, MODE, HOW>(A, i0, j0, j1, i, false, false);
+    stream_strip<T, R, EQF, false, MODE, HOW, WIDE>(A, i0, j0, j1, i, false, false);
 }
 
 template <int T, typename R, bool EQF>
@@ -388,6 +396,15 @@ hipError_t launch_t(bgk_handle* h, const MomStep& st) {
                      (int64_t)(sizeof(double2) + sizeof(typename Vec<R>::V4) +
                                sizeof(typename CType<R, EQF>::T) + sizeof(double)) >> 20;
   const bool cached = mb >= (sizeof(R) == sizeof(float) ? 96 : 64) && mb < 256;
+  if constexpr (T == 1) {
+    if (wide_rows(h)) {
+      const auto k = st.write_all   ? k_stream_mom<T, R, EQF, kFinal, kNonTemporal, true>
+                     : st.probe_out ? k_stream_mom<T, R, EQF, kProbes, kNonTemporal, true>
+                                    : k_stream_mom<T, R, EQF, kPlain, kNonTemporal, true>;
+      hipLaunchKernelGGL(k, grd, dim3(kLanes), 0, h->stream, a);
+      return hipGetLastError();
+    }
+  }
   if constexpr (T == 2) {
     if (st.mid.a) {
       const auto k = st.probe_out ? k_stream_mom<T, R, EQF, kKeepProbes, kNonTemporal>

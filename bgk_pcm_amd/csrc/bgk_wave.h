@@ -55,12 +55,21 @@ __device__ __forceinline__ float from_east(float x) {
 // Buffer descriptor of n elements at p (wave-uniform), and a store of one
 // element at offset q that the hardware drops where q >= n.  kPastStrip times
 // an element's size (4 to 32 bytes) stays within 32 bits and past any strip
-// (kMaxStrip elements, see make_wave_grid).
-constexpr int kPastStrip = 0x07ffffff;
+// (kMaxStrip elements, see make_wave_grid).  Where a row alone is more (wide_rows),
+// the moment kernels count columns from the wave's first one.  The population
+// kernels store row by row, elements of at most 16 bytes: row_buffer and kPastRow,
+// just below 2^32 bytes, hold for any row that fits a device.
+constexpr int kPastStrip = 0x07ffffff, kPastRow = -16;
 constexpr int kMaxStrip = 0x03ffffff;
+inline bool wide_rows(const bgk_handle* h) { return h->pitch > kMaxStrip; }
 template <typename E>
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t strip_buffer(E* p, int n) {
   return __builtin_amdgcn_make_buffer_rsrc(p, 0, n * (int)sizeof(E), 0x00020000);
+}
+template <typename E>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_buffer(E* p, int64_t n) {
+  return __builtin_amdgcn_make_buffer_rsrc(p, 0, (int)((unsigned)n * (unsigned)sizeof(E)),
+                                           0x00020000);
 }
 constexpr int kCached = 0, kNonTemporal = 2;
 template <int HOW = kNonTemporal, typename E>
@@ -141,7 +150,7 @@ __device__ __forceinline__ scalar_ptr as_scalar(const double* p) {
 constexpr int kMaxRows = 64;
 struct WaveGrid {
   int nseg, nright;  // segments; those that meet the east wall
-  int ne;            // segments whose every strip meets a wall: 1 + nright, or all
+  int ne;            // segments whose every strip runs the walls' code: 1 + nright, or all
   int re, nse;       // rows per strip of those, strips
   int ra;            // rows of the lowest and highest strip of the others
   int rows, nmid;    // rows per strip between them, strips
@@ -182,14 +191,17 @@ __device__ __forceinline__ bool wave_tile(const WaveGrid& g, int ny, int* seg, i
 
 // The split with strips of h rows (walls: of equal duration, at `slow` times
 // the cost per row iteration).  A strip of h rows takes h + extra iterations.
-inline WaveGrid split_waves(int nx, int ny, int cols, int T, int extra, double slow, int h) {
+// most: the rows that a strip may have; where the T + 1 rows that keep the others
+// off the walls are more, every strip runs the walls' code.
+inline WaveGrid split_waves(int nx, int ny, int cols, int T, int extra, double slow, int h,
+                            int most) {
   WaveGrid g{};
   g.nseg = (nx + cols - 1) / cols;
   const int last = nx - (g.nseg - 1) * cols;  // columns of the last segment
   g.nright = last <= T ? 2 : 1;
   g.re = std::max(1, std::min({ny, h, (int)((h + extra) / slow) - extra}));
   g.ra = std::max(g.re, T + 1);
-  g.ne = g.nseg <= 1 + g.nright || ny <= 2 * g.ra ? g.nseg : 1 + g.nright;
+  g.ne = g.nseg <= 1 + g.nright || ny <= 2 * g.ra || g.ra > most ? g.nseg : 1 + g.nright;
   g.nse = (ny + g.re - 1) / g.re;
   g.rows = h;
   const int64_t inner = g.nseg - g.ne;
@@ -208,13 +220,14 @@ inline WaveGrid split_waves(int nx, int ny, int cols, int T, int extra, double s
 inline WaveGrid make_wave_grid(int nx, int ny, int cols, int T, int extra, double slow, int most,
                                int n_cu, int rows_override, int deep = 2) {
   // (offsets within a strip stay below kMaxStrip elements)
-  most = std::max(1, std::min({most, ny, kMaxRows, (int)(kMaxStrip / (int64_t)(nx + 256))}));
+  const int room = (int)std::max((int64_t)1, kMaxStrip / ((int64_t)nx + 256));
+  most = std::min({most, ny, kMaxRows, room});
   if (rows_override > 0)
-    return split_waves(nx, ny, cols, T, extra, slow, std::min(rows_override, most));
+    return split_waves(nx, ny, cols, T, extra, slow, std::min(rows_override, most), room);
   WaveGrid best{};
   double cost = -1.0;
   for (int h = 1; h <= most; ++h) {
-    const WaveGrid g = split_waves(nx, ny, cols, T, extra, slow, h);
+    const WaveGrid g = split_waves(nx, ny, cols, T, extra, slow, h, room);
     const double inner = g.nseg - g.ne, slots = 4.0 * deep * n_cu;
     const double shared = deep > 1 ? 1.35 : 1.0;
     const double waves = g.nedge + inner * g.nmid;
