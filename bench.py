@@ -54,7 +54,9 @@ Printed JSON line (one):
                  memory holds, 16 seeded probes): device bytes of the handle
                  and of the adjoint's checkpoints, the forward steps the
                  backward pass recomputes, forward and backward time per
-                 step and their ratio; and the same gradient by the FP32 and
+                 step and their ratio, against the plain step as bgk_step
+                 takes it at this size (one per launch) and with two per
+                 launch (BGK_MOM_VARIANT=2); and the same gradient by the FP32 and
                  the FP64 adjoint at 1024^2 with their relative difference
   cpu_baseline   the reference's own STEP_OPENMP time step (compiled from its
                  sources into oracle/_ref) timed on this host's cores on a
@@ -499,12 +501,25 @@ def adjoint_large(nsteps: int = 5000, seg_outer: int = 289, seg: int = 17,
     # plain forward steps of the same handle type over the same steps (the
     # step gets slower as the melting front widens), for the cost ratio
     progress(f"adjoint {n}^2: plain forward steps")
-    with Lattice(w.params) as lat:
-        lat.synchronize()
-        t0 = time.perf_counter()
-        lat.step(nsteps)
-        lat.synchronize()
-        t_plain = (time.perf_counter() - t0) / nsteps
+    def plain():
+        with Lattice(w.params) as lat:
+            lat.synchronize()
+            t0 = time.perf_counter()
+            lat.step(nsteps)
+            lat.synchronize()
+            return (time.perf_counter() - t0) / nsteps
+
+    t_plain = plain()
+    # the same with two steps per launch, which bgk_step leaves out at this size
+    old = os.environ.get("BGK_MOM_VARIANT")
+    os.environ["BGK_MOM_VARIANT"] = "2"
+    try:
+        t_two = plain()
+    finally:
+        if old is None:
+            del os.environ["BGK_MOM_VARIANT"]
+        else:
+            os.environ["BGK_MOM_VARIANT"] = old
     res = {"workload": f"{w.note}, {nsteps} steps, binomial checkpointing in the free "
                        "device memory, 16 probes",
            "grad": [float(x) for x in g],
@@ -515,7 +530,9 @@ def adjoint_large(nsteps: int = 5000, seg_outer: int = 289, seg: int = 17,
            "forward_ms_per_step": round(t_plain * 1e3, 4),
            "recorded_forward_ms_per_step": round(tf / nsteps * 1e3, 4),
            "backward_ms_per_step": round(tb / nsteps * 1e3, 4),
-           "backward_over_forward": round(tb / nsteps / t_plain, 3)}
+           "backward_over_forward": round(tb / nsteps / t_plain, 3),
+           "forward_two_steps_per_launch_ms_per_step": round(t_two * 1e3, 4),
+           "backward_over_forward_two_steps_per_launch": round(tb / nsteps / t_two, 3)}
     if check_n:
         g32, g64 = out[(check_n, FP32_MOM)][0], out[(check_n, FP64_MOM)][0]
         rel = [float(abs(a - b) / abs(b)) for a, b in zip(g32, g64)]

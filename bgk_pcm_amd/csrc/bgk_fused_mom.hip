@@ -383,12 +383,14 @@ void launch_init(bgk_handle* h, const MomOut& st, dim3 grd) {
 
 // Most steps per launch.  Two halve the HBM bytes of a step; three pay only
 // where a node is large and its update small (FP64 moments with omega_f = 1:
-// 4096^2 188 against 239 us per step, 2048^2 62 against 64, smaller lattices
-// lose).  FP32 moments with omega_f = 1 take one step per launch beyond 2^25
-// nodes: there the cost of the adjoint is held to three plain forward steps,
-// and its own kernel, at 58% of the memory rate, cannot follow a forward step
-// of half the time (8192^2: 1.80 ms; the forward step 1.13, or 0.69 with two per
-// launch).  The adjoint's own forward runs (`adjoint`) take two.
+// 4096^2 181 against 240 us per step, 2048^2 50 against 63).
+//
+// FP32 moments with omega_f = 1 take one step per launch beyond 2^25 nodes although
+// two are faster there too (8192^2: 1.15 against 0.72 ms per step).  The reason is
+// no measurement but a bound on a ratio: the backward pass is held to three plain
+// forward steps at 8192^2, and at 2.87 ms a step (its kernel alone takes 1.80, at
+// 89% of a copy's rate) it is four of the faster ones.  BGK_MOM_VARIANT=2 takes two
+// at every size; the adjoint's own forward runs (`adjoint`) always do.
 int mom_most_steps(const bgk_handle* h, bool adjoint) {
   const bool f64 = h->prm.precision == BGK_FP64_MOM;
   const int64_t nodes = (int64_t)h->nx * h->ny;

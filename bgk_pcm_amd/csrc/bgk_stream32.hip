@@ -12,8 +12,8 @@
 // the populations are rounded to what the planes would hold.
 //
 // What bounds it: both HBM (80 B per node and step, 160 with one step per
-// launch; 3.8 TB/s at 4096^2) and VALU issue at two waves per SIMD (half of a
-// row's time); the rest is the latency of 512-byte row pieces.  Measured in
+// launch; 3.8 TB/s at 4096^2) and VALU issue at two waves per SIMD (65% of the
+// time); the rest is the latency of 512-byte row pieces.  Measured in
 // stream32.
 #include <algorithm>
 

@@ -360,7 +360,8 @@ __device__ __forceinline__ void strip_edge(const Args64& A, int j0, int j1, int 
     load_pulled_edge(A.A, P, ny, offs, min(r + 1, ny), in);
     pn = phi_row(r + 2);
     __builtin_amdgcn_sched_barrier(0);
-    if (FINAL && T == 2 && r >= j0 && r <= j1 && own) halo(A, r, i, averaged(o), o.phi);
+    static_assert(T == 2, "level 0 gives the state before the last step");
+    if (FINAL && r >= j0 && r <= j1 && own) halo(A, r, i, averaged(o), o.phi);
 #pragma unroll
     for (int t = 1; t < T; ++t) {
       const int j = r - t + 1;  // row fed to level t
@@ -370,8 +371,6 @@ __device__ __forceinline__ void strip_edge(const Args64& A, int j0, int j1, int 
       o = node_step<STEP7>(A.c, fp, gp, tap);
       tav = averaged_T(o);
       if (ghost) o.phi = tap[0];
-      if (FINAL && T > 2 && t == T - 2 && j - 1 >= j0 && j - 1 <= j1 && own)
-        halo(A, j - 1, i, averaged(o), o.phi);
     }
     const int jc = r - (T - 1);  // row completed by the last level
     Store64<FINAL>::put(A, jc, j0, j1, i, own, own_phi, o);

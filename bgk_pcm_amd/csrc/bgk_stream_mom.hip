@@ -14,7 +14,7 @@
 // VALU issue at two waves per SIMD (FP32 moments: 212 VGPRs).  Measured at
 // 4096^2, us per step, against one step per launch of the ring kernel:
 // FP32 moments 203 (362), with omega_f = 1 168 (290), FP64 moments 323 (648),
-// with omega_f = 1 180 (462, three steps per launch).  FP32 moments with three
+// with omega_f = 1 181 (462, three steps per launch).  FP32 moments with three
 // steps per launch: 230 (spills), with omega_f = 1 172.
 #include <algorithm>
 

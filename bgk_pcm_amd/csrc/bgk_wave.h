@@ -1,5 +1,6 @@
-// bgk_wave.h -- building blocks of the wave-streaming kernels that advance
-// several time steps per launch (bgk_stream_mom.hip).
+// bgk_wave.h -- building blocks of the wave-streaming kernels: the steps of several
+// levels per launch (bgk_stream_mom.hip, bgk_stream32.hip, bgk_stream64.hip) and the
+// adjoint (bgk_adjoint.hip).
 //
 // One wavefront owns 64 neighbouring columns and walks up a strip of rows.
 // Lane L holds column i0 - T + L of the row being processed, so a pull from
