@@ -386,7 +386,7 @@ void launch_init(bgk_handle* h, const MomOut& st, dim3 grd) {
 // 4096^2 181 against 240 us per step, 2048^2 50 against 63).
 //
 // FP32 moments with omega_f = 1 take one step per launch beyond 2^25 nodes although
-// two are faster there too (8192^2: 1.15 against 0.72 ms per step).  The reason is
+// two are faster there too (8192^2: 1.14 against 0.68 ms per step).  The reason is
 // no measurement but a bound on a ratio: the backward pass is held to three plain
 // forward steps at 8192^2, and at 2.87 ms a step (its kernel alone takes 1.80, at
 // 89% of a copy's rate) it is four of the faster ones.  BGK_MOM_VARIANT=2 takes two
