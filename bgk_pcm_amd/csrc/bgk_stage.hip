@@ -316,10 +316,9 @@ __device__ __forceinline__ void bc_g_ns(const Pops64& G, const Macro& m, double*
 // BC_f and/or BC_g in one launch.  The sides depend on each other in the
 // reference's order (west and east, then north and south; f before g), but
 // only in the columns 0, 1, Nx, Nx+1 and the rows 0, 1, Ny-1, Ny, Ny+1: the first
-// workgroup does these, waiting between the four parts; every other row of the
-// west and east and column of the north and south is a thread of its own
-// elsewhere, f before g.  On lattices of fewer than 8 rows or columns the first
-// workgroup does everything.
+// workgroup does these (each once, where they coincide), waiting between the four
+// parts; every other row of the west and east and column of the north and south
+// is a thread of its own elsewhere, f before g.
 // What bounds it: the latency of a launch and of a few dependent accesses.
 // Measured, us per step of a channel (this launch and k_general64): 2048 x 1024
 // 186 with one workgroup for all, 132 so; 1024 x 512 71 / 48; 64^2 13.3 / 12.8.
@@ -332,38 +331,38 @@ struct BcArgs {
   Geom gm;
   Walls w;
   int do_f, do_g;
-  int small;
 };
 __global__ __launch_bounds__(kBcThreads) void k_bc(BcArgs a) {
   const int nx = a.gm.nx, ny = a.gm.ny;
   if (blockIdx.x > 0) {
     int t = ((int)blockIdx.x - 1) * kBcThreads + (int)threadIdx.x;
-    if (t < ny - 3) {
+    const int rows = max(ny - 3, 0);
+    if (t < rows) {
       const int j = t + 2;  // 2..Ny-2
       if (a.do_f) bc_f_we(a.F, a.m, a.c, a.gm, a.w, j);
       if (a.do_g) bc_g_we(a.G, a.m, a.c, a.gm, j);
-    } else if ((t -= ny - 3) < nx - 2) {
+    } else if ((t -= rows) < nx - 2) {
       const int i = t + 2;  // 2..Nx-1
       if (a.do_f) bc_f_ns(a.F, a.m, a.c, a.gm, a.w, i);
       if (a.do_g) bc_g_ns(a.G, a.m, a.phi, a.gm, i);
     }
     return;
   }
-  // rows and columns of the first workgroup
-  const int nr = a.small ? ny + 2 : 5, nc = a.small ? nx + 2 : 4;
-  auto row = [&](int e) { return a.small || e < 2 ? e : ny - 3 + e; };
-  auto col = [&](int e) { return a.small || e < 2 ? e : nx - 2 + e; };
+  // this thread's row (0, 1, Ny-1..Ny+1) and column (0, 1, Nx, Nx+1) of the first
+  // workgroup; -1: none
+  const int e = (int)threadIdx.x;
+  const int row = e < 2 ? e : e < 5 && ny - 3 + e > 1 ? ny - 3 + e : -1;
+  const int col = e < 2 ? e : e < 4 && nx - 2 + e > 1 ? nx - 2 + e : -1;
   if (a.do_f) {
-    for (int e = threadIdx.x; e < nr; e += kBcThreads) bc_f_we(a.F, a.m, a.c, a.gm, a.w, row(e));
+    if (row >= 0) bc_f_we(a.F, a.m, a.c, a.gm, a.w, row);
     __syncthreads();
-    for (int e = threadIdx.x; e < nc; e += kBcThreads) bc_f_ns(a.F, a.m, a.c, a.gm, a.w, col(e));
+    if (col >= 0) bc_f_ns(a.F, a.m, a.c, a.gm, a.w, col);
     __syncthreads();
   }
   if (a.do_g) {
-    for (int e = threadIdx.x; e < nr; e += kBcThreads)
-      if (row(e) >= 1 && row(e) <= ny) bc_g_we(a.G, a.m, a.c, a.gm, row(e));
+    if (row >= 1 && row <= ny) bc_g_we(a.G, a.m, a.c, a.gm, row);
     __syncthreads();
-    for (int e = threadIdx.x; e < nc; e += kBcThreads) bc_g_ns(a.G, a.m, a.phi, a.gm, col(e));
+    if (col >= 0) bc_g_ns(a.G, a.m, a.phi, a.gm, col);
   }
 }
 
@@ -498,11 +497,11 @@ hipError_t launch_initialization(bgk_handle* h) {
 
 hipError_t launch_bc(bgk_handle* h, bool do_f, bool do_g) {
   const Geom& g = h->geom;
-  const bool small = g.nx < 8 || g.ny < 8;
   BcArgs a{pops(h->f[h->cur]), pops(h->g[h->cur]), macro_of(h), h->phi[h->pc], h->c, g,
            Walls{h->prm.west_bc, h->prm.east_bc, h->prm.north_bc, h->prm.south_bc},
-           do_f ? 1 : 0, do_g ? 1 : 0, small ? 1 : 0};
-  const unsigned rest = small ? 0 : blocks1d(g.ny - 3 + g.nx - 2, kBcThreads);
+           do_f ? 1 : 0, do_g ? 1 : 0};
+  // rows 2..Ny-2 and columns 2..Nx-1
+  const unsigned rest = blocks1d(std::max(g.ny - 3, 0) + std::max(g.nx - 2, 0), kBcThreads);
   hipLaunchKernelGGL(k_bc, dim3(1 + rest), dim3(kBcThreads), 0, h->stream, a);
   return hipGetLastError();
 }
