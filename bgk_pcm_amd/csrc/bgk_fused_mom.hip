@@ -364,9 +364,13 @@ int ring_width(const bgk_handle* h) {
 //   128 x 8000    47 / 39       42 / 35      66 / 55       54 / 43
 //   120 x 6000    29 / 28       27 / 27      38 / 41       31 / 33
 //   250 x 1000    15 / 19       14 / 18      17 / 23       15 / 20
-// (of few columns a wave's last segment is a large share).
+//   1 x 3000      14 / 8.2      14 / 8.1     15 / 8.4     15 / 8.3
+//   2 x 300      9.8 / 7.3     9.7 / 7.5     10 / 7.3
+// (of few columns a wave's last segment is a large share; of one or two every node
+// is a boundary node, a thread of its own in the ring kernel).
 bool ring_step(const bgk_handle* h) {
   if (h->mom_variant != 0) return h->mom_variant >= 4;
+  if (h->nx <= 2) return true;
   const int64_t least = h->nx <= 384 ? (int64_t)1 << 19 : (int64_t)3 << 20;
   return (int64_t)h->nx * h->ny >= least && ring_width(h) > 0;
 }
