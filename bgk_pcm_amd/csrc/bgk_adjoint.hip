@@ -1060,7 +1060,6 @@ hipError_t fwd_steps(bgk_handle* h, int T, const StatePtrs& in, const StatePtrs*
   st.probe_idx = probe_idx;
   st.probe_out = probe_out;
   st.probe_np = np;
-  st.adjoint = true;
   if (mid) {
     st.mid = mom::MomOut{mid->a, mid->b, mid->c};
     st.phi_mid = mid->phi;
@@ -1189,7 +1188,7 @@ hipError_t adj_forward(bgk_handle* h, double* probe_T_host) {
     const bool kept = keep && n + T == stop;
     const StatePtrs out = kept ? *keep : own;
     e = fwd_steps(h, T, in, mid, out, x->np > 0 ? x->probe_T + (size_t)n * x->np : nullptr,
-                  x->probe_idx, x->np, mom_write_all(h, T, x->nsteps - n - T, true));
+                  x->probe_idx, x->np, mom_write_all(x->nsteps - n - T, false));
     if (e != hipSuccess) return e;
     if (kept) {
       ++next_chain;

@@ -338,19 +338,23 @@ hipError_t launch_ring_layout(bgk_handle* h, const MomStep& st) {
 }
 
 // Width of the ring kernel's workgroups: the widest that adds at most a quarter to
-// the columns, or the narrowest that adds at most half; 0: none.  (The wider, the
-// longer the contiguous pieces of a row; FP64 rows wider than 256 do not fit
-// the LDS of a resident workgroup twice.)
+// the columns, or the widest of those that add least; 0: none adds less than half.
+// (The wider, the longer the contiguous pieces of a row; FP64 rows wider than 256
+// do not fit the LDS of a resident workgroup twice.)
 int ring_width(const bgk_handle* h) {
   const auto columns = [h](int w) { return ((int64_t)h->nx + w - 1) / w * w; };
-  for (int w = h->prm.precision == BGK_FP32_MOM ? 512 : 256; w >= 128; w /= 2)
+  int best = 64;
+  for (int w = h->prm.precision == BGK_FP32_MOM ? 512 : 256; w >= 64; w /= 2) {
     if (4 * columns(w) <= 5 * (int64_t)h->nx) return w;
-  return 2 * columns(128) <= 3 * (int64_t)h->nx ? 128 : 0;
+    if (columns(w) < columns(best) || (columns(w) == columns(best) && w > best)) best = w;
+  }
+  return 2 * columns(best) <= 3 * (int64_t)h->nx ? best : 0;
 }
 
-// Whether one step alone goes through the ring kernel: its loads go past the caches,
-// which leaves these to the macroscopic fields that a call's last step writes,
-// and its rows are longer pieces than a wave's.  Measured, us per call of one
+// Whether a step alone goes through the ring kernel: its loads go past the caches,
+// which leaves these to the macroscopic fields that a call's last step writes;
+// its rows are longer pieces than a wave's; and its boundary nodes are a thread
+// each, where the streaming kernel walks rows.  Measured, us per call of one
 // step, streaming kernel with T = 1 / ring:
 //              FP32 moments  omega_f = 1  FP64 moments  omega_f = 1
 //   1700^2        85 / 84       71 / 73     151 / 133     105 / 96
@@ -358,21 +362,41 @@ int ring_width(const bgk_handle* h) {
 //   2048^2       146 / 107     121 / 89     211 / 172     165 / 129
 //   4096^2       551 / 510     475 / 427    812 / 767     631 / 587
 //   90 x 40000   157 / 125     136 / 105    215 / 186     170 / 140
-//   130 x 40000  234 / 208     208 / 189    319 / 369     254 / 279  (width 0)
+//   130 x 40000  228 / 198     207 / 172    320 / 290     253 / 222
 //   512 x 1500    30 / 37       25 / 35      42 / 44       32 / 35
 //   250 x 2200    31 / 24       28 / 22      37 / 31       31 / 26
-//   128 x 8000    47 / 39       42 / 35      66 / 55       54 / 43
-//   120 x 6000    29 / 28       27 / 27      38 / 41       31 / 33
 //   250 x 1000    15 / 19       14 / 18      17 / 23       15 / 20
+//   60 x 60000   132 / 128     110 / 108    188 / 201     144 / 151
+//   60 x 2500     16 / 12       15 / 12      17 / 15       16 / 13
+//   7 x 3000      14 / 10       14 / 10      15 / 10       15 / 10
 //   1 x 3000      14 / 8.2      14 / 8.1     15 / 8.4     15 / 8.3
-//   2 x 300      9.8 / 7.3     9.7 / 7.5     10 / 7.3
-// (of few columns a wave's last segment is a large share; of one or two every node
-// is a boundary node, a thread of its own in the ring kernel).
 bool ring_step(const bgk_handle* h) {
   if (h->mom_variant != 0) return h->mom_variant >= 4;
+  const int64_t nodes = (int64_t)h->nx * h->ny;
   if (h->nx <= 2) return true;
-  const int64_t least = h->nx <= 384 ? (int64_t)1 << 19 : (int64_t)3 << 20;
-  return (int64_t)h->nx * h->ny >= least && ring_width(h) > 0;
+  if (h->nx <= 64) return nodes <= 160000;
+  return nodes >= (h->nx <= 384 ? (int64_t)1 << 19 : (int64_t)3 << 20) && ring_width(h) > 0;
+}
+
+// Whether the last two steps of a call go one by one, through the ring kernel: on
+// small or narrow lattices of the general layout the launch of two that writes the
+// fields takes up to four plain ones' time.  Measured, us per step of calls of two, one
+// launch / two ring launches:
+//              FP32 moments  FP64 moments
+//   16 x 16     9.7 / 6.7     11.2 / 7.1
+//   97 x 61     9.5 / 8.7     11.0 / 8.8
+//   300^2      11.4 / 9.6     15.9 / 11.0
+//   512^2        16 / 26        22 / 22
+//   100 x 1500   16 / 11        22 / 15
+//   30 x 6000    22 / 20        28 / 22
+//   60 x 60000  117 / 128      195 / 198
+//   90 x 40000  139 / 121      248 / 184
+//   130 x 40000 203 / 188      307 / 279
+bool ends_in_singles(const bgk_handle* h) {
+  if (h->mom_variant != 0 || h->mom_eqf) return false;
+  const int64_t nodes = (int64_t)h->nx * h->ny;
+  if (h->nx <= 144) return h->nx > 64 || nodes <= (int64_t)1 << 18;
+  return nodes <= (h->prm.precision == BGK_FP64_MOM ? (int64_t)1 << 17 : 100000);
 }
 
 template <typename R, bool EQF>
@@ -412,22 +436,17 @@ int mom_next_steps(const bgk_handle* h, int left, bool adjoint) {
   return left % most ? left % most : most;
 }
 
-// Whether a launch of T steps has to write the macroscopic fields: the last of
-// a call; and the one before a last launch of one step, which takes the halo
-// from them, unless it is a ring launch (these keep the boundary nodes
-// current).
-bool mom_write_all(const bgk_handle* h, int T, int left, bool adjoint) {
-  return left == 0 || (left == 1 && !(T == 1 && !adjoint && ring_step(h)));
-}
-
 hipError_t launch_mom_steps(bgk_handle* h, const MomStep& st, int T) {
-  if (T > 1 || st.adjoint || !ring_step(h)) return launch_mom_stream(h, st, T);
+  if (!st.ring) return launch_mom_stream(h, st, T);
   const int w = ring_width(h);
   if (h->prm.precision == BGK_FP64_MOM)
-    return w == 256 ? launch_ring_layout<256, double>(h, st) : launch_ring_layout<128, double>(h, st);
+    return w == 256   ? launch_ring_layout<256, double>(h, st)
+           : w == 128 ? launch_ring_layout<128, double>(h, st)
+                      : launch_ring_layout<64, double>(h, st);
   return w == 512   ? launch_ring_layout<512, float>(h, st)
          : w == 256 ? launch_ring_layout<256, float>(h, st)
-                    : launch_ring_layout<128, float>(h, st);
+         : w == 128 ? launch_ring_layout<128, float>(h, st)
+                    : launch_ring_layout<64, float>(h, st);
 }
 
 hipError_t launch_fused_steps_mom(bgk_handle* h, int nsteps) {
@@ -435,8 +454,11 @@ hipError_t launch_fused_steps_mom(bgk_handle* h, int nsteps) {
   // not fill whole ones, two of them where `most` is even, goes step by step.
   const int most = mom_most_steps(h), group = most % 2 == 0 ? 2 * most : most;
   const int whole = nsteps / group * group;
+  const bool alone = ring_step(h), pair = nsteps >= 2 && ends_in_singles(h);
   for (int left = nsteps; left > 0;) {
-    const int T = !h->recorded ? mom_next_steps(h, left) : left > whole ? 1 : most;
+    const int T = h->recorded          ? (left > whole ? 1 : most)
+                  : pair && left == 2 ? 1
+                                      : mom_next_steps(h, left);
     left -= T;
     const int a = h->cur, b = 1 - h->cur;
     MomStep st;
@@ -446,7 +468,10 @@ hipError_t launch_fused_steps_mom(bgk_handle* h, int nsteps) {
     st.pb = h->phi[1 - h->pc];
     st.te_in = h->teast[h->te_cur];
     st.te_out = h->teast[1 - h->te_cur];
-    st.write_all = mom_write_all(h, T, left);
+    // (an odd step before others writes no fields: through the ring only where the
+    // lattice is large, 2048^2 103 us for 106, FP64 162 for 170)
+    st.ring = T == 1 && (left <= 1 ? alone || pair : alone && h->nx > 384);
+    st.write_all = mom_write_all(left, alone || pair);
     st.probe_idx = nullptr;
     st.probe_out = nullptr;
     st.probe_np = 0;

@@ -247,7 +247,7 @@ __device__ __forceinline__ CoreT<A> core_from_sums(const C& c, const PullSumsT<A
 // adjoint's runs keep to the streaming kernel, whose steps have the same bits
 // however a run is split.
 struct MomStep {
-  bool adjoint = false;
+  bool ring = false;  // (one step) through the ring kernel
   MomIn in;
   MomOut out;
   const double* pa;
@@ -272,8 +272,12 @@ struct MomStep {
 hipError_t launch_mom_steps(bgk_handle* h, const mom::MomStep& st, int T);
 hipError_t launch_mom_stream(bgk_handle* h, const mom::MomStep& st, int T);
 int mom_next_steps(const bgk_handle* h, int left, bool adjoint = false);
+// Whether a launch has to write the macroscopic fields, `left` steps of the call
+// after it: the last one; and the one before a last launch of one step, which takes
+// the halo from them, unless that is a ring launch after another one (these keep
+// the boundary nodes current).
+inline bool mom_write_all(int left, bool ring) { return left == 0 || (left == 1 && !ring); }
 int mom_most_steps(const bgk_handle* h, bool adjoint = false);
-bool mom_write_all(const bgk_handle* h, int T, int left, bool adjoint = false);
 }  // namespace bgk
 
 #endif  // BGK_MOM_H
