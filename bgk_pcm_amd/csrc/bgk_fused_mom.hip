@@ -411,7 +411,9 @@ void launch_init(bgk_handle* h, const MomOut& st, dim3 grd) {
 
 // Most steps per launch.  Two halve the HBM bytes of a step; three pay only
 // where a node is large and its update small (FP64 moments with omega_f = 1:
-// 4096^2 181 against 240 us per step, 2048^2 50 against 63).
+// 4096^2 181 against 240 us per step, 2048^2 50 against 63) and most strips run no
+// wall's code (200 x 20000 67 against 75, 130 x 40000 109 against 106, 60 x 60000
+// 128 against 64; 60000 x 40 37 against 39, 400000 x 6 68 against 50).
 //
 // FP32 moments with omega_f = 1 take one step per launch beyond 2^25 nodes although
 // two are faster there too (8192^2: 1.14 against 0.68 ms per step).  The reason is
@@ -425,7 +427,8 @@ int mom_most_steps(const bgk_handle* h, bool adjoint) {
   if (h->mom_variant >= 4 || wave::wide_rows(h)) return 1;
   if (h->mom_variant > 0) return h->mom_variant == 3 && !(f64 && h->mom_eqf) ? 2 : h->mom_variant;
   if (!adjoint && !f64 && h->mom_eqf && nodes > (int64_t)1 << 25) return 1;
-  return f64 && h->mom_eqf && nodes >= (int64_t)1 << 21 ? 3 : 2;
+  const bool walls = h->nx <= 160 || h->ny <= 32;
+  return f64 && h->mom_eqf && nodes >= (int64_t)1 << 21 && !walls ? 3 : 2;
 }
 
 // Of `left` steps, how many the next launch takes: an odd rest first, so that
