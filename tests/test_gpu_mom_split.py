@@ -47,6 +47,26 @@ def test_ring_and_stream(monkeypatch, nx, ny, precision, tau_f, cold, rows):
             assert np.array_equal(got[f], want[f]), (variant, split, f)
 
 
+@pytest.mark.parametrize("nx,ny", [(1, 300), (2, 300), (3, 50), (16, 16), (64, 2500), (64, 2600), (64, 4097),
+                                   (65, 40), (97, 61), (144, 30), (145, 689), (145, 690), (145, 904),
+                                   (160, 13200), (161, 13100)])
+@pytest.mark.parametrize("precision", [FP32_MOM, FP64_MOM])
+@pytest.mark.parametrize("tau_f", [1.0, 0.8])
+def test_short_calls_on_small_and_narrow_lattices(monkeypatch, nx, ny, precision, tau_f):
+    """The rule's own launches (ring launches alone, two at a call's end, and none),
+    at its lines, against one strip launch per step of one call."""
+    want = None
+    for variant, split in [(1, [10]), (0, [10]), (0, [1] * 10), (0, [2, 3, 5]), (0, [4, 6])]:
+        monkeypatch.setenv("BGK_MOM_VARIANT", str(variant))
+        with Lattice(params(nx, ny, precision, tau_f), **EXT) as lat:
+            for n in split:
+                lat.step(n)
+            got = fields(lat)
+        want = want or got
+        for f in FIELDS:
+            assert np.array_equal(got[f], want[f]), (variant, split, f)
+
+
 @pytest.mark.parametrize("nx,ny,precision", [(4100, 2050, FP32_MOM), (2900, 2899, FP64_MOM),
                                              (250, 2200, FP64_MOM), (130, 30000, FP32_MOM)])
 @pytest.mark.parametrize("tau_f", [1.0, 0.8])
